@@ -22,7 +22,7 @@ BWD_DS_WORKSPACE = 1  # AXL_BWD_DS_WORKSPACE
 AXL_OK, AXL_ERR_INVALID_ARGUMENT, AXL_ERR_UNSUPPORTED, AXL_ERR_WORKSPACE, AXL_ERR_LAUNCH = 0, -1, -2, -3, -4
 
 
-ABI_VERSION = 7  # AXL_ATTN_ABI_VERSION of include/axl_attn.h these structures mirror
+ABI_VERSION = 8  # AXL_ATTN_ABI_VERSION of include/axl_attn.h these structures mirror
 
 
 class AxlError(RuntimeError):
@@ -64,6 +64,24 @@ class AxlFlashFwdParams(ctypes.Structure):
         ("logit_sink", ctypes.c_void_p),
         ("aux", AxlAttnAux),
         ("q_pos_offsets", ctypes.c_void_p),
+    ]
+
+
+class AxlFlashChunkParams(ctypes.Structure):
+    _fields_ = [
+        ("q", ctypes.c_void_p), ("k", ctypes.c_void_p), ("v", ctypes.c_void_p), ("out", ctypes.c_void_p),
+        ("q_strides", AxlStrides), ("k_strides", AxlStrides), ("v_strides", AxlStrides),
+        ("out_strides", AxlStrides),
+        ("batch", ctypes.c_int32), ("q_len", ctypes.c_int32), ("kv_len", ctypes.c_int32),
+        ("num_q_heads", ctypes.c_int32), ("num_kv_heads", ctypes.c_int32),
+        ("head_dim", ctypes.c_int32),
+        ("dtype", ctypes.c_int32), ("mask_kind", ctypes.c_int32),
+        ("sliding_window", ctypes.c_int32),
+        ("softmax_scale", ctypes.c_float),
+        ("logit_sink", ctypes.c_void_p), ("positions", ctypes.c_void_p),
+        ("pos_batch_stride", ctypes.c_int64), ("pos_row_stride", ctypes.c_int64),
+        ("pos_is_i64", ctypes.c_int32),
+        ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
     ]
 
 
@@ -142,6 +160,8 @@ class AxlPageInsertParams(ctypes.Structure):
 
 EXPORTED_SYMBOLS = (
     "axl_flash_fwd",
+    "axl_flash_chunk",
+    "axl_flash_chunk_workspace_bytes",
     "axl_flash_bwd",
     "axl_flash_bwd_phases",
     "axl_flash_bwd_workspace_bytes",
@@ -178,6 +198,7 @@ def load() -> ctypes.CDLL:
         )
     for name, ptype in (
         ("axl_flash_fwd", AxlFlashFwdParams),
+        ("axl_flash_chunk", AxlFlashChunkParams),
         ("axl_flash_bwd", AxlFlashBwdParams),
         ("axl_paged_decode", AxlPagedDecodeParams),
         ("axl_paged_decode_static", AxlPagedDecodeParams),
@@ -190,6 +211,7 @@ def load() -> ctypes.CDLL:
     lib.axl_flash_bwd_phases.restype = ctypes.c_int
     lib.axl_flash_bwd_phases.argtypes = [ctypes.POINTER(AxlFlashBwdParams), ctypes.c_int, ctypes.c_void_p]
     for name, ptype in (
+        ("axl_flash_chunk_workspace_bytes", AxlFlashChunkParams),
         ("axl_flash_bwd_workspace_bytes", AxlFlashBwdParams),
         ("axl_paged_decode_workspace_bytes", AxlPagedDecodeParams),
         ("axl_decode_workspace_bytes", AxlDecodeParams),

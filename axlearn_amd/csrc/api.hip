@@ -22,6 +22,8 @@ int set_error(int code, const char* fmt, ...) {
 }
 
 int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream);
+int launch_flash_chunk(const AxlFlashChunkParams& p, hipStream_t stream);
+size_t flash_chunk_workspace_bytes(const AxlFlashChunkParams& p);
 int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream);
 size_t flash_bwd_workspace_bytes(const AxlFlashBwdParams& p);
 int launch_paged_decode(const AxlPagedDecodeParams& p, hipStream_t stream);
@@ -221,6 +223,39 @@ int axl_flash_fwd(const AxlFlashFwdParams* p, void* stream) {
                           {&p->q_strides, &p->k_strides, &p->v_strides, &p->out_strides});
   if (rc != AXL_OK) return rc;
   return launch_flash_fwd(*p, (hipStream_t)stream);
+}
+
+size_t axl_flash_chunk_workspace_bytes(const AxlFlashChunkParams* p) {
+  if (!p || p->batch <= 0 || p->q_len <= 0 || p->num_kv_heads <= 0 || p->num_q_heads < p->num_kv_heads) return 0;
+  return flash_chunk_workspace_bytes(*p);
+}
+
+int axl_flash_chunk(const AxlFlashChunkParams* p, void* stream) {
+  const char* who = "axl_flash_chunk";
+  if (!p) return set_error(AXL_ERR_INVALID_ARGUMENT, "%s: params is NULL", who);
+  // any number of query rows: the length rule is checked for the cache alone
+  int rc = check_flash_shapes(who, p->batch, p->q_len > 0 ? 128 : p->q_len, p->kv_len, p->num_q_heads, p->num_kv_heads,
+                              p->head_dim, p->dtype, p->mask_kind, p->sliding_window, p->softmax_scale, nullptr);
+  if (rc != AXL_OK) return rc;
+  if (p->dtype == AXL_F32) return set_error(AXL_ERR_UNSUPPORTED, "%s: dtype fp32 (supported: bf16, f16)", who);
+  if (p->mask_kind == AXL_MASK_NONE) return set_error(AXL_ERR_UNSUPPORTED, "%s: needs a causal or sliding-window mask", who);
+  if (!p->q || !p->k || !p->v || !p->out || !p->positions)
+    return set_error(AXL_ERR_INVALID_ARGUMENT, "%s: NULL tensor pointer", who);
+  if (p->pos_batch_stride < 0 || p->pos_row_stride < 0)
+    return set_error(AXL_ERR_INVALID_ARGUMENT, "%s: position strides must be >= 0", who);
+  if ((int64_t)p->q_len * (p->num_q_heads / p->num_kv_heads) > (int64_t)1 << 30)
+    return set_error(AXL_ERR_UNSUPPORTED, "%s: q_len * query heads per kv head above 2^30", who);
+  if (!aligned16(p->q) || !aligned16(p->k) || !aligned16(p->v) || !aligned16(p->out) ||
+      !strides_ok(p->q_strides, 2) || !strides_ok(p->k_strides, 2) || !strides_ok(p->v_strides, 2) ||
+      !strides_ok(p->out_strides, 2))
+    return set_error(AXL_ERR_UNSUPPORTED, "%s: tensors must be 16-byte aligned rows", who);
+  rc = check_odd_head_dim(who, p->head_dim, false, {&p->k_strides, &p->v_strides});
+  if (rc != AXL_OK) return rc;
+  const size_t need = flash_chunk_workspace_bytes(*p);
+  if (need && (!p->workspace || p->workspace_bytes < need || !aligned16(p->workspace)))
+    return set_error(AXL_ERR_WORKSPACE, "%s: workspace needs %zu bytes, 16-byte aligned (got %zu)", who, need,
+                     p->workspace ? p->workspace_bytes : (size_t)0);
+  return launch_flash_chunk(*p, (hipStream_t)stream);
 }
 
 size_t axl_flash_bwd_workspace_bytes(const AxlFlashBwdParams* p) {

@@ -42,6 +42,12 @@ struct FwdArgs {
   int mask_kind, window, q_off;
   float scale;
   int d_real;  // head_dim of the tensors: a multiple of 8, at most the compiled width D (16-bit kernels)
+  // Chunk form only (see flash_fwd_body):
+  const char* pos;        // positions of the query rows, int32 or int64
+  int64_t pos_sb, pos_ss; // its strides in BYTES
+  int pos_i64;
+  int slots;              // workgroups of the launch if they share the keys of a row block, else 0
+  char* part;             // their partial results
 };
 
 // NW wavefronts of 32 query rows each.  The kernels are launched with 4 (two workgroups per CU); 8
@@ -65,9 +71,89 @@ struct FwdTile {
 constexpr int kMaxSegTiles = 1024;               // key tiles whose segment ids the forward classifies
 constexpr int kSegNotUniform = -0x7fffffff - 1;  // marks a tile with more than one segment id
 
-template <typename E, int D, bool AUX, int NW = 4>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(AUX ? 1 : 2, AUX ? 1 : 2)))
-void flash_fwd_kernel(const FwdArgs a) {
+// Partial results of the chunk form: per workgroup and wavefront the accumulators as they lie in
+// registers, [D / 8 pieces][64 lanes] float4, so that a store instruction writes 1 KB in one piece, then
+// (log2-scaled running maximum, sum) of the wavefront's 32 rows.
+template <int D>
+struct ChunkPart {
+  static constexpr int O_BYTES = 32 * D * 4;
+  static constexpr int BYTES = O_BYTES + 32 * 8;
+};
+
+// Which sequence a workgroup of the chunk form works on and how many share its key range.  The live
+// lengths are known on the device only, and they differ: with the same number of workgroups for every
+// sequence the longest one would finish alone.  So every wavefront derives the same plan: a workgroup takes about `target` tiles of 64 keys, a sequence of n
+// tiles gets ceil(n / target) workgroups per row block, and target is the smallest of a few growing ones
+// with which the whole plan fits the launch (at the latest when it exceeds the sum of n over
+// slots - groups, with groups the row blocks of the call: ceil(x) < x + 1).  The length is taken from the
+// sequence's last row; any figure would give right results.
+struct ChunkShare {
+  int b, nsplit, first;   // sequence, workgroups per row block, number of its first (row block, split)
+};
+// by_slot: the sequence that (row block, split) number `key` belongs to (b = -1 past the last); else that of b = key.
+__device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, int nqb, bool by_slot, int key) {
+  if (a.slots == 0) return by_slot ? ChunkShare{key / nqb, 1, key / nqb * nqb} : ChunkShare{key, 1, key * nqb};
+  auto tiles = [&](int b) -> int {
+    if (b >= a.B) return 0;
+    const char* pp = a.pos + b * a.pos_sb + (a.T - 1) * a.pos_ss;
+    const int end = min(a.S, max(0, (a.pos_i64 ? (int)*(const int64_t*)pp : *(const int32_t*)pp) + 1));
+    const int begin = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? max(0, end - a.T - a.window) : 0;
+    return (max(end, begin + 1) - begin + 63) / 64;
+  };
+  int total = 0;
+  for (int b = lane; b < a.B; b += 64) total += tiles(b);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
+  const int per = nqb * a.Hkv;
+  // at least 8 tiles (512 keys) each: below that a workgroup's fixed costs weigh more than what it takes over
+  int target = max(8, (int)((int64_t)total * per / a.slots));
+  for (;; target += 1 + target / 16) {
+    int n = 0;
+    for (int b = lane; b < a.B; b += 64) n += (tiles(b) + target - 1) / target;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+    if (n * per <= a.slots) break;
+  }
+  ChunkShare r{-1, 1, 0};
+  int before = 0;
+  for (int base = 0; base < a.B; base += 64) {
+    const int n = (tiles(base + lane) + target - 1) / target;
+    int incl = n;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int up = __shfl_up(incl, o);
+      if (lane >= o) incl += up;
+    }
+    const uint64_t m = __builtin_amdgcn_ballot_w64(by_slot ? (before + incl) * nqb > key && n > 0 : base + lane == key);
+    if (m) {
+      const int l = __builtin_ctzll(m);
+      r.b = base + l;
+      r.nsplit = __builtin_amdgcn_readlane(n, l);
+      r.first = (before + __builtin_amdgcn_readlane(incl, l) - r.nsplit) * nqb;
+      break;
+    }
+    before += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return r;
+}
+
+// The body of flash_fwd_kernel and flash_chunk_kernel (CHUNK).
+//
+// CHUNK: a chunk of query rows per sequence at positions of their own over a longer cache (incremental
+// prefill).  What bounds it is that such calls hold few rows: padded to 128 per (sequence, query head)
+// and one workgroup to a block, 200 rows of 2 x 32 heads over 8192 keys were 128 workgroups, most of them
+// walking the whole cache, on 256 CUs (119 us; the operations alone are 22 us at the rate of a large GEMM).  So
+//   * the rows of all query heads of a kv head form one list, row r = (token r / G, head r % G): only the
+//     last block of the list is padded, and a block of 128 rows reads the K / V tiles once for G heads;
+//   * several workgroups share the key range of a block, together as many as fill two workgroups per CU
+//     (chunk_share); each leaves its accumulators for flash_chunk_combine_kernel;
+//   * the position of every row comes from the caller's tensor as it is (int32 or int64): nothing about
+//     the positions is looked at on the host.
+// That call now takes 55 us for the 42 GFLOP of offsets 7552 and 4996 (760 TFLOP/s; the forward at full
+// occupancy runs at 1000) and 10 us for the merge, 172 -> 99 us as a call of the layer.
+template <typename E, int D, bool AUX, int NW, bool CHUNK>
+__device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
+  static_assert(!(AUX && CHUNK), "the chunk form takes no bias or dropout mask");
   using Tile = FwdTile<D, NW>;
   constexpr int KK = D / 16;  // MFMA k-steps over head_dim
   constexpr int DT = D / 32;  // 32-row output tiles over head_dim
@@ -79,14 +165,36 @@ void flash_fwd_kernel(const FwdArgs a) {
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-  int qb, b, h;
-  decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h);
-  const int hk = h / (a.Hq / a.Hkv);
-  const int q_off = a.q_off + (a.q_offs ? a.q_offs[b] : 0);  // position of this sequence's query row 0
+  int qb, b, h, hk, split = 0, nsplit = 1;
+  const int G = a.Hq / a.Hkv;
+  if constexpr (CHUNK) {
+    // The kv head counts fastest: workgroup i is dispatched to XCD i % 8, so with 8 kv heads the workgroups
+    // that read the same K / V share an L2; the row blocks of a split follow one another.
+    const int nqb = (a.T * G + Tile::BQ - 1) / Tile::BQ;
+    const int slot = blockIdx.x / a.Hkv;
+    const ChunkShare sh = chunk_share(a, lane, nqb, true, slot);
+    if (sh.b < 0) return;   // the plan needs fewer workgroups than were launched
+    b = sh.b;
+    nsplit = sh.nsplit;
+    split = (slot - sh.first) / nqb;
+    qb = slot - sh.first - split * nqb;
+    hk = blockIdx.x - slot * a.Hkv;
+  } else {
+    decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h);
+    hk = h / G;
+  }
+  const int q_off = CHUNK ? 0 : a.q_off + (a.q_offs ? a.q_offs[b] : 0);  // position of this sequence's query row 0
   const int q0_wg = qb * Tile::BQ;
   const int q0 = q0_wg + wave * 32;
+  int row = q0 + l32;          // this lane's query row
+  const int chunk_rows = CHUNK ? a.T * G : 0;
+  if constexpr (CHUNK) {       // rows past the list repeat its last one and are not stored
+    const int r = min(row, chunk_rows - 1);
+    row = r / G;
+    h = hk * G + r - row * G;  // differs from lane to lane
+  }
 
-  const __bf16* qp = (const __bf16*)a.q + b * a.qs.b + (int64_t)(q0 + l32) * a.qs.s + h * a.qs.h;
+  const __bf16* qp = (const __bf16*)a.q + b * a.qs.b + (int64_t)row * a.qs.s + h * a.qs.h;
   const __bf16* kp = (const __bf16*)a.k + b * a.ks.b + hk * a.ks.h;
   const __bf16* vp = (const __bf16*)a.v + b * a.vs.b + hk * a.vs.h;
 
@@ -101,14 +209,46 @@ void flash_fwd_kernel(const FwdArgs a) {
     qf[kk] = 16 * kk + 8 * g < a.d_real ? *(const bf16x8*)(qp + 16 * kk + 8 * g) : zero8;
   }
 
+  int qpos = row + q_off;                                 // this lane's query position
+  int qpos_min = q0 + q_off, qpos_max = q0 + 31 + q_off;  // of the wavefront
+  int wg_min = q0_wg + q_off, wg_max = q0_wg + Tile::BQ - 1 + q_off;  // of the workgroup
+  if constexpr (CHUNK) {
+    const char* pp = a.pos + b * a.pos_sb + row * a.pos_ss;
+    qpos = a.pos_i64 ? (int)*(const int64_t*)pp : *(const int32_t*)pp;
+    qpos_min = qpos_max = qpos;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {   // the lanes l and l ^ 32 hold the same row
+      qpos_min = min(qpos_min, __shfl_xor(qpos_min, o));
+      qpos_max = max(qpos_max, __shfl_xor(qpos_max, o));
+    }
+    __shared__ int s_pos[2 * NW];
+    if (lane == 0) {
+      s_pos[2 * wave] = qpos_min;
+      s_pos[2 * wave + 1] = qpos_max;
+    }
+    __syncthreads();
+    wg_min = qpos_min;
+    wg_max = qpos_max;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      wg_min = min(wg_min, s_pos[2 * w]);
+      wg_max = max(wg_max, s_pos[2 * w + 1]);
+    }
+    // the same in every lane: say so, scalar addresses and loop bounds are formed from them
+    qpos_min = __builtin_amdgcn_readfirstlane(qpos_min);
+    qpos_max = __builtin_amdgcn_readfirstlane(qpos_max);
+    wg_min = __builtin_amdgcn_readfirstlane(wg_min);
+    wg_max = __builtin_amdgcn_readfirstlane(wg_max);
+  }
+
   // Visible key range of this workgroup.
   int k_begin = 0, k_end = a.S;
   if (a.mask_kind != AXL_MASK_NONE) {
-    k_end = min(a.S, q0_wg + Tile::BQ + q_off);
-    if (a.mask_kind == AXL_MASK_SLIDING_WINDOW) k_begin = max(0, q0_wg + q_off - a.window);
+    k_end = max(0, min(a.S, wg_max + 1));
+    if (a.mask_kind == AXL_MASK_SLIDING_WINDOW) k_begin = min(k_end, max(0, wg_min - a.window));
   }
-  const int seg_q = a.seg ? a.seg[(int64_t)b * a.T + q0 + l32] : 0;
-  const int32_t* seg_k = a.seg ? a.seg + (int64_t)b * a.T : nullptr;
+  const int seg_q = !CHUNK && a.seg ? a.seg[(int64_t)b * a.T + q0 + l32] : 0;
+  const int32_t* seg_k = !CHUNK && a.seg ? a.seg + (int64_t)b * a.T : nullptr;
   // With segment ids: one pass over the ids of the key range shrinks it to the hull of the keys whose
   // id lies between the smallest and the largest id of this workgroup's queries, and records for
   // every 64-key tile whether it carries a single id.  A tile whose keys all carry the one id that
@@ -117,8 +257,13 @@ void flash_fwd_kernel(const FwdArgs a) {
   int seg_t0 = 0;          // tile that s_tile_id[0] describes
   if (seg_k) seg_t0 = classify_segment_groups<Tile::BK, 64 * NW>(seg_q, seg_k, tid, k_begin, k_end, s_tile_id, kMaxSegTiles,
                                                             kSegNotUniform);
-  const int t_begin = k_begin / Tile::BK;
-  const int t_end = (k_end + Tile::BK - 1) / Tile::BK;
+  int t_begin = k_begin / Tile::BK;
+  int t_end = (k_end + Tile::BK - 1) / Tile::BK;
+  if constexpr (CHUNK) {       // this workgroup's share of the tiles
+    const int per = (t_end - t_begin + nsplit - 1) / nsplit;
+    t_begin = min(t_end, t_begin + split * per);
+    t_end = min(t_end, t_begin + per);
+  }
   bool seg_fast = false;   // this wavefront's queries share one id and the table covers the tiles
   int wq_id = 0;
   if (seg_k && t_end - seg_t0 <= kMaxSegTiles) {
@@ -134,8 +279,6 @@ void flash_fwd_kernel(const FwdArgs a) {
     if (a.aux.bias) bias_row = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh + (int64_t)(q0 + l32) * a.aux.bias_sr;
     if (a.aux.drop) drop_row = a.aux.drop + b * a.aux.drop_sb + h * a.aux.drop_sh + (int64_t)(q0 + l32) * a.aux.drop_sr;
   }
-  const int qpos = q0 + l32 + q_off;       // this lane's query position
-  const int qpos_min = q0 + q_off, qpos_max = q0 + 31 + q_off;  // of the wavefront
   // Tiles this wavefront has to process (the others it only helps to load): [tw_begin, tw_end).
   int tw_begin = t_begin, tw_end = t_end;
   if (a.mask_kind != AXL_MASK_NONE) {
@@ -143,6 +286,7 @@ void flash_fwd_kernel(const FwdArgs a) {
     if (a.mask_kind == AXL_MASK_SLIDING_WINDOW) tw_begin = max(t_begin, (qpos_min - a.window) / Tile::BK);
     tw_begin = max(tw_begin, t_begin);
   }
+  if (CHUNK && q0 >= chunk_rows) tw_end = tw_begin;   // a wavefront without rows only helps to load
 
   floatx16 o[DT];
 #pragma unroll
@@ -152,7 +296,7 @@ void flash_fwd_kernel(const FwdArgs a) {
   float m_run = kNegInf;  // running row max of the raw (unscaled) logits
   float l_run = 0.f;      // this lane's share of the running row sum (lanes l and l^32 split it)
   const float c = a.scale * kLog2e;
-  if (a.sink) {
+  if (a.sink && split == 0) {
     // The sink is one more logit per row, with no value row (attention.py:608-626): it enters the
     // running softmax state as an already-processed key of weight exp(sink - m) = 1.
     m_run = a.sink[h] / a.scale;
@@ -570,9 +714,25 @@ void flash_fwd_kernel(const FwdArgs a) {
 
   // Epilogue: out = acc / l ; lse = m*scale + ln(l).
   const float l_tot = xor32_sum(l_run);
+  if constexpr (CHUNK) {
+    if (nsplit > 1) {
+      if (q0 >= chunk_rows) return;
+      char* part = a.part + ((int64_t)blockIdx.x * NW + wave) * ChunkPart<D>::BYTES;
+      if (g == 0) *(floatx2*)(part + ChunkPart<D>::O_BYTES + 8 * l32) = floatx2{m_run * c, l_tot};
+      if (tw_begin < tw_end || split == 0) {   // (elsewhere l is zero and the accumulators are not read)
+#pragma unroll
+        for (int i = 0; i < 4 * DT; i++) {
+          const floatx4 w = {o[i / 4][4 * (i % 4)], o[i / 4][4 * (i % 4) + 1], o[i / 4][4 * (i % 4) + 2], o[i / 4][4 * (i % 4) + 3]};
+          *(floatx4*)(part + i * 1024 + 16 * lane) = w;
+        }
+      }
+      return;
+    }
+    if (q0 + l32 >= chunk_rows) return;
+  }
   float inv_l = l_tot > 0.f ? 1.0f / l_tot : 0.f;  // a row with no visible key yields zeros
   if constexpr (AUX) inv_l *= a.aux.keep_scale;
-  __bf16* op = (__bf16*)a.out + b * a.os.b + (int64_t)(q0 + l32) * a.os.s + h * a.os.h;
+  __bf16* op = (__bf16*)a.out + b * a.os.b + (int64_t)row * a.os.s + h * a.os.h;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++) {
 #pragma unroll
@@ -586,8 +746,66 @@ void flash_fwd_kernel(const FwdArgs a) {
       if (32 * dt + 8 * rq + 4 * g < a.d_real) *(uint2*)(op + 32 * dt + 8 * rq + 4 * g) = w.u;
     }
   }
-  if (a.lse && g == 0) {
+  if (!CHUNK && a.lse && g == 0) {
     a.lse[((int64_t)b * a.Hq + h) * a.T + q0 + l32] = (m_run * c + fast_log2(l_tot)) * kLn2;
+  }
+}
+
+template <typename E, int D, bool AUX, int NW = 4>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(AUX ? 1 : 2, AUX ? 1 : 2)))
+void flash_fwd_kernel(const FwdArgs a) {
+  flash_fwd_body<E, D, AUX, NW, false>(a);
+}
+
+template <typename E, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_chunk_kernel(const FwdArgs a) {
+  flash_fwd_body<E, D, false, 4, true>(a);
+}
+
+// Merges the partial results of the chunk form, out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s in the
+// order of the splits.  One workgroup per 32-row block, a wavefront per 32 columns of head_dim, the
+// pieces read as they were written (1 KB per instruction, four per split in flight).  Bound by the
+// bytes: the partials of the chunk above (504 workgroups) are 30 MB in 10 us.
+template <typename E, int D>
+__global__ __launch_bounds__(2 * D) void flash_chunk_combine_kernel(const FwdArgs a) {
+  const int lane = threadIdx.x & 63, dt = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
+  const int G = a.Hq / a.Hkv, chunk_rows = a.T * G, blocks = (chunk_rows + 31) / 32, nqb = (chunk_rows + 127) / 128;
+  const int pair = blockIdx.x / blocks, blk = blockIdx.x - pair * blocks;
+  const int b = pair / a.Hkv, hk = pair - b * a.Hkv;
+  const ChunkShare sh = chunk_share(a, lane, nqb, false, b);
+  if (sh.nsplit == 1) return;   // stored by the one workgroup that had the keys
+  const char* part = a.part + (((int64_t)(sh.first + blk / 4) * a.Hkv + hk) * 4 + blk % 4) * ChunkPart<D>::BYTES;
+  const int64_t split_bytes = (int64_t)nqb * a.Hkv * 4 * ChunkPart<D>::BYTES;
+  float mx = 2.f * kNegInf;
+  for (int s = 0; s < sh.nsplit; s++)
+    mx = fmaxf(mx, *(const float*)(part + s * split_bytes + ChunkPart<D>::O_BYTES + 8 * l32));
+  floatx4 acc[4] = {};
+  float l = 0.f;
+#pragma unroll 2
+  for (int s = 0; s < sh.nsplit; s++) {
+    const char* p = part + s * split_bytes;
+    const floatx2 ml = *(const floatx2*)(p + ChunkPart<D>::O_BYTES + 8 * l32);
+    const float w = ml[1] > 0.f ? fast_exp2(ml[0] - mx) : 0.f;
+    l += w * ml[1];
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) {
+      const floatx4 o = *(const floatx4*)(p + (4 * dt + rq) * 1024 + 16 * lane);
+#pragma unroll
+      for (int j = 0; j < 4; j++) acc[rq][j] = ml[1] > 0.f ? __builtin_fmaf(w, o[j], acc[rq][j]) : acc[rq][j];
+    }
+  }
+  const int r = 32 * blk + l32;
+  if (r >= chunk_rows) return;
+  const float inv_l = l > 0.f ? 1.0f / l : 0.f;
+  const int t = r / G, h = hk * G + r - t * G;
+  __bf16* op = (__bf16*)a.out + b * a.os.b + (int64_t)t * a.os.s + h * a.os.h;
+#pragma unroll
+  for (int rq = 0; rq < 4; rq++) {
+    union { bf16x2 p[2]; uint2 u; } w;
+    w.p[0] = E::pack(acc[rq][0] * inv_l, acc[rq][1] * inv_l);
+    w.p[1] = E::pack(acc[rq][2] * inv_l, acc[rq][3] * inv_l);
+    if (32 * dt + 8 * rq + 4 * g < a.d_real) *(uint2*)(op + 32 * dt + 8 * rq + 4 * g) = w.u;
   }
 }
 
@@ -1146,6 +1364,56 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
 #undef AXL_LAUNCH_FWD
   if (err != hipSuccess)
     return set_error(AXL_ERR_LAUNCH, "axl_flash_fwd: launch failed: %s", hipGetErrorString(err));
+  return AXL_OK;
+}
+
+// Workgroups of a chunk launch whose row blocks share their key ranges out (chunk_share): two per CU, if
+// that is at least two per row block and the range that can be live is worth two (1024 keys: a cache of
+// 512 is never split, so that its rows are those of a full forward bit for bit); else 0, one per row block.
+static int chunk_slots(const AxlFlashChunkParams& p) {
+  const int64_t rows = (int64_t)p.q_len * (p.num_q_heads / p.num_kv_heads);
+  const int64_t groups = (rows + 127) / 128 * p.batch * p.num_kv_heads;
+  int64_t live = p.kv_len;
+  if (p.mask_kind == AXL_MASK_SLIDING_WINDOW && (int64_t)p.sliding_window + p.q_len < live) live = p.sliding_window + p.q_len;
+  const int slots = 2 * cu_count();
+  return 2 * groups <= slots && live >= 1024 ? slots : 0;
+}
+
+size_t flash_chunk_workspace_bytes(const AxlFlashChunkParams& p) {
+  return (size_t)chunk_slots(p) * 4 * (p.head_dim <= 64 ? ChunkPart<64>::BYTES : ChunkPart<128>::BYTES);
+}
+
+template <typename E, int D>
+static hipError_t launch_chunk(const FwdArgs& a, hipStream_t stream) {
+  auto kern = flash_chunk_kernel<E, D>;
+  const hipError_t err = allow_dynamic_lds((const void*)kern, FwdTile<D>::LDS_BYTES);
+  if (err != hipSuccess) return err;
+  const int rows = a.T * (a.Hq / a.Hkv), pairs = a.B * a.Hkv;
+  hipLaunchKernelGGL(kern, dim3(a.slots ? a.slots : (rows + 127) / 128 * pairs), dim3(256), FwdTile<D>::LDS_BYTES, stream, a);
+  if (a.slots)
+    hipLaunchKernelGGL((flash_chunk_combine_kernel<E, D>), dim3((rows + 31) / 32 * pairs), dim3(2 * D), 0, stream, a);
+  return hipGetLastError();
+}
+
+int launch_flash_chunk(const AxlFlashChunkParams& p, hipStream_t stream) {
+  FwdArgs a{};
+  a.q = p.q; a.k = p.k; a.v = p.v; a.out = p.out;
+  a.sink = p.logit_sink;
+  a.qs = to_s3(p.q_strides); a.ks = to_s3(p.k_strides); a.vs = to_s3(p.v_strides); a.os = to_s3(p.out_strides);
+  a.B = p.batch; a.T = p.q_len; a.S = p.kv_len; a.Hq = p.num_q_heads; a.Hkv = p.num_kv_heads;
+  a.mask_kind = p.mask_kind; a.window = p.sliding_window;
+  a.scale = p.softmax_scale;
+  a.d_real = p.head_dim;
+  const int es = p.pos_is_i64 ? 8 : 4;
+  a.pos = (const char*)p.positions; a.pos_i64 = p.pos_is_i64;
+  a.pos_sb = p.pos_batch_stride * es; a.pos_ss = p.pos_row_stride * es;
+  a.slots = chunk_slots(p);
+  a.part = (char*)p.workspace;
+  hipError_t err;
+  if (p.dtype == AXL_BF16) err = p.head_dim <= 64 ? launch_chunk<ElemBf16, 64>(a, stream) : launch_chunk<ElemBf16, 128>(a, stream);
+  else err = p.head_dim <= 64 ? launch_chunk<ElemF16, 64>(a, stream) : launch_chunk<ElemF16, 128>(a, stream);
+  if (err != hipSuccess)
+    return set_error(AXL_ERR_LAUNCH, "axl_flash_chunk: launch failed: %s", hipGetErrorString(err));
   return AXL_OK;
 }
 

@@ -314,12 +314,23 @@ class HipFlashAttention(BaseFlashAttention):
         return True
 
     def _incremental_prefill(self, input_batch: Nested) -> Tensor:
-        """Queries at per-sequence offsets into the cache; rows padded up to the 128-row block."""
+        """A chunk of queries per sequence at positions of its own in the cache.
+
+        16-bit types: any number of rows at any positions, as the bias gives them.  float32: rows padded
+        up to the 128-row block of the plain forward, positions consecutive (looked at on the host)."""
         query, key, value = input_batch["query"], input_batch["key"], input_batch["value"]
         mask, _, _ = split(input_batch["bias"], MaskFnAttentionBias, SegmentIdAttentionBias)
         kind = classify_mask_bias(mask)
         b, t, _, head_dim = query.shape
         positions = mask.target_positions.to(query.device)
+        if query.dtype != torch.float32:
+            width = head_dim if runs_at_native_head_dim(query, key, value, aux=False) else padded_head_dim(head_dim)
+            out = ops.flash_chunk(
+                _pad_last(query.detach(), width), _pad_last(key.detach(), width), _pad_last(value.detach(), width),
+                positions, softmax_scale=float(self.cfg.softmax_scale), mask_kind=kind[0], sliding_window=kind[1],
+                logit_sink=input_batch.get("logit_sink", None),
+            )
+            return out if width == head_dim else out[..., :head_dim]
         offsets = positions[:, 0].to(torch.int32).expand(b).contiguous()
         consecutive = positions[:, :1] + torch.arange(t, device=query.device)[None]
         if not torch.equal(positions, consecutive.to(positions.dtype)):

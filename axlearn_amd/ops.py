@@ -20,6 +20,7 @@ from axlearn_amd._lib import (
     AxlDecodeParams,
     AxlError,
     AxlFlashBwdParams,
+    AxlFlashChunkParams,
     AxlFlashFwdParams,
     AxlPagedDecodeParams,
     AxlPageInsertParams,
@@ -30,6 +31,7 @@ __all__ = [
     "MASK_CAUSAL",
     "MASK_SLIDING_WINDOW",
     "flash_fwd",
+    "flash_chunk",
     "flash_bwd",
     "flash_bwd_buffers",
     "flash_bwd_ds_workspace_bytes",
@@ -185,6 +187,46 @@ def flash_fwd(
     )
     _lib.check(lib.axl_flash_fwd(ctypes.byref(p), _lib.current_stream_ptr()))
     return out, lse
+
+
+def flash_chunk(
+    q: torch.Tensor,
+    k: torch.Tensor,
+    v: torch.Tensor,
+    positions: torch.Tensor,
+    *,
+    softmax_scale: float = 1.0,
+    mask_kind: int = MASK_CAUSAL,
+    sliding_window: int = 0,
+    logit_sink: Optional[torch.Tensor] = None,
+) -> torch.Tensor:
+    """Incremental prefill: q [B,T,Hq,D] (any T) at positions [B|1,T] (int32 / int64, on the GPU) over a
+    cache k, v [B,S,Hkv,D] -> out [B,T,Hq,D].  bf16 / f16, forward only."""
+    b, t, hq, d, s, hkv = _check_qkv(q, k, v)
+    if positions.dim() != 2 or positions.shape[0] not in (1, b) or positions.shape[1] != t:
+        raise _bad(f"positions must be [{b}|1, {t}], got {list(positions.shape)}")
+    _require_cuda(q, k, v, positions, logit_sink)
+    lib = _lib.load()
+    if positions.dtype not in (torch.int32, torch.int64):
+        positions = positions.to(torch.int32)
+    out = torch.empty((b, t, hq, d), dtype=q.dtype, device=q.device)
+    sink = _sink(logit_sink, hq)
+    p = AxlFlashChunkParams(
+        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), out=out.data_ptr(),
+        q_strides=_lib.strides4(q), k_strides=_lib.strides4(k), v_strides=_lib.strides4(v),
+        out_strides=_lib.strides4(out),
+        batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
+        dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind, sliding_window=int(sliding_window),
+        softmax_scale=float(softmax_scale), logit_sink=_lib.ptr(sink), positions=positions.data_ptr(),
+        pos_batch_stride=positions.stride(0) if positions.shape[0] > 1 else 0, pos_row_stride=positions.stride(1),
+        pos_is_i64=int(positions.dtype == torch.int64),
+    )
+    need = int(lib.axl_flash_chunk_workspace_bytes(ctypes.byref(p)))
+    if need:
+        ws = torch.empty((need,), dtype=torch.uint8, device=q.device)
+        p.workspace, p.workspace_bytes = ws.data_ptr(), need
+    _lib.check(lib.axl_flash_chunk(ctypes.byref(p), _lib.current_stream_ptr()))
+    return out
 
 
 def flash_bwd(

@@ -1351,3 +1351,43 @@ def test_baseline_c5_full_size(ds_workspace):
     _sampled_fwd_bwd_check(1, 32768, 64, 8, 128, "causal", None, False,
                            samples=[(0, 3)], dq_rows=[(0, 128), (16384, 16512), (32640, 32768)],
                            key_blocks=[(32384, 32512), (32000, 32128)], ds_workspace=ds_workspace)
+
+
+# ----------------------------------------------------------------------------- chunks over a long cache
+
+
+@pytest.mark.parametrize("b,rows,hq,hkv,d,kv_len,window,dtype,sink", [
+    (2, 1, 4, 4, 128, 512, None, torch.bfloat16, False),       # one row, one workgroup per block
+    (2, 7, 8, 2, 128, 4096, None, torch.bfloat16, True),       # 28 packed rows: one wavefront, split keys
+    (2, 32, 4, 4, 64, 2048, None, torch.float16, False),       # exactly one wavefront's rows
+    (2, 33, 12, 4, 64, 3968, 700, torch.bfloat16, True),       # 99 packed rows (3 per token), window
+    (3, 130, 5, 1, 128, 1152, None, torch.float16, False),     # 650 packed rows, 5 per token: last block of 10
+    (2, 200, 16, 2, 80, 8192, 3000, torch.bfloat16, False),    # head_dim below the compiled width
+    (70, 3, 4, 1, 64, 2048, None, torch.bfloat16, False),      # more sequences than lanes, some of them not split
+    (2, 1100, 8, 8, 64, 1280, None, torch.bfloat16, False),    # enough row blocks: nothing is split
+])
+def test_chunk_of_rows_over_a_long_cache(b, rows, hq, hkv, d, kv_len, window, dtype, sink):
+    # Rows packed over the query heads of a kv head, keys shared by several workgroups: every remainder of
+    # the packing, positions that are neither consecutive nor sorted, the first and the last of the cache,
+    # and a row at position -1 that sees no key (zeros).
+    q, k, v, _ = _inputs(b, rows, hq, hkv, d, dtype, s=kv_len)
+    g = torch.Generator().manual_seed(rows)
+    positions = torch.randint(0, kv_len, (b, rows), generator=g)
+    positions[0, 0], positions[1, -1] = kv_len - 1, 0
+    if rows > 8:
+        positions[0, 5] = -1
+    sk = torch.randn(hq, generator=g) if sink else None
+    mask_kind = ops.MASK_CAUSAL if window is None else ops.MASK_SLIDING_WINDOW
+    spec = ref.MaskSpec(causal=window is None, sliding_window=window, target_positions=positions,
+                        source_positions=torch.arange(kv_len)[None])
+    want = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5, **({} if sk is None else dict(logit_sink=sk)))
+    outs = []
+    for pos in (positions.cuda(), positions.to(torch.int32).cuda(), positions.cuda()):
+        outs.append(ops.flash_chunk(q.cuda(), k.cuda(), v.cuda(), pos, softmax_scale=d ** -0.5, mask_kind=mask_kind,
+                                    sliding_window=window or 0, logit_sink=None if sk is None else sk.cuda()))
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    got = outs[0].cpu()
+    seen = positions >= 0
+    assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
+    # outputs over thousands of keys are small: the relative bar alone, an eighth of it for f16
+    assert ref.rel_l2(got[seen], want[seen]) < (1e-2 if dtype == torch.bfloat16 else 1.25e-3)

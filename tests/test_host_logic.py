@@ -678,3 +678,9 @@ def test_ffi_shim_and_jax_side_stay_in_step_with_the_abi():
     # the version the shim and the binding were written against
     assert _lib.ABI_VERSION == int(re.search(r"#define AXL_ATTN_ABI_VERSION (\d+)",
                                              open(os.path.join(ROOT, "include", "axl_attn.h")).read()).group(1))
+
+
+def test_chunk_kernel_keeps_the_distance_behind_its_assembly_mfma_chains():
+    """The form of the forward for chunks over a long cache shares its body: the same check."""
+    asm, _ = _device_asm("flash_fwd.hip", extra=("-mllvm", "-amdgpu-mfma-vgpr-form"))
+    _assert_asm_mfma_distances(asm, r"_ZN3axl18flash_chunk_kernel", 4)
