@@ -199,8 +199,8 @@ class CompositeAttentionBias(BaseAttentionBias):
         members = self._nonzero()
         if not members:
             return None
-        total = 0.0
-        for b in members:
+        total = members[0].value()
+        for b in members[1:]:
             total = total + b.value()
         return total
 
