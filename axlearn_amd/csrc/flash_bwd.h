@@ -62,10 +62,11 @@ __host__ __device__ inline int64_t ds_run_start(int64_t pair, int T, int G, int 
 }
 
 // Enqueues the dK/dV kernel for `dtype` AXL_BF16 or AXL_F16 and head_dim 64 or 128; `aux` selects
-// the instantiation that reads the dense bias / dropout mask.  With a.ds set (and no bias / dropout
-// mask, causal or sliding-window mask, q_off 0, T == S) the kernel also stores dS for
-// launch_bwd_dq_stream, and with a.kb_tbl set the range of query tiles each key block stored.
+// the instantiation that reads the dense bias / dropout mask.  With a.ds set (causal or sliding-window
+// mask, q_off 0, T == S) the kernel also stores dS for launch_bwd_dq_stream, and with a.kb_tbl set the
+// range of query tiles each key block stored.
 hipError_t launch_bwd_dkdv(const BwdArgs& a, int dtype, int head_dim, bool aux, hipStream_t stream);
+hipError_t launch_bwd_dkdv_aux(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 
 // Enqueues the streaming dQ kernel, dq = scale * dS k from the dS blocks in a.ds (with a.kb_tbl set:
 // from the blocks that table says were stored).

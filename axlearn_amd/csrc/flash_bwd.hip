@@ -394,14 +394,14 @@ static size_t stats_bytes(const AxlFlashBwdParams& p) {
 
 // The dS-spill path: the dK/dV kernel stores dS and the dQ kernel becomes one streaming GEMM
 // (5 executed GEMMs instead of 7).  Causal or sliding-window attention over equal lengths, with or
-// without segment ids.
+// without segment ids, a dense bias or a dropout mask.
 static bool spill_ranged(const AxlFlashBwdParams& p) {
   return p.mask_kind == AXL_MASK_SLIDING_WINDOW || p.segment_ids;
 }
 static bool spill_eligible(const AxlFlashBwdParams& p) {
   return (p.dtype == AXL_BF16 || p.dtype == AXL_F16) &&
          (p.mask_kind == AXL_MASK_CAUSAL || p.mask_kind == AXL_MASK_SLIDING_WINDOW) && p.q_pos_offset == 0 &&
-         p.q_len == p.kv_len && !p.aux.bias && !p.aux.dropout_mask && (p.flags & AXL_BWD_DS_WORKSPACE) &&
+         p.q_len == p.kv_len && (p.flags & AXL_BWD_DS_WORKSPACE) &&
          // the ranged kernel keeps the table in LDS beside its ring: 256-row blocks at head_dim 128
          (!spill_ranged(p) || (p.kv_len / 128 <= kMaxKbRanged && (p.head_dim <= 64 || p.q_len % 256 == 0)));
 }
@@ -530,7 +530,9 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       s.dv = (char*)a.dv + h0 * a.dvs.h * es;
       s.ndelta = a.ndelta + hq0 * p.q_len;
       s.lse2 = a.lse2 + hq0 * p.q_len;
-      if (phases & AXL_BWD_DKDV) err = launch_bwd_dkdv(s, dt, width, false, stream);
+      if (a.aux.bias) s.aux.bias = a.aux.bias + hq0 * a.aux.bias_sh;
+      if (a.aux.drop) s.aux.drop = a.aux.drop + hq0 * a.aux.drop_sh;
+      if (phases & AXL_BWD_DKDV) err = launch_bwd_dkdv(s, dt, width, aux, stream);
       if ((phases & AXL_BWD_DQ) && err == hipSuccess) err = launch_bwd_dq_stream(s, dt, width, stream);
     }
     phases &= AXL_BWD_DELTA;  // what is left for the code below: the sink gradient

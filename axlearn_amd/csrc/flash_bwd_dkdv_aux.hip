@@ -1,0 +1,30 @@
+// The dK / dV kernel's instantiations with a dense bias and / or a dropout mask: one per combination of the
+// two, with and without segment ids, leaving dS for the streaming dQ kernel or not.
+#include "flash_bwd_dkdv_kernel.h"
+
+namespace axl {
+
+template <typename E, int D, int AUX>
+static hipError_t launch_mode(const BwdArgs& a, hipStream_t stream) {
+  if (a.ds) return a.seg ? launch_one<E, D, true, AUX, true>(a, stream) : launch_one<E, D, false, AUX, true>(a, stream);
+  return a.seg ? launch_one<E, D, true, AUX>(a, stream) : launch_one<E, D, false, AUX>(a, stream);
+}
+
+template <typename E, int D>
+static hipError_t launch_for(const BwdArgs& a, hipStream_t stream) {
+  const int bias = a.aux.bias ? (a.aux.bias_f32 ? kAuxBias32 : kAuxBias16) : 0;
+  switch (bias | (a.aux.drop ? kAuxDrop : 0)) {
+    case kAuxBias16: return launch_mode<E, D, kAuxBias16>(a, stream);
+    case kAuxBias32: return launch_mode<E, D, kAuxBias32>(a, stream);
+    case kAuxDrop: return launch_mode<E, D, kAuxDrop>(a, stream);
+    case kAuxBias16 | kAuxDrop: return launch_mode<E, D, kAuxBias16 | kAuxDrop>(a, stream);
+    default: return launch_mode<E, D, kAuxBias32 | kAuxDrop>(a, stream);
+  }
+}
+
+hipError_t launch_bwd_dkdv_aux(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream) {
+  if (dtype == AXL_F16) return head_dim == 128 ? launch_for<ElemF16, 128>(a, stream) : launch_for<ElemF16, 64>(a, stream);
+  return head_dim == 128 ? launch_for<ElemBf16, 128>(a, stream) : launch_for<ElemBf16, 64>(a, stream);
+}
+
+}  // namespace axl

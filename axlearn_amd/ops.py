@@ -259,7 +259,7 @@ def flash_bwd(
     = (dq, dk, dv, workspace) reuses caller-provided outputs instead of allocating.  bias,
     dropout_mask and dropout_rate must be the ones the forward was given (the bias gets no gradient,
     as in gpu_attention.py:786).  `ds_workspace=True` (AXL_BWD_DS_WORKSPACE; causal or sliding-window
-    attention over equal lengths without offsets, bias or dropout; ignored otherwise) keeps dS in a
+    attention over equal lengths without offsets; ignored otherwise) keeps dS in a
     larger workspace instead of recomputing it for dq; with `ds_slice_kv_heads=n` the workspace holds
     the dS of n kv heads at a time and the two kernels run slice after slice
     (AXL_BWD_DS_SLICE_KV_HEADS).  `ds_workspace=None` decides by size (`select_ds_slice`): the dS
@@ -270,7 +270,7 @@ def flash_bwd(
     _check_segment_ids(segment_ids, b, t, s)
     if ds_workspace is None:
         ds_workspace, ds_slice_kv_heads = False, 0
-        if phases == 7 and bias is None and dropout_mask is None and q_pos_offset == 0:
+        if phases == 7 and q_pos_offset == 0:
             ds_workspace, ds_slice_kv_heads = select_ds_slice(q, k, mask_kind=mask_kind, segment_ids=segment_ids,
                                                               limit=ds_workspace_limit)
     _want_shape("out", out, q.shape)
@@ -340,7 +340,7 @@ def flash_bwd_buffers(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, mask
 
     The workspace holds delta and the scaled lse (fp32 [B,Hq,T] each); with `segment_ids` (the ones the
     calls will pass) also the table of id ranges per 32 rows; with `ds_workspace=True` and a causal or
-    sliding-window `mask_kind` (equal lengths, no offsets / bias / dropout) also dS, about T*S bytes per
+    sliding-window `mask_kind` (equal lengths, no offsets) also dS, about T*S bytes per
     (batch, head), for `flash_bwd(..., ds_workspace=True)` - of `ds_slice_kv_heads` kv heads at a time if that
     is given (the calls must pass the same number)."""
     b, t, hq, d = q.shape

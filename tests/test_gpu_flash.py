@@ -1391,3 +1391,30 @@ def test_chunk_of_rows_over_a_long_cache(b, rows, hq, hkv, d, kv_len, window, dt
     assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
     # outputs over thousands of keys are small: the relative bar alone, an eighth of it for f16
     assert ref.rel_l2(got[seen], want[seen]) < (1e-2 if dtype == torch.bfloat16 else 1.25e-3)
+
+
+@pytest.mark.parametrize("t,hq,hkv,d,mask,window,packed,bias_dtype,drop", [
+    (128, 2, 1, 64, "causal", None, False, torch.bfloat16, False),     # one row block, one key block
+    (384, 4, 2, 128, "causal", None, False, torch.float32, True),      # an odd number of key blocks
+    (512, 4, 2, 128, "causal", None, False, None, True),
+    (768, 6, 2, 128, "sliding", 200, True, torch.bfloat16, True),      # stored tiles by key block
+    (512, 4, 4, 64, "sliding", 96, False, torch.float32, False),
+])
+def test_ds_workspace_backward_with_bias_and_dropout(t, hq, hkv, d, mask, window, packed, bias_dtype, drop):
+    # dS kept in the workspace beside a dense bias per head and / or a dropout mask: dk and dv are the bits
+    # of the recomputing pair (the same arithmetic), dq the same products summed in another order; whole and
+    # one kv head at a time.
+    b = 2
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, torch.bfloat16))
+    g = torch.Generator().manual_seed(t)
+    seg = ref.packed_segment_ids(3, b, t) if packed else None
+    spec, kw = _mask_args(mask, window, seg)
+    bias = None if bias_dtype is None else torch.randn(1, hq, t, t, generator=g).to(bias_dtype).cuda()
+    mask_bytes = (torch.rand(b, hq, t, t, generator=g) < 0.2).cuda() if drop else None
+    kw.update(softmax_scale=d ** -0.5, bias=bias, dropout_mask=mask_bytes, dropout_rate=0.2 if drop else 0.0)
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    want = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=False, **kw)
+    for heads in (0, 1):
+        got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=True, ds_slice_kv_heads=heads, **kw)
+        assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
+        assert ref.rel_l2(got[0].cpu(), want[0].cpu()) < 4e-3   # both rounded to bf16 once: 2^-8 apart at most
