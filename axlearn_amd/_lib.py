@@ -18,6 +18,7 @@ LIB_PATH = os.path.join(_HERE, "libaxl_attn_hip.so")
 AXL_BF16, AXL_F32, AXL_F16 = 0, 1, 2
 MASK_NONE, MASK_CAUSAL, MASK_SLIDING_WINDOW = 0, 1, 2
 DECODE_DETERMINISTIC, DECODE_WORKSPACE_REUSED = 1, 2  # AXL_DECODE_* flags
+DECODE_LENGTHS_ARE_POSITIONS, DECODE_LENGTHS_I64 = 4, 8
 BWD_DS_WORKSPACE = 1  # AXL_BWD_DS_WORKSPACE
 AXL_OK, AXL_ERR_INVALID_ARGUMENT, AXL_ERR_UNSUPPORTED, AXL_ERR_WORKSPACE, AXL_ERR_LAUNCH = 0, -1, -2, -3, -4
 
@@ -127,6 +128,7 @@ class AxlPagedDecodeParams(ctypes.Structure):
         ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
         ("flags", ctypes.c_int32),
         ("bias", AxlDecodeBias),
+        ("lengths_stride", ctypes.c_int64),
     ]
 
 
@@ -142,6 +144,7 @@ class AxlDecodeParams(ctypes.Structure):
         ("workspace", ctypes.c_void_p), ("workspace_bytes", ctypes.c_size_t),
         ("flags", ctypes.c_int32),
         ("bias", AxlDecodeBias),
+        ("lengths_stride", ctypes.c_int64),
     ]
 
 

@@ -5,12 +5,15 @@
 // gpu_decoding.py:71-283 (`_attn_forward_kernel`, `_decode_attn_unbatched`).
 //
 // The operation is bound by HBM: every K and V byte of the live context is read exactly once.
-//   * split-K over the context in blocks of `chunk_pages` logical pages (16 tokens each) of one
-//     (sequence, kv head).  The split kernel is persistent (two workgroups of 4 wavefronts per CU):
-//     every workgroup derives the list of live blocks from the lengths and draws runs of
-//     consecutive blocks from a global counter, long runs first and single blocks at the end, so
-//     that blocks past a sequence's length cost nothing and CUs that are served faster by the
-//     memory system take more of the work;
+//   * split-K over the context, by one of two rules (DecArgs::even):
+//     calls whose context capacity gives a workgroup at most 256 tiles of 16 tokens: the live tiles of all
+//     (sequence, kv head) pairs form one list and every workgroup (two of 4 wavefronts per CU) takes an
+//     equal, contiguous share of it.  Nothing is drawn, so there is no counter, no kernel that zeroes it and
+//     no half-empty last round;
+//     other calls: blocks of `chunk_pages` tiles of one pair.  The split kernel is persistent: every workgroup derives the list of live blocks from the lengths and
+//     draws runs of consecutive blocks from a global counter, long runs first and single blocks at the
+//     end, so that blocks past a sequence's length cost nothing and CUs that are served faster by the
+//     memory system take more of the work (over the milliseconds of such a call that is worth 4 %);
 //   * K and V pages stream from HBM straight into a private LDS ring per wavefront
 //     (global_load_lds), so the bytes in flight cost no registers; a stage is refilled as soon as
 //     its fragments sit in registers.  The pages of a run are handed to the 4 wavefronts through a
@@ -25,7 +28,7 @@
 // Work is handed out by timing, so the grouping of the fp32 partial sums - not the set of keys -
 // can differ between two calls; the AXL_DECODE_DETERMINISTIC flag of the call (or
 // AXL_DECODE_DETERMINISTIC=1 in the environment, read once, as the default for every call) selects
-// a fixed decomposition (one block per record, pages dealt round-robin) whose result is
+// a fixed decomposition (equal shares, or one block per record; pages dealt round-robin) whose result is
 // reproducible bit for bit.
 // Keys at index >= length are masked (gpu_paged_attention.py:100, gpu_decoding.py:109); the query
 // position is length-1, so a sliding window w also masks keys with (length-1) - j > w.  A page
@@ -42,7 +45,9 @@ struct DecArgs {
   const __bf16* k;        // paged: [Hkv, P, page_size, D]; contiguous: [B, S, Hkv, D] (strided)
   const __bf16* v;
   const int32_t* page_tables;  // [B, pt_stride] (paged only)
-  const int32_t* lengths;      // [B]
+  const char* lengths;         // [B] at `len_stride` bytes: lengths, or positions of the query (len_add = 1)
+  int64_t len_stride;
+  int len_i64, len_add;        // int64 instead of int32; what to add to get the length
   __bf16* out;                 // [B, Hq, D]
   float* ws_o;                 // [records, GP, D]; at most B * Hkv * NCH records
   float* ws_m;                 // [records, GP]
@@ -67,7 +72,9 @@ struct DecArgs {
   int* ticket;                 // [0] blocks handed out: zero when the split kernel starts (zeroed by
                                // decode_plan_kernel, or left at zero by the previous call's combine kernel)
   int deterministic;           // fixed work decomposition: results reproducible bit for bit
-  int static_only;             // no more blocks than workgroups: block i goes to workgroup i, the counter is not used
+  int even;                    // equal shares of the live tiles instead of blocks (see the head of this file)
+  int n_wg;                    // ... over this many workgroups
+  int min_share;               // ... of at least this many tiles
 };
 
 // Tokens per tile: the unit the kernels stream and compute on.  A pool page of 16 << page_shift
@@ -99,21 +106,41 @@ __device__ __forceinline__ int v_swizzle(int row) {
   return 2 * ((row >> 1) & 3);
 }
 
+// Records per (sequence, kv head) pair: bounds the combine kernel's LDS tables.
+constexpr int kMaxChunks = 256;
+
 // Sequences per launch: bounds the work-item tables each workgroup keeps in LDS.
 constexpr int kMaxBatch = 512;
 
-// Live chunk range [ch0, ch1) of a sequence of length `len`.
-__device__ __forceinline__ void live_chunks(const DecArgs& a, int len, int& ch0, int& ch1) {
-  const int npages = min((len + kPage - 1) / kPage, a.pps);
-  const int first_page = a.window >= 0 ? max(0, len - 1 - a.window) / kPage : 0;
-  ch0 = first_page / a.chunk_pages;
-  ch1 = max(ch0, (npages + a.chunk_pages - 1) / a.chunk_pages);
+// Length of sequence b.  Lengths outside [0, capacity] are clamped: a sequence cannot hold more keys than
+// its page table (or its cache rows) can address, and a non-positive length is an empty context.
+__device__ __forceinline__ int length_of(const DecArgs& a, int b) {
+  const char* p = a.lengths + b * a.len_stride;
+  const int64_t len = (a.len_i64 ? *(const int64_t*)p : (int64_t)*(const int32_t*)p) + a.len_add;
+  return (int)max((int64_t)0, min(len, (int64_t)a.kv_len));
 }
 
-// Lengths outside [0, capacity] are clamped: a sequence cannot hold more keys than its page table
-// (or its cache rows) can address, and a non-positive length is an empty context.
-__device__ __forceinline__ int clamp_length(const DecArgs& a, int len) {
-  return max(0, min(len, a.kv_len));
+// Live tiles [t0, t1) of a sequence of length `len`.
+__device__ __forceinline__ void live_tiles(const DecArgs& a, int len, int& t0, int& t1) {
+  t0 = a.window >= 0 ? max(0, len - 1 - a.window) / kPage : 0;
+  t1 = max(t0, min((len + kPage - 1) / kPage, a.pps));
+}
+// Live units of work [u0, u1) of a sequence, a unit being `unit` tiles (numbered from the first of the cache).
+__device__ __forceinline__ void live_units(const DecArgs& a, int len, int unit, int& u0, int& u1) {
+  int t0, t1;
+  live_tiles(a, len, t0, t1);
+  u0 = t0 / unit;
+  u1 = max(u0, (t1 + unit - 1) / unit);
+}
+// Equal shares (DecArgs::even): the unit and the units per workgroup, from the call's live blocks and tiles.
+// No more blocks than workgroups: a block each, the decomposition of AXL_DECODE_DETERMINISTIC.  Otherwise
+// tiles, in whole rounds of the 4 wavefronts.
+struct EvenPlan {
+  int unit, share;
+};
+__device__ __forceinline__ EvenPlan even_plan(const DecArgs& a, int blocks, int tiles) {
+  if (blocks <= a.n_wg) return EvenPlan{a.chunk_pages, 1};
+  return EvenPlan{1, max(a.min_share, ((tiles + a.n_wg - 1) / a.n_wg + 3) & ~3)};
 }
 
 template <int D, int GP, int NST>
@@ -158,33 +185,56 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   // ---- every workgroup builds the same exclusive prefix of live-block counts over the batch.
   int* pfx = (int*)(smem + Tile::PFX_BASE);
   int* lens = (int*)(smem + Tile::LEN_BASE);
+  int unit = a.chunk_pages, share = 0;
   {
     constexpr int PER = kMaxBatch / 256;  // consecutive sequences per thread
-    int cnt[PER], tsum = 0;
+    int cnt[PER], cnt_t[PER], tsum = 0, tsum_t = 0;   // live blocks, live tiles
 #pragma unroll
     for (int i = 0; i < PER; i++) {
       const int bi = tid * PER + i;
-      int n = 0;
+      int n = 0, nt = 0;
       if (bi < a.B) {
-        const int l = clamp_length(a, a.lengths[bi]);
+        const int l = length_of(a, bi);
         lens[bi] = l;
-        int c0, c1;
-        live_chunks(a, l, c0, c1);
-        n = c1 - c0;
+        int u0, u1;
+        live_units(a, l, a.chunk_pages, u0, u1);
+        n = u1 - u0;
+        live_tiles(a, l, u0, u1);
+        nt = u1 - u0;
       }
       cnt[i] = n;
+      cnt_t[i] = nt;
       tsum += n;
+      tsum_t += nt;
     }
-    int incl = tsum;  // inclusive scan over the wavefront
+    int incl = tsum, incl_t = tsum_t;  // inclusive scans over the wavefront
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-      const int up = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += up;
+      const int up = __shfl_up(incl, d, 64), up_t = __shfl_up(incl_t, d, 64);
+      if (lane >= d) {
+        incl += up;
+        incl_t += up_t;
+      }
     }
     int* wsum = (int*)(smem + Tile::RED_BASE);
-    if (lane == 63) wsum[wave] = incl;
+    if (lane == 63) {
+      wsum[wave] = incl;
+      wsum[4 + wave] = incl_t;
+    }
     __syncthreads();
     int run = incl - tsum;
+    if (a.even) {
+      const EvenPlan p = even_plan(a, (wsum[0] + wsum[1] + wsum[2] + wsum[3]) * a.Hv,
+                                   (wsum[4] + wsum[5] + wsum[6] + wsum[7]) * a.Hv);
+      unit = p.unit;
+      share = p.share;
+      if (unit == 1) {
+        run = incl_t - tsum_t;
+        wsum += 4;
+#pragma unroll
+        for (int i = 0; i < PER; i++) cnt[i] = cnt_t[i];
+      }
+    }
     for (int w = 0; w < wave; w++) run += wsum[w];
 #pragma unroll
     for (int i = 0; i < PER; i++) {
@@ -206,7 +256,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   // The ids of at most 256 pages are kept in registers.  A fixed decomposition (one block per
   // record, pages dealt round-robin) makes the result independent of timing.
   const int max_run = a.deterministic ? 1 : max(1, 256 / a.chunk_pages);
-  const int run0 = min(max_run, max(1, n_blocks / (2 * n_wg)));
+  const int run0 = a.even ? share : min(max_run, max(1, n_blocks / (2 * n_wg)));
   int* s_next = (int*)(smem + Tile::NEXT_BASE);
   int* s_page = s_next + 3;  // next page of the segment to hand to a wavefront
   if (tid == 0) *s_page = 4 * NST;
@@ -225,7 +275,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   }
   const int len = lens[b];
   int ch0, ch1;
-  live_chunks(a, len, ch0, ch1);
+  live_units(a, len, unit, ch0, ch1);
   const int rem = run_e - pfx[b] * a.Hv;
   const int hv = rem / (ch1 - ch0), cl = rem % (ch1 - ch0);
   // Virtual head -> kv head and group of (at most) 16 of its query heads.
@@ -234,10 +284,9 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   const int gcount = min(16, a.G - 16 * grp);
   const int hbase = hk * a.G + 16 * grp;
   const int seg = min(run_end - run_e, ch1 - ch0 - cl);
-  int first_page = 0;
-  if (a.window >= 0) first_page = max(0, (len - 1 - a.window)) / kPage;
-  const int c_begin = max((ch0 + cl) * a.chunk_pages, first_page);
-  const int c_end = min((ch0 + cl + seg) * a.chunk_pages, min((len + kPage - 1) / kPage, a.pps));
+  int t0, t1;
+  live_tiles(a, len, t0, t1);
+  const int c_begin = max((ch0 + cl) * unit, t0), c_end = min((ch0 + cl + seg) * unit, t1);
   // Pages of the segment are numbered 0 .. n_pg-1.  A wavefront starts with pages wave + 4*i,
   // i < NST, and draws further ones from a counter in LDS whenever a ring stage frees up, so that
   // the 4 wavefronts finish together however unevenly the memory system serves them.
@@ -245,11 +294,14 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
 
   // Draw the next run; the round trip overlaps the loads of Q and of the page ids below.  The
   // segment's record slot is the number of its first block: unique, and below the B * Hkv * NCH
-  // records the workspace holds.
-  const int rec = run_e;
+  // records the workspace holds.  With equal shares it is workgroup + pair: from one segment of the list
+  // to the next one of the two or both go up, so it is unique too, and the records of a pair lie side
+  // by side in context order.
+  const int rec = a.even ? (int)blockIdx.x + b * a.Hv + hv : run_e;
+  const bool whole = a.even && seg == ch1 - ch0;   // all of the pair's keys: the result, not a record
   if (tid == 0 && first_segment) {
     next_n = min(max_run, max(1, (n_blocks - handed) / (4 * n_wg)));
-    next_e = a.static_only ? n_blocks : atomicAdd(&a.ticket[0], next_n);
+    next_e = a.even ? n_blocks : atomicAdd(&a.ticket[0], next_n);
   }
   first_segment = false;
 
@@ -487,11 +539,28 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   __syncthreads();
   const int64_t slot = rec;
   float* out_ws = a.ws_o + slot * (GP * D);
-  for (int idx = tid; idx < GP * D; idx += 256) {
-    const int gq = idx / D, d = idx % D;
-    out_ws[idx] = red_o[gq][d] + red_o[GP + gq][d] + red_o[2 * GP + gq][d] + red_o[3 * GP + gq][d];
+  if (whole) {
+    for (int idx = tid; idx < GP * D / 2; idx += 256) {
+      const int gq = 2 * idx / D, d = 2 * idx % D;
+      if (gq >= gcount || d >= a.d_real) continue;
+      const float mw = fmaxf(fmaxf(red_m[0][gq], red_m[1][gq]), fmaxf(red_m[2][gq], red_m[3][gq]));
+      float lw = 0.f;
+#pragma unroll
+      for (int w = 0; w < 4; w++) lw += red_l[w][gq] * fast_exp2((red_m[w][gq] - mw) * c);
+      const float inv = lw > 0.f ? 1.f / lw : 0.f;
+      float x[2];
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+        x[j] = (red_o[gq][d + j] + red_o[GP + gq][d + j] + red_o[2 * GP + gq][d + j] + red_o[3 * GP + gq][d + j]) * inv;
+      *(bf16x2*)(a.out + ((int64_t)b * a.Hq + hbase + gq) * a.d_real + d) = E::pack(x[0], x[1]);
+    }
+  } else {
+    for (int idx = tid; idx < GP * D; idx += 256) {
+      const int gq = idx / D, d = idx % D;
+      out_ws[idx] = red_o[gq][d] + red_o[GP + gq][d] + red_o[2 * GP + gq][d] + red_o[3 * GP + gq][d];
+    }
   }
-  if (tid < GP) {
+  if (!whole && tid < GP) {
     const float mw = fmaxf(fmaxf(red_m[0][tid], red_m[1][tid]), fmaxf(red_m[2][tid], red_m[3][tid]));
     float lw = 0.f;
 #pragma unroll
@@ -500,7 +569,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
     a.ws_l[slot * GP + tid] = lw;
   }
   // Table entries of the segment's chunks: the record at its first chunk, "none" at the others.
-  for (int i = tid; i < seg; i += 256) a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + cl + i] = i == 0 ? (int)slot : -1;
+  for (int i = tid; i < seg && !a.even; i += 256) a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + cl + i] = i == 0 ? (int)slot : -1;
   if (tid == 0) *s_page = 4 * NST;
   __syncthreads();  // the ring (and red_m/red_l) are reused by the next segment
   run_e += seg;
@@ -523,7 +592,6 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int* ticket) {
 
 // Merges the per-chunk partials of one (sequence, kv head): the "final round of flash"
 // (gpu_paged_attention.py:287-296, gpu_decoding.py:277-283).
-constexpr int kMaxChunks = 256;  // per sequence; bounds the combine kernel's LDS tables
 
 template <typename E, int D, int GP>
 __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
@@ -539,13 +607,51 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
   const int gcount = min(16, a.G - 16 * grp);   // query heads of this group
   const int hbase = hk * a.G + 16 * grp;
   const int tid = threadIdx.x;
-  const int len = clamp_length(a, a.lengths[b]);
+  const int len = length_of(a, b);
   int ch0, ch1;
-  live_chunks(a, len, ch0, ch1);
-  const int nc = ch1 - ch0;               // live chunks = upper bound on records of this (b, hk)
+  live_units(a, len, a.chunk_pages, ch0, ch1);
+  int nc = ch1 - ch0;                     // live chunks = upper bound on records of this (b, hk)
   // The split kernel has finished: leave the work counter at zero for the next call on this workspace.
   if (hv == 0 && b == 0 && tid == 0) a.ticket[0] = 0;
   const float c = a.scale * kLog2e;
+  if (a.even) {
+    // Where the pair's units lie in the list says which workgroups took them.
+    int before[2] = {0, 0}, all[2] = {0, 0};   // of blocks, of tiles
+    for (int i = tid; i < a.B; i += 256) {
+      const int l = length_of(a, i);
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        int u0, u1;
+        live_units(a, l, k == 0 ? a.chunk_pages : 1, u0, u1);
+        all[k] += u1 - u0;
+        before[k] += i < b ? u1 - u0 : 0;
+      }
+    }
+    __shared__ int s_sum[4][4];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+#pragma unroll
+      for (int o = 32; o > 0; o >>= 1) {
+        before[k] += __shfl_xor(before[k], o);
+        all[k] += __shfl_xor(all[k], o);
+      }
+      if ((tid & 63) == 0) {
+        s_sum[k][tid >> 6] = before[k];
+        s_sum[2 + k][tid >> 6] = all[k];
+      }
+    }
+    __syncthreads();
+    auto sum4 = [&](int k) { return s_sum[k][0] + s_sum[k][1] + s_sum[k][2] + s_sum[k][3]; };
+    const EvenPlan p = even_plan(a, sum4(2) * a.Hv, sum4(3) * a.Hv);
+    live_units(a, len, p.unit, ch0, ch1);
+    nc = ch1 - ch0;
+    const int first = sum4(p.unit == 1 ? 1 : 0) * a.Hv + hv * nc;
+    const int w0 = first / p.share, w1 = nc > 0 ? (first + nc - 1) / p.share : w0 - 1;
+    if (w0 == w1) return;                 // one workgroup had all of it and stored the result
+    const int n = min(w1 - w0 + 1, kMaxChunks);
+    if (tid < n) s_list[tid] = w0 + tid + b * a.Hv + hv;
+    if (tid == 0) s_count = n;
+  } else {
   // The whole table row in one round trip, then compacted in chunk order by one wavefront.
   s_raw[tid] = tid < nc ? a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + tid] : -1;
   __syncthreads();
@@ -558,6 +664,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
       count += __builtin_popcountll(mask);
     }
     if (tid == 0) s_count = count;
+  }
   }
   __syncthreads();
   const int nl = s_count;
@@ -647,9 +754,9 @@ __global__ __launch_bounds__(256) void decode_split_f32_kernel(const DecArgs a) 
   const int gcount = min(16, a.G - 16 * grp);   // query heads of this group
   const int hbase = hk * a.G + 16 * grp;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, sub = lane >> 4, l16 = lane & 15;
-  const int len = clamp_length(a, a.lengths[b]);
+  const int len = length_of(a, b);
   int ch0, ch1;
-  live_chunks(a, len, ch0, ch1);
+  live_units(a, len, a.chunk_pages, ch0, ch1);
   if (ch0 + c >= ch1) return;
   const int npages = min((len + kPage - 1) / kPage, a.pps);
   const int first_page = a.window >= 0 ? max(0, len - 1 - a.window) / kPage : 0;
@@ -804,23 +911,65 @@ static int page_shift_of(int page_size) {
   return -1;
 }
 
-static size_t ws_bytes_for(int batch, int hq, int hkv, int d, int tiles, bool bias) {
+// Tiles of a (sequence, kv head) pair that a call can have to read, from its shapes.
+static int64_t capacity_tiles(int tiles, int window) {
+  const int64_t w = window >= 0 ? (int64_t)window / kPage + 2 : tiles;
+  return w < tiles ? w : tiles;
+}
+
+// Equal shares (see the head of this file) where the capacity makes them at most 256 tiles, the page ids a
+// segment keeps in registers.  Measured at 8 sequences of 2000 to 8190 tokens, 8 kv heads (40 tiles a
+// workgroup): split kernel 42.8 us drawing blocks of 32 tiles (640 blocks for 512 workgroups), 39.6 us in
+// equal shares, and the call is two launches instead of three; at 64 sequences of up to 32768 tokens (1024
+// tiles a workgroup) drawing is 4 % faster.  Fills in the launch's part of `a`; a.B, a.Hv, a.pps, a.window
+// and a.nch are set.
+static void plan_even(DecArgs& a, bool deterministic) {
+  const int64_t pair = capacity_tiles(a.pps, a.window), total = pair * a.B * a.Hv;
+  const int slots = 2 * cu_count();
+  // at least 8 tiles (one round of the wavefronts' rings: a shorter share ends no sooner), and few enough
+  // records per pair for the tables of the combine kernel
+  const int64_t by_table = (pair + kMaxChunks - 2) / (kMaxChunks - 1);
+  a.min_share = (int)((by_table > 8 ? by_table : 8) + 3) & ~3;
+  a.n_wg = (int)(total < (int64_t)slots * a.min_share ? (total + a.min_share - 1) / a.min_share : slots);
+  const int64_t share = ((total + a.n_wg - 1) / a.n_wg + 3) & ~(int64_t)3;
+  a.even = a.B <= kMaxBatch && share <= 256 && a.min_share <= 256;
+  // A deterministic call keeps to the blocks, whose bits depend on a pair's own keys alone: equal shares only
+  // where the shapes leave no more blocks than workgroups.
+  if (deterministic && (int64_t)a.B * a.Hv * a.nch > a.n_wg) a.even = 0;
+}
+
+static size_t ws_bytes_for(int batch, int hq, int hkv, int d, int tiles, bool bias, int dtype) {
   const int G = hq / hkv;
   const int cp = pick_chunk_pages(tiles, (int64_t)batch * hkv * groups_of(G));
   const int nch = (tiles + cp - 1) / cp;
-  return ws_bytes(batch, hkv * groups_of(G), nch, gp_of(G, bias), width_of(d));
+  const size_t drawn = ws_bytes(batch, hkv * groups_of(G), nch, gp_of(G, bias), width_of(d));
+  if (dtype == AXL_F32 || batch > kMaxBatch) return drawn;
+  // Equal shares: one record per workgroup and pair at most.  The size does not depend on the window (a query
+  // may leave it out): with one there are no more tiles, in shares of 8 or more.
+  const int64_t pairs = (int64_t)batch * hkv * groups_of(G), wgs = (pairs * tiles + 7) / 8, slots = 2 * (int64_t)cu_count();
+  const size_t even = ws_bytes(1, 1, (int)((wgs < slots ? wgs : slots) + pairs), gp_of(G, bias), width_of(d));
+  return even > drawn ? even : drawn;
 }
 
 size_t paged_decode_workspace_bytes(const AxlPagedDecodeParams& p) {
   const int sh = page_shift_of(p.page_size);
   if (p.pages_per_seq <= 0 || p.num_kv_heads <= 0 || p.num_q_heads < p.num_kv_heads || sh < 0) return 0;
-  return ws_bytes_for(p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.pages_per_seq << sh, p.bias.bias != nullptr);
+  return ws_bytes_for(p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, p.pages_per_seq << sh, p.bias.bias != nullptr,
+                      p.dtype);
 }
 
 size_t decode_workspace_bytes(const AxlDecodeParams& p) {
   if (p.kv_len <= 0 || p.num_kv_heads <= 0 || p.num_q_heads < p.num_kv_heads) return 0;
   return ws_bytes_for(p.batch, p.num_q_heads, p.num_kv_heads, p.head_dim, (p.kv_len + kPage - 1) / kPage,
-                      p.bias.bias != nullptr);
+                      p.bias.bias != nullptr, p.dtype);
+}
+
+static void set_lengths(DecArgs& a, const int32_t* lengths, int64_t stride, int flags) {
+  a.lengths = (const char*)lengths;
+  a.len_i64 = (flags & AXL_DECODE_LENGTHS_I64) != 0;
+  a.len_add = (flags & AXL_DECODE_LENGTHS_ARE_POSITIONS) != 0;
+  const bool strided = a.len_i64 || a.len_add;
+  a.len_stride = (strided ? stride : 1) * (a.len_i64 ? 8 : 4);
 }
 
 static void set_bias(DecArgs& a, const AxlDecodeBias& x, float scale) {
@@ -857,19 +1006,17 @@ static int launch_common(DecArgs a, int flags, hipStream_t stream, const char* w
   a.ticket = (int*)a.ws_o;
   a.ws_o += kWsHeaderFloats;
   float* ws = a.ws_o;
-  const size_t n_o = (size_t)a.B * a.Hv * a.nch * gp * D;
-  const size_t n_s = (size_t)a.B * a.Hv * a.nch * gp;
+  a.deterministic = (flags & AXL_DECODE_DETERMINISTIC) != 0 || deterministic_by_default();
+  plan_even(a, a.deterministic);
+  const size_t records = a.even ? (size_t)a.n_wg + (size_t)a.B * a.Hv : (size_t)a.B * a.Hv * a.nch;
+  const size_t n_o = records * gp * D, n_s = records * gp;
   a.ws_m = ws + n_o;
   a.ws_l = ws + n_o + n_s;
   a.ws_tab = (int32_t*)(ws + n_o + 2 * n_s);
-  a.deterministic = (flags & AXL_DECODE_DETERMINISTIC) != 0 || deterministic_by_default();
   // Two workgroups fit a CU (LDS); the split kernel is persistent and strides over its work items.
-  const dim3 grid(2 * cu_count());
+  const dim3 grid(a.even ? a.n_wg : 2 * cu_count());
   hipError_t err = hipSuccess;
-  // With at most one block per workgroup (a bound the shapes give: the lengths live on the device) the
-  // blocks are dealt by workgroup index and the counter is neither read nor zeroed.
-  a.static_only = (int64_t)(a.B < kMaxBatch ? a.B : kMaxBatch) * a.Hv * a.nch <= (int64_t)grid.x;
-  if (!(flags & AXL_DECODE_WORKSPACE_REUSED) && !a.static_only)
+  if (!(flags & AXL_DECODE_WORKSPACE_REUSED) && !a.even)
     hipLaunchKernelGGL(decode_plan_kernel, dim3(1), dim3(64), 0, stream, a.ticket);
 #define AXL_DEC(E, DD, GG, NS, BB)                                                              \
   do {                                                                                          \
@@ -888,7 +1035,7 @@ static int launch_common(DecArgs a, int flags, hipStream_t stream, const char* w
     s.B = a.B - b0 < kMaxBatch ? a.B - b0 : kMaxBatch;
     s.q = a.q + (size_t)b0 * a.Hq * a.d_real;
     s.out = a.out + (size_t)b0 * a.Hq * a.d_real;
-    s.lengths = a.lengths + b0;
+    s.lengths = a.lengths + b0 * a.len_stride;
     if (PAGED) s.page_tables = a.page_tables + (size_t)b0 * a.pt_stride;
     else { s.k = a.k + b0 * a.ks.b; s.v = a.v + b0 * a.vs.b; }
     if (bias) s.bias = a.bias + b0 * a.bias_sb;
@@ -956,7 +1103,8 @@ static int launch_f32(DecArgs a, hipStream_t stream, const char* who) {
 int launch_paged_decode(const AxlPagedDecodeParams& p, hipStream_t stream) {
   DecArgs a{};
   a.q = (const __bf16*)p.q; a.k = (const __bf16*)p.k_pages; a.v = (const __bf16*)p.v_pages;
-  a.page_tables = p.page_tables; a.lengths = p.lengths; a.out = (__bf16*)p.out;
+  a.page_tables = p.page_tables; a.out = (__bf16*)p.out;
+  set_lengths(a, p.lengths, p.lengths_stride, p.flags);
   a.ws_o = (float*)p.workspace;
   a.B = p.batch; a.Hq = p.num_q_heads; a.Hkv = p.num_kv_heads; a.G = p.num_q_heads / p.num_kv_heads;
   a.page_shift = page_shift_of(p.page_size);   // the entry point has checked the page size
@@ -1024,7 +1172,8 @@ int launch_paged_decode_static(const AxlPagedDecodeParams& p, hipStream_t stream
 int launch_decode(const AxlDecodeParams& p, hipStream_t stream) {
   DecArgs a{};
   a.q = (const __bf16*)p.q; a.k = (const __bf16*)p.k; a.v = (const __bf16*)p.v;
-  a.page_tables = nullptr; a.lengths = p.lengths; a.out = (__bf16*)p.out;
+  a.page_tables = nullptr; a.out = (__bf16*)p.out;
+  set_lengths(a, p.lengths, p.lengths_stride, p.flags);
   a.ws_o = (float*)p.workspace;
   a.ks = Strides3{p.k_strides.batch, p.k_strides.seq, p.k_strides.head};
   a.vs = Strides3{p.v_strides.batch, p.v_strides.seq, p.v_strides.head};

@@ -50,14 +50,18 @@ def _decode_window(mask: BaseAttentionBias) -> Optional[int]:
     return -1 if kind[0] == ops.MASK_CAUSAL else kind[1]
 
 
-def _lengths(mask: MaskFnAttentionBias, batch_size: int, device) -> Tensor:
+def _positions(mask: MaskFnAttentionBias, batch_size: int, device) -> Tensor:
+    """[batch_size] position of each sequence's query token: a view of the bias's own tensor where that is
+    on the GPU (the kernels take either integer type and any stride, so nothing is launched for it)."""
     if mask is None or getattr(mask, "target_positions", None) is None:
         raise ValueError("Cannot retrieve MaskFnAttentionBias or target_positions.")
-    lengths = (mask.target_positions[:, -1] + 1).to(device=device, dtype=torch.int32)
-    return lengths.expand(batch_size).contiguous()
+    positions = mask.target_positions[:, -1]
+    if positions.device != device or positions.dtype not in (torch.int32, torch.int64):
+        positions = positions.to(device=device, dtype=torch.int32)
+    return positions.expand(batch_size)
 
 
-def _mask_and_bias(input_batch: Nested, lengths: Tensor, kv_len: int) -> Tuple[int, Optional[Tensor]]:
+def _mask_and_bias(input_batch: Nested, positions: Tensor, kv_len: int) -> Tuple[int, Optional[Tensor]]:
     """(sliding window for the kernel or -1, bias `[B|1, Hq|1, kv_len]` or None) of a decode call."""
     mask, explicit_bias = split(input_batch["bias"], MaskFnAttentionBias)
     query = input_batch["query"]
@@ -70,9 +74,9 @@ def _mask_and_bias(input_batch: Nested, lengths: Tensor, kv_len: int) -> Tuple[i
     window = _decode_window(mask)
     if window is None:
         # mask_fn(kv_len - 1, indices), per sequence (gpu_decoding.py:110): a row of 0 / NEG_INF.
-        qpos = (lengths.to(torch.int64) - 1)[:, None]
+        qpos = positions.to(torch.int64)[:, None]
         kpos = torch.arange(kv_len, device=query.device)[None, :]
-        keep = torch.as_tensor(mask.mask(qpos, kpos), device=query.device).expand(lengths.shape[0], kv_len)
+        keep = torch.as_tensor(mask.mask(qpos, kpos), device=query.device).expand(positions.shape[0], kv_len)
         row = torch.where(keep, 0.0, NEG_INF).to(torch.float32)[:, None, :]
         bias = row if bias is None else bias.to(torch.float32) + row
         window = -1
@@ -119,11 +123,12 @@ class HipDecoding(BaseSingleStepDecoding):
         query, key, value = input_batch["query"], input_batch["key"], input_batch["value"]
         mask, _ = split(input_batch["bias"], MaskFnAttentionBias)
         batch_size, _, q_heads, head_dim = query.shape
-        lengths = _lengths(mask, batch_size, query.device)
-        window, bias = _mask_and_bias(input_batch, lengths, key.shape[1])
+        positions = _positions(mask, batch_size, query.device)
+        window, bias = _mask_and_bias(input_batch, positions, key.shape[1])
         out = ops.decode(
             query.reshape(batch_size, q_heads, head_dim), _as_query_dtype(key, query), _as_query_dtype(value, query),
-            lengths, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window, bias=bias,
+            positions, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window, bias=bias,
+            lengths_are_positions=True,
         )
         return out.reshape(batch_size, 1, q_heads, head_dim)
 
@@ -153,11 +158,11 @@ class HipPagedAttention(BasePagedAttention):
         page_tables = input_batch["page_tables"]
         mask, _ = split(input_batch["bias"], MaskFnAttentionBias)
         batch_size, _, q_heads, head_dim = query.shape
-        lengths = _lengths(mask, batch_size, query.device)
-        window, bias = _mask_and_bias(input_batch, lengths, key.shape[2] * page_tables.shape[1])
+        positions = _positions(mask, batch_size, query.device)
+        window, bias = _mask_and_bias(input_batch, positions, key.shape[2] * page_tables.shape[1])
         out = ops.paged_decode(
             query.reshape(batch_size, q_heads, head_dim), _as_query_dtype(key, query), _as_query_dtype(value, query),
-            page_tables.contiguous(), lengths, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window,
-            bias=bias,
+            page_tables.contiguous(), positions, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window,
+            bias=bias, lengths_are_positions=True,
         )
         return out.reshape(batch_size, 1, q_heads, head_dim)

@@ -408,8 +408,19 @@ def select_ds_workspace(q: torch.Tensor, k: torch.Tensor, *, mask_kind: int,
     return select_ds_slice(q, k, mask_kind=mask_kind, segment_ids=segment_ids, limit=limit)[0]
 
 
-def _decode_flags(deterministic: bool, workspace_reused: bool) -> int:
-    return (_lib.DECODE_DETERMINISTIC if deterministic else 0) | (_lib.DECODE_WORKSPACE_REUSED if workspace_reused else 0)
+def _decode_flags(deterministic: bool, workspace_reused: bool, lengths: torch.Tensor, are_positions: bool) -> int:
+    return ((_lib.DECODE_DETERMINISTIC if deterministic else 0) | (_lib.DECODE_WORKSPACE_REUSED if workspace_reused else 0)
+            | (_lib.DECODE_LENGTHS_ARE_POSITIONS if are_positions else 0)
+            | (_lib.DECODE_LENGTHS_I64 if lengths.dtype == torch.int64 else 0))
+
+
+def _check_lengths(lengths: torch.Tensor, b: int, are_positions: bool) -> None:
+    _want_shape("lengths", lengths, (b,))
+    if are_positions:
+        if lengths.dtype not in (torch.int32, torch.int64) or lengths.stride(0) < 0:
+            raise _bad("positions must be int32 or int64")
+    elif lengths.dtype != torch.int32:
+        raise _bad("lengths must be int32")
 
 
 def _check_decode_out_ws(q, out, workspace):
@@ -453,13 +464,15 @@ def paged_decode(
     deterministic: bool = False,
     workspace_reused: bool = False,
     bias: Optional[torch.Tensor] = None,
+    lengths_are_positions: bool = False,
 ) -> torch.Tensor:
     """q [B,Hq,D]; pools [Hkv,P,page,D]; page_tables [B,pps] int32; lengths [B] int32 -> [B,Hq,D].
 
     Lengths are clamped to [0, pps * page]; a sequence of length 0 yields zeros.  `deterministic`
     fixes the work decomposition (bit-reproducible); `workspace_reused` promises that `workspace` was
     last touched by an earlier decode call (skips the launch that zeroes its work counter).
-    bias [B|1,Hq|1,pps*page] bf16/fp32: additive logit bias per key position."""
+    bias [B|1,Hq|1,pps*page] bf16/fp32: additive logit bias per key position.  `lengths_are_positions`:
+    `lengths` holds positions of the query tokens (length - 1), int32 or int64, with any stride."""
     if q.dim() != 3 or k_pages.dim() != 4:
         raise _bad(f"q must be [B,Hq,D] and k_pages [Hkv,P,page,D], got {list(q.shape)}, {list(k_pages.shape)}")
     b, hq, d = q.shape
@@ -471,13 +484,13 @@ def paged_decode(
         raise _bad(f"num_q_heads {hq} is not divisible by num_kv_heads {hkv}")
     if page_tables.dim() != 2 or page_tables.shape[0] != b:
         raise _bad(f"page_tables must be [{b}, pages_per_seq], got {list(page_tables.shape)}")
-    _want_shape("lengths", lengths, (b,))
-    if page_tables.dtype != torch.int32 or lengths.dtype != torch.int32:
+    _check_lengths(lengths, b, lengths_are_positions)
+    if page_tables.dtype != torch.int32:
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "page_tables and lengths must be int32")
     if k_pages.dtype != q.dtype or v_pages.dtype != q.dtype:
         raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "q and the pools must share one dtype")
     for name, x in (("q", q), ("k_pages", k_pages), ("v_pages", v_pages), ("page_tables", page_tables), ("lengths", lengths)):
-        if not x.is_contiguous():
+        if not x.is_contiguous() and not (name == "lengths" and lengths_are_positions):
             raise AxlError(_lib.AXL_ERR_UNSUPPORTED, f"{name} must be contiguous")
     _check_decode_out_ws(q, out, workspace)
     if workspace_reused and workspace is None:
@@ -494,7 +507,8 @@ def paged_decode(
         page_size=page_size, pages_per_seq=page_tables.shape[1],
         dtype=_lib.dtype_code(q.dtype), sliding_window=int(sliding_window),
         softmax_scale=float(softmax_scale), workspace=None, workspace_bytes=0,
-        flags=_decode_flags(deterministic, workspace_reused), bias=bias_blk,
+        flags=_decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), bias=bias_blk,
+        lengths_stride=lengths.stride(0),
     )
     need = int(lib.axl_paged_decode_workspace_bytes(ctypes.byref(p)))
     if workspace is None or workspace.numel() < need:
@@ -533,10 +547,11 @@ def decode(
     deterministic: bool = False,
     workspace_reused: bool = False,
     bias: Optional[torch.Tensor] = None,
+    lengths_are_positions: bool = False,
 ) -> torch.Tensor:
     """q [B,Hq,D]; k/v [B,S,Hkv,D]; lengths [B] int32 -> [B,Hq,D].  Lengths are clamped to [0, S]; a
     sequence of length 0 yields zeros.  `deterministic` / `workspace_reused`: see `paged_decode`.
-    bias [B|1,Hq|1,S] bf16/fp32: additive logit bias per key position."""
+    bias [B|1,Hq|1,S] bf16/fp32: additive logit bias per key position.  `lengths_are_positions`: as there."""
     if q.dim() != 3 or k.dim() != 4:
         raise _bad(f"q must be [B,Hq,D] and k [B,S,Hkv,D], got {list(q.shape)}, {list(k.shape)}")
     b, hq, d = q.shape
@@ -546,12 +561,12 @@ def decode(
     _want_shape("v", v, k.shape)
     if hkv <= 0 or hq % hkv != 0:
         raise _bad(f"num_q_heads {hq} is not divisible by num_kv_heads {hkv}")
-    _want_shape("lengths", lengths, (b,))
+    _check_lengths(lengths, b, lengths_are_positions)
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "q, k, v must share one dtype")
     if not q.is_contiguous():
         raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "q must be contiguous")
-    if lengths.dtype != torch.int32 or not lengths.is_contiguous():
+    if not lengths_are_positions and not lengths.is_contiguous():
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "lengths must be contiguous int32")
     _check_decode_out_ws(q, out, workspace)
     if workspace_reused and workspace is None:
@@ -567,7 +582,8 @@ def decode(
         batch=b, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
         dtype=_lib.dtype_code(q.dtype), sliding_window=int(sliding_window),
         softmax_scale=float(softmax_scale), workspace=None, workspace_bytes=0,
-        flags=_decode_flags(deterministic, workspace_reused), bias=bias_blk,
+        flags=_decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), bias=bias_blk,
+        lengths_stride=lengths.stride(0),
     )
     need = int(lib.axl_decode_workspace_bytes(ctypes.byref(p)))
     if workspace is None or workspace.numel() < need:

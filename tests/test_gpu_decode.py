@@ -828,3 +828,30 @@ def test_decode_kv_dtype_other_than_the_query_dtype(q_dtype, kv_dtype):
                                           kv_cache_type=KVCache)
     assert impl is not None and isinstance(impl.fn, HipDecoding)
     assert _bar(impl.fn(dict(query=q.cuda(), key=kk, value=vv, bias=bias)).cpu(), want, q_dtype)
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,pps,window", [
+    (1, 8, 1, 128, 4096, -1),      # one pair over all workgroups, its records bounded by the merge's tables
+    (8, 8, 8, 64, 512, -1),        # more blocks than workgroups: tile shares that straddle pairs and sequences
+    (40, 16, 16, 64, 60, -1),      # shares longer than most pairs: whole pairs stored without a record
+    (16, 32, 8, 128, 260, 3000),   # a window that starts inside a tile
+    (512, 4, 4, 64, 20, -1),       # the most sequences one launch takes
+])
+def test_decode_in_equal_shares(b, hq, hkv, d, pps, window):
+    # Calls whose capacity gives a workgroup at most 256 tiles divide the live tiles evenly: lengths of 0, 1,
+    # a tile and the capacity among random ones; the bits of the lengths read as positions in either
+    # integer type (int64 with a stride), and the oracle within the bar.
+    q, kp, vp, tables, lengths = ref.paged_inputs(31, batch=b, num_heads=hq, num_kv_heads=hkv, head_dim=d, page_size=16,
+                                                  pages_per_seq=pps, min_len=1, max_len=16 * pps)
+    for i, n in enumerate((16 * pps, 0, 1, 16, 17)):
+        if i < b and b > 1:
+            lengths[i] = n
+    args = (q[:, 0].cuda(), kp.cuda(), vp.cuda(), tables.cuda())
+    want = ref.reference_decode(q, kp, vp, lengths, softmax_scale=0.1, page_tables=tables,
+                                sliding_window=None if window < 0 else window)[:, 0]
+    live = lengths > 0
+    pos = torch.stack([lengths.long() - 1, torch.zeros(b, dtype=torch.int64)], 1).cuda()[:, 0]
+    for lens, kw in ((lengths.cuda(), {}), (pos, dict(lengths_are_positions=True)),
+                     (pos.to(torch.int32), dict(lengths_are_positions=True))):
+        got = ops.paged_decode(*args, lens, softmax_scale=0.1, sliding_window=window, **kw).cpu()
+        assert _ok(got[live], want[live]) and torch.equal(got[~live], torch.zeros_like(got[~live]))
