@@ -249,7 +249,7 @@ def strides4(t: torch.Tensor) -> AxlStrides:
 
 
 def current_stream_ptr() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())  # no Stream object around it
 
 
 def ptr(t: Optional[torch.Tensor]) -> Optional[int]:

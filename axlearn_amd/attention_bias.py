@@ -137,7 +137,11 @@ class BaseAttentionBias:
         return self._broadcast_value(value)
 
     def astype(self, dtype: torch.dtype) -> "BaseAttentionBias":
-        return dataclasses.replace(self, dtype=dtype)
+        # the fields as they are, without running __init__ and __post_init__ over them again
+        new = object.__new__(type(self))
+        new.__dict__.update(self.__dict__)
+        new.dtype = dtype
+        return new
 
     def __add__(self, other: "BaseAttentionBias") -> "CompositeAttentionBias":
         return CompositeAttentionBias([self, other])
@@ -217,10 +221,14 @@ class CompositeAttentionBias(BaseAttentionBias):
         direct = super().bias_and_residual(cls)
         if direct.bias is not None:
             return direct
-        pending = list(self._nonzero())
+        pending = self._nonzero()
         found, rest = [], []
         while pending:
             member = pending.pop()
+            if type(member).bias_and_residual is BaseAttentionBias.bias_and_residual:
+                # not a composite: all of it is of type `cls` or none is
+                (found if isinstance(member, cls) else rest).append(member)
+                continue
             part = member.bias_and_residual(cls)
             if part.bias is not None:
                 found.append(part.bias)
@@ -229,7 +237,8 @@ class CompositeAttentionBias(BaseAttentionBias):
                 target = rest
             if part.residual.has_value():
                 target.append(part.residual)
-        return BiasAndResidual(bias=cls.from_sequence(found), residual=CompositeAttentionBias(rest))
+        bias = found[0] if len(found) == 1 else cls.from_sequence(found)
+        return BiasAndResidual(bias=bias, residual=CompositeAttentionBias(rest))
 
     def _flatten(self) -> "CompositeAttentionBias":
         todo, flat = [self], []

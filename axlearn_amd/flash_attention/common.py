@@ -129,6 +129,14 @@ class BaseFlashAttention(Configurable):
         if key.shape != value.shape:
             raise ValueError(f"Expects {key.shape=} to be equal to {value.shape=}")
 
+    @classmethod
+    def serves(cls, query: Tensor, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
+        """Whether the class is meant for such calls at all: False makes the dispatch pass it over without
+        building it (a decode kernel in every prefill call cost 20 us, most of it for the warning that
+        it does not take one)."""
+        del query, kv_cache_type
+        return True
+
     def is_supported(self, input_batch: Nested, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
         del kv_cache_type
         self._validate_input_batch(input_batch)
@@ -173,6 +181,10 @@ class BaseFlashAttention(Configurable):
 class BaseSingleStepDecoding(BaseFlashAttention):
     """Checks shared by the single-token decode kernels (common.py:322-340)."""
 
+    @classmethod
+    def serves(cls, query: Tensor, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
+        return kv_cache_type is not None and query.dim() == 4 and query.shape[1] == 1
+
     def is_supported(self, input_batch: Nested, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
         if not super().is_supported(input_batch, kv_cache_type=kv_cache_type):
             return False
@@ -195,6 +207,10 @@ class BasePagedAttention(BaseSingleStepDecoding):
     @config_class
     class Config(BaseSingleStepDecoding.Config):
         sparse_ratio: float = 0.8
+
+    @classmethod
+    def serves(cls, query: Tensor, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
+        return True  # the only candidate for its cache type: `is_supported` says why it declines
 
     def _validate_input_batch(self, input_batch: Nested) -> None:
         super()._validate_input_batch(input_batch)

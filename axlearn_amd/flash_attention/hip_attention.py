@@ -129,11 +129,19 @@ def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, lo
         raise NotImplementedError(f"{head_dim=} > 128 is not supported by the HIP kernels.")
     if runs_at_native_head_dim(query, key, value, aux=bias is not None or dropout_mask is not None):
         width = head_dim
-    out = _FlashAttentionFn.apply(
-        _pad_last(query, width), _pad_last(key, width), _pad_last(value, width), segment_ids,
-        softmax_scale, mask_kind, window, logit_sink, bias, dropout_mask, dropout_rate, save_residuals,
-        bwd_ds_workspace, bwd_workspace_limit_bytes,
-    )
+    query, key, value = _pad_last(query, width), _pad_last(key, width), _pad_last(value, width)
+    if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad
+                                    or (logit_sink is not None and logit_sink.requires_grad)):
+        out = _FlashAttentionFn.apply(
+            query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink, bias, dropout_mask,
+            dropout_rate, save_residuals, bwd_ds_workspace, bwd_workspace_limit_bytes,
+        )
+    else:  # nothing to differentiate: no autograd node, no lse
+        out, _ = ops.flash_fwd(
+            query, key, value, softmax_scale=softmax_scale, mask_kind=mask_kind, sliding_window=window,
+            segment_ids=segment_ids, return_lse=False, logit_sink=logit_sink, bias=bias, dropout_mask=dropout_mask,
+            dropout_rate=dropout_rate,
+        )
     return out if width == head_dim else out[..., :head_dim]
 
 

@@ -73,7 +73,7 @@ class FlashAttention(Configurable):
         for the base layer's standard attention, which the reference calls when no kernel supports the
         request (layer.py:278-285).  This package computes nothing outside its HIP kernels: without a
         fallback such a request raises."""
-        cfg = self.config
+        cfg = self._config  # read only: no copy per call
         attention_logit_biases = attention_logit_biases.astype(q_proj.dtype)
         softmax_scale = cfg.softmax_scale if cfg.softmax_scale is not None else 1.0
         flash_specs = flash_attention_implementation(

@@ -65,6 +65,8 @@ def flash_attention_implementation(
         query=query, key=key, value=value, page_tables=page_tables, bias=bias, logit_sink=logit_sink
     )
     for klass in candidates:
+        if not klass.serves(query, kv_cache_type):
+            continue
         attn_fn = klass.default_config().set(**common_cfg).instantiate()
         if attn_fn.is_supported(input_batch=input_batch, kv_cache_type=kv_cache_type):
             logging.info("Using %s for flash attention.", attn_fn.name())
