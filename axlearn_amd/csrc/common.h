@@ -448,8 +448,11 @@ __device__ __forceinline__ int classify_segment_groups_tbl(const int2* tbl, int 
 // that many query blocks x query heads), heaviest query blocks (most visible keys under a causal
 // mask) first across the group.  The workgroups that run together then read the K/V of one or two
 // kv heads, which that XCD's L2 holds, and a group still has enough workgroups to keep every CU busy.
+// `batch_fastest`: an XCD takes the pairs of one kv head after one another over the batch, for inputs that
+// the batch shares: a broadcast bias is then read by all of it while that XCD's L2 or the memory-side cache
+// holds it (kv heads a multiple of 8, so that the batch stays on one XCD).
 __device__ __forceinline__ void decode_block(int bid, int nqb, int B, int Hq, int Hkv, int slots, int& qb,
-                                             int& b, int& h) {
+                                             int& b, int& h, bool batch_fastest = false) {
   const int G = Hq / Hkv;
   const int npairs = B * Hkv;
   if (npairs % 8 == 0) {
@@ -461,10 +464,11 @@ __device__ __forceinline__ void decode_block(int bid, int nqb, int B, int Hq, in
     const int r = slot - grp * (pgn * per_pair);
     const int pg = min(pgn, ppx - grp * pgn);          // the last group may be smaller
     const int rem = r % (pg * G);
-    const int pair = xcd + 8 * (grp * pgn + rem / G);
+    const int i = grp * pgn + rem / G;                 // pair of this XCD
+    const bool by_head = batch_fastest && Hkv % 8 == 0;
     qb = nqb - 1 - r / (pg * G);
-    b = pair / Hkv;
-    h = (pair % Hkv) * G + rem % G;
+    b = by_head ? i % B : (xcd + 8 * i) / Hkv;
+    h = (by_head ? xcd + 8 * (i / B) : (xcd + 8 * i) % Hkv) * G + rem % G;
   } else {
     const int per_qb = B * Hq;
     const int qb_rev = bid / per_qb, rem = bid % per_qb;

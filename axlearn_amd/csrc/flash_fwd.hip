@@ -71,6 +71,9 @@ struct FwdTile {
 constexpr int kMaxSegTiles = 1024;               // key tiles whose segment ids the forward classifies
 constexpr int kSegNotUniform = -0x7fffffff - 1;  // marks a tile with more than one segment id
 
+// Optional inputs of the body: none; a bf16 bias and nothing else; whatever the arguments say.
+constexpr int kFwdPlain = 0, kFwdBias16 = 1, kFwdAux = 2;
+
 // Partial results of the chunk form: per workgroup and wavefront the accumulators as they lie in
 // registers, [D / 8 pieces][64 lanes] float4, so that a store instruction writes 1 KB in one piece, then
 // (log2-scaled running maximum, sum) of the wavefront's 32 rows.
@@ -151,8 +154,10 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
 //     the positions is looked at on the host.
 // That call now takes 55 us for the 42 GFLOP of offsets 7552 and 4996 (760 TFLOP/s; the forward at full
 // occupancy runs at 1000) and 10 us for the merge, 172 -> 99 us as a call of the layer.
-template <typename E, int D, bool AUX, int NW, bool CHUNK>
+template <typename E, int D, int INPUTS, int NW, bool CHUNK>
 __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
+  // BIAS16: a bf16 bias and nothing else, known at compile time; AUX without it: whatever there is.
+  constexpr bool AUX = INPUTS != kFwdPlain, BIAS16 = INPUTS == kFwdBias16;
   static_assert(!(AUX && CHUNK), "the chunk form takes no bias or dropout mask");
   using Tile = FwdTile<D, NW>;
   constexpr int KK = D / 16;  // MFMA k-steps over head_dim
@@ -180,7 +185,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     qb = slot - sh.first - split * nqb;
     hk = blockIdx.x - slot * a.Hkv;
   } else {
-    decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h);
+    decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h, BIAS16 && a.aux.bias_sb == 0);
     hk = h / G;
   }
   const int q_off = CHUNK ? 0 : a.q_off + (a.q_offs ? a.q_offs[b] : 0);  // position of this sequence's query row 0
@@ -275,7 +280,13 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // the raw logits as bias / scale, so the scale folded into the exponent applies to both.
   const char* bias_row = nullptr;
   const uint8_t* drop_row = nullptr;
-  if constexpr (AUX) {
+  // BIAS16: the same as a scalar base and one 32-bit offset per lane (the launcher checks that it fits).
+  const char* bias_head = nullptr;
+  unsigned bias_off = 0;
+  if constexpr (BIAS16) {
+    bias_head = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh;
+    bias_off = (unsigned)(q0 + l32) * (unsigned)a.aux.bias_sr + 16 * g;
+  } else if constexpr (AUX) {
     if (a.aux.bias) bias_row = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh + (int64_t)(q0 + l32) * a.aux.bias_sr;
     if (a.aux.drop) drop_row = a.aux.drop + b * a.aux.drop_sb + h * a.aux.drop_sh + (int64_t)(q0 + l32) * a.aux.drop_sr;
   }
@@ -317,29 +328,64 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     k_src[i] = (unsigned)(row * (int)a.ks.s + chunk * 8) * 2 - (i % 2) * 1024;
     v_src[i] = (unsigned)(row * (int)a.vs.s + chunk * 8) * 2 - (i % 2) * 1024;
   }
+  // The bias form has no registers for the eight offsets (three of them went to scratch, and each reload
+  // waited for all loads in flight, the bias's among them: 83 instead of 68 us at B2 H16 T2048).  Row
+  // 4 i of a lane's rows holds its chunk XOR a constant of i, so an offset is that of row 0 plus a uniform
+  // step plus a difference that K and V share; it is formed where it is used, in assembly so that the
+  // compiler does not move the sums out of the loop again.
+  constexpr bool kFormOffsets = BIAS16 && D == 128;
+  unsigned src_delta[kFormOffsets ? Tile::DMA_PER_WAVE : 1];
+  if constexpr (kFormOffsets) {
+#pragma unroll
+    for (int i = 0; i < Tile::DMA_PER_WAVE; i++)
+      src_delta[i] = k_src[i] - k_src[0] - (unsigned)(RPI * i * (int)a.ks.s) * 2 + (i % 2) * 1024;
+  }
+  auto src_off = [&](const unsigned (&src)[Tile::DMA_PER_WAVE], int64_t stride, int i) __attribute__((always_inline)) {
+    if constexpr (kFormOffsets) {
+      if (i == 0) return src[0];
+      unsigned r;
+      asm volatile("v_add3_u32 %0, %1, %2, %3"
+                   : "=v"(r)
+                   : "v"(src[0]), "v"(src_delta[i]), "s"((unsigned)(RPI * i * (int)stride) * 2 - (i % 2) * 1024));
+      return r;
+    } else {
+      return src[i];
+    }
+  };
+  auto seg_off = [&]() __attribute__((always_inline)) -> unsigned {   // 16 bytes per lane, lanes 0..15
+    if constexpr (kFormOffsets) {
+      unsigned r;
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_lshlrev_b32 %0, 4, %0" : "=v"(r));
+      return r;
+    } else {
+      return 16 * (lane & 15);
+    }
+  };
   const unsigned lds0 = lds_address(smem);
   auto issue_k = [&](int t, int buf) {
     const __bf16* src = kp + (int64_t)t * Tile::BK * a.ks.s;
     const unsigned dst = lds0 + buf * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB);
 #pragma unroll
-    for (int i = 0; i < Tile::DMA_PER_WAVE; i += 2) dma16x2(k_src[i], k_src[i + 1], src, dst + i * 1024);
+    for (int i = 0; i < Tile::DMA_PER_WAVE; i += 2)
+      dma16x2(src_off(k_src, a.ks.s, i), src_off(k_src, a.ks.s, i + 1), src, dst + i * 1024);
     if (seg_k && wave == 0 && lane < Tile::BK / 4)  // 64 ids = 16 lanes x 16 bytes
       dma16(seg_k + t * Tile::BK + 4 * lane, lds0 + Tile::SEG_BASE + (t % Tile::NSEG) * (Tile::BK * 4));
   };
   // One pair of a tile's loads (FAST tiles deal the pairs out over their MFMA slots).
   auto issue_k_pair = [&](int t, int buf, int i) __attribute__((always_inline)) {
     const __bf16* src = kp + (int64_t)t * Tile::BK * a.ks.s;
-    dma16x2(k_src[i], k_src[i + 1], src, lds0 + buf * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB) + i * 1024);
+    dma16x2(src_off(k_src, a.ks.s, i), src_off(k_src, a.ks.s, i + 1), src, lds0 + buf * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB) + i * 1024);
   };
   auto issue_v_pair = [&](int t, int buf, int i) __attribute__((always_inline)) {
     const __bf16* src = vp + (int64_t)t * Tile::BK * a.vs.s;
-    dma16x2(v_src[i], v_src[i + 1], src, lds0 + (2 + buf) * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB) + i * 1024);
+    dma16x2(src_off(v_src, a.vs.s, i), src_off(v_src, a.vs.s, i + 1), src, lds0 + (2 + buf) * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB) + i * 1024);
   };
   auto issue_v = [&](int t, int buf) {
     const __bf16* src = vp + (int64_t)t * Tile::BK * a.vs.s;
     const unsigned dst = lds0 + (2 + buf) * Tile::TILE_BYTES + wave * (Tile::WROWS * Tile::ROWB);
 #pragma unroll
-    for (int i = 0; i < Tile::DMA_PER_WAVE; i += 2) dma16x2(v_src[i], v_src[i + 1], src, dst + i * 1024);
+    for (int i = 0; i < Tile::DMA_PER_WAVE; i += 2)
+      dma16x2(src_off(v_src, a.vs.s, i), src_off(v_src, a.vs.s, i + 1), src, dst + i * 1024);
   };
 
   // ---- per-lane LDS read offsets (bytes).  K row reads: row swap_bits_2_3(l32) (+32 per sub-tile),
@@ -384,14 +430,18 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // AUX: raw bias words and dropout bytes of the lane's 4 runs of 8 keys, requested one tile ahead
   // with ordinary (compiler-tracked) loads.  Run i covers keys 32(i/2) + 16(i%2) + 8g .. +7 of the tile;
   // an fp32 bias fills both vectors of a run, a bf16 bias the first.
-  u32x4 bias_nx[AUX ? 8 : 1];
-  uint2 drop_nx[AUX ? 4 : 1];
+  u32x4 bias_nx[BIAS16 ? 4 : (AUX ? 8 : 1)];
+  uint2 drop_nx[AUX && !BIAS16 ? 4 : 1];
   // Both tests are uniform (the row pointers are not: they differ by lane).  A bf16 bias repeats its
   // one load so that the request is the same straight-line code for both element types.
-  const bool has_bias = AUX && a.aux.bias != nullptr, has_drop = AUX && a.aux.drop != nullptr;
+  const bool has_bias = AUX && (BIAS16 || a.aux.bias != nullptr), has_drop = AUX && !BIAS16 && a.aux.drop != nullptr;
   const int bias_shift = a.aux.bias_f32 ? 2 : 1, bias_second = a.aux.bias_f32 ? 16 : 0;
   auto aux_request = [&](int t) __attribute__((always_inline)) {
-    if constexpr (AUX) {
+    if constexpr (BIAS16) {
+      const char* p = bias_head + (int64_t)t * (2 * Tile::BK);
+#pragma unroll
+      for (int i = 0; i < 4; i++) bias_nx[i] = *(const u32x4*)(p + 64 * (i / 2) + 32 * (i % 2) + bias_off);
+    } else if constexpr (AUX) {
       const int k0 = t * Tile::BK + 8 * g;
       if (has_bias) {
 #pragma unroll
@@ -440,7 +490,21 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     // ago, ahead of that tile's K / V loads); they are consumed here, before anything else is
     // requested, so the compiler's own wait for them finds the counter at zero already.
     uint2 dm[2][2] = {};  // dropout bytes of the lane's 4 runs of 8 keys
-    if constexpr (AUX && !FAST) {
+    if constexpr (BIAS16) {
+      if (do_sm) {
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            // (a copy first: a bit cast applied to the vector element itself reads element 0)
+            const unsigned w = bias_nx[i][j / 2];
+            const float x = s[i / 2][8 * (i % 2) + j];
+            s[i / 2][8 * (i % 2) + j] =
+                __builtin_fmaf(__builtin_bit_cast(float, j % 2 ? w & 0xffff0000u : w << 16), a.aux.inv_scale, x);
+          }
+      }
+      if (do_s) aux_request(t + 1);
+    } else if constexpr (AUX) {
       if (do_sm) {
         if (has_bias) {
 #pragma unroll
@@ -488,7 +552,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     // ---- masks of tile t.  Register r of sub-tile ks in lane group g is key k0 + 32ks + 16(r/8) + 8g + (r%8).
     // Probability that enters P V: zero where the dropout mask says so (the row sum keeps it).
     auto after_dropout = [&](int idx, float p) {
-      if constexpr (AUX) {
+      if constexpr (AUX && !BIAS16) {
         const int ks = idx / 16, r = idx % 16;
         const unsigned w = (r % 8) < 4 ? dm[ks][r / 8].x : dm[ks][r / 8].y;
         return ((w >> (8 * (r % 4))) & 0xffu) ? 0.f : p;
@@ -535,7 +599,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     // moves when the new max exceeds it by more than 2^kLazyLog2 in the exponent; until then exp2 is
     // taken against the stale max, which scales numerator and denominator alike.
     float mx = m_run;
-    if constexpr (FAST) {
+    if constexpr (FAST && !BIAS16) {
       mx = fmaxf(mx, mx_carry);
     } else {
 #pragma unroll
@@ -584,7 +648,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
           // the ids of tile t+2 for a general tile that may follow (every wavefront fetches the same
           // 256 bytes: no branch on the wavefront number inside the slot sequence)
           if (n == 4 * kPairs && seg_k)
-            dma16s_first16(16 * (lane & 15), seg_k + t_k2 * Tile::BK, lds0 + Tile::SEG_BASE + (t_k2 % Tile::NSEG) * (Tile::BK * 4));
+            dma16s_first16(seg_off(), seg_k + t_k2 * Tile::BK, lds0 + Tile::SEG_BASE + (t_k2 % Tile::NSEG) * (Tile::BK * 4));
           // The chain in vector registers where the next tile's softmax reads it, started from a
           // literal zero: no register is cleared and none is copied.  (The 16 P V MFMAs of this tile lie
           // between the end of the chain and the first read of its result.)
@@ -638,7 +702,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     for (int n = 0; n < kPvSteps; n++) {
       if (n + kPvAhead < kPvSteps) AXL_PV_READ(n + kPvAhead)
       o[n % DT] = E::mfma_32x32x16(vfr[n].v, pb.v[n / DT], o[n % DT]);
-      if constexpr (FAST) {
+      if constexpr (FAST && !BIAS16) {
         // Row maximum of the next tile's logits, two per slot from slot 2 on: by then two MFMAs have
         // been issued after the last one of the S chains, whose results these reads therefore find
         // complete.  Four independent partial maxima keep the chains short.
@@ -649,7 +713,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
       }
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (FAST) mx_carry = fmaxf(fmaxf(pm[0], pm[1]), fmaxf(pm[2], pm[3]));
+    if constexpr (FAST && !BIAS16) mx_carry = fmaxf(fmaxf(pm[0], pm[1]), fmaxf(pm[2], pm[3]));
 #undef AXL_PV_READ
   };
   {
@@ -661,7 +725,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     const std::integral_constant<int, 0> c0{};
     const std::integral_constant<int, 1> c1{};
     int f_lo = t_end, f_hi = t_end;
-    if (!AUX && (!seg_k || seg_fast)) {
+    if ((!AUX || BIAS16) && (!seg_k || seg_fast)) {
       f_lo = tw_begin;
       f_hi = tw_end - 1;
       if (a.mask_kind != AXL_MASK_NONE) {
@@ -692,9 +756,9 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
         tile_step(t + 1, c1, s_odd, s_even, std::false_type{});
       }
     };
-    if constexpr (!AUX) {
+    if constexpr (!AUX || BIAS16) {
       generic_pairs_to(min(f_lo, t_end));
-      if (t + 1 < f_hi) {  // the first FAST tile's lane-local maximum (later ones get theirs from the tile before)
+      if (!BIAS16 && t + 1 < f_hi) {  // the first FAST tile's lane-local maximum (later ones get theirs from the tile before)
         mx_carry = kMasked;
 #pragma unroll
         for (int ks = 0; ks < 2; ks++)
@@ -731,7 +795,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     if (q0 + l32 >= chunk_rows) return;
   }
   float inv_l = l_tot > 0.f ? 1.0f / l_tot : 0.f;  // a row with no visible key yields zeros
-  if constexpr (AUX) inv_l *= a.aux.keep_scale;
+  if constexpr (AUX && !BIAS16) inv_l *= a.aux.keep_scale;
   __bf16* op = (__bf16*)a.out + b * a.os.b + (int64_t)row * a.os.s + h * a.os.h;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++) {
@@ -754,13 +818,27 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
 template <typename E, int D, bool AUX, int NW = 4>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(AUX ? 1 : 2, AUX ? 1 : 2)))
 void flash_fwd_kernel(const FwdArgs a) {
-  flash_fwd_body<E, D, AUX, NW, false>(a);
+  flash_fwd_body<E, D, AUX ? kFwdAux : kFwdPlain, NW, false>(a);
+}
+
+// A bf16 bias without a dropout mask.  Knowing that at compile time takes the run-time tests, the fp32
+// copies' registers and the dropout arithmetic out: interior tiles take the plain kernel's FAST form (32 more
+// multiply-adds and 32 conversions per tile) and two wavefronts fit a SIMD.  Causal, bias [1,H,T,T]:
+// B2 H16 T2048 D128 104 -> 68 us (plain 52), D64 73 -> 43 us (plain 31); B4 H32 T4096 D128 1.53 -> 0.80 ms
+// (plain 0.59; of it, taking the batch's workgroups of one head together, so that the bias comes from memory
+// once: 1.01 -> 0.88, no scratch reload in the FAST loop: 0.88 -> 0.80).
+// (Requesting the bias after the exponentials, where registers are free, made the compiler spill more
+// of the loop, 108 us.)
+template <typename E, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_fwd_bias_kernel(const FwdArgs a) {
+  flash_fwd_body<E, D, kFwdBias16, 4, false>(a);
 }
 
 template <typename E, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_chunk_kernel(const FwdArgs a) {
-  flash_fwd_body<E, D, false, 4, true>(a);
+  flash_fwd_body<E, D, kFwdPlain, 4, true>(a);
 }
 
 // Merges the partial results of the chunk form, out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s in the
@@ -1305,6 +1383,8 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   a.sink = p.logit_sink;
   a.aux = make_aux_args(p.aux, p.softmax_scale);
   const bool aux = p.aux.bias || p.aux.dropout_mask;
+  const bool bias16 = p.aux.bias && p.aux.bias_dtype == AXL_BF16 && !p.aux.dropout_mask &&
+                      (int64_t)p.q_len * a.aux.bias_sr < (int64_t)1 << 32;  // 32-bit row offsets
   a.qs = to_s3(p.q_strides); a.ks = to_s3(p.k_strides); a.vs = to_s3(p.v_strides);
   a.os = to_s3(p.out_strides);
   a.B = p.batch; a.T = p.q_len; a.S = p.kv_len; a.Hq = p.num_q_heads; a.Hkv = p.num_kv_heads;
@@ -1325,7 +1405,10 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   } while (0)
 #define AXL_LAUNCH_FWD16(E)                                                                     \
   do {                                                                                          \
-    if (width == 128) {                                                                         \
+    if (bias16) {                                                                               \
+      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128>), FwdTile<128>);          \
+      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64>), FwdTile<64>);                         \
+    } else if (width == 128) {                                                                  \
       if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, true>), FwdTile<128>);                  \
       else AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, false>), FwdTile<128>);                     \
     } else {                                                                                    \

@@ -1418,3 +1418,25 @@ def test_ds_workspace_backward_with_bias_and_dropout(t, hq, hkv, d, mask, window
         got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=True, ds_slice_kv_heads=heads, **kw)
         assert torch.equal(got[1], want[1]) and torch.equal(got[2], want[2])
         assert ref.rel_l2(got[0].cpu(), want[0].cpu()) < 4e-3   # both rounded to bf16 once: 2^-8 apart at most
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,shared", [
+    (1, 128, 2, 1, 128, "causal", None, False, True),     # two tiles: none in the interior form
+    (2, 384, 8, 8, 64, "none", None, False, True),        # every tile but the last in it, pairs a multiple of 8
+    (2, 640, 8, 4, 128, "causal", None, False, True),     # batch-fastest order of the pairs
+    (2, 512, 4, 2, 128, "sliding", 150, True, False),     # a bias per batch element, masks of every kind
+])
+def test_forward_with_bf16_bias_alone(b, t, hq, hkv, d, mask, window, packed, shared):
+    # The forward's form for a bf16 bias and nothing else, against the oracle and against the general form
+    # (which the same bias in fp32 takes: the same values, so outputs at most one rounding of P apart).
+    q, k, v, _ = _inputs(b, t, hq, hkv, d, torch.bfloat16)
+    bias = ref.normal_tensor(9, (1 if shared else b, hq, t, t), torch.bfloat16)
+    seg = ref.packed_segment_ids(6, b, t) if packed else None
+    spec, kw = _mask_args(mask, window, seg)
+    spec.dense_bias = bias.float()
+    want, want_lse = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5, return_lse=True)
+    args = (q.cuda(), k.cuda(), v.cuda())
+    out, lse = ops.flash_fwd(*args, softmax_scale=d ** -0.5, bias=bias.cuda(), **kw)
+    out32, lse32 = ops.flash_fwd(*args, softmax_scale=d ** -0.5, bias=bias.float().cuda(), **kw)
+    assert ref.rel_l2(out.cpu(), want) < 1e-2 and ref.rel_l2(out.cpu(), out32.cpu()) < 4e-3
+    assert ref.max_abs(lse.cpu(), want_lse) < 1e-3 and ref.max_abs(lse.cpu(), lse32.cpu()) < 1e-4

@@ -680,7 +680,7 @@ def test_ffi_shim_and_jax_side_stay_in_step_with_the_abi():
                                              open(os.path.join(ROOT, "include", "axl_attn.h")).read()).group(1))
 
 
-def test_chunk_kernel_keeps_the_distance_behind_its_assembly_mfma_chains():
-    """The form of the forward for chunks over a long cache shares its body: the same check."""
+def test_chunk_and_bias_kernels_keep_the_distance_behind_their_assembly_mfma_chains():
+    """The forms of the forward for chunks over a long cache and for a bf16 bias share its body: the same check."""
     asm, _ = _device_asm("flash_fwd.hip", extra=("-mllvm", "-amdgpu-mfma-vgpr-form"))
-    _assert_asm_mfma_distances(asm, r"_ZN3axl18flash_chunk_kernel", 4)
+    _assert_asm_mfma_distances(asm, r"_ZN3axl(18flash_chunk_kernel|21flash_fwd_bias_kernel)", 8)
