@@ -252,6 +252,10 @@ __device__ __forceinline__ void store16x2(unsigned voff, void* sbase, bf16x8 d0,
                : "v"(voff), "v"(d0), "v"(d1), "s"(sbase)
                : "memory");
 }
+// One such store of four fp32.
+__device__ __forceinline__ void store16_stream(unsigned voff, const void* sbase, floatx4 d) {
+  asm volatile("global_store_dwordx4 %0, %1, %2 sc0 sc1 nt" : : "v"(voff), "v"(d), "s"(sbase) : "memory");
+}
 #pragma clang diagnostic pop
 template <int N>
 __device__ __forceinline__ void wait_vmem_le() {

@@ -15,6 +15,8 @@ struct BwdArgs {
   float* ndelta; // workspace [B, Hq, T]: -rowsum(out * dO); negated so that a dP accumulator chain can start from it
   float* lse2;   // workspace [B, Hq, T]: -lse * log2(e), the exponent offset of the dK/dV kernel
   void* ds;      // workspace: dS blocks left by the dK/dV kernel for the streaming dQ kernel (spill path), or nullptr
+  const char* q_planes;   // workspace (fp32): the 32-row tiles of Q and of dO as bf16 planes, [B, Hq, T / 32] tiles
+  const char* do_planes;
   void* dq;
   void* dk;
   void* dv;
@@ -61,6 +63,17 @@ __host__ __device__ inline int64_t ds_run_start(int64_t pair, int T, int G, int 
   return G * (pair * ds_blocks_per_head(T) + ds_tile_offset(t)) + hh * ds_run_blocks(t);
 }
 
+// dS workspace of the fp32 kernels: 4 KB blocks of 32 queries x 32 keys (fp32; inside a block see
+// flash_bwd_f32x.hip).  Query tile t of a head has a run of t + 1 blocks; runs are ordered as above.
+constexpr int kDs32BlockElems = 1024;
+__host__ __device__ inline int64_t ds32_blocks_per_head(int T) {
+  const int64_t n = T / 32;
+  return n * (n + 1) / 2;
+}
+__host__ __device__ inline int64_t ds32_run_start(int64_t pair, int T, int G, int t, int hh) {
+  return G * (pair * ds32_blocks_per_head(T) + (int64_t)t * (t + 1) / 2) + (int64_t)hh * (t + 1);
+}
+
 // Enqueues the dK/dV kernel for `dtype` AXL_BF16 or AXL_F16 and head_dim 64 or 128; `aux` selects
 // the instantiation that reads the dense bias / dropout mask.  With a.ds set (causal or sliding-window
 // mask, q_off 0, T == S) the kernel also stores dS for launch_bwd_dq_stream, and with a.kb_tbl set the
@@ -80,5 +93,15 @@ hipError_t launch_bwd_dq(const BwdArgs& a, int dtype, int head_dim, bool fuse_de
 // Enqueues the fp32 dK/dV and / or dQ kernels (`phases`: AXL_BWD_DKDV, AXL_BWD_DQ) for head_dim 64
 // or 128; they read delta from the workspace and honour the dense bias / dropout mask.
 hipError_t launch_bwd_f32(const BwdArgs& a, int head_dim, int phases, hipStream_t stream);
+
+// AXL_F32_MFMA=1 in the environment (read once): fp32 on the fp32 matrix instruction, for comparison.
+bool f32_on_fp32_mfma();
+
+// Fills the workspace's Q and dO planes, which the fp32 dK/dV kernel reads.
+hipError_t launch_bwd_split_f32x(const BwdArgs& a, int head_dim, hipStream_t stream);
+
+// The fp32 kernels behind launch_bwd_f32: dK/dV (with a.ds set it also stores dS) and dQ from the stored dS.
+hipError_t launch_bwd_dkdv_f32x(const BwdArgs& a, int head_dim, hipStream_t stream);
+hipError_t launch_bwd_dq_ds_f32(const BwdArgs& a, int head_dim, hipStream_t stream);
 
 }  // namespace axl

@@ -395,11 +395,12 @@ static size_t stats_bytes(const AxlFlashBwdParams& p) {
 // The dS-spill path: the dK/dV kernel stores dS and the dQ kernel becomes one streaming GEMM
 // (5 executed GEMMs instead of 7).  Causal or sliding-window attention over equal lengths, with or
 // without segment ids, a dense bias or a dropout mask.
+// 16-bit kernels: which tiles of dS there are depends on the key block (fp32: on the tile's place alone).
 static bool spill_ranged(const AxlFlashBwdParams& p) {
-  return p.mask_kind == AXL_MASK_SLIDING_WINDOW || p.segment_ids;
+  return p.dtype != AXL_F32 && (p.mask_kind == AXL_MASK_SLIDING_WINDOW || p.segment_ids);
 }
 static bool spill_eligible(const AxlFlashBwdParams& p) {
-  return (p.dtype == AXL_BF16 || p.dtype == AXL_F16) &&
+  return (p.dtype == AXL_BF16 || p.dtype == AXL_F16 || (p.dtype == AXL_F32 && !f32_on_fp32_mfma())) &&
          (p.mask_kind == AXL_MASK_CAUSAL || p.mask_kind == AXL_MASK_SLIDING_WINDOW) && p.q_pos_offset == 0 &&
          p.q_len == p.kv_len && (p.flags & AXL_BWD_DS_WORKSPACE) &&
          // the ranged kernel keeps the table in LDS beside its ring: 256-row blocks at head_dim 128
@@ -414,6 +415,7 @@ static int spill_slice_heads(const AxlFlashBwdParams& p) {
 }
 static size_t spill_bytes(const AxlFlashBwdParams& p) {
   const int heads = spill_slice_heads(p) * (p.num_q_heads / p.num_kv_heads);
+  if (p.dtype == AXL_F32) return (size_t)p.batch * heads * (size_t)ds32_blocks_per_head(p.q_len) * kDs32BlockElems * 4;
   return (size_t)p.batch * heads * (size_t)ds_blocks_per_head(p.q_len) * kDsBlockBytes;
 }
 
@@ -429,12 +431,18 @@ static size_t kb_table_bytes(const AxlFlashBwdParams& p) {
   return ((size_t)p.batch * (p.kv_len / 128) * sizeof(int2) + 255) & ~(size_t)255;
 }
 
+// fp32: the planes of Q (and, of the same size, of dO), six bytes per element of the compiled width.
+static size_t planes_bytes(const AxlFlashBwdParams& p) {
+  if (p.dtype != AXL_F32 || f32_on_fp32_mfma()) return 0;
+  return (size_t)p.batch * p.num_q_heads * p.q_len * (p.head_dim <= 64 ? 64 : 128) * 6;
+}
+
 // The parts of the workspace start on 256-byte boundaries; the caller's pointer only has to be
 // 16-byte aligned (allocators that slice one arena, XLA's buffer assignment among them, promise less
 // than 256), so the size includes the slack for rounding it up.
 constexpr size_t kWsAlign = 256;
 size_t flash_bwd_workspace_bytes(const AxlFlashBwdParams& p) {
-  return stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p) + (spill_eligible(p) ? spill_bytes(p) : 0) +
+  return stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p) + 2 * planes_bytes(p) + (spill_eligible(p) ? spill_bytes(p) : 0) +
          (kWsAlign - 16);
 }
 
@@ -449,7 +457,10 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   const bool spill = spill_eligible(p);  // the entry point has checked that the workspace holds dS as well
   a.seg_tbl = p.segment_ids ? (const int2*)(ws + stats_bytes(p)) : nullptr;
   a.kb_tbl = kb_table_bytes(p) ? (int2*)(ws + stats_bytes(p) + seg_table_bytes(p)) : nullptr;
-  a.ds = spill ? ws + stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p) : nullptr;
+  char* const ws_planes = ws + stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p);
+  a.q_planes = ws_planes;
+  a.do_planes = ws_planes + planes_bytes(p);
+  a.ds = spill ? ws_planes + 2 * planes_bytes(p) : nullptr;
   a.qs = to_s3(p.q_strides); a.ks = to_s3(p.k_strides); a.vs = to_s3(p.v_strides);
   a.os = to_s3(p.out_strides); a.dos = to_s3(p.d_out_strides); a.dqs = to_s3(p.dq_strides);
   a.dks = to_s3(p.dk_strides); a.dvs = to_s3(p.dv_strides);
@@ -497,6 +508,9 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       if (width == 128) AXL_LAUNCH((bwd_delta_kernel<float, 128>), delta_grid, 0);
       else AXL_LAUNCH((bwd_delta_kernel<float, 64>), delta_grid, 0);
     }
+    if ((phases & AXL_BWD_DKDV) && !f32_on_fp32_mfma() && err == hipSuccess) err = launch_bwd_split_f32x(a, width, stream);
+  }
+  if (dt == AXL_F32 && !spill) {
     if (err == hipSuccess) err = launch_bwd_f32(a, width, phases, stream);
   } else if (spill) {
     // delta, then the dK/dV kernel (which leaves dS behind), then dq = scale * dS k.
@@ -508,14 +522,14 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       if (dt == AXL_BF16) {
         if (width == 128) AXL_LAUNCH((bwd_delta_kernel<__bf16, 128>), delta_grid, 0);
         else AXL_LAUNCH((bwd_delta_kernel<__bf16, 64>), delta_grid, 0);
-      } else {
+      } else if (dt == AXL_F16) {
         if (width == 128) AXL_LAUNCH((bwd_delta_kernel<_Float16, 128>), delta_grid, 0);
         else AXL_LAUNCH((bwd_delta_kernel<_Float16, 64>), delta_grid, 0);
       }
     }
     // One slice of kv heads after the other: the kernels see a problem of that many heads (tensors
     // and statistics offset to the slice's first head) and the same dS workspace.
-    const int slice = spill_slice_heads(p), G = p.num_q_heads / p.num_kv_heads, es = 2;
+    const int slice = spill_slice_heads(p), G = p.num_q_heads / p.num_kv_heads, es = dt == AXL_F32 ? 4 : 2;
     for (int h0 = 0; h0 < p.num_kv_heads && err == hipSuccess; h0 += slice) {
       BwdArgs s = a;
       s.Hkv = min(slice, p.num_kv_heads - h0);
@@ -530,8 +544,14 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       s.dv = (char*)a.dv + h0 * a.dvs.h * es;
       s.ndelta = a.ndelta + hq0 * p.q_len;
       s.lse2 = a.lse2 + hq0 * p.q_len;
+      s.q_planes = a.q_planes + hq0 * p.q_len * width * 6;
+      s.do_planes = a.do_planes + hq0 * p.q_len * width * 6;
       if (a.aux.bias) s.aux.bias = a.aux.bias + hq0 * a.aux.bias_sh;
       if (a.aux.drop) s.aux.drop = a.aux.drop + hq0 * a.aux.drop_sh;
+      if (dt == AXL_F32) {
+        err = launch_bwd_f32(s, width, phases, stream);
+        continue;
+      }
       if (phases & AXL_BWD_DKDV) err = launch_bwd_dkdv(s, dt, width, aux, stream);
       if ((phases & AXL_BWD_DQ) && err == hipSuccess) err = launch_bwd_dq_stream(s, dt, width, stream);
     }

@@ -340,7 +340,7 @@ def flash_bwd_buffers(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, mask
 
     The workspace holds delta and the scaled lse (fp32 [B,Hq,T] each); with `segment_ids` (the ones the
     calls will pass) also the table of id ranges per 32 rows; with `ds_workspace=True` and a causal or
-    sliding-window `mask_kind` (equal lengths, no offsets) also dS, about T*S bytes per
+    sliding-window `mask_kind` (equal lengths, no offsets) also dS, about T*S bytes (float32: twice that) per
     (batch, head), for `flash_bwd(..., ds_workspace=True)` - of `ds_slice_kv_heads` kv heads at a time if that
     is given (the calls must pass the same number)."""
     b, t, hq, d = q.shape

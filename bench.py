@@ -348,7 +348,7 @@ def bench_f32_row(steps, warmup):
         arithmetic="fp32 operands as three bf16 parts each, six bf16 MFMA partial products per product, fp32 accumulation",
         fwd_ms=ms_fwd, bwd_ms=ms_bwd, fwd_tflops=fl_fwd / (ms_fwd * 1e-3) / 1e12,
         bwd_tflops=2.5 * fl_fwd / (ms_bwd * 1e-3) / 1e12, fp32_mfma_peak_tflops=MFMA_F32_PEAK_TFLOPS,
-        kernels=["flash_fwd_f32x_kernel", "flash_bwd_dkdv_f32x_kernel", "flash_bwd_dq_f32x_kernel"],
+        kernels=["flash_fwd_f32x_kernel", "split_planes_kernel", "flash_bwd_dkdv_f32x_kernel", "flash_bwd_dq_f32x_kernel"],
     )
 
 

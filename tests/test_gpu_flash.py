@@ -1440,3 +1440,40 @@ def test_forward_with_bf16_bias_alone(b, t, hq, hkv, d, mask, window, packed, sh
     out32, lse32 = ops.flash_fwd(*args, softmax_scale=d ** -0.5, bias=bias.float().cuda(), **kw)
     assert ref.rel_l2(out.cpu(), want) < 1e-2 and ref.rel_l2(out.cpu(), out32.cpu()) < 4e-3
     assert ref.max_abs(lse.cpu(), want_lse) < 1e-3 and ref.max_abs(lse.cpu(), lse32.cpu()) < 1e-4
+
+
+@pytest.mark.parametrize("t,hq,hkv,d,mask,window,packed,drop", [
+    (128, 2, 1, 64, "causal", None, False, False),      # half of dQ's block of 256 rows, one key block
+    (384, 6, 2, 128, "causal", None, False, True),      # an odd number of key blocks (one per workgroup), a last half block
+    (512, 8, 8, 128, "causal", None, True, False),      # two key blocks per workgroup, pairs a multiple of 8
+    (640, 4, 2, 128, "sliding", 33, False, False),      # windows that leave whole key tiles of a block without dS
+    (768, 4, 1, 64, "sliding", 0, True, True),          # every query sees itself alone
+    (512, 4, 2, 128, "sliding", 511, False, False),
+])
+def test_float32_ds_workspace_backward(t, hq, hkv, d, mask, window, packed, drop):
+    # fp32 with dS kept in the workspace: dk and dv are the bits of the call without it (the same kernel), dq,
+    # a kernel of its own, meets the fp32 bar against the oracle; whole and one kv head at a time.  The
+    # workspace starts as NaN, so a block that is read without having been written shows.
+    b = 2
+    q, k, v, do = _inputs(b, t, hq, hkv, d, torch.float32)
+    g = torch.Generator().manual_seed(t)
+    seg = ref.packed_segment_ids(3, b, t) if packed else None
+    spec, kw = _mask_args(mask, window, seg)
+    drop_mask = torch.rand(b, hq, t, t, generator=g) < 0.2 if drop else None
+    spec.dropout_mask, spec.dropout_rate = drop_mask, 0.2 if drop else 0.0
+    want = ref.reference_mha_grads(q, k, v, do, spec, softmax_scale=d ** -0.5, dropout_mask=drop_mask,
+                                   dropout_rate=0.2 if drop else 0.0)
+    kw.update(softmax_scale=d ** -0.5, dropout_mask=None if drop_mask is None else drop_mask.cuda(),
+              dropout_rate=0.2 if drop else 0.0)
+    args = (q.cuda(), k.cuda(), v.cuda())
+    out, lse = ops.flash_fwd(*args, **kw)
+    plain = ops.flash_bwd(*args, out, lse, do.cuda(), ds_workspace=False, **kw)
+    for heads in (0, 1):
+        bufs = ops.flash_bwd_buffers(*args, mask_kind=kw["mask_kind"], ds_workspace=True,
+                                     segment_ids=kw.get("segment_ids"), ds_slice_kv_heads=heads)
+        bufs[3].fill_(255)   # NaN in every word
+        got = ops.flash_bwd(*args, out, lse, do.cuda(), ds_workspace=True, ds_slice_kv_heads=heads, buffers=bufs, **kw)
+        assert torch.equal(got[1], plain[1]) and torch.equal(got[2], plain[2])
+        for name, x, y in zip(("dq", "dk", "dv"), got, want):
+            top = max(1.0, float(y.abs().max()))
+            assert ref.max_abs(x.cpu(), y) <= FP32_MAX_ABS * top, name
