@@ -80,6 +80,7 @@ __host__ __device__ inline int64_t ds32_run_start(int64_t pair, int T, int G, in
 // range of query tiles each key block stored.
 hipError_t launch_bwd_dkdv(const BwdArgs& a, int dtype, int head_dim, bool aux, hipStream_t stream);
 hipError_t launch_bwd_dkdv_aux(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
+hipError_t launch_bwd_dkdv_bias(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 
 // Enqueues the streaming dQ kernel, dq = scale * dS k from the dS blocks in a.ds (with a.kb_tbl set:
 // from the blocks that table says were stored).

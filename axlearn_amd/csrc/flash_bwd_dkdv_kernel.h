@@ -1,5 +1,5 @@
 // dK / dV kernel of the flash-attention backward for gfx950 (16-bit types), compiled in flash_bwd_dkdv.hip
-// (plain) and flash_bwd_dkdv_aux.hip (dense bias, dropout mask).
+// (plain), flash_bwd_dkdv_bias.hip (a bf16 bias alone) and flash_bwd_dkdv_aux.hip (other dense biases, dropout mask).
 //
 // Replaces axlearn/common/flash_attention/gpu_attention.py:436-528 (`_mha_backward_kernel_dkdv`):
 //   p = exp(qk - lse); dv += p^T dO; dp = dO v^T; ds = p * (dp - delta) * scale; dk += ds^T q,
@@ -37,7 +37,8 @@
 
 namespace axl {
 
-template <int D>
+// BIAS: with the bf16 bias of the tile's queries and the workgroup's keys beside it.
+template <int D, bool BIAS>
 struct DkvTile {
   static constexpr int BKV = 128;            // keys per workgroup (32 per wavefront)
   static constexpr int BQ = 32;              // query rows per LDS tile
@@ -45,13 +46,17 @@ struct DkvTile {
   static constexpr int TILE_BYTES = BQ * ROWB;                   // Q tile, then the dO tile
   static constexpr int STAT_BASE = 2 * TILE_BYTES;
   static constexpr int STAT_BYTES = 4 * BQ * 4;  // -lse*log2e | -delta | segment id | (unused) per query row
-  static constexpr int BUF_BYTES = STAT_BASE + STAT_BYTES;
+  static constexpr int BIAS_BASE = STAT_BASE + STAT_BYTES;
+  static constexpr int BIAS_ROWB = BKV * 2;                      // [query][key], 16-byte chunks swizzled by the query
+  static constexpr int BUF_BYTES = BIAS_BASE + (BIAS ? BQ * BIAS_ROWB : 0);
   static constexpr int NBUF = 6;
   static constexpr int RPI = 1024 / ROWB;                        // rows per direct-to-LDS instruction
   static constexpr int DMA_PER_WAVE = BQ / 4 / RPI;              // per tensor per tile (8 rows per wavefront)
-  static constexpr int DMA_PER_TILE = 2 * DMA_PER_WAVE + 1;      // Q, dO and one row of statistics
+  static constexpr int DMA_PER_TILE = 2 * DMA_PER_WAVE + 1 + (BIAS ? 2 : 0);  // Q, dO, one row of statistics, 8 rows of bias
   static constexpr int LDS_BYTES = NBUF * BUF_BYTES;
 };
+
+constexpr bool bias_through_lds(bool has_seg, int aux) { return aux == kAuxBias16 && !has_seg; }
 
 constexpr int kMaxSubDkv = 1024;                 // query tiles whose segment ids the dK/dV kernel classifies
 constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than one segment id
@@ -65,7 +70,13 @@ constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than 
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void flash_bwd_dkdv_kernel(const BwdArgs a) {
-  using Tile = DkvTile<D>;
+  // A bf16 bias alone comes through the tile ring like Q and dO, its elements read from LDS where they are used;
+  // everything else is the plain kernel.  The other inputs (fp32 bias, dropout mask, both, a bias beside segment
+  // ids, whose form of this kernel has no registers left) are fetched element by element into registers an
+  // iteration ahead: no room for mask-free loops and accumulators in vector registers, and half a microsecond
+  // for a load from HBM, which takes longer.  B2 H16 T2048 D128 causal with dS: 125 -> 104 us.
+  constexpr bool BIAS_LDS = bias_through_lds(HAS_SEG, AUX), LEAN = AUX == 0 || BIAS_LDS;
+  using Tile = DkvTile<D, BIAS_LDS>;
   constexpr bool HAS_BIAS = (AUX & (kAuxBias16 | kAuxBias32)) != 0, BIAS_F32 = (AUX & kAuxBias32) != 0;
   constexpr bool HAS_DROP = (AUX & kAuxDrop) != 0;
   constexpr int KK = D / 16, DT = D / 32;
@@ -137,12 +148,12 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   // between the smallest and the largest id of this workgroup's keys, and s_sub records for every query
   // tile from sub_g0 on whether its rows carry a single id (both from the table of per-group id ranges
   // that a small kernel leaves in the workspace).
-  __shared__ int s_sub[HAS_SEG && !AUX ? kMaxSubDkv : 1];
+  __shared__ int s_sub[HAS_SEG && LEAN ? kMaxSubDkv : 1];
   int sub_g0 = 0;
   if (HAS_SEG)
     sub_g0 = classify_segment_groups_tbl<256>(a.seg_tbl + (int64_t)b * (a.T / kSegGroupRows), k0_wg / kSegGroupRows,
                                               Tile::BKV / kSegGroupRows, tid, q_begin, q_end, s_sub,
-                                              AUX ? 0 : kMaxSubDkv, kNotUniformDkv);
+                                              LEAN ? kMaxSubDkv : 0, kNotUniformDkv);
   const int t_begin = q_begin / Tile::BQ;
   const int nt = max(0, (q_end + Tile::BQ - 1) / Tile::BQ - t_begin);
   if constexpr (SPILL) {
@@ -213,25 +224,51 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   // statistics rows are [B, Hq, T] fp32; segment ids do not depend on the head
   const int64_t s_step = s_is_seg ? 0 : (int64_t)a.T * 4;
   const int64_t s_wrap = s_is_seg ? dir * (int64_t)Tile::BQ * 4 : (-(int64_t)(G - 1) * a.T + dir * Tile::BQ) * 4;
+  // Bias rows 8 wave .. + 7 of the tile, four per load; the chunk a lane fetches is the one the swizzle puts at
+  // its slot.  64-bit lane offsets: a row stride has no bound.
+  const char* b_src = nullptr;
+  int64_t b_lane = 0, b_step = 0, b_wrap = 0;
+  if constexpr (BIAS_LDS) {
+    b_src = a.aux.bias + b * a.aux.bias_sb + (int64_t)(hk * G) * a.aux.bias_sh +
+            ((int64_t)t_first * Tile::BQ + 8 * wave) * a.aux.bias_sr + (int64_t)k0_wg * 2;
+    b_lane = (lane >> 4) * a.aux.bias_sr + (((lane & 15) ^ ((lane >> 4) << 2)) << 4);
+    b_step = a.aux.bias_sh;
+    b_wrap = -(int64_t)(G - 1) * a.aux.bias_sh + dir * (int64_t)Tile::BQ * a.aux.bias_sr;
+  }
   const unsigned lds0 = lds_address(smem);
-  // The k-th group of loads (Q rows, dO rows, statistics) of the cursor's tile into the buffer at LDS
-  // address BUF_; all from scalar bases, no vector instruction forms an address.
-  constexpr int NGRP = 3;
+  // The k-th group of loads (Q rows, dO rows, statistics, bias rows) of the cursor's tile into the buffer at LDS
+  // address BUF_; all but the bias from scalar bases, no vector instruction forms an address.
+  constexpr int NGRP = BIAS_LDS ? 4 : 3;
+  // The loads' scalar bases are wave-uniform, but with the bias's cursor beside the others the compiler keeps some of
+  // them in vector registers.
+  auto uni = [](const auto* p) __attribute__((always_inline)) {
+    if constexpr (BIAS_LDS) {
+      const uint64_t u = (uint64_t)p;
+      return (decltype(p))(((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32) |
+                           (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)u));
+    } else {
+      return p;
+    }
+  };
 #define AXL_DMA(BUF_, K_)                                                                          \
   {                                                                                               \
     if ((K_) == 0) {                                                                              \
-      if constexpr (PAIRS) dma16x2(q_lane[0], q_lane[Tile::DMA_PER_WAVE - 1], q_src, (BUF_) + wave * (8 * Tile::ROWB)); \
-      else dma16s(q_lane[0], q_src, (BUF_) + wave * (8 * Tile::ROWB));                            \
+      if constexpr (PAIRS) dma16x2(q_lane[0], q_lane[Tile::DMA_PER_WAVE - 1], uni(q_src), (BUF_) + wave * (8 * Tile::ROWB)); \
+      else dma16s(q_lane[0], uni(q_src), (BUF_) + wave * (8 * Tile::ROWB));                            \
     } else if ((K_) == 1) {                                                                       \
-      if constexpr (PAIRS) dma16x2(d_lane[0], d_lane[Tile::DMA_PER_WAVE - 1], d_src, (BUF_) + Tile::TILE_BYTES + wave * (8 * Tile::ROWB)); \
-      else dma16s(d_lane[0], d_src, (BUF_) + Tile::TILE_BYTES + wave * (8 * Tile::ROWB));         \
-    } else {                                                                                      \
-      dma16s_first8(s_lane, s_src, (BUF_) + Tile::STAT_BASE + st_kind * (Tile::BQ * 4));          \
+      if constexpr (PAIRS) dma16x2(d_lane[0], d_lane[Tile::DMA_PER_WAVE - 1], uni(d_src), (BUF_) + Tile::TILE_BYTES + wave * (8 * Tile::ROWB)); \
+      else dma16s(d_lane[0], uni(d_src), (BUF_) + Tile::TILE_BYTES + wave * (8 * Tile::ROWB));         \
+    } else if ((K_) == 2) {                                                                       \
+      dma16s_first8(s_lane, uni(s_src), (BUF_) + Tile::STAT_BASE + st_kind * (Tile::BQ * 4));          \
+    } else if constexpr (BIAS_LDS) {                                                              \
+      const unsigned bdst_ = (BUF_) + Tile::BIAS_BASE + wave * (8 * Tile::BIAS_ROWB);             \
+      dma16(b_src + b_lane, bdst_);                                                               \
+      dma16(b_src + 4 * a.aux.bias_sr + b_lane, bdst_ + 1024);                                    \
     }                                                                                             \
   }
 #define AXL_DMA_TILE(BUF_)                                                                         \
   {                                                                                               \
-    AXL_DMA(BUF_, 0) AXL_DMA(BUF_, 1) AXL_DMA(BUF_, 2)                                            \
+    AXL_DMA(BUF_, 0) AXL_DMA(BUF_, 1) AXL_DMA(BUF_, 2) AXL_DMA(BUF_, 3)                           \
   }
   // Prefetch cursor; it stops at the last tile (re-fetching that tile is harmless).
   int pf_idx = 0, pf_t = t_first - t_begin, pf_h = 0;  // tile number, query tile (from t_begin), head within the group
@@ -245,6 +282,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     q_src += adv_ ? (wrap_ ? q_wrap : q_step) : 0;                          \
     d_src += adv_ ? (wrap_ ? d_wrap : d_step) : 0;                          \
     s_src += adv_ ? (wrap_ ? s_wrap : s_step) : 0;                          \
+    if constexpr (BIAS_LDS) b_src += adv_ ? (wrap_ ? b_wrap : b_step) : 0;  \
   }
 
   char* buf_b = smem;                         // tile j     (stage B reads)
@@ -288,6 +326,13 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   for (int r = 0; r < 16; r++) s_e[r] = dp_e[r] = 0.f;
 
   floatx4 lse_v[4], del_v[4];
+  // BIAS_LDS: bias of this lane's key and queries 16 (i/2) + 8 g + 4 (i%2) .. + 3, by transposing reads.
+  shortx4 bias_v[4];
+  const int bias_off = (8 * g + ((lane & 15) >> 2)) * Tile::BIAS_ROWB + Tile::BIAS_BASE + (lane & 1) * 8 +
+                       (((4 * wave + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (((lane & 15) >> 2) << 2)) << 4);
+#define AXL_READ_BIAS(BUF_, I_) \
+  if constexpr (BIAS_LDS)       \
+    bias_v[I_] = lds_read_tr16((BUF_) + bias_off + (16 * ((I_) / 2) + 4 * ((I_) % 2)) * Tile::BIAS_ROWB);
   intx4 seg_v[4];
   int diff0 = 0;
   // Row statistics of the tile in BUF_: register r of lane group g is query q0 + 16(r/8) + 8g + (r%8).
@@ -317,7 +362,10 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
       if (HAS_SEG) sv_ = seg_v[r_ / 4][r_ % 4] == seg_k ? sv_ : kMasked;                       \
     }                                                                                          \
     float off_ = lse_v[r_ / 4][r_ % 4]; /* -lse * log2 e */                                    \
-    if constexpr (HAS_BIAS) {                                                                  \
+    if constexpr (BIAS_LDS) {                                                                  \
+      const unsigned bw_ = (unsigned)(uint16_t)bias_v[r_ / 4][r_ % 4] << 16;                   \
+      off_ = __builtin_fmaf(__builtin_bit_cast(float, bw_), kLog2e, off_);                     \
+    } else if constexpr (HAS_BIAS) {                                                           \
       /* bias raw bits: fp32 as loaded, bf16 in the low half.  The empty statement keeps the    \
          first use of the loaded register here, an iteration after its load: without it the     \
          shift (and the test of the dropout byte below) moves up to the load and waits there    \
@@ -341,7 +389,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
       dpv_ = kept_ ? dpv_ * a.aux.keep_scale : 0.f; /* gpu_attention.py:509-512 */            \
       s_e[r_] = kept_ ? p_ : 0.f; /* P that multiplies dO: dropped entries removed */          \
     }                                                                                          \
-    if constexpr (AUX) dp_e[r_] = p_ * (dpv_ + del_v[r_ / 4][r_ % 4]); /* del_v holds -delta */ \
+    if constexpr (!LEAN) dp_e[r_] = p_ * (dpv_ + del_v[r_ / 4][r_ % 4]); /* del_v holds -delta */ \
     else dp_e[r_] = p_ * dpv_; /* the dP chain started from -delta */                          \
   }
 #define AXL_ELEM(R_)                                                                           \
@@ -389,13 +437,13 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   // compiler, which keeps that distance for its own MFMAs, does not know what the assembly is.  The
   // wait below is placed after whatever wrote the registers and before the first MFMA.
 #define AXL_CHAIN_START(S_, DP_) \
-  if constexpr (!AUX) asm volatile("s_nop 7" : "+v"(S_), "+v"(DP_));
+  if constexpr (LEAN) asm volatile("s_nop 7" : "+v"(S_), "+v"(DP_));
   // Stage A of the tile in BUF_ into (S_, DP_), not interleaved with anything (pipeline fill).
 #define AXL_STAGE_A_PLAIN(BUF_, S_, DP_)                                                        \
   _Pragma("unroll") for (int kk = 0; kk < KK; kk++) {                                           \
     const bf16x8 qa_ = AXL_A_FRAG(BUF_, 0, kk);                                                 \
     const bf16x8 da_ = AXL_A_FRAG(BUF_, 1, kk);                                                 \
-    if constexpr (AUX) {                                                                        \
+    if constexpr (!LEAN) {                                                                      \
       S_ = E::mfma_32x32x16(qa_, kf[kk], S_);                                                   \
       DP_ = E::mfma_32x32x16(da_, vf[kk], DP_);                                                 \
     } else if (kk + 1 < KK) {                                                                   \
@@ -466,7 +514,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     q0_s2 = (t_begin + pf_t) * Tile::BQ;
     h_s2 = pf_h;
     AXL_DMA_TILE(lds_address(buf_s))
-    if constexpr (AUX) {                 // bias / dropout columns of tile 0
+    if constexpr (!LEAN) {               // bias / dropout columns of tile 0
       const char* bp_;
       const uint8_t* dp_;
       AXL_AUX_ROW0(0, t_first * Tile::BQ, bp_, dp_)
@@ -478,7 +526,9 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     // Pipeline fill: stage A and the elementwise stage of tile 0, stage A of tile 1.
     AXL_READ_STATS_PART(buf_b, 0, lse_v, del_v, seg_v)
     AXL_READ_STATS_PART(buf_b, 1, lse_v, del_v, seg_v)
-    if constexpr (!AUX) {  // the dP chain starts from -delta
+#pragma unroll
+    for (int i = 0; i < 4; i++) AXL_READ_BIAS(buf_b, i)
+    if constexpr (LEAN) {  // the dP chain starts from -delta
 #pragma unroll
       for (int r = 0; r < 16; r++) dp_e[r] = del_v[r / 4][r % 4];
     }
@@ -493,13 +543,15 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     for (int r = 0; r < 16; r++) s_e[r] = dp_e[r] = 0.f;
     AXL_READ_STATS_PART(buf_e, 0, lse_v, del_v, seg_v)
     AXL_READ_STATS_PART(buf_e, 1, lse_v, del_v, seg_v)
-    if constexpr (!AUX) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) AXL_READ_BIAS(buf_e, i)
+    if constexpr (LEAN) {
 #pragma unroll
       for (int r = 0; r < 16; r++) dp_e[r] = del_v[r / 4][r % 4];
     }
     AXL_CHAIN_START(s_e, dp_e)
     AXL_STAGE_A_PLAIN(buf_e, s_e, dp_e)
-    if constexpr (AUX) {                 // ... and of tile 1, for the first iteration
+    if constexpr (!LEAN) {               // ... and of tile 1, for the first iteration
       const char* bp_;
       const uint8_t* dp_;
       AXL_AUX_ROW0(h_1, q0_1, bp_, dp_)
@@ -525,10 +577,10 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     constexpr bool MASKED = decltype(masked_c)::value;
   // One iteration.  (s_e, dp_e): tile j + 1; (pb, dsb): tile j, packed; (s_a, dp_a): the stage-A
   // accumulators of tile j + 2; (pb_n, dsb_n): tile j + 1, packed as its elements complete.
-  // Without a bias / dropout mask the stage-A chains accumulate in vector registers
+  // Without a dropout mask or an fp32 bias the stage-A chains accumulate in vector registers
   // (mfma_32x32x16_vgpr): the next iteration's elementwise stage reads them where they are.  Its first
   // read of s comes after that iteration's first MFMA and after the last MFMA of the dP chain, its
-  // first read of dp two slots later.  The bias / dropout instantiations, which run out of vector
+  // first read of dp two slots later.  The other instantiations, which run out of vector
   // registers, keep the compiler's own form.
   auto iter = [&](floatx16& s_e, floatx16& dp_e, PackedOperand& pb, PackedOperand& dsb, floatx16& s_a, floatx16& dp_a,
                   PackedOperand& pb_n, PackedOperand& dsb_n, uint32_t (&braw_v)[16], uint32_t (&draw_v)[16],
@@ -553,7 +605,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     }
     const char* bias_t = nullptr;        // bias / dropout columns of tile j + 2 go to (braw_n, draw_n)
     const uint8_t* drop_t = nullptr;
-    if constexpr (AUX) AXL_AUX_ROW0(h_a, q0_a, bias_t, drop_t)
+    if constexpr (!LEAN) AXL_AUX_ROW0(h_a, q0_a, bias_t, drop_t)
     if constexpr (SPILL) {
       // dS of tile j (this iteration's stage-B operand), ahead of the iteration's tile loads: by the
       // end of the iteration the stores have long been accepted.
@@ -589,7 +641,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
           dk_acc[dt] = E::mfma_32x32x16(bfr[n].v, dsb.v[t8], dk_acc[dt]);
       } else {
         constexpr int x = n - NB;
-        if constexpr (AUX) {
+        if constexpr (!LEAN) {
           if constexpr (x % 2 == 0) s_a = E::mfma_32x32x16(afr[x], kf[x / 2], x == 0 ? zero16 : s_a);
           else dp_a = E::mfma_32x32x16(afr[x], vf[x / 2], x == 1 ? zero16 : dp_a);
         } else {
@@ -618,7 +670,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
         q0_p = (t_begin + pf_t) * Tile::BQ;
         h_p = pf_h;
       }
-      if constexpr (AUX) {
+      if constexpr (!LEAN) {
         if (n % ESTEP == 0) AXL_AUX_LOAD(bias_t, drop_t, n / ESTEP, braw_n, draw_n)
       }
       if constexpr (n >= LD_SLOT0 && n < LD_SLOT0 + NGRP) AXL_DMA(lds_s, n - LD_SLOT0)
@@ -630,8 +682,9 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
         if (n == (4 * i + 3) * (NS - 3) / 16 + 1) {
           lse_v[i] = *(const floatx4*)st_;
           if (HAS_SEG) seg_v[i] = *(const intx4*)(st_ + 2 * Tile::BQ * 4);
+          AXL_READ_BIAS(buf_a, i)
         }
-        if constexpr (AUX) {
+        if constexpr (!LEAN) {
           if (n == (4 * i + 3) * (NS - 3) / 16 + 3) del_v[i] = *(const floatx4*)(st_ + Tile::BQ * 4);
         } else {
           // -delta of tile j+2's rows: what its dP chain starts from (slot NB + 1), loaded into the
@@ -652,13 +705,13 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     // iteration refills.  (With a bias or a dropout mask, at least 43 of their element loads - 11 of
     // the iteration before last, 16 of each iteration since - are younger than tile j+3's loads as
     // well; 40 leaves a margin.)
-    wait_vmem_le<2 * NLD + (AUX ? 40 : 0)>();
+    wait_vmem_le<2 * NLD + (LEAN ? 0 : 40)>();
     __syncthreads();
     // The stage-A chains of the last slots were issued through inline assembly, so the compiler places
     // no wait states behind them; where a run of iterations ends it may move values into their
     // registers a few instructions after this barrier.  Eight wait states here bring every such write
     // to at least the 12 the hardware wants after the last MFMA of a chain, whatever the barrier took.
-    if constexpr (!AUX) asm volatile("s_nop 7");
+    if constexpr (LEAN) asm volatile("s_nop 7");
     char* const tmp = buf_b;
     buf_b = buf_e;
     buf_e = buf_a;
@@ -682,12 +735,12 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     if (j < j_to) {
       // odd count: one more iteration, then the sets go back to their roles with one copy per run
       iter(s_e, dp_e, pb, dsb, s_x, dp_x, pb_x, dsb_x, braw_v, draw_v, braw_w, draw_w);
-      if constexpr (!AUX) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(s_x), "+v"(dp_x));  // the chains have just ended
+      if constexpr (LEAN) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(s_x), "+v"(dp_x));  // the chains have just ended
       s_e = s_x;
       dp_e = dp_x;
       pb = pb_x;
       dsb = dsb_x;
-      if constexpr (AUX) {
+      if constexpr (!LEAN) {
 #pragma unroll
         for (int r = 0; r < 16; r++) {
           braw_v[r] = braw_w[r];
@@ -707,7 +760,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     if (a.mask_kind == AXL_MASK_SLIDING_WINDOW)
       u_hi = min(nt - 1, floor_div(a.window + k0 - 31 - a.q_off, Tile::BQ) - t_begin);
   }
-  if (HAS_SEG && !AUX) {
+  if (HAS_SEG && LEAN) {
     // Query tiles whose 32 rows all carry the segment id that all 32 keys of this wavefront carry
     // need no segment mask either: take the first run [tA, tB) of such tiles (the masked loop is
     // always correct, so whatever lies outside that run simply stays on it).
@@ -735,7 +788,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   }
   u_lo = min(u_lo, nt);
   u_hi = max(u_hi, u_lo - 1);
-  if constexpr (AUX) {
+  if constexpr (!LEAN) {
     run(0, total, std::true_type{});  // every tile takes the masked path
   } else {
     int j = 0;
@@ -750,6 +803,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     run_to(total, std::true_type{});
     run(j, total, std::true_type{});  // the last iteration (its elementwise tile is past the end)
   }
+#undef AXL_READ_BIAS
 #undef AXL_AUX_ROW0
 #undef AXL_AUX_LOAD
   // The cursor re-requests the last tile during the final iterations (which keeps the count of
@@ -785,7 +839,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
       w.p[1] = E::pack(dk_acc[dt][4 * rq + 2] * a.scale, dk_acc[dt][4 * rq + 3] * a.scale);
       const bool in_row = 32 * dt + 8 * rq + 4 * g < a.d_real;
       if (in_row) *(uint2*)(dkp + 32 * dt + 8 * rq + 4 * g) = w.u;
-      const float vs = AUX ? a.aux.keep_scale : 1.0f;  // kept probabilities are P / (1 - rate)
+      const float vs = LEAN ? 1.0f : a.aux.keep_scale;  // kept probabilities are P / (1 - rate)
       w.p[0] = E::pack(dv_acc[dt][4 * rq + 0] * vs, dv_acc[dt][4 * rq + 1] * vs);
       w.p[1] = E::pack(dv_acc[dt][4 * rq + 2] * vs, dv_acc[dt][4 * rq + 3] * vs);
       if (in_row) *(uint2*)(dvp + 32 * dt + 8 * rq + 4 * g) = w.u;
@@ -796,7 +850,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
-  using Tile = DkvTile<D>;
+  using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
   auto kernel = flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;

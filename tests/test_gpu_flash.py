@@ -1477,3 +1477,31 @@ def test_float32_ds_workspace_backward(t, hq, hkv, d, mask, window, packed, drop
         for name, x, y in zip(("dq", "dk", "dv"), got, want):
             top = max(1.0, float(y.abs().max()))
             assert ref.max_abs(x.cpu(), y) <= FP32_MAX_ABS * top, name
+
+
+@pytest.mark.parametrize("b,t,s,hq,hkv,d,dtype,mask,window,kind,ds", [
+    (1, 128, 128, 2, 1, 128, torch.bfloat16, "causal", None, "bh", True),    # four tiles: the ring is deeper than the walk
+    (2, 384, 384, 6, 2, 64, torch.bfloat16, "causal", None, "1h", True),     # three heads a group: the bias cursor wraps
+    (2, 512, 512, 8, 4, 128, torch.bfloat16, "causal", None, "11", True),    # two key blocks, up and down, one bias for all
+    (1, 640, 640, 4, 2, 128, torch.float16, "sliding", 150, "b1", True),
+    (2, 256, 384, 4, 2, 128, torch.bfloat16, "none", None, "bh", False),
+    (1, 512, 512, 4, 4, 64, torch.bfloat16, "causal", None, "strided", False),  # rows further apart than they are long
+])
+def test_dkdv_with_bf16_bias_alone(b, t, s, hq, hkv, d, dtype, mask, window, kind, ds):
+    # dK/dV with the bias tiles in LDS, against the oracle and against the form that reads elements from global
+    # memory, which the same values in fp32 take: P and dS round alike there, one rounding of the results apart.
+    q, k, v, do = _inputs(b, t, hq, hkv, d, dtype, s=s)
+    shape = dict(bh=(b, hq), b1=(b, 1)).get(kind, (1, hq)) if kind != "11" else (1, 1)
+    bias = ref.normal_tensor(9, (*shape, t, s + (24 if kind == "strided" else 0)), torch.bfloat16)[..., :s]
+    spec, kw = _mask_args(mask, window, None)
+    spec.dense_bias = bias.float()
+    want = ref.reference_mha_grads(q, k, v, do, spec, softmax_scale=d ** -0.5)
+    args = (q.cuda(), k.cuda(), v.cuda())
+    kw.update(softmax_scale=d ** -0.5)
+    full = ref.normal_tensor(9, (*shape, t, s + (24 if kind == "strided" else 0)), torch.bfloat16).cuda()[..., :s]
+    out, lse = ops.flash_fwd(*args, bias=full, **kw)
+    got = ops.flash_bwd(*args, out, lse, do.cuda(), bias=full, ds_workspace=ds, **kw)
+    other = ops.flash_bwd(*args, out, lse, do.cuda(), bias=full.float(), ds_workspace=ds, **kw)
+    for name, x, y, w in zip(("dq", "dk", "dv"), got, other, want):
+        assert ref.rel_l2(x.cpu(), y.cpu()) < 4e-3, name       # two roundings to 16 bits of the same sums
+        assert ref.rel_l2(x.cpu(), w) < (1e-2 if dtype == torch.bfloat16 else 1.25e-3), name

@@ -615,6 +615,16 @@ def test_dkdv_kernel_keeps_its_vector_register_accumulators_in_place():
     _assert_asm_mfma_distances(asm, r"_ZN3axl21flash_bwd_dkdv_kernel", 16)
 
 
+def test_dkdv_kernel_with_a_bf16_bias_keeps_its_chains_in_place():
+    """The dK/dV instantiations with a bf16 bias alone use the plain ones' inline-assembly chains, with the bias
+    tiles' cursor and fragments beside them: nothing spills to scratch memory, every direct-to-LDS load has a
+    scalar base, and the hazard distances hold on every path."""
+    asm, remarks = _device_asm("flash_bwd_dkdv_bias.hip")
+    assert re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", remarks) == ["0"] * 8
+    assert not re.search(r"global_load_lds_dwordx4 v\d+, v\[", asm)
+    _assert_asm_mfma_distances(asm, r"_ZN3axl21flash_bwd_dkdv_kernel", 8)
+
+
 def test_forward_kernel_keeps_the_distance_behind_its_assembly_mfma_chains():
     """The same for the forward's interior tiles, whose S^T chains of the next tile are inline-assembly
     MFMAs read by the softmax of the next step: the hazard distance on every path of the four
