@@ -1140,7 +1140,7 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
   constexpr int QS = Tile::QSTRIDE / 4;
 
   const int tid = threadIdx.x;
-  const int wave = tid >> 6, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   int qb, b, h;
   decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 1 << 20, qb, b, h);
   const int hk = h / (a.Hq / a.Hkv);
@@ -1191,10 +1191,6 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
   const int qpos_min = q0 + q_off, qpos_max = q0 + 31 + q_off;
   const int seg_q = a.seg ? a.seg[(int64_t)b * a.T + q0 + l32] : 0;
   const int32_t* seg_k = a.seg ? a.seg + (int64_t)b * a.T : nullptr;
-  const char* bias_row = nullptr;
-  const uint8_t* drop_row = nullptr;
-  if (a.aux.bias) bias_row = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh + (int64_t)(q0 + l32) * a.aux.bias_sr;
-  if (a.aux.drop) drop_row = a.aux.drop + b * a.aux.drop_sb + h * a.aux.drop_sh + (int64_t)(q0 + l32) * a.aux.drop_sr;
 
   floatx16 o[DT];
 #pragma unroll
@@ -1209,12 +1205,13 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
   // The K / V tile of 32 keys from global memory into this thread's registers, and from there, split, into
   // a ring buffer: the next tile's round trip runs under the current tile's MFMAs, one barrier per tile.
   float4 kx[Tile::LD4], vx[Tile::LD4];
+  const int64_t k_lane = (tid / (D / 4)) * a.ks.s + tid % (D / 4) * 4, v_lane = (tid / (D / 4)) * a.vs.s + tid % (D / 4) * 4;
+  constexpr int ROW_STEP = Tile::NT / (D / 4);
   auto request = [&](int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < Tile::LD4; i++) {
-      const int e = tid + i * Tile::NT, row = e / (D / 4), c4 = e % (D / 4);
-      kx[i] = *(const float4*)(kp + (int64_t)(k0 + row) * a.ks.s + c4 * 4);
-      vx[i] = *(const float4*)(vp + (int64_t)(k0 + row) * a.vs.s + c4 * 4);
+      kx[i] = *(const float4*)(kp + (int64_t)(k0 + i * ROW_STEP) * a.ks.s + k_lane);
+      vx[i] = *(const float4*)(vp + (int64_t)(k0 + i * ROW_STEP) * a.vs.s + v_lane);
     }
   };
   auto deposit = [&](int t) __attribute__((always_inline)) {
@@ -1238,8 +1235,23 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
   if (t_begin < t_end) {
     request(t_begin * Tile::BK);
     deposit(t_begin);
+    if (t_begin + 1 < t_end) request((t_begin + 1) * Tile::BK);
   }
   __syncthreads();
+  // Tile t + 1 from registers into LDS (that buffer was last read a tile ago, before the barrier that ended it), tile
+  // t + 2 on its way.  Of the two wavefronts of a SIMD (NW = 8) one does it ahead of its MFMAs, the other behind
+  // them: its splitting falls on the other one's MFMAs.
+  auto advance = [&](int t) __attribute__((always_inline)) {
+    if (t + 1 < t_end) deposit(t + 1);
+    if (t + 2 < t_end) request((t + 2) * Tile::BK);
+  };
+  // l32, hidden from the compiler: addresses that are rarely needed are not kept in registers from tile to tile.
+  auto own_row = [&]() __attribute__((always_inline)) {
+    int r = l32;
+    asm volatile("" : "+v"(r));
+    return r;
+  };
+  const bool advance_first = NW == 8 && wave >= 4;
 
   // Per-lane read offsets.  K: the row of key swap_bits_2_3(l32), 16 bytes at d = 16 s + 8 g.  V: transposing
   // reads at row 8 g + j16 / 4 (+4 for the second half, +16 for the tile's second 16 keys), columns
@@ -1250,8 +1262,7 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
 
   for (int t = t_begin; t < t_end; t++) {
     const int k0 = t * Tile::BK;
-    const bool more = t + 1 < t_end;
-    if (more) request(k0 + Tile::BK);
+    if (advance_first) advance(t);
     const char* k_lds = smem + (t & 1) * Tile::BUF_BYTES;
     const char* v_lds = k_lds + 3 * Tile::KPLANE;
     bool skip = false;
@@ -1265,15 +1276,23 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
     floatx16 s;
 #pragma unroll
     for (int r = 0; r < 16; r++) s[r] = 0.f;
+    // the fragments of the next step are read ahead of the current step's MFMAs, here and for V below
+    bf16x8 kf[2][3];
+    auto read_k = [&](int ks) __attribute__((always_inline)) {
+#pragma unroll
+      for (int p = 0; p < 3; p++) kf[ks & 1][p] = *(const bf16x8*)(k_lds + p * Tile::KPLANE + k_off + 32 * ks);
+    };
+    read_k(0);
 #pragma unroll
     for (int ks = 0; ks < KSTEPS; ks++) {
-      bf16x8 kf[3];
-#pragma unroll
-      for (int p = 0; p < 3; p++) kf[p] = *(const bf16x8*)(k_lds + p * Tile::KPLANE + k_off + 32 * ks);
-      s = mfma_split(kf, q_mine[ks], s);
+      if (ks + 1 < KSTEPS) read_k(ks + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      s = mfma_split(kf[ks & 1], q_mine[ks], s);
+      __builtin_amdgcn_sched_barrier(0);
     }
     // Register r of lane group g is key k0 + 16 (r / 8) + 8 g + r % 8.
-    if (bias_row) {  // logits = scale * qk + bias, in units of log2
+    if (a.aux.bias) {  // logits = scale * qk + bias, in units of log2
+      const char* bias_row = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh + (int64_t)(q0 + own_row()) * a.aux.bias_sr;
 #pragma unroll
       for (int r4 = 0; r4 < 4; r4++) {
         float bv[4];
@@ -1326,7 +1345,8 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
       lsum += s[r];
     }
     l_run += lsum;
-    if (drop_row) {  // dropped probabilities leave P V but stay in the row sum
+    if (a.aux.drop) {  // dropped probabilities leave P V but stay in the row sum
+      const uint8_t* drop_row = a.aux.drop + b * a.aux.drop_sb + h * a.aux.drop_sh + (int64_t)(q0 + own_row()) * a.aux.drop_sr;
 #pragma unroll
       for (int r4 = 0; r4 < 4; r4++) {
         const unsigned w = *(const unsigned*)(drop_row + k0 + 16 * (r4 / 2) + 8 * g + 4 * (r4 % 2));
@@ -1335,29 +1355,36 @@ __global__ __launch_bounds__(64 * NW) void flash_fwd_f32x_kernel(const FwdArgs a
       }
     }
     // O^T[d][q] += V^T[d][key] P^T[key][q], 16 keys per step.
+    bf16x8 vf[2][3], pf[3];
+    auto read_v = [&](int n) __attribute__((always_inline)) {
 #pragma unroll
-    for (int kk = 0; kk < 2; kk++) {
-      float pr[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) pr[j] = s[8 * kk + j];
-      Split3x8 ps;
-      split3x8(pr, ps);
-      const bf16x8 pf[3] = {ps.part[0].v, ps.part[1].v, ps.part[2].v};
-#pragma unroll
-      for (int dt = 0; dt < DT; dt++) {
-        union { bf16x8 v; shortx4 hlf[2]; } vf[3];
-#pragma unroll
-        for (int p = 0; p < 3; p++) {
-          const char* va = v_lds + p * Tile::VPLANE + v_off + 16 * kk * Tile::VSTRIDE + 64 * dt;
-          vf[p].hlf[0] = lds_read_tr16(va);
-          vf[p].hlf[1] = lds_read_tr16(va + 4 * Tile::VSTRIDE);
-        }
-        const bf16x8 vfa[3] = {vf[0].v, vf[1].v, vf[2].v};
-        o[dt] = mfma_split(vfa, pf, o[dt]);
+      for (int p = 0; p < 3; p++) {
+        union { bf16x8 v; shortx4 hlf[2]; } u;
+        const char* va = v_lds + p * Tile::VPLANE + v_off + 16 * (n / DT) * Tile::VSTRIDE + 64 * (n % DT);
+        u.hlf[0] = lds_read_tr16(va);
+        u.hlf[1] = lds_read_tr16(va + 4 * Tile::VSTRIDE);
+        vf[n & 1][p] = u.v;
       }
+    };
+    read_v(0);
+#pragma unroll
+    for (int n = 0; n < 2 * DT; n++) {
+      if (n % DT == 0) {
+        float pr[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) pr[j] = s[8 * (n / DT) + j];
+        Split3x8 ps;
+        split3x8(pr, ps);
+#pragma unroll
+        for (int p = 0; p < 3; p++) pf[p] = ps.part[p].v;
+      }
+      if (n + 1 < 2 * DT) read_v(n + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      o[n % DT] = mfma_split(vf[n & 1], pf, o[n % DT]);
+      __builtin_amdgcn_sched_barrier(0);
     }
     }  // tile not skipped
-    if (more) deposit(t + 1);  // that buffer was last read a tile ago, before the barrier that ended it
+    if (!advance_first) advance(t);
     __syncthreads();
   }
 
