@@ -103,27 +103,33 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
     const int begin = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? max(0, end - a.T - a.window) : 0;
     return (max(end, begin + 1) - begin + 63) / 64;
   };
+  // The plan stands at the head of both kernels' chains of latencies: the lengths of the first 64 sequences are read
+  // once, and the reductions go over no more lanes than there are sequences (2 x 200 rows of 32 heads over 8192 keys:
+  // chunk kernel 40.5 -> 38.5 us, merge 10.4 -> 9.2 us).
+  const int own = tiles(lane);
+  auto tiles_of = [&](int b) -> int { return b == lane ? own : tiles(b); };
+  const int span = a.B >= 64 ? 64 : a.B <= 1 ? 1 : 2 << (31 - __builtin_clz(a.B - 1));   // power of two, lanes with work
+  auto sum = [&](int x) -> int {
+    for (int o = span >> 1; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return __builtin_amdgcn_readfirstlane(x);
+  };
   int total = 0;
-  for (int b = lane; b < a.B; b += 64) total += tiles(b);
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o);
+  for (int b = lane; b < a.B; b += 64) total += tiles_of(b);
+  total = sum(total);
   const int per = nqb * a.Hkv;
   // at least 8 tiles (512 keys) each: below that a workgroup's fixed costs weigh more than what it takes over
   int target = max(8, (int)((int64_t)total * per / a.slots));
   for (;; target += 1 + target / 16) {
     int n = 0;
-    for (int b = lane; b < a.B; b += 64) n += (tiles(b) + target - 1) / target;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
-    if (n * per <= a.slots) break;
+    for (int b = lane; b < a.B; b += 64) n += (tiles_of(b) + target - 1) / target;
+    if (sum(n) * per <= a.slots) break;
   }
   ChunkShare r{-1, 1, 0};
   int before = 0;
   for (int base = 0; base < a.B; base += 64) {
-    const int n = (tiles(base + lane) + target - 1) / target;
+    const int n = (tiles_of(base + lane) + target - 1) / target;
     int incl = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
+    for (int o = 1; o < span; o <<= 1) {
       const int up = __shfl_up(incl, o);
       if (lane >= o) incl += up;
     }
@@ -135,7 +141,7 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
       r.first = (before + __builtin_amdgcn_readlane(incl, l) - r.nsplit) * nqb;
       break;
     }
-    before += __builtin_amdgcn_readlane(incl, 63);
+    before += __builtin_amdgcn_readlane(incl, span - 1);
   }
   return r;
 }
@@ -844,7 +850,7 @@ void flash_chunk_kernel(const FwdArgs a) {
 // Merges the partial results of the chunk form, out = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s in the
 // order of the splits.  One workgroup per 32-row block, a wavefront per 32 columns of head_dim, the
 // pieces read as they were written (1 KB per instruction, four per split in flight).  Bound by the
-// bytes: the partials of the chunk above (504 workgroups) are 30 MB in 10 us.
+// bytes: the partials of the chunk above (504 workgroups) are 30 MB in 8.6 us.
 template <typename E, int D>
 __global__ __launch_bounds__(2 * D) void flash_chunk_combine_kernel(const FwdArgs a) {
   const int lane = threadIdx.x & 63, dt = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
@@ -855,22 +861,40 @@ __global__ __launch_bounds__(2 * D) void flash_chunk_combine_kernel(const FwdArg
   if (sh.nsplit == 1) return;   // stored by the one workgroup that had the keys
   const char* part = a.part + (((int64_t)(sh.first + blk / 4) * a.Hkv + hk) * 4 + blk % 4) * ChunkPart<D>::BYTES;
   const int64_t split_bytes = (int64_t)nqb * a.Hkv * 4 * ChunkPart<D>::BYTES;
+  // One pass with a running maximum, kBatch parts in flight: each part's statistics and values come together
+  // (maxima first and the values two parts at a time: 9.2 us instead of 8.6 for 2 x 200 rows of 32 heads).
+  constexpr int kBatch = 4;
   float mx = 2.f * kNegInf;
-  for (int s = 0; s < sh.nsplit; s++)
-    mx = fmaxf(mx, *(const float*)(part + s * split_bytes + ChunkPart<D>::O_BYTES + 8 * l32));
   floatx4 acc[4] = {};
   float l = 0.f;
-#pragma unroll 2
-  for (int s = 0; s < sh.nsplit; s++) {
-    const char* p = part + s * split_bytes;
-    const floatx2 ml = *(const floatx2*)(p + ChunkPart<D>::O_BYTES + 8 * l32);
-    const float w = ml[1] > 0.f ? fast_exp2(ml[0] - mx) : 0.f;
-    l += w * ml[1];
+  for (int s0 = 0; s0 < sh.nsplit; s0 += kBatch) {
+    floatx2 ml[kBatch];
+    floatx4 o[kBatch][4];
 #pragma unroll
-    for (int rq = 0; rq < 4; rq++) {
-      const floatx4 o = *(const floatx4*)(p + (4 * dt + rq) * 1024 + 16 * lane);
+    for (int i = 0; i < kBatch; i++) {
+      const char* p = part + min(s0 + i, sh.nsplit - 1) * split_bytes;   // past the end: the last one, not counted
+      ml[i] = *(const floatx2*)(p + ChunkPart<D>::O_BYTES + 8 * l32);
 #pragma unroll
-      for (int j = 0; j < 4; j++) acc[rq][j] = ml[1] > 0.f ? __builtin_fmaf(w, o[j], acc[rq][j]) : acc[rq][j];
+      for (int rq = 0; rq < 4; rq++) o[i][rq] = *(const floatx4*)(p + (4 * dt + rq) * 1024 + 16 * lane);
+    }
+    float mn = mx;
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) mn = fmaxf(mn, ml[i][0]);
+    const float f = fast_exp2(mx - mn);
+    mx = mn;
+    l *= f;
+#pragma unroll
+    for (int rq = 0; rq < 4; rq++) acc[rq] *= f;
+#pragma unroll
+    for (int i = 0; i < kBatch; i++) {
+      if (s0 + i >= sh.nsplit) continue;
+      const bool any = ml[i][1] > 0.f;
+      const float w = any ? fast_exp2(ml[i][0] - mx) : 0.f;
+      l += w * ml[i][1];
+#pragma unroll
+      for (int rq = 0; rq < 4; rq++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc[rq][j] = any ? __builtin_fmaf(w, o[i][rq][j], acc[rq][j]) : acc[rq][j];
     }
   }
   const int r = 32 * blk + l32;
