@@ -204,6 +204,10 @@ class CompositeAttentionBias(BaseAttentionBias):
         if not members:
             return None
         total = members[0].value()
+        # Not `0.0 + total`: that read and wrote every element of a lone dense bias.  It stays where it
+        # changes what a kernel sees: integers become floats, an expanded or strided view becomes dense rows.
+        if len(members) == 1 and not (total.is_floating_point() and total.is_contiguous()):
+            total = 0.0 + total
         for b in members[1:]:
             total = total + b.value()
         return total

@@ -367,6 +367,8 @@ class HipFlashAttention(BaseFlashAttention):
             kind = (ops.MASK_NONE, 0)
         if dense is not None:
             dense = dense.to(query.device)
+            if dense.data_ptr() % 16:  # a view into a larger tensor; the kernels load 16 bytes at a time
+                dense = dense.clone()
         seg = get_segment_ids(query=query, key=key, segment_ids=segment_ids)
         rate = float(self.cfg.dropout_rate)
         dropout_mask = None

@@ -1505,3 +1505,29 @@ def test_dkdv_with_bf16_bias_alone(b, t, s, hq, hkv, d, dtype, mask, window, kin
     for name, x, y, w in zip(("dq", "dk", "dv"), got, other, want):
         assert ref.rel_l2(x.cpu(), y.cpu()) < 4e-3, name       # two roundings to 16 bits of the same sums
         assert ref.rel_l2(x.cpu(), w) < (1e-2 if dtype == torch.bfloat16 else 1.25e-3), name
+
+
+def _layer_call(q, k, v, biases, **kw):
+    bias = ab.CompositeAttentionBias(biases)
+    fn = flash_attention_implementation("gpu", query=q, key=k, value=v, bias=bias, softmax_scale=q.shape[-1] ** -0.5, **kw)
+    return fn(dict(query=q, key=k, value=v, bias=bias))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_dense_bias_given_as_a_view(dtype):
+    # One row for all queries, a window into a larger tensor whose rows start between two 16-byte boundaries,
+    # a storage that starts there: the same bits as from a dense copy, forward and gradients.
+    b, t, h, d = 2, 256, 2, 64
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, h, h, d, torch.bfloat16))
+    gen = torch.Generator().manual_seed(5)
+    wide = torch.randn(1, h, t, t + 8, generator=gen).to(dtype).cuda()
+    flat = torch.randn(h * t * t + 8, generator=gen).to(dtype).cuda()
+    pos = dict(target_positions=torch.arange(t)[None], source_positions=torch.arange(t)[None])
+    for view in (wide[:, :, :1, :t].expand(1, h, t, t), wide[..., 1:t + 1], wide[..., :t].transpose(2, 3),
+                 flat[1:1 + h * t * t].view(1, h, t, t)):
+        got = []
+        for bias in (view, view.clone(memory_format=torch.contiguous_format)):
+            leaves = [x.clone().requires_grad_(True) for x in (q, k, v)]
+            out = _layer_call(*leaves, [ab.CausalAttentionBias(**pos), ab.TensorAttentionBias(bias)])
+            got.append([out, *torch.autograd.grad(out, leaves, do)])
+        assert all(torch.equal(x, y) for x, y in zip(*got))

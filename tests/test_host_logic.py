@@ -80,6 +80,17 @@ def test_composite_bias_and_split():
         ab.CompositeAttentionBias([]).eval_shape()
 
 
+def test_value_of_a_lone_member_is_what_adding_zero_gives():
+    """A lone float bias in dense rows comes back as it is; everything else as `0.0 + bias` makes it."""
+    base = torch.randn(1, 4, 8, 24, generator=torch.Generator().manual_seed(0))
+    assert ab.CompositeAttentionBias([ab.TensorAttentionBias(base)]).value() is base
+    for view in (base[:, :, :1].expand(1, 4, 8, 24), base[..., 1:17], base.transpose(2, 3), base[..., ::2],
+                 torch.arange(192).reshape(1, 1, 8, 24), base > 0):
+        got = ab.CompositeAttentionBias([ab.TensorAttentionBias(view)]).value()
+        want = 0.0 + view
+        assert torch.equal(got, want) and got.dtype == want.dtype and got.stride() == want.stride()
+
+
 def test_structured_masks_combine():
     t = 8
     pos = dict(target_positions=torch.arange(t)[None], source_positions=torch.arange(t)[None])
