@@ -21,6 +21,7 @@ import logging
 from typing import Optional, Tuple
 
 import torch
+from torch.autograd import forward_ad
 
 from axlearn_amd import ops
 from axlearn_amd.attention_bias import (
@@ -130,8 +131,7 @@ def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, lo
     if runs_at_native_head_dim(query, key, value, aux=bias is not None or dropout_mask is not None):
         width = head_dim
     query, key, value = _pad_last(query, width), _pad_last(key, width), _pad_last(value, width)
-    if torch.is_grad_enabled() and (query.requires_grad or key.requires_grad or value.requires_grad
-                                    or (logit_sink is not None and logit_sink.requires_grad)):
+    if _differentiated(query, key, value, logit_sink, bias):
         out = _FlashAttentionFn.apply(
             query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink, bias, dropout_mask,
             dropout_rate, save_residuals, bwd_ds_workspace, bwd_workspace_limit_bytes,
@@ -143,6 +143,15 @@ def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, lo
             dropout_rate=dropout_rate,
         )
     return out if width == head_dim else out[..., :head_dim]
+
+
+def _differentiated(*tensors: Optional[Tensor]) -> bool:
+    """Whether autograd has to see the call.  A bias that wants a gradient counts (it gets none, but the
+    output then still hangs in the graph), and so does forward mode, which the node refuses: past the
+    node a tangent would be dropped without a word."""
+    if forward_ad._current_level >= 0:  # pylint: disable=protected-access
+        return True
+    return torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors)
 
 
 class _FlashAttentionFn(torch.autograd.Function):

@@ -12,7 +12,7 @@ import torch
 
 from axlearn_amd import _lib
 from axlearn_amd import attention_bias as ab
-from axlearn_amd.flash_attention import common
+from axlearn_amd.flash_attention import common, hip_attention
 from axlearn_amd.flash_attention.hip_attention import (
     HipFlashAttention,
     classify_mask_bias,
@@ -89,6 +89,20 @@ def test_value_of_a_lone_member_is_what_adding_zero_gives():
         got = ab.CompositeAttentionBias([ab.TensorAttentionBias(view)]).value()
         want = 0.0 + view
         assert torch.equal(got, want) and got.dtype == want.dtype and got.stride() == want.stride()
+
+
+def test_autograd_sees_calls_that_only_the_bias_or_a_tangent_marks(monkeypatch):
+    monkeypatch.setattr(ops, "flash_fwd", lambda q, k, v, **kw: (q + 0.0, torch.zeros(1, 2, 128)))
+    q, k, v = (torch.randn(1, 128, 2, 64) for _ in range(3))
+    bias = torch.zeros(1, 2, 128, 128)
+    call = lambda q, b: hip_attention._attend(q, k, v, None, 1.0, ops.MASK_NONE, 0, bias=b)
+    assert not call(q, bias).requires_grad
+    assert call(q, bias.clone().requires_grad_(True)).requires_grad
+    with torch.no_grad():
+        assert not call(q, bias.clone().requires_grad_(True)).requires_grad
+    with torch.autograd.forward_ad.dual_level():
+        with pytest.raises(RuntimeError, match="(?i)jvp"):
+            call(torch.autograd.forward_ad.make_dual(q, torch.ones_like(q)), bias)
 
 
 def test_structured_masks_combine():
