@@ -170,17 +170,20 @@ class _FlashAttentionFn(torch.autograd.Function):
     def forward(ctx, query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink,
                 bias, dropout_mask, dropout_rate, save_residuals, bwd_ds_workspace=None,
                 bwd_workspace_limit_bytes=None):
-        aux = dict(bias=bias, dropout_mask=dropout_mask, dropout_rate=dropout_rate)
+        # neither is differentiated (gpu_attention.py:786)
+        aux = dict(dropout_mask=dropout_mask, dropout_rate=dropout_rate)
         out, lse = ops.flash_fwd(
             query, key, value, softmax_scale=softmax_scale, mask_kind=mask_kind,
-            sliding_window=window, segment_ids=segment_ids, logit_sink=logit_sink, **aux,
+            sliding_window=window, segment_ids=segment_ids, logit_sink=logit_sink, bias=bias, **aux,
         )
+        # The bias may be the caller's own tensor: saved like the others, so that writing to it ahead of the
+        # backward is an error and not a wrong gradient.
         if save_residuals:
-            ctx.save_for_backward(query, key, value, out, lse, logit_sink)
+            ctx.save_for_backward(query, key, value, out, lse, logit_sink, bias)
         else:
-            ctx.save_for_backward(query, key, value, None, None, logit_sink)
+            ctx.save_for_backward(query, key, value, None, None, logit_sink, bias)
         ctx.segment_ids = segment_ids
-        ctx.aux = aux  # not differentiated: the bias gets no gradient (gpu_attention.py:786)
+        ctx.aux = aux
         ctx.args = (softmax_scale, mask_kind, window)
         ctx.bwd_ds_workspace = None if bwd_ds_workspace is None else bool(bwd_ds_workspace)
         ctx.bwd_workspace_limit_bytes = bwd_workspace_limit_bytes
@@ -188,19 +191,20 @@ class _FlashAttentionFn(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, d_out):
-        query, key, value, out, lse, logit_sink = ctx.saved_tensors
+        query, key, value, out, lse, logit_sink, bias = ctx.saved_tensors
+        aux = dict(ctx.aux, bias=bias)
         softmax_scale, mask_kind, window = ctx.args
         if out is None:  # residuals were not saved: recompute them
             out, lse = ops.flash_fwd(
                 query, key, value, softmax_scale=softmax_scale, mask_kind=mask_kind,
-                sliding_window=window, segment_ids=ctx.segment_ids, logit_sink=logit_sink, **ctx.aux,
+                sliding_window=window, segment_ids=ctx.segment_ids, logit_sink=logit_sink, **aux,
             )
         if d_out.stride(-1) != 1:
             d_out = d_out.contiguous()
         grads = ops.flash_bwd(
             query, key, value, out, lse, d_out, softmax_scale=softmax_scale, mask_kind=mask_kind,
             sliding_window=window, segment_ids=ctx.segment_ids, logit_sink=logit_sink,
-            ds_workspace=ctx.bwd_ds_workspace, ds_workspace_limit=ctx.bwd_workspace_limit_bytes, **ctx.aux,
+            ds_workspace=ctx.bwd_ds_workspace, ds_workspace_limit=ctx.bwd_workspace_limit_bytes, **aux,
         )
         d_sink = grads[3].to(logit_sink.dtype) if logit_sink is not None else None
         return grads[0], grads[1], grads[2], None, None, None, None, d_sink, None, None, None, None, None, None

@@ -105,6 +105,19 @@ def test_autograd_sees_calls_that_only_the_bias_or_a_tangent_marks(monkeypatch):
             call(torch.autograd.forward_ad.make_dual(q, torch.ones_like(q)), bias)
 
 
+def test_bias_written_to_ahead_of_the_backward_is_an_error(monkeypatch):
+    monkeypatch.setattr(ops, "flash_fwd", lambda q, k, v, **kw: (q + 0.0, torch.zeros(1, 2, 128)))
+    monkeypatch.setattr(ops, "flash_bwd", lambda q, k, v, *a, **kw: (q + kw["bias"].sum(), k + 0.0, v + 0.0))
+    q, k, v = (torch.randn(1, 128, 2, 64, requires_grad=True) for _ in range(3))
+    bias = torch.ones(1, 2, 128, 128)
+    composite = ab.CompositeAttentionBias([ab.TensorAttentionBias(bias)])
+    out = hip_attention._attend(q, k, v, None, 1.0, ops.MASK_NONE, 0, bias=composite.value())
+    assert torch.equal(torch.autograd.grad(out.sum(), q, retain_graph=True)[0], q + bias.sum())
+    bias.add_(1)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        torch.autograd.grad(out.sum(), q)
+
+
 def test_structured_masks_combine():
     t = 8
     pos = dict(target_positions=torch.arange(t)[None], source_positions=torch.arange(t)[None])
