@@ -97,6 +97,14 @@ def _pad_last(x: Tensor, width: int) -> Tensor:
     return x if x.shape[-1] == width else torch.nn.functional.pad(x, (0, width - x.shape[-1]))
 
 
+def _aligned_rows(x: Tensor) -> Tensor:
+    """`x` where the kernels' 16-byte loads can read its rows in place, else a dense copy."""
+    step = 16 // x.element_size()
+    if x.stride(-1) == 1 and x.data_ptr() % 16 == 0 and not any(n % step for n in x.stride()[:-1]):
+        return x
+    return x.clone(memory_format=torch.contiguous_format)
+
+
 def get_dropout_mask(shape, *, prng_key, rate: float, device) -> Tensor:
     """Bool mask of `shape`, True = dropped with probability `rate` (layers.py:140-142).
 
@@ -347,8 +355,8 @@ class HipFlashAttention(BaseFlashAttention):
         if query.dtype != torch.float32:
             width = head_dim if runs_at_native_head_dim(query, key, value, aux=False) else padded_head_dim(head_dim)
             out = ops.flash_chunk(
-                _pad_last(query.detach(), width), _pad_last(key.detach(), width), _pad_last(value.detach(), width),
-                positions, softmax_scale=float(self.cfg.softmax_scale), mask_kind=kind[0], sliding_window=kind[1],
+                _aligned_rows(_pad_last(query.detach(), width)), _pad_last(key.detach(), width),
+                _pad_last(value.detach(), width), positions, softmax_scale=float(self.cfg.softmax_scale), mask_kind=kind[0], sliding_window=kind[1],
                 logit_sink=input_batch.get("logit_sink", None),
             )
             return out if width == head_dim else out[..., :head_dim]

@@ -13,6 +13,7 @@ from axlearn_amd import attention_bias as ab
 from axlearn_amd import _lib, ops
 from axlearn_amd.flash_attention.hip_attention import HipFlashAttention, flash_attention
 from axlearn_amd.flash_attention.utils import flash_attention_implementation
+from axlearn_amd.kv_cache import KVCache
 from oracle import brute
 from oracle import ref_attention as ref
 
@@ -1510,7 +1511,7 @@ def test_dkdv_with_bf16_bias_alone(b, t, s, hq, hkv, d, dtype, mask, window, kin
 def _layer_call(q, k, v, biases, **kw):
     bias = ab.CompositeAttentionBias(biases)
     fn = flash_attention_implementation("gpu", query=q, key=k, value=v, bias=bias, softmax_scale=q.shape[-1] ** -0.5, **kw)
-    return fn(dict(query=q, key=k, value=v, bias=bias))
+    return fn.fn(dict(query=q, key=k, value=v, bias=bias))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
@@ -1531,3 +1532,18 @@ def test_dense_bias_given_as_a_view(dtype):
             out = _layer_call(*leaves, [ab.CausalAttentionBias(**pos), ab.TensorAttentionBias(bias)])
             got.append([out, *torch.autograd.grad(out, leaves, do)])
         assert all(torch.equal(x, y) for x, y in zip(*got))
+
+
+@pytest.mark.parametrize("rows,d", [(128, 64), (40, 128), (7, 80)])
+def test_chunk_query_given_as_a_view(rows, d):
+    # Rows that start between two 16-byte boundaries or are not dense, heads before tokens: as from a copy.
+    b, hq, hkv, kv_len = 2, 4, 2, 512
+    _, k, v, _ = (x.cuda() for x in _inputs(b, rows, hq, hkv, d, torch.bfloat16, s=kv_len))
+    wide = ref.normal_tensor(7, (b, rows, hq, 2 * d + 3), torch.bfloat16).cuda()
+    pos = dict(target_positions=torch.tensor([[100], [301]]).cuda() + torch.arange(rows).cuda()[None],
+               source_positions=torch.arange(kv_len)[None].cuda())
+    heads_first = wide[..., :d].transpose(1, 2).contiguous().transpose(1, 2)
+    for view in (wide[..., 1:d + 1], wide[..., :2 * d:2], wide[..., :d], heads_first):
+        got = [_layer_call(q, k, v, [ab.CausalAttentionBias(**pos)], kv_cache_type=KVCache)
+               for q in (view, view.clone(memory_format=torch.contiguous_format))]
+        assert torch.equal(*got)

@@ -118,6 +118,15 @@ def test_bias_written_to_ahead_of_the_backward_is_an_error(monkeypatch):
         torch.autograd.grad(out.sum(), q)
 
 
+def test_rows_of_a_view_are_copied_only_where_the_kernels_cannot_read_them():
+    base = torch.randn(2, 8, 4, 72).to(torch.bfloat16)
+    for x in (base, base[..., :64], base[:, :, 1:], base.transpose(1, 2), base[..., 8:40]):
+        assert hip_attention._aligned_rows(x) is x
+    for x in (base[..., 1:65], base[..., ::2], base.reshape(2, 8, 96, 3)):
+        got = hip_attention._aligned_rows(x)
+        assert torch.equal(got, x) and got.is_contiguous()
+
+
 def test_structured_masks_combine():
     t = 8
     pos = dict(target_positions=torch.arange(t)[None], source_positions=torch.arange(t)[None])
