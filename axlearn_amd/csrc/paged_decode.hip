@@ -932,6 +932,16 @@ static int64_t capacity_tiles(int tiles, int window) {
   return w < tiles ? w : tiles;
 }
 
+// Workspace of equal shares: one record per workgroup and pair at most.  The size does not depend on the window
+// (a query may leave it out): with one there are no more tiles, in shares of 8 or more.
+static size_t even_ws_bytes(int64_t pairs, int tiles, int gp, int width) {
+  const int64_t wgs = (pairs * tiles + 7) / 8, slots = 2 * (int64_t)cu_count();
+  return ws_bytes(1, 1, (int)((wgs < slots ? wgs : slots) + pairs), gp, width);
+}
+// The workgroups' records must not push a call whose blocks fit it past the buffer of axl_paged_decode_static
+// (thousands of pairs of a block each; blocks are drawn there).
+static bool even_fits(size_t even, size_t drawn) { return even <= drawn || even <= AXL_PAGED_DECODE_STATIC_MAX_BYTES; }
+
 // Equal shares (see the head of this file) where the capacity makes them at most 256 tiles, the page ids a
 // segment keeps in registers.  Measured at 8 sequences of 2000 to 8190 tokens, 8 kv heads (40 tiles a
 // workgroup): split kernel 42.8 us drawing blocks of 32 tiles (640 blocks for 512 workgroups), 39.6 us in
@@ -951,6 +961,8 @@ static void plan_even(DecArgs& a, bool deterministic) {
   // A deterministic call keeps to the blocks, whose bits depend on a pair's own keys alone: equal shares only
   // where the shapes leave no more blocks than workgroups.
   if (deterministic && (int64_t)a.B * a.Hv * a.nch > a.n_wg) a.even = 0;
+  const int gp = gp_of(a.G, a.bias != nullptr), width = width_of(a.d_real);
+  if (!even_fits(even_ws_bytes((int64_t)a.B * a.Hv, a.pps, gp, width), ws_bytes(a.B, a.Hv, a.nch, gp, width))) a.even = 0;
 }
 
 static size_t ws_bytes_for(int batch, int hq, int hkv, int d, int tiles, bool bias, int dtype) {
@@ -959,11 +971,8 @@ static size_t ws_bytes_for(int batch, int hq, int hkv, int d, int tiles, bool bi
   const int nch = (tiles + cp - 1) / cp;
   const size_t drawn = ws_bytes(batch, hkv * groups_of(G), nch, gp_of(G, bias), width_of(d));
   if (dtype == AXL_F32 || batch > kMaxBatch) return drawn;
-  // Equal shares: one record per workgroup and pair at most.  The size does not depend on the window (a query
-  // may leave it out): with one there are no more tiles, in shares of 8 or more.
-  const int64_t pairs = (int64_t)batch * hkv * groups_of(G), wgs = (pairs * tiles + 7) / 8, slots = 2 * (int64_t)cu_count();
-  const size_t even = ws_bytes(1, 1, (int)((wgs < slots ? wgs : slots) + pairs), gp_of(G, bias), width_of(d));
-  return even > drawn ? even : drawn;
+  const size_t even = even_ws_bytes((int64_t)batch * hkv * groups_of(G), tiles, gp_of(G, bias), width_of(d));
+  return even > drawn && even_fits(even, drawn) ? even : drawn;
 }
 
 size_t paged_decode_workspace_bytes(const AxlPagedDecodeParams& p) {

@@ -127,6 +127,16 @@ def test_rows_of_a_view_are_copied_only_where_the_kernels_cannot_read_them():
         assert torch.equal(got, x) and got.is_contiguous()
 
 
+@pytest.mark.parametrize("batch,page,pages", [(480, 16, 8), (500, 64, 2), (500, 128, 1)])
+def test_decode_workspace_of_many_short_sequences_fits_the_built_in_buffer(batch, page, pages):
+    # A block, and so a record, per pair: 500 sequences x 8 kv heads of 16 query heads make 33.3 MB of its 33.6 MB.
+    p = _lib.AxlPagedDecodeParams(batch=batch, num_q_heads=128, num_kv_heads=8, head_dim=128, num_pages=4096,
+                                  page_size=page, pages_per_seq=pages, dtype=_lib.dtype_code(torch.bfloat16))
+    need = _lib.load().axl_paged_decode_workspace_bytes(ctypes.byref(p))
+    record = (16 * 128 + 2 * 16 + 1) * 4
+    assert need == batch * 8 * record + 256 <= 32 << 20
+
+
 def test_structured_masks_combine():
     t = 8
     pos = dict(target_positions=torch.arange(t)[None], source_positions=torch.arange(t)[None])
