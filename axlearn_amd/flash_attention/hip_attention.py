@@ -154,10 +154,13 @@ def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, lo
 
 
 def _differentiated(*tensors: Optional[Tensor]) -> bool:
-    """Whether autograd has to see the call.  A bias that wants a gradient counts (it gets none, but the
-    output then still hangs in the graph), and so does forward mode, which the node refuses: past the
-    node a tangent would be dropped without a word."""
-    if forward_ad._current_level >= 0:  # pylint: disable=protected-access
+    """Whether autograd has to see the call.
+
+    A bias that wants a gradient counts: it gets none, but the output then still hangs in the graph.  So does
+    whatever looks at a call by its operations, for past the node there are none that it could see: a trace
+    (`torch.jit.trace`) keeps the node as a call into Python, and would hold the allocation of the output alone
+    without it; forward mode, which the node refuses, would drop a tangent without a word."""
+    if torch.jit.is_tracing() or forward_ad._current_level >= 0:  # pylint: disable=protected-access
         return True
     return torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors)
 

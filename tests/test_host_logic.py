@@ -105,6 +105,26 @@ def test_autograd_sees_calls_that_only_the_bias_or_a_tangent_marks(monkeypatch):
             call(torch.autograd.forward_ad.make_dual(q, torch.ones_like(q)), bias)
 
 
+def _kernel_behind_a_pointer(monkeypatch):
+    """`flash_fwd` as a trace sees it: an output allocated by torch and filled where torch cannot look."""
+    def flash_fwd(q, k, v, **kw):
+        out, result = torch.empty_like(q), (q + 2 * k).detach().contiguous()
+        ctypes.memmove(out.data_ptr(), result.data_ptr(), 4 * out.numel())
+        return out, torch.zeros(1, 2, 128)
+    monkeypatch.setattr(ops, "flash_fwd", flash_fwd)
+    return lambda q, k, v: hip_attention._attend(q, k, v, None, 1.0, ops.MASK_NONE, 0)
+
+
+@pytest.mark.parametrize("grad", [True, False])
+def test_a_trace_keeps_the_kernel(monkeypatch, grad):
+    call = _kernel_behind_a_pointer(monkeypatch)
+    q, k, v, other = (torch.randn(1, 128, 2, 64) for _ in range(4))
+    with torch.set_grad_enabled(grad):
+        traced = torch.jit.trace(call, (q, k, v), check_trace=False)
+        assert "aten::empty" not in str(traced.graph)
+        assert torch.equal(traced(other, k, v), other + 2 * k)
+
+
 def test_bias_written_to_ahead_of_the_backward_is_an_error(monkeypatch):
     monkeypatch.setattr(ops, "flash_fwd", lambda q, k, v, **kw: (q + 0.0, torch.zeros(1, 2, 128)))
     monkeypatch.setattr(ops, "flash_bwd", lambda q, k, v, *a, **kw: (q + kw["bias"].sum(), k + 0.0, v + 0.0))
