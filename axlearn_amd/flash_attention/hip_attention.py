@@ -159,8 +159,10 @@ def _differentiated(*tensors: Optional[Tensor]) -> bool:
     A bias that wants a gradient counts: it gets none, but the output then still hangs in the graph.  So does
     whatever looks at a call by its operations, for past the node there are none that it could see: a trace
     (`torch.jit.trace`) keeps the node as a call into Python, and would hold the allocation of the output alone
-    without it; forward mode, which the node refuses, would drop a tangent without a word."""
-    if torch.jit.is_tracing() or forward_ad._current_level >= 0:  # pylint: disable=protected-access
+    without it; forward mode would drop a tangent without a word, and the transforms of `torch.func` would
+    hand over wrappers without storage, where the node refuses."""
+    # pylint: disable=protected-access
+    if torch.jit.is_tracing() or torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0:
         return True
     return torch.is_grad_enabled() and any(x is not None and x.requires_grad for x in tensors)
 

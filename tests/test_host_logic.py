@@ -125,6 +125,18 @@ def test_a_trace_keeps_the_kernel(monkeypatch, grad):
         assert torch.equal(traced(other, k, v), other + 2 * k)
 
 
+def test_function_transforms_are_refused(monkeypatch):
+    # of the tensors the kernel reads and of others alike
+    call = _kernel_behind_a_pointer(monkeypatch)
+    q, k, v = (torch.randn(1, 128, 2, 64) for _ in range(3))
+    for transformed in (lambda: torch.func.vmap(call)(q[None], k[None], v[None]),
+                        lambda: torch.func.vmap(lambda x: call(q, k, v) * x)(torch.ones(2)),
+                        lambda: torch.func.grad(lambda x: (call(q, k, v) * x).sum())(torch.tensor(1.0)),
+                        lambda: torch.func.functionalize(call)(q, k, v)):
+        with pytest.raises(RuntimeError, match="setup_context"):
+            transformed()
+
+
 def test_bias_written_to_ahead_of_the_backward_is_an_error(monkeypatch):
     monkeypatch.setattr(ops, "flash_fwd", lambda q, k, v, **kw: (q + 0.0, torch.zeros(1, 2, 128)))
     monkeypatch.setattr(ops, "flash_bwd", lambda q, k, v, *a, **kw: (q + kw["bias"].sum(), k + 0.0, v + 0.0))
