@@ -150,6 +150,41 @@ def test_bias_written_to_ahead_of_the_backward_is_an_error(monkeypatch):
         torch.autograd.grad(out.sum(), q)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_layer_takes_a_bias_buffer_that_is_refilled_ahead_of_the_backward(monkeypatch, dtype):
+    # One buffer for the biases of two calls: each backward has the bias its forward had.  Nothing is copied where no
+    # backward follows, nor where the bias came as a sum or in another type, a tensor of the call's own already.
+    seen = []
+
+    def flash_fwd(q, k, v, **kw):
+        seen.append(kw["bias"])
+        return q + 0.0, torch.zeros(1, 2, 128)
+
+    monkeypatch.setattr(ops, "flash_fwd", flash_fwd)
+    monkeypatch.setattr(ops, "flash_bwd", lambda q, k, v, *a, **kw: (q * 0 + kw["bias"].float().mean(), k + 0.0, v + 0.0))
+    q, k, v = (torch.randn(1, 128, 2, 64, requires_grad=True) for _ in range(3))
+    buffer = torch.empty(1, 2, 128, 128, dtype=dtype)
+    fn = HipFlashAttention.default_config().instantiate()
+    bias = ab.TensorAttentionBias(buffer)
+    batch = lambda b: dict(query=q, key=k, value=v, bias=ab.CompositeAttentionBias(b))
+    outs = []
+    for value in (1.0, 3.0):
+        buffer.fill_(value)
+        outs.append(fn(batch([bias])))
+    for out, value in zip(outs, (1.0, 3.0)):
+        assert torch.equal(torch.autograd.grad(out.sum(), q)[0], torch.full_like(q, value))
+    storage = lambda x: x.untyped_storage().data_ptr()
+    assert len({storage(seen[0]), storage(seen[1]), storage(buffer)}) == 3
+    with torch.no_grad():
+        fn(batch([bias]))
+    assert storage(seen[2]) == storage(buffer)
+    clones = []
+    monkeypatch.setattr(torch.Tensor, "clone", lambda x, **kw: clones.append(x))
+    fn(batch([bias.astype(torch.float16)]))
+    fn(batch([bias, bias]))
+    assert not clones
+
+
 def test_rows_of_a_view_are_copied_only_where_the_kernels_cannot_read_them():
     base = torch.randn(2, 8, 4, 72).to(torch.bfloat16)
     for x in (base, base[..., :64], base[:, :, 1:], base.transpose(1, 2), base[..., 8:40]):
