@@ -889,7 +889,9 @@ __global__ __launch_bounds__(2 * D) void flash_chunk_combine_kernel(const FwdArg
 #pragma unroll
     for (int i = 0; i < kBatch; i++) {
       if (s0 + i >= sh.nsplit) continue;
-      const bool any = ml[i][1] > 0.f;
+      // A part without a visible key has a sum of exactly zero, and its values may never have been written.  (Not
+      // `> 0`: a NaN sum, which the unsplit form stores as NaN, would be left out like an empty part.)
+      const bool any = ml[i][1] != 0.f;
       const float w = any ? fast_exp2(ml[i][0] - mx) : 0.f;
       l += w * ml[i][1];
 #pragma unroll

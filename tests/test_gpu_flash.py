@@ -1547,3 +1547,36 @@ def test_chunk_query_given_as_a_view(rows, d):
         got = [_layer_call(q, k, v, [ab.CausalAttentionBias(**pos)], kv_cache_type=KVCache)
                for q in (view, view.clone(memory_format=torch.contiguous_format))]
         assert torch.equal(*got)
+
+
+@pytest.mark.parametrize("kv_len", [512, 4096])   # one workgroup per row block; its keys shared by several
+def test_chunk_passes_nan_and_infinity_on(kv_len):
+    # A query row that is NaN, a key that is NaN and one whose logits are +inf (which the softmax turns into NaN):
+    # every row that sees one is NaN throughout, the others are what they are without it.
+    b, rows, hq, hkv, d, bad_key = 2, 7, 4, 2, 64, 300
+    q, k, v, _ = (x.cuda() for x in _inputs(b, rows, hq, hkv, d, torch.bfloat16, s=kv_len))
+    q[..., 0] = q[..., 0].abs() + 1
+    positions = (kv_len - rows + torch.arange(rows))[None].repeat(b, 1)
+    positions[1, 0], positions[1, 1] = 3, bad_key - 1
+    positions = positions.cuda()
+
+    def run(q, k):
+        return ops.flash_chunk(q, k, v, positions, softmax_scale=d ** -0.5)
+
+    clean = run(q, k)
+    assert torch.isfinite(clean).all()
+    bad_q = q.clone()
+    bad_q[0, 2, 1] = float("nan")
+    hit_q = torch.zeros(b, rows, hq, dtype=torch.bool)
+    hit_q[0, 2, 1] = True
+    hit_k = torch.zeros(b, rows, hq, dtype=torch.bool)
+    hit_k[1, 2:, 2:] = True    # sequence 1, the rows from bad_key on, the two heads of kv head 1
+    calls = [(bad_q, k, hit_q)]
+    for value in (float("nan"), float("inf")):
+        bad_k = k.clone()
+        bad_k[1, bad_key, 1, 0] = value
+        calls.append((q, bad_k, hit_k))
+    for qq, kk, hit in calls:
+        got = run(qq, kk).cpu()
+        assert torch.isnan(got[hit]).all()
+        assert ref.rel_l2(got[~hit], clean.cpu()[~hit]) < 4e-3   # at most another rounding of P
