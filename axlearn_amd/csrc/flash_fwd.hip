@@ -304,7 +304,9 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     if (a.mask_kind == AXL_MASK_SLIDING_WINDOW) tw_begin = max(t_begin, (qpos_min - a.window) / Tile::BK);
     tw_begin = max(tw_begin, t_begin);
   }
-  if (CHUNK && q0 >= chunk_rows) tw_end = tw_begin;   // a wavefront without rows only helps to load
+  // A wavefront without rows only helps to load: no tile of its own, stated inside [t_begin, t_end).  (It repeats the
+  // last row, whose window may begin past t_end: `tw_end = tw_begin` sent it through the loops beyond t_end.)
+  if (CHUNK && q0 >= chunk_rows) tw_begin = tw_end = t_begin;
 
   floatx16 o[DT];
 #pragma unroll

@@ -1580,3 +1580,26 @@ def test_chunk_passes_nan_and_infinity_on(kv_len):
         got = run(qq, kk).cpu()
         assert torch.isnan(got[hit]).all()
         assert ref.rel_l2(got[~hit], clean.cpu()[~hit]) < 4e-3   # at most another rounding of P
+
+
+@pytest.mark.parametrize("kv_len,rows,window", [
+    (512, 9, 300),        # not split: three of the four wavefronts have no rows
+    (4096, 9, 1100),      # split
+    (4096, 40, 3000),     # 80 rows in a block: the third wavefront is half full
+])
+def test_chunk_whose_last_row_lies_past_the_others(kv_len, rows, window):
+    # Under a window, the last row of a block past the range of the keys that the others see: late in the cache, at its
+    # end, past it and past the window behind it (where it sees nothing).
+    b, hq, hkv, d = 2, 4, 2, 64
+    q, k, v, _ = _inputs(b, rows, hq, hkv, d, torch.bfloat16, s=kv_len)
+    for last in (kv_len - 1, kv_len + window // 2, kv_len + window, 3 * kv_len + window):
+        positions = torch.arange(rows)[None].repeat(b, 1) + 70
+        positions[:, -1] = last
+        seen = positions - window < kv_len
+        spec = ref.MaskSpec(causal=False, sliding_window=window, target_positions=positions,
+                            source_positions=torch.arange(kv_len)[None])
+        want = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5)
+        got = ops.flash_chunk(q.cuda(), k.cuda(), v.cuda(), positions.cuda(), softmax_scale=d ** -0.5,
+                              mask_kind=ops.MASK_SLIDING_WINDOW, sliding_window=window).cpu()
+        assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
+        assert ref.rel_l2(got[seen], want[seen]) < 1e-2
