@@ -83,6 +83,15 @@ struct ChunkPart {
   static constexpr int BYTES = O_BYTES + 32 * 8;
 };
 
+// Position of row t of sequence b, brought into [-1, 2^31 - 129]: every position below 0 sees no key, and the bounds of
+// tiles and differences that are formed from it stay within 32 bits, whatever stands in rows that mean nothing.
+// (A row past the end of the cache sees what the mask says: all of it, or under a window the keys within that.)
+__device__ __forceinline__ int chunk_position(const FwdArgs& a, int b, int t) {
+  const char* p = a.pos + b * a.pos_sb + t * a.pos_ss;
+  const int64_t x = a.pos_i64 ? *(const int64_t*)p : (int64_t)*(const int32_t*)p;
+  return (int)max((int64_t)-1, min(x, (int64_t)0x7fffffff - 128));
+}
+
 // Which sequence a workgroup of the chunk form works on and how many share its key range.  The live
 // lengths are known on the device only, and they differ: with the same number of workgroups for every
 // sequence the longest one would finish alone.  So every wavefront derives the same plan: a workgroup takes about `target` tiles of 64 keys, a sequence of n
@@ -98,9 +107,8 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
   if (a.slots == 0) return by_slot ? ChunkShare{key / nqb, 1, key / nqb * nqb} : ChunkShare{key, 1, key * nqb};
   auto tiles = [&](int b) -> int {
     if (b >= a.B) return 0;
-    const char* pp = a.pos + b * a.pos_sb + (a.T - 1) * a.pos_ss;
-    const int end = min(a.S, max(0, (a.pos_i64 ? (int)*(const int64_t*)pp : *(const int32_t*)pp) + 1));
-    const int begin = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? max(0, end - a.T - a.window) : 0;
+    const int end = min(a.S, chunk_position(a, b, a.T - 1) + 1);
+    const int begin = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? max(0, end - a.T - min(a.window, a.S)) : 0;
     return (max(end, begin + 1) - begin + 63) / 64;
   };
   // The plan stands at the head of both kernels' chains of latencies: the lengths of the first 64 sequences are read
@@ -225,8 +233,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   int qpos_min = q0 + q_off, qpos_max = q0 + 31 + q_off;  // of the wavefront
   int wg_min = q0_wg + q_off, wg_max = q0_wg + Tile::BQ - 1 + q_off;  // of the workgroup
   if constexpr (CHUNK) {
-    const char* pp = a.pos + b * a.pos_sb + row * a.pos_ss;
-    qpos = a.pos_i64 ? (int)*(const int64_t*)pp : *(const int32_t*)pp;
+    qpos = chunk_position(a, b, row);
     qpos_min = qpos_max = qpos;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {   // the lanes l and l ^ 32 hold the same row

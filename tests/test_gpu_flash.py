@@ -1603,3 +1603,32 @@ def test_chunk_whose_last_row_lies_past_the_others(kv_len, rows, window):
                               mask_kind=ops.MASK_SLIDING_WINDOW, sliding_window=window).cpu()
         assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
         assert ref.rel_l2(got[seen], want[seen]) < 1e-2
+
+
+@pytest.mark.parametrize("window", [None, 300])
+@pytest.mark.parametrize("kv_len", [512, 4096])
+def test_chunk_rows_at_positions_of_any_size(kv_len, window):
+    # The largest and the smallest of either integer type, and int64 positions that are others when cut to 32 bits,
+    # among ordinary rows: a row past the cache sees all of it (under the window none), one before it none, and the
+    # rows beside them are what they are without them, in the first, middle and last row (from which the shares of the
+    # keys are taken).
+    b, rows, hq, hkv, d = 2, 9, 4, 2, 64
+    q, k, v, _ = _inputs(b, rows, hq, hkv, d, torch.bfloat16, s=kv_len)
+    base = (kv_len - rows + torch.arange(rows))[None].repeat(b, 1)
+    i32, i64 = torch.iinfo(torch.int32), torch.iinfo(torch.int64)
+    for dtype, values in ((torch.int32, (i32.max, i32.min, i32.max - 1)),
+                          (torch.int64, (i64.max, i64.min, 1 << 31, (1 << 32) + 5, -(1 << 32) + 5))):
+        for value in values:
+            for row in (0, 4, rows - 1):
+                positions = base.clone()
+                positions[1, row] = value
+                seen = torch.ones(b, rows, dtype=torch.bool)
+                seen[1, row] = value > 0 and window is None
+                spec = ref.MaskSpec(causal=window is None, sliding_window=window, source_positions=torch.arange(kv_len)[None],
+                                    target_positions=positions.clamp(-1, 2 * kv_len))
+                want = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5)
+                got = ops.flash_chunk(q.cuda(), k.cuda(), v.cuda(), positions.to(dtype).cuda(), softmax_scale=d ** -0.5,
+                                      mask_kind=ops.MASK_CAUSAL if window is None else ops.MASK_SLIDING_WINDOW,
+                                      sliding_window=window or 0).cpu()
+                assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
+                assert ref.rel_l2(got[seen], want[seen]) < 1e-2
