@@ -15,7 +15,7 @@ struct BwdArgs {
   float* ndelta; // workspace [B, Hq, T]: -rowsum(out * dO); negated so that a dP accumulator chain can start from it
   float* lse2;   // workspace [B, Hq, T]: -lse * log2(e), the exponent offset of the dK/dV kernel
   void* ds;      // workspace: dS blocks left by the dK/dV kernel for the streaming dQ kernel (spill path), or nullptr
-  const char* q_planes;   // workspace (fp32): the 32-row tiles of Q and of dO as bf16 planes, [B, Hq, T / 32] tiles
+  const char* q_planes;   // workspace (fp32): the 32-row tiles of Q and of dO as bf16 planes, [B, Hq, T / 32] tiles; or nullptr
   const char* do_planes;
   void* dq;
   void* dk;

@@ -399,8 +399,12 @@ static size_t stats_bytes(const AxlFlashBwdParams& p) {
 static bool spill_ranged(const AxlFlashBwdParams& p) {
   return p.dtype != AXL_F32 && (p.mask_kind == AXL_MASK_SLIDING_WINDOW || p.segment_ids);
 }
+// fp32 whose dK/dV kernel reads Q and dO as planes from the workspace.
+static bool f32_planes(const AxlFlashBwdParams& p) {
+  return p.dtype == AXL_F32 && !f32_on_fp32_mfma() && !(p.flags & AXL_BWD_F32_NO_PLANES);
+}
 static bool spill_eligible(const AxlFlashBwdParams& p) {
-  return (p.dtype == AXL_BF16 || p.dtype == AXL_F16 || (p.dtype == AXL_F32 && !f32_on_fp32_mfma())) &&
+  return (p.dtype == AXL_BF16 || p.dtype == AXL_F16 || f32_planes(p)) &&
          (p.mask_kind == AXL_MASK_CAUSAL || p.mask_kind == AXL_MASK_SLIDING_WINDOW) && p.q_pos_offset == 0 &&
          p.q_len == p.kv_len && (p.flags & AXL_BWD_DS_WORKSPACE) &&
          // the ranged kernel keeps the table in LDS beside its ring: 256-row blocks at head_dim 128
@@ -433,7 +437,7 @@ static size_t kb_table_bytes(const AxlFlashBwdParams& p) {
 
 // fp32: the planes of Q (and, of the same size, of dO), six bytes per element of the compiled width.
 static size_t planes_bytes(const AxlFlashBwdParams& p) {
-  if (p.dtype != AXL_F32 || f32_on_fp32_mfma()) return 0;
+  if (!f32_planes(p)) return 0;
   return (size_t)p.batch * p.num_q_heads * p.q_len * (p.head_dim <= 64 ? 64 : 128) * 6;
 }
 
@@ -458,8 +462,8 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   a.seg_tbl = p.segment_ids ? (const int2*)(ws + stats_bytes(p)) : nullptr;
   a.kb_tbl = kb_table_bytes(p) ? (int2*)(ws + stats_bytes(p) + seg_table_bytes(p)) : nullptr;
   char* const ws_planes = ws + stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p);
-  a.q_planes = ws_planes;
-  a.do_planes = ws_planes + planes_bytes(p);
+  a.q_planes = f32_planes(p) ? ws_planes : nullptr;
+  a.do_planes = f32_planes(p) ? ws_planes + planes_bytes(p) : nullptr;
   a.ds = spill ? ws_planes + 2 * planes_bytes(p) : nullptr;
   a.qs = to_s3(p.q_strides); a.ks = to_s3(p.k_strides); a.vs = to_s3(p.v_strides);
   a.os = to_s3(p.out_strides); a.dos = to_s3(p.d_out_strides); a.dqs = to_s3(p.dq_strides);
@@ -508,7 +512,7 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       if (width == 128) AXL_LAUNCH((bwd_delta_kernel<float, 128>), delta_grid, 0);
       else AXL_LAUNCH((bwd_delta_kernel<float, 64>), delta_grid, 0);
     }
-    if ((phases & AXL_BWD_DKDV) && !f32_on_fp32_mfma() && err == hipSuccess) err = launch_bwd_split_f32x(a, width, stream);
+    if ((phases & AXL_BWD_DKDV) && a.q_planes && err == hipSuccess) err = launch_bwd_split_f32x(a, width, stream);
   }
   if (dt == AXL_F32 && !spill) {
     if (err == hipSuccess) err = launch_bwd_f32(a, width, phases, stream);
@@ -544,8 +548,10 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       s.dv = (char*)a.dv + h0 * a.dvs.h * es;
       s.ndelta = a.ndelta + hq0 * p.q_len;
       s.lse2 = a.lse2 + hq0 * p.q_len;
-      s.q_planes = a.q_planes + hq0 * p.q_len * width * 6;
-      s.do_planes = a.do_planes + hq0 * p.q_len * width * 6;
+      if (a.q_planes) {
+        s.q_planes = a.q_planes + hq0 * p.q_len * width * 6;
+        s.do_planes = a.do_planes + hq0 * p.q_len * width * 6;
+      }
       if (a.aux.bias) s.aux.bias = a.aux.bias + hq0 * a.aux.bias_sh;
       if (a.aux.drop) s.aux.drop = a.aux.drop + hq0 * a.aux.drop_sh;
       if (dt == AXL_F32) {

@@ -591,7 +591,7 @@ static hipError_t launch_f32(const BwdArgs& a, int phases, hipStream_t stream) {
   const bool true_f32 = f32_on_fp32_mfma();
   hipError_t err = hipSuccess;
   if (phases & AXL_BWD_DKDV) {
-    if (true_f32) {
+    if (!a.q_planes) {   // AXL_F32_MFMA=1, or a workspace without them
       err = allow_dynamic_lds((const void*)flash_bwd_dkdv_f32_kernel<D>, Tile::LDS_BYTES_DKDV);
       if (err != hipSuccess) return err;
       hipLaunchKernelGGL(flash_bwd_dkdv_f32_kernel<D>, dim3((a.S / Tile::ROWS) * a.B * a.Hkv), dim3(Tile::NT),
@@ -603,7 +603,7 @@ static hipError_t launch_f32(const BwdArgs& a, int phases, hipStream_t stream) {
     if (err != hipSuccess) return err;
   }
   if (phases & AXL_BWD_DQ) {
-    if (a.ds && !true_f32) return launch_bwd_dq_ds_f32(a, D, stream);
+    if (a.ds) return launch_bwd_dq_ds_f32(a, D, stream);
     auto kernel = true_f32 ? flash_bwd_dq_f32_kernel<D> : flash_bwd_dq_f32x_kernel<D>;
     const int lds = true_f32 ? Tile::LDS_BYTES : TileX::LDS_BYTES;
     err = allow_dynamic_lds((const void*)kernel, lds);

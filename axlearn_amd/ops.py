@@ -265,10 +265,12 @@ def flash_bwd(
     (AXL_BWD_DS_SLICE_KV_HEADS).  `ds_workspace=None` decides by size (`select_ds_slice`): the dS
     workspace is used when that path applies and fits `ds_workspace_limit` bytes (default:
     `default_bwd_workspace_limit`, a sixteenth of the device's memory), whole or in slices of kv
-    heads that still fill the GPU."""
+    heads that still fill the GPU.  A workspace that there is no room for (on the device, or in `buffers`) gives
+    way to a smaller one as `_bwd_workspace` says."""
     b, t, hq, d, s, hkv = _check_qkv(q, k, v)
     _check_segment_ids(segment_ids, b, t, s)
-    if ds_workspace is None:
+    by_size = ds_workspace is None
+    if by_size:
         ds_workspace, ds_slice_kv_heads = False, 0
         if phases == 7 and q_pos_offset == 0:
             ds_workspace, ds_slice_kv_heads = select_ds_slice(q, k, mask_kind=mask_kind, segment_ids=segment_ids,
@@ -312,17 +314,40 @@ def flash_bwd(
         workspace=None, workspace_bytes=0, logit_sink=_lib.ptr(sink), d_logit_sink=_lib.ptr(d_sink),
         aux=aux, flags=_bwd_flags(ds_workspace, ds_slice_kv_heads),
     )
-    need = int(lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)))
-    if ws is None:
-        ws = torch.empty((max(need, 256),), dtype=torch.uint8, device=q.device)
-    elif ws.numel() * ws.element_size() < need:
-        raise AxlError(_lib.AXL_ERR_WORKSPACE, f"buffers workspace holds {ws.numel() * ws.element_size()} bytes, {need} needed")
+    ws = _bwd_workspace(lib, p, by_size or bias is not None or dropout_mask is not None, ws, q.device)
     p.workspace = ws.data_ptr()
     p.workspace_bytes = ws.numel() * ws.element_size()
     _lib.check(lib.axl_flash_bwd_phases(ctypes.byref(p), int(phases), _lib.current_stream_ptr()))
     if sink is not None:
         return dq, dk, dv, d_sink
     return dq, dk, dv
+
+
+def _bwd_workspace(lib, p: AxlFlashBwdParams, ds_optional: bool, ws: Optional[torch.Tensor], device) -> torch.Tensor:
+    """The backward's workspace: `ws`, or a new one where that is None.
+
+    Where there is no room for the workspace of `p.flags`, the largest that there is room for: without dS if that is
+    optional (the size rule's choice, a float32 call, or one with a bias or dropout mask), in float32 at last
+    without the planes.  `p.flags` is set to match; the kernels that make do with less are slower."""
+    choices = [p.flags]
+    if p.flags and (ds_optional or p.dtype == _lib.AXL_F32):
+        choices.append(0)
+    if p.dtype == _lib.AXL_F32:
+        choices.append(_lib.BWD_F32_NO_PLANES)
+    error = None
+    for p.flags in choices:
+        need = int(lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)))
+        if ws is not None:
+            have = ws.numel() * ws.element_size()
+            if have >= need:
+                return ws
+            error = error or AxlError(_lib.AXL_ERR_WORKSPACE, f"buffers workspace holds {have} bytes, {need} needed")
+            continue
+        try:
+            return torch.empty((max(need, 256),), dtype=torch.uint8, device=device)
+        except torch.OutOfMemoryError as e:
+            error = error or e
+    raise error
 
 
 def _bwd_flags(ds_workspace: bool, ds_slice_kv_heads: int = 0) -> int:
@@ -348,8 +373,7 @@ def flash_bwd_buffers(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, mask
                           head_dim=d, dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind,
                           segment_ids=_lib.ptr(_seg(segment_ids)),
                           flags=_bwd_flags(ds_workspace, ds_slice_kv_heads))
-    nbytes = int(_lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p)))
-    ws = torch.empty((max(nbytes, 256),), dtype=torch.uint8, device=q.device)
+    ws = _bwd_workspace(_lib.load(), p, False, None, q.device)
     return torch.empty_like(q), torch.empty_like(k), torch.empty_like(v), ws
 
 

@@ -1480,6 +1480,32 @@ def test_float32_ds_workspace_backward(t, hq, hkv, d, mask, window, packed, drop
             assert ref.max_abs(x.cpu(), y) <= FP32_MAX_ABS * top, name
 
 
+@pytest.mark.parametrize("t,hq,hkv,d,mask,window,packed,drop", [
+    (128, 2, 1, 64, "causal", None, False, False),
+    (384, 6, 2, 128, "sliding", 33, True, True),
+])
+def test_float32_backward_in_a_workspace_without_planes(t, hq, hkv, d, mask, window, packed, drop):
+    # Buffers of the statistics and the segment table alone: dk and dv from the kernel on the fp32 matrix instruction,
+    # dq, recomputed, the bits of the call with planes.  The workspace starts as NaN.
+    b = 2
+    q, k, v, do = _inputs(b, t, hq, hkv, d, torch.float32)
+    g = torch.Generator().manual_seed(t)
+    spec, kw = _mask_args(mask, window, ref.packed_segment_ids(3, b, t) if packed else None)
+    drop_mask = torch.rand(b, hq, t, t, generator=g) < 0.2 if drop else None
+    dropped = dict(dropout_mask=drop_mask, dropout_rate=0.2 if drop else 0.0)
+    want = ref.reference_mha_grads(q, k, v, do, spec, softmax_scale=d ** -0.5, **dropped)
+    kw.update(dropped, softmax_scale=d ** -0.5, dropout_mask=None if drop_mask is None else drop_mask.cuda())
+    args = (q.cuda(), k.cuda(), v.cuda())
+    out, lse = ops.flash_fwd(*args, **kw)
+    plain = ops.flash_bwd(*args, out, lse, do.cuda(), ds_workspace=False, **kw)
+    room = 2 * b * hq * t * 4 + 240 + (256 if packed else 0)
+    bufs = (*(torch.empty_like(x) for x in args), torch.full((room,), 255, dtype=torch.uint8, device="cuda"))
+    got = ops.flash_bwd(*args, out, lse, do.cuda(), ds_workspace=None, buffers=bufs, **kw)
+    assert torch.equal(got[0], plain[0]) and not torch.equal(got[1], plain[1])
+    for name, x, y in zip(("dq", "dk", "dv"), got, want):
+        assert ref.max_abs(x.cpu(), y) <= FP32_MAX_ABS * max(1.0, float(y.abs().max())), name
+
+
 @pytest.mark.parametrize("b,t,s,hq,hkv,d,dtype,mask,window,kind,ds", [
     (1, 128, 128, 2, 1, 128, torch.bfloat16, "causal", None, "bh", True),    # four tiles: the ring is deeper than the walk
     (2, 384, 384, 6, 2, 64, torch.bfloat16, "causal", None, "1h", True),     # three heads a group: the bias cursor wraps

@@ -185,6 +185,63 @@ def test_layer_takes_a_bias_buffer_that_is_refilled_ahead_of_the_backward(monkey
     assert not clones
 
 
+@pytest.mark.parametrize("dtype,kind,forced,flags", [
+    # (the flags of each call as the room shrinks: for all of it, for the statistics and planes, for the statistics)
+    (torch.bfloat16, "plain", None, (1, 0, 0)),
+    (torch.bfloat16, "plain", True, (1, None, None)),   # asked for, not the rule's choice
+    (torch.bfloat16, "bias", True, (1, 0, 0)),
+    (torch.float32, "plain", None, (1, 0, 2)),
+    (torch.float32, "plain", True, (1, 0, 2)),
+    (torch.float32, "drop", False, (0, 0, 2)),
+])
+@pytest.mark.parametrize("own_buffers", [False, True])
+def test_backward_takes_the_workspace_there_is_room_for(monkeypatch, dtype, kind, forced, flags, own_buffers):
+    b, t, h, d = 1, 1024, 2, 64
+    seen = []
+
+    def phases(p, *_):
+        seen.append(p._obj.flags)
+        assert p._obj.workspace_bytes >= lib.axl_flash_bwd_workspace_bytes(p)
+        return _lib.AXL_OK
+
+    lib = _lib.load()
+    size = lib.axl_flash_bwd_workspace_bytes
+    fake = type("Lib", (), dict(axl_flash_bwd_workspace_bytes=staticmethod(size), axl_flash_bwd_phases=staticmethod(phases)))
+    monkeypatch.setattr(_lib, "load", lambda: fake)
+    monkeypatch.setattr(_lib, "current_stream_ptr", lambda: None)
+    monkeypatch.setattr(ops, "_require_cuda", lambda *x: None)
+    q, k, v, out, do = (torch.zeros(b, t, h, d, dtype=dtype) for _ in range(5))
+    p = _lib.AxlFlashBwdParams(batch=b, q_len=t, kv_len=t, num_q_heads=h, num_kv_heads=h, head_dim=d,
+                               dtype=_lib.dtype_code(dtype), mask_kind=ops.MASK_CAUSAL)
+    need = []
+    for p.flags in (1, 0, 2):
+        need.append(size(ctypes.byref(p)))
+    assert need[0] > need[1] and need[2] == 2 * b * h * t * 4 + 240 and (need[1] > need[2]) == (dtype == torch.float32)
+    kw = dict(mask_kind=ops.MASK_CAUSAL, ds_workspace=forced, ds_workspace_limit=1 << 30)
+    if kind == "bias":
+        kw["bias"] = torch.zeros(1, h, t, t, dtype=torch.bfloat16)
+    if kind == "drop":
+        kw.update(dropout_mask=torch.zeros(b, h, t, t, dtype=torch.bool), dropout_rate=0.1)
+    empty = torch.empty
+    for room, want in zip(need, flags):
+        def limited(*size, **opts):
+            if opts.get("dtype") == torch.uint8 and size[0][0] > room:
+                raise torch.OutOfMemoryError("no room")
+            return empty(*size, **opts)
+
+        buffers = (*(torch.empty_like(x) for x in (q, k, v)), torch.empty((room,), dtype=torch.uint8)) if own_buffers else None
+        with monkeypatch.context() as m:
+            if not own_buffers:
+                m.setattr(torch, "empty", limited)
+            call = lambda: ops.flash_bwd(q, k, v, out, torch.zeros(b, h, t), do, buffers=buffers, **kw)
+            if want is None:
+                with pytest.raises(_lib.AxlError if own_buffers else torch.OutOfMemoryError):
+                    call()
+            else:
+                call()
+                assert seen[-1] == want
+
+
 def test_rows_of_a_view_are_copied_only_where_the_kernels_cannot_read_them():
     base = torch.randn(2, 8, 4, 72).to(torch.bfloat16)
     for x in (base, base[..., :64], base[:, :, 1:], base.transpose(1, 2), base[..., 8:40]):
