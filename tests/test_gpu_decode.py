@@ -839,8 +839,8 @@ def test_decode_kv_dtype_other_than_the_query_dtype(q_dtype, kv_dtype):
 ])
 def test_decode_in_equal_shares(b, hq, hkv, d, pps, window):
     # Calls whose capacity gives a workgroup at most 256 tiles divide the live tiles evenly: lengths of 0, 1,
-    # a tile and the capacity among random ones; the bits of the lengths read as positions in either
-    # integer type (int64 with a stride), and the oracle within the bar.
+    # a tile and the capacity among random ones, and the oracle within the bar.  Lengths, or positions in either integer
+    # type (int64 with a stride): the same bits where the decomposition is fixed.
     q, kp, vp, tables, lengths = ref.paged_inputs(31, batch=b, num_heads=hq, num_kv_heads=hkv, head_dim=d, page_size=16,
                                                   pages_per_seq=pps, min_len=1, max_len=16 * pps)
     for i, n in enumerate((16 * pps, 0, 1, 16, 17)):
@@ -851,7 +851,12 @@ def test_decode_in_equal_shares(b, hq, hkv, d, pps, window):
                                 sliding_window=None if window < 0 else window)[:, 0]
     live = lengths > 0
     pos = torch.stack([lengths.long() - 1, torch.zeros(b, dtype=torch.int64)], 1).cuda()[:, 0]
+    fixed = []
     for lens, kw in ((lengths.cuda(), {}), (pos, dict(lengths_are_positions=True)),
                      (pos.to(torch.int32), dict(lengths_are_positions=True))):
-        got = ops.paged_decode(*args, lens, softmax_scale=0.1, sliding_window=window, **kw).cpu()
-        assert _ok(got[live], want[live]) and torch.equal(got[~live], torch.zeros_like(got[~live]))
+        for deterministic in (False, True):
+            got = ops.paged_decode(*args, lens, softmax_scale=0.1, sliding_window=window, deterministic=deterministic,
+                                   **kw).cpu()
+            assert _ok(got[live], want[live]) and torch.equal(got[~live], torch.zeros_like(got[~live]))
+        fixed.append(got)
+    assert torch.equal(fixed[0], fixed[1]) and torch.equal(fixed[0], fixed[2])
