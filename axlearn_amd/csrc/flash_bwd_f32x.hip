@@ -31,7 +31,7 @@ namespace axl {
 // than one accumulator set (64 registers), so both operands fit 256 registers and two wavefronts a SIMD.
 // Rings: Q planes of three tiles (e-1, e, e+1), dO planes of two, P of two, statistics of three.
 //
-// B2 H32 T4096 D128 causal: 2.67 ms, matrix cores 73 % busy (at the 1.7 GHz that the power limit leaves; one wavefront
+// B2 H32 T4096 D128 causal: 2.55 ms, matrix cores 73 % busy (at the 1.7 GHz that the power limit leaves; one wavefront
 // per SIMD: 6.4 ms, 20 %).
 // ---------------------------------------------------------------------------------------------
 template <int D>
@@ -340,7 +340,7 @@ void flash_bwd_dkdv_f32x_kernel(const BwdArgs a) {
 // two tiles ahead.  Bound by the matrix cores (six bf16 products per pair and
 // element of d) with dS read from HBM once, 4 bytes per visible pair.
 //
-// B2 H32 T4096 D128 causal: 0.96 ms, matrix cores 53 % busy (recomputing S and dP: 4.3 ms).
+// B2 H32 T4096 D128 causal: 0.94 ms, matrix cores 53 % busy (recomputing S and dP: 4.3 ms).
 // ---------------------------------------------------------------------------------------------
 template <int D>
 struct DqDsF32 : TileF32x<D> {

@@ -112,8 +112,8 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
     return (max(end, begin + 1) - begin + 63) / 64;
   };
   // The plan stands at the head of both kernels' chains of latencies: the lengths of the first 64 sequences are read
-  // once, and the reductions go over no more lanes than there are sequences (2 x 200 rows of 32 heads over 8192 keys:
-  // chunk kernel 40.5 -> 38.5 us, merge 10.4 -> 9.2 us).
+  // once, and the reductions go over no more lanes than there are sequences (2 x 200 rows of 32 heads over a cache of
+  // 8192 keys, at one pair of offsets: chunk kernel 40.5 -> 38.5 us, merge 10.4 -> 9.2 us).
   const int own = tiles(lane);
   auto tiles_of = [&](int b) -> int { return b == lane ? own : tiles(b); };
   const int span = a.B >= 64 ? 64 : a.B <= 1 ? 1 : 2 << (31 - __builtin_clz(a.B - 1));   // power of two, lanes with work
@@ -168,7 +168,8 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
 //     the positions is looked at on the host.
 // A call of 42 GFLOP (offsets 7552 and 4996) took 55 us this way (760 TFLOP/s; the forward at full occupancy runs
 // at 1000) and 10 us for the merge; since, with the plan's reads shortened, 38.5 instead of 40.5 and 8.6 instead
-// of 10.4 us at other offsets.  As a call of the layer 172 -> 45 us (host path included).
+// of 10.4 us at other offsets.  Over pairs of offsets drawn from the cache the chunk kernel takes 38 to 53 us and the
+// merge 8.0 to 8.9.  As a call of the layer 172 -> 45 us (host path included).
 template <typename E, int D, int INPUTS, int NW, bool CHUNK>
 __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // BIAS16: a bf16 bias and nothing else, known at compile time; AUX without it: whatever there is.
@@ -735,8 +736,9 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   {
     // Tiles [f_lo, f_hi) of this wavefront take the FAST form: inside its own range, the tile after
     // them inside it too, no positional mask (every key of the tile at or before the wavefront's first
-    // query and, under a sliding window, within the window of its last query), no segment ids, no bias
-    // or dropout mask.  f_lo has the parity of t_begin so that a pair of FAST tiles uses the register
+    // query and, under a sliding window, within the window of its last query), no segment ids other than
+    // the one id of the wavefront's queries, no fp32 bias or dropout mask (a bf16 bias alone is added in the FAST
+    // form too).  f_lo has the parity of t_begin so that a pair of FAST tiles uses the register
     // sets and the buffers in the order (even, odd).
     const std::integral_constant<int, 0> c0{};
     const std::integral_constant<int, 1> c1{};
