@@ -19,7 +19,7 @@ AXL_BF16, AXL_F32, AXL_F16 = 0, 1, 2
 MASK_NONE, MASK_CAUSAL, MASK_SLIDING_WINDOW = 0, 1, 2
 DECODE_DETERMINISTIC, DECODE_WORKSPACE_REUSED = 1, 2  # AXL_DECODE_* flags
 DECODE_LENGTHS_ARE_POSITIONS, DECODE_LENGTHS_I64 = 4, 8
-BWD_DS_WORKSPACE, BWD_F32_NO_PLANES = 1, 2  # AXL_BWD_* flags
+BWD_DS_WORKSPACE, BWD_F32_NO_PLANES, BWD_NO_SPLIT = 1, 2, 4  # AXL_BWD_* flags
 AXL_OK, AXL_ERR_INVALID_ARGUMENT, AXL_ERR_UNSUPPORTED, AXL_ERR_WORKSPACE, AXL_ERR_LAUNCH = 0, -1, -2, -3, -4
 
 

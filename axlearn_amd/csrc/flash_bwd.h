@@ -35,6 +35,8 @@ struct BwdArgs {
                 // place of the slices past it (finite values that only ever meet those zeros or end up in
                 // output columns that are not stored), stores leave the columns past it out.
   int kb_per_wg;  // key blocks (of 128 keys) a dK/dV workgroup works through: 1, or 2 (a block and its mirror image)
+  int splits;     // 16-bit dK/dV: workgroups that share the query tiles of a key block (plan_dkdv); with more than
+  char* part;     // one, the workspace's partial sums, DkvPart<width>::BYTES per (pair, key block, split, wavefront)
   AuxArgs aux;  // dense bias / dropout mask (read only by the AUX instantiations)
 };
 
@@ -74,10 +76,18 @@ __host__ __device__ inline int64_t ds32_run_start(int64_t pair, int T, int G, in
   return G * (pair * ds32_blocks_per_head(T) + (int64_t)t * (t + 1) / 2) + (int64_t)hh * (t + 1);
 }
 
+// Partial sums of a split dK/dV launch: the fp32 accumulators of a wavefront's 32 keys as they lie in registers, dK
+// then dV, each [D / 8 pieces][64 lanes] float4, so that a store instruction writes 1 KB in one piece.
+template <int D>
+struct DkvPart {
+  static constexpr int TENSOR_BYTES = 32 * D * 4;
+  static constexpr int BYTES = 2 * TENSOR_BYTES;
+};
+
 // Enqueues the dK/dV kernel for `dtype` AXL_BF16 or AXL_F16 and head_dim 64 or 128; `aux` selects
 // the instantiation that reads the dense bias / dropout mask.  With a.ds set (causal or sliding-window
 // mask, q_off 0, T == S) the kernel also stores dS for launch_bwd_dq_stream, and with a.kb_tbl set the
-// range of query tiles each key block stored.
+// range of query tiles each key block stored.  With a.splits > 1 the sum over the splits follows.
 hipError_t launch_bwd_dkdv(const BwdArgs& a, int dtype, int head_dim, bool aux, hipStream_t stream);
 hipError_t launch_bwd_dkdv_aux(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 hipError_t launch_bwd_dkdv_bias(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);

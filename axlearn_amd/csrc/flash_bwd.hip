@@ -18,6 +18,8 @@
 //   dQ: a workgroup owns 128 queries (32 per wavefront, Q and dO fragments in registers) and
 //     streams 64-key K/V tiles through LDS exactly like the forward; S^T = K Q^T, dP^T = V dO^T,
 //     dQ^T += K^T dS^T with K^T from transposing LDS reads.
+#include <algorithm>
+
 #include "flash_bwd.h"
 
 namespace axl {
@@ -441,13 +443,85 @@ static size_t planes_bytes(const AxlFlashBwdParams& p) {
   return (size_t)p.batch * p.num_q_heads * p.q_len * (p.head_dim <= 64 ? 64 : 128) * 6;
 }
 
+// How the 16-bit dK/dV kernel's work is cut: key blocks per workgroup (kb_per_wg) and workgroups that share the query
+// tiles of a key block (splits).
+//
+// The kernel's own parallelism is (batch, kv head, key block): a call with few kv heads leaves CUs idle while each
+// workgroup walks G x T / 32 tiles (batch 1, 64 / 8 heads, 1792 tokens: 56 workgroups of 480 tiles on 256 CUs).  There the
+// query tiles are split, fp32 partial sums go through the workspace and a second kernel adds them.  Costs, in tiles
+// (0.87 us at the compiled width 128, 0.5 at 64): 12 per key block that a workgroup starts and ends (11 us), 8 for
+// the second launch and 16 per 256 blocks of partial sums written and read.  The split is taken where the
+// longest workgroup walks kSplitTiles or more and this estimate falls by a sixth; below that a call is bound by its
+// caller's host work (kernels of less than 110 us in a step of about 200).  Causal, bf16, dK/dV without / with the split
+// and the sum: batch 1, 8 / 1 heads, 4096 tokens 840 / 91 + 14 us; 64 / 8 heads, 1024 tokens 253 / 63 + 10 us; 32 / 8
+// heads, 2048 tokens 248 / 97 + 12 us; 12 / 4 heads of 64, 4096 tokens 241 / 88 + 7 us; batch 2, 8 / 1 heads with a bias,
+// 1920 tokens 427 / 58 + 12 us; batch 1, 8 / 1 heads, 16384 tokens, window 1024: 257 / 161 + 11 us.
+struct DkdvPlan {
+  int kb_per_wg, splits;
+};
+constexpr int kSplitTiles = 128, kMaxSplits = 32, kMaxSplitBlocks = 512;
+static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind) {
+  // Two key blocks per workgroup under a causal mask, where a block and its mirror image see
+  // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
+  // environment (read once) keeps one block per workgroup.
+  static const bool single = [] { const char* e = getenv("AXL_DKDV_KB_PER_WG"); return e && e[0] == '1'; }();
+  const int nkb = p.kv_len / 128;
+  const bool mirror = !single && mask_kind == AXL_MASK_CAUSAL && nkb % 2 == 0;
+  const DkdvPlan whole{mirror ? 2 : 1, 1};
+  if (p.dtype == AXL_F32 || nkb < 1) return whole;
+  const int64_t pairs = (int64_t)p.batch * p.num_kv_heads, blocks = pairs * nkb;
+  const int G = p.num_q_heads / p.num_kv_heads, cus = cu_count();
+  if (blocks >= 4 * (int64_t)cus) return whole;
+  // query tiles x heads of the longest key block, of a block and its mirror image, and of all blocks
+  int64_t longest = 0, total = 0;
+  for (int kb = 0; kb < nkb; kb++) {
+    int64_t lo = 0, hi = p.q_len;
+    if (mask_kind != AXL_MASK_NONE) lo = std::max<int64_t>(0, std::min<int64_t>(p.q_len, (int64_t)kb * 128 - p.q_pos_offset));
+    if (mask_kind == AXL_MASK_SLIDING_WINDOW)
+      hi = std::max<int64_t>(lo, std::min<int64_t>(p.q_len, (int64_t)kb * 128 + 128 + p.sliding_window - p.q_pos_offset));
+    const int64_t n = (hi - lo + 31) / 32 * G;
+    longest = std::max(longest, n);
+    total += n;
+  }
+  const double both = mirror ? 2.0 * total / nkb : 0;   // the mirror images add up to the same for every workgroup
+  if ((mirror ? both : (double)longest) < kSplitTiles) return whole;
+  const double start = p.head_dim <= 64 ? 22 : 12, bytes = 16 / 256.0;   // (64: half the bytes, half the time per tile)
+  auto cost = [&](const DkdvPlan& x) {
+    const int64_t wgs = blocks / x.kb_per_wg * x.splits;
+    double c;
+    if (x.kb_per_wg == 2) c = (double)((wgs + cus - 1) / cus) * (both / x.splits + 2 * start);
+    else c = std::max((double)longest / x.splits + start, 1.1 * ((double)total * pairs + start * (double)wgs) / cus);
+    return x.splits == 1 ? c : c + 8 + bytes * (double)(blocks * x.splits);
+  };
+  DkdvPlan best = whole;
+  double best_cost = cost(whole) / 1.2;
+  for (int kpw = 1; kpw <= whole.kb_per_wg; kpw++)
+    for (int n = 2; n <= kMaxSplits && blocks * n <= kMaxSplitBlocks; n++)
+      if (cost(DkdvPlan{kpw, n}) < best_cost) {
+        best = DkdvPlan{kpw, n};
+        best_cost = cost(best);
+      }
+  return best;
+}
+// Bytes of the partial sums.  The same for every mask, so that a workspace sized without it fits: a window's calls,
+// which the size does not look at, take no more splits than there is room for.
+static int max_splits(const AxlFlashBwdParams& p) {
+  if (p.flags & AXL_BWD_NO_SPLIT) return 1;
+  return std::max(plan_dkdv(p, AXL_MASK_NONE).splits, plan_dkdv(p, AXL_MASK_CAUSAL).splits);
+}
+static size_t split_bytes(const AxlFlashBwdParams& p) {
+  const int n = max_splits(p);
+  if (n <= 1) return 0;
+  return (size_t)p.batch * p.num_kv_heads * (p.kv_len / 128) * n * 4 * (p.head_dim <= 64 ? DkvPart<64>::BYTES : DkvPart<128>::BYTES);
+}
+
 // The parts of the workspace start on 256-byte boundaries; the caller's pointer only has to be
 // 16-byte aligned (allocators that slice one arena, XLA's buffer assignment among them, promise less
 // than 256), so the size includes the slack for rounding it up.
 constexpr size_t kWsAlign = 256;
 size_t flash_bwd_workspace_bytes(const AxlFlashBwdParams& p) {
-  return stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p) + 2 * planes_bytes(p) + (spill_eligible(p) ? spill_bytes(p) : 0) +
-         (kWsAlign - 16);
+  return stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p) + 2 * planes_bytes(p) + split_bytes(p) +
+         (spill_eligible(p) ? spill_bytes(p) : 0) + (kWsAlign - 16);
 }
 
 int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream) {
@@ -464,7 +538,8 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   char* const ws_planes = ws + stats_bytes(p) + seg_table_bytes(p) + kb_table_bytes(p);
   a.q_planes = f32_planes(p) ? ws_planes : nullptr;
   a.do_planes = f32_planes(p) ? ws_planes + planes_bytes(p) : nullptr;
-  a.ds = spill ? ws_planes + 2 * planes_bytes(p) : nullptr;
+  a.part = ws_planes + 2 * planes_bytes(p);
+  a.ds = spill ? a.part + split_bytes(p) : nullptr;
   a.qs = to_s3(p.q_strides); a.ks = to_s3(p.k_strides); a.vs = to_s3(p.v_strides);
   a.os = to_s3(p.out_strides); a.dos = to_s3(p.d_out_strides); a.dqs = to_s3(p.dq_strides);
   a.dks = to_s3(p.dk_strides); a.dvs = to_s3(p.dv_strides);
@@ -474,11 +549,9 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   a.d_real = p.head_dim;
   a.stat_hq = p.num_q_heads;
   {
-    // Two key blocks per dK/dV workgroup under a causal mask, where a block and its mirror image see
-    // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
-    // environment (read once) keeps one block per workgroup.
-    static const bool single = [] { const char* e = getenv("AXL_DKDV_KB_PER_WG"); return e && e[0] == '1'; }();
-    a.kb_per_wg = (!single && p.mask_kind == AXL_MASK_CAUSAL && (p.kv_len / 128) % 2 == 0) ? 2 : 1;
+    const DkdvPlan plan = plan_dkdv(p, p.mask_kind);   // of all kv heads, whatever the slices: the same sums
+    a.kb_per_wg = plan.kb_per_wg;
+    a.splits = std::min(plan.splits, max_splits(p));
   }
   const int width = p.head_dim <= 64 ? 64 : 128;   // the compiled width that serves this head_dim
   a.aux = make_aux_args(p.aux, p.softmax_scale);

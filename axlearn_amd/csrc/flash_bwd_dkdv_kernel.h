@@ -97,7 +97,10 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   // them brings a Q / dO tile into L2, the others find it there), half as many workgroups start and
   // end, and the launch divides evenly over the CUs.
   const int npairs = a.B * a.Hkv, nkb = a.S / Tile::BKV;
-  const int nkb_wg = nkb / a.kb_per_wg;              // key blocks the blockIdx mapping numbers
+  // With a.splits > 1 (plan_dkdv: launches that would leave CUs idle) that many workgroups share the query tiles of
+  // a key block, or of both, each leaving fp32 partial sums for flash_bwd_dkdv_combine_kernel; the splits of a key
+  // block have neighbouring numbers.
+  const int nkb_wg = nkb / a.kb_per_wg * a.splits;   // (key block, split) pairs the blockIdx mapping numbers
   int kb0, pair;
   if (npairs % 8 == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -110,6 +113,11 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   } else {
     kb0 = blockIdx.x / npairs;
     pair = blockIdx.x % npairs;
+  }
+  int split = 0;
+  if (a.splits > 1) {
+    split = kb0 % a.splits;
+    kb0 /= a.splits;
   }
   const int b = pair / a.Hkv, hk = pair % a.Hkv;
   for (int pass = 0; pass < a.kb_per_wg; pass++) {
@@ -154,11 +162,16 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
     sub_g0 = classify_segment_groups_tbl<256>(a.seg_tbl + (int64_t)b * (a.T / kSegGroupRows), k0_wg / kSegGroupRows,
                                               Tile::BKV / kSegGroupRows, tid, q_begin, q_end, s_sub,
                                               LEAN ? kMaxSubDkv : 0, kNotUniformDkv);
-  const int t_begin = q_begin / Tile::BQ;
-  const int nt = max(0, (q_end + Tile::BQ - 1) / Tile::BQ - t_begin);
+  int t_begin = q_begin / Tile::BQ;
+  int nt = max(0, (q_end + Tile::BQ - 1) / Tile::BQ - t_begin);
   if constexpr (SPILL) {
-    // which tiles' dS this key block stores, for the streaming dQ kernel (the same for every kv head)
-    if (a.kb_tbl && hk == 0 && tid == 0) a.kb_tbl[b * nkb + kb] = make_int2(t_begin, t_begin + nt);
+    // which tiles' dS this key block stores, for the streaming dQ kernel (the same for every kv head and split)
+    if (a.kb_tbl && hk == 0 && split == 0 && tid == 0) a.kb_tbl[b * nkb + kb] = make_int2(t_begin, t_begin + nt);
+  }
+  if (a.splits > 1) {  // this workgroup's share of the tiles
+    const int lo = nt * split / a.splits, hi = nt * (split + 1) / a.splits;
+    t_begin += lo;
+    nt = hi - lo;
   }
   // Tiles in processing order: query tile (outer, from the LAST one down to the diagonal) x query head
   // (inner).  Every workgroup of a (batch, kv head) pair starts at the same last tile and walks down
@@ -825,6 +838,18 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 #undef AXL_A_FRAG
 #undef AXL_ADVANCE
 
+  if (a.splits > 1) {
+    char* part = a.part + (((int64_t)pair * nkb + kb) * a.splits + split) * (4 * DkvPart<D>::BYTES) + wave * DkvPart<D>::BYTES;
+#pragma unroll
+    for (int i = 0; i < 4 * DT; i++) {
+      const floatx4 wk = {dk_acc[i / 4][4 * (i % 4)], dk_acc[i / 4][4 * (i % 4) + 1], dk_acc[i / 4][4 * (i % 4) + 2], dk_acc[i / 4][4 * (i % 4) + 3]};
+      const floatx4 wv = {dv_acc[i / 4][4 * (i % 4)], dv_acc[i / 4][4 * (i % 4) + 1], dv_acc[i / 4][4 * (i % 4) + 2], dv_acc[i / 4][4 * (i % 4) + 3]};
+      *(floatx4*)(part + i * 1024 + 16 * lane) = wk;
+      *(floatx4*)(part + DkvPart<D>::TENSOR_BYTES + i * 1024 + 16 * lane) = wv;
+    }
+    __syncthreads();  // as below
+    continue;
+  }
   __bf16* dkp = (__bf16*)a.dk + b * a.dks.b + (int64_t)(k0 + l32) * a.dks.s + hk * a.dks.h;
   __bf16* dvp = (__bf16*)a.dv + b * a.dvs.b + (int64_t)(k0 + l32) * a.dvs.s + hk * a.dvs.h;
 #pragma unroll
@@ -848,13 +873,51 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   }  // key blocks of this workgroup
 }
 
+// Sums the partial dK (blockIdx.y 0) and dV (1) of a split launch in the order of the splits, and scales and rounds
+// as the kernel above does at its end.  One workgroup per 32 keys, a wavefront per 32 columns of head_dim, the pieces read
+// as they were written (1 KB per instruction, four splits in flight).  Bound by the bytes.
+template <typename E, int D>
+__global__ __launch_bounds__(2 * D) void flash_bwd_dkdv_combine_kernel(const BwdArgs a) {
+  const int lane = threadIdx.x & 63, dt = threadIdx.x >> 6, l32 = lane & 31, g = lane >> 5;
+  const int nkb = a.S / 128, blk = blockIdx.x >> 2, wave = blockIdx.x & 3, is_v = blockIdx.y;
+  const int pair = blk / nkb, kb = blk - pair * nkb, b = pair / a.Hkv, hk = pair - b * a.Hkv;
+  const char* part = a.part + (int64_t)blk * a.splits * (4 * DkvPart<D>::BYTES) + wave * DkvPart<D>::BYTES +
+                     is_v * DkvPart<D>::TENSOR_BYTES + dt * 4096 + 16 * lane;
+  constexpr int kBatch = 4;
+  floatx4 acc[4] = {};
+  for (int s0 = 0; s0 < a.splits; s0 += kBatch) {
+    floatx4 x[kBatch][4];
+#pragma unroll
+    for (int i = 0; i < kBatch; i++)
+#pragma unroll
+      for (int rq = 0; rq < 4; rq++)   // past the end: the last split, not counted
+        x[i][rq] = *(const floatx4*)(part + (int64_t)min(s0 + i, a.splits - 1) * (4 * DkvPart<D>::BYTES) + rq * 1024);
+#pragma unroll
+    for (int i = 0; i < kBatch; i++)
+      if (s0 + i < a.splits) {
+#pragma unroll
+        for (int rq = 0; rq < 4; rq++) acc[rq] += x[i][rq];
+      }
+  }
+  const Strides3 st = is_v ? a.dvs : a.dks;
+  const float f = is_v ? a.aux.keep_scale : a.scale;
+  __bf16* row = (__bf16*)(is_v ? a.dv : a.dk) + b * st.b + (int64_t)(kb * 128 + wave * 32 + l32) * st.s + hk * st.h;
+#pragma unroll
+  for (int rq = 0; rq < 4; rq++) {
+    union { bf16x2 p[2]; uint2 u; } w;
+    w.p[0] = E::pack(acc[rq][0] * f, acc[rq][1] * f);
+    w.p[1] = E::pack(acc[rq][2] * f, acc[rq][3] * f);
+    if (32 * dt + 8 * rq + 4 * g < a.d_real) *(uint2*)(row + 32 * dt + 8 * rq + 4 * g) = w.u;
+  }
+}
+
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
   auto kernel = flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
-  const int grid = (a.S / Tile::BKV) * a.B * a.Hkv / a.kb_per_wg;
+  const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), Tile::LDS_BYTES, stream, a);
   return hipGetLastError();
 }

@@ -326,17 +326,21 @@ def flash_bwd(
 def _bwd_workspace(lib, p: AxlFlashBwdParams, ds_optional: bool, ws: Optional[torch.Tensor], device) -> torch.Tensor:
     """The backward's workspace: `ws`, or a new one where that is None.
 
-    Where there is no room for the workspace of `p.flags`, the largest that there is room for: without dS if that is
-    optional (the size rule's choice, a float32 call, or one with a bias or dropout mask), in float32 at last
-    without the planes.  `p.flags` is set to match; the kernels that make do with less are slower."""
-    choices = [p.flags]
+    Where there is no room for the workspace of `p.flags`, the largest that there is room for: in a 16-bit type without
+    partial sums of dK and dV, then without dS if that is optional (the size rule's choice, a float32 call, or one with a
+    bias or dropout mask), in float32 at last without the planes.  `p.flags` is set to match; the kernels that make do with less are slower."""
+    no_split = 0 if p.dtype == _lib.AXL_F32 else _lib.BWD_NO_SPLIT
+    choices = [p.flags, p.flags | no_split]
     if p.flags and (ds_optional or p.dtype == _lib.AXL_F32):
-        choices.append(0)
+        choices += [0, no_split]
     if p.dtype == _lib.AXL_F32:
         choices.append(_lib.BWD_F32_NO_PLANES)
-    error = None
+    error, smallest = None, None
     for p.flags in choices:
         need = int(lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)))
+        if smallest is not None and need >= smallest:
+            continue
+        smallest = need
         if ws is not None:
             have = ws.numel() * ws.element_size()
             if have >= need:

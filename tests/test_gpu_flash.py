@@ -5,6 +5,8 @@ max-abs OR <= 1e-2 relative-L2, measured against the oracle's float64 evaluation
 bf16-rounded inputs.  Masking is checked bit-exactly through poison tests.
 """
 
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -1658,3 +1660,47 @@ def test_chunk_rows_at_positions_of_any_size(kv_len, window):
                                       sliding_window=window or 0).cpu()
                 assert torch.equal(got[~seen], torch.zeros_like(got[~seen]))
                 assert ref.rel_l2(got[seen], want[seen]) < 1e-2
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,bias,dtype", [
+    (1, 1024, 8, 1, 128, "causal", None, False, False, torch.bfloat16),    # 4 workgroups of two key blocks
+    (2, 896, 16, 2, 64, "causal", None, True, False, torch.float16),       # an odd number of key blocks, documents
+    (1, 640, 32, 2, 128, "none", None, False, False, torch.float16),
+    (1, 1280, 16, 1, 128, "sliding", 300, True, False, torch.bfloat16),    # key blocks of unequal ranges, some tiles empty
+    (1, 1280, 16, 2, 80, "causal", None, False, False, torch.bfloat16),    # a head dim below the compiled width
+    (1, 1152, 8, 1, 64, "causal", None, False, True, torch.bfloat16),      # bias through the tile ring
+    (1, 1024, 16, 1, 128, "causal", None, True, True, torch.bfloat16),     # bias beside documents: the general form
+    (1, 128, 256, 2, 64, "none", None, False, False, torch.bfloat16),      # one key block, four tiles of 128 heads
+])
+@pytest.mark.parametrize("ds", [False, True])
+def test_query_tiles_of_a_key_block_shared_by_workgroups(b, t, hq, hkv, d, mask, window, packed, bias, dtype, ds):
+    """Calls with few kv heads: several workgroups share a key block's query tiles.  Against the same call
+    without room for partial sums (AXL_BWD_NO_SPLIT): dq is the same bits, dk and dv are fp32 sums in another
+    order, rounded once, so an element moves by at most one step of its type (2^-8 / 2^-11 of its size, the sums themselves
+    differ by less than 1e-5 of the rms).  The workspace starts as NaN: no partial sum is read unwritten."""
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, dtype))
+    segs = ref.packed_segment_ids(3, b, t).cuda() if packed else None
+    mk = {"none": ops.MASK_NONE, "causal": ops.MASK_CAUSAL, "sliding": ops.MASK_SLIDING_WINDOW}[mask]
+    kw = dict(mask_kind=mk, sliding_window=window or 0, softmax_scale=d ** -0.5, segment_ids=segs)
+    if bias:
+        kw["bias"] = torch.randn(1, hq, t, t, device="cuda", generator=torch.Generator("cuda").manual_seed(1)).to(torch.bfloat16)
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    bufs = ops.flash_bwd_buffers(q, k, v, mask_kind=mk, ds_workspace=ds, segment_ids=segs)
+    p = _lib.AxlFlashBwdParams(batch=b, q_len=t, kv_len=t, num_q_heads=hq, num_kv_heads=hkv, head_dim=d, mask_kind=mk,
+                               dtype=_lib.dtype_code(dtype), segment_ids=256 if packed else None,
+                               flags=_lib.BWD_NO_SPLIT | (_lib.BWD_DS_WORKSPACE if ds else 0))
+    small = _lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p))
+    assert small < bufs[3].numel()
+    whole = (*(torch.empty_like(x) for x in (q, k, v)), torch.empty(small, dtype=torch.uint8, device="cuda"))
+    for x in (bufs[3], whole[3]):
+        x.fill_(0xff)
+    got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=bufs, **kw)
+    want = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=whole, **kw)
+    step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    assert torch.equal(got[0], want[0])
+    for name, x, y in (("dk", got[1].float(), want[1].float()), ("dv", got[2].float(), want[2].float())):
+        rms = y.square().mean().sqrt()
+        assert ((x - y).abs() <= 2 * step * y.abs() + 2e-5 * rms).all(), name
+        assert ref.rel_l2(x.cpu(), y.cpu()) < step / 4, name
+    again = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=bufs, **kw)
+    assert all(torch.equal(x, y) for x, y in zip(again, got))
