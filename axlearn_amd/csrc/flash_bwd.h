@@ -84,7 +84,8 @@ struct DkvPart {
   static constexpr int BYTES = 2 * TENSOR_BYTES;
 };
 
-// Enqueues the dK/dV kernel for `dtype` AXL_BF16 or AXL_F16 and head_dim 64 or 128; `aux` selects
+// Enqueues the dK/dV kernel for `dtype` AXL_BF16 or AXL_F16 and head_dim (rounded up) 64, 128 or, without `aux`, 96
+// (also for the dQ kernels below); `aux` selects
 // the instantiation that reads the dense bias / dropout mask.  With a.ds set (causal or sliding-window
 // mask, q_off 0, T == S) the kernel also stores dS for launch_bwd_dq_stream, and with a.kb_tbl set the
 // range of query tiles each key block stored.  With a.splits > 1 the sum over the splits follows.
@@ -96,8 +97,8 @@ hipError_t launch_bwd_dkdv_bias(const BwdArgs& a, int dtype, int head_dim, hipSt
 // from the blocks that table says were stored).
 hipError_t launch_bwd_dq_stream(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 
-// Enqueues the dQ kernel (no dense bias / dropout mask) for `dtype` AXL_BF16 or AXL_F16 and head_dim
-// 64 or 128.  With `fuse_delta` it also writes delta and the scaled lse into the workspace (instead
+// Enqueues the dQ kernel (no dense bias / dropout mask) for `dtype` AXL_BF16 or AXL_F16.
+// With `fuse_delta` it also writes delta and the scaled lse into the workspace (instead
 // of reading them), for a dK/dV kernel enqueued after it.
 hipError_t launch_bwd_dq(const BwdArgs& a, int dtype, int head_dim, bool fuse_delta, hipStream_t stream);
 

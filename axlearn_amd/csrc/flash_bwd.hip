@@ -556,6 +556,8 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   const int width = p.head_dim <= 64 ? 64 : 128;   // the compiled width that serves this head_dim
   a.aux = make_aux_args(p.aux, p.softmax_scale);
   const bool aux = p.aux.bias || p.aux.dropout_mask;
+  // 16-bit dK/dV and dQ: head dims 72 to 96 leave the last 32 columns of the width 128 out (no bias or mask there)
+  const int live = width == 128 && p.head_dim <= 96 && !aux ? 96 : width;
   hipError_t err = hipSuccess;
   const int64_t rows = (int64_t)p.batch * p.q_len * p.num_q_heads;
   const int delta_grid = (int)((rows + 15) / 16);
@@ -631,8 +633,8 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
         err = launch_bwd_f32(s, width, phases, stream);
         continue;
       }
-      if (phases & AXL_BWD_DKDV) err = launch_bwd_dkdv(s, dt, width, aux, stream);
-      if ((phases & AXL_BWD_DQ) && err == hipSuccess) err = launch_bwd_dq_stream(s, dt, width, stream);
+      if (phases & AXL_BWD_DKDV) err = launch_bwd_dkdv(s, dt, live, aux, stream);
+      if ((phases & AXL_BWD_DQ) && err == hipSuccess) err = launch_bwd_dq_stream(s, dt, live, stream);
     }
     phases &= AXL_BWD_DELTA;  // what is left for the code below: the sink gradient
     phases = (phases & AXL_BWD_DELTA) && p.d_logit_sink ? AXL_BWD_DELTA : 0;
@@ -645,8 +647,8 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       return set_error(AXL_ERR_LAUNCH, "axl_flash_bwd: launch failed: %s", hipGetErrorString(err));
     return AXL_OK;
   } else if ((phases & all) == all && !aux && !p.d_logit_sink) {
-    err = launch_bwd_dq(a, dt, width, true, stream);
-    if (err == hipSuccess) err = launch_bwd_dkdv(a, dt, width, false, stream);
+    err = launch_bwd_dq(a, dt, live, true, stream);
+    if (err == hipSuccess) err = launch_bwd_dkdv(a, dt, live, false, stream);
     if (err != hipSuccess)
       return set_error(AXL_ERR_LAUNCH, "axl_flash_bwd: launch failed: %s", hipGetErrorString(err));
     return AXL_OK;
@@ -654,10 +656,10 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
 #define AXL_BWD_PHASES(E, T, DD)                                                                  \
   do {                                                                                            \
     if (phases & AXL_BWD_DELTA) AXL_LAUNCH((bwd_delta_kernel<T, DD>), delta_grid, 0);             \
-    if ((phases & AXL_BWD_DKDV) && err == hipSuccess) err = launch_bwd_dkdv(a, dt, DD, aux, stream); \
+    if ((phases & AXL_BWD_DKDV) && err == hipSuccess) err = launch_bwd_dkdv(a, dt, live, aux, stream); \
     if ((phases & AXL_BWD_DQ) && aux)                                                             \
       AXL_LAUNCH((flash_bwd_dq_aux_kernel<E, DD, true>), dq_grid, DqTile<DD>::LDS_BYTES);         \
-    if ((phases & AXL_BWD_DQ) && !aux && err == hipSuccess) err = launch_bwd_dq(a, dt, DD, false, stream); \
+    if ((phases & AXL_BWD_DQ) && !aux && err == hipSuccess) err = launch_bwd_dq(a, dt, live, false, stream); \
   } while (0)
   if (dt == AXL_F32) {
     // enqueued above

@@ -67,7 +67,11 @@ constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than 
 // With a dense bias or a dropout mask too: the recomputing dQ kernel reads those a second time and is the
 // slower the more it has to read (causal, B2 H16 T2048 D128, bias bf16: 117 us; from dS 46 us, for 5 us
 // more in this kernel).
-template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
+//
+// W: live width, the head_dim rounded up to a multiple of 32 (D: the width of a row in LDS).  The MFMAs and fragment
+// reads past it, whose operands or results are nothing but padding, are left out (B2 H32/8 T4096, head_dim 96 causal
+// with dS 557 -> 481 us, 80 unmasked 931 -> 775 us; the recomputing dQ kernel there 708 -> 590 us).
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false, int W = D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void flash_bwd_dkdv_kernel(const BwdArgs a) {
   // A bf16 bias alone comes through the tile ring like Q and dO, its elements read from LDS where they are used;
@@ -79,7 +83,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   using Tile = DkvTile<D, BIAS_LDS>;
   constexpr bool HAS_BIAS = (AUX & (kAuxBias16 | kAuxBias32)) != 0, BIAS_F32 = (AUX & kAuxBias32) != 0;
   constexpr bool HAS_DROP = (AUX & kAuxDrop) != 0;
-  constexpr int KK = D / 16, DT = D / 32;
+  constexpr int KK = W / 16, DT = W / 32;
   constexpr int NA = 2 * KK;          // stage-A MFMAs per tile
   constexpr int NB = 4 * DT;          // stage-B MFMAs per tile
   static_assert(Tile::BQ == 32, "tiling");
@@ -498,7 +502,7 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 
   constexpr int NS = NA + NB;          // MFMAs per iteration: stage B of tile j, then stage A of tile j+2
   constexpr int ESTEP = NS / 16;       // bias / dropout loads: one of the 16 elements per lane every ESTEP slots
-  static_assert(NS % 16 == 0, "the 16 elements per lane are spread evenly over the MFMA slots");
+  static_assert(LEAN || NS % 16 == 0, "the 16 elements per lane are spread evenly over the MFMA slots");
   constexpr int kAheadA = 6, kAheadB = 4;
   constexpr int NLD = Tile::DMA_PER_TILE;     // direct-to-LDS loads of a tile per wavefront
   constexpr int LD_SLOT0 = 2;                 // one per slot from here on, after the cursor moved in slot 1
@@ -839,13 +843,13 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 #undef AXL_ADVANCE
 
   if (a.splits > 1) {
-    char* part = a.part + (((int64_t)pair * nkb + kb) * a.splits + split) * (4 * DkvPart<D>::BYTES) + wave * DkvPart<D>::BYTES;
+    char* part = a.part + (((int64_t)pair * nkb + kb) * a.splits + split) * (4 * DkvPart<W>::BYTES) + wave * DkvPart<W>::BYTES;
 #pragma unroll
     for (int i = 0; i < 4 * DT; i++) {
       const floatx4 wk = {dk_acc[i / 4][4 * (i % 4)], dk_acc[i / 4][4 * (i % 4) + 1], dk_acc[i / 4][4 * (i % 4) + 2], dk_acc[i / 4][4 * (i % 4) + 3]};
       const floatx4 wv = {dv_acc[i / 4][4 * (i % 4)], dv_acc[i / 4][4 * (i % 4) + 1], dv_acc[i / 4][4 * (i % 4) + 2], dv_acc[i / 4][4 * (i % 4) + 3]};
       *(floatx4*)(part + i * 1024 + 16 * lane) = wk;
-      *(floatx4*)(part + DkvPart<D>::TENSOR_BYTES + i * 1024 + 16 * lane) = wv;
+      *(floatx4*)(part + DkvPart<W>::TENSOR_BYTES + i * 1024 + 16 * lane) = wv;
     }
     __syncthreads();  // as below
     continue;
@@ -911,10 +915,10 @@ __global__ __launch_bounds__(2 * D) void flash_bwd_dkdv_combine_kernel(const Bwd
   }
 }
 
-template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
-  auto kernel = flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
+  auto kernel = flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL, W>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
   const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;

@@ -48,11 +48,12 @@ constexpr int kNotUniform = -0x7fffffff - 1;  // marks a sub-tile with more than
 // FUSE_DELTA: the kernel also computes delta = rowsum(out * dO) (gpu_attention.py:653-658) and the
 // scaled lse of its own rows and leaves both in the workspace for the dK/dV kernel, which then has to
 // run after this one; the separate delta pass is not needed.
-template <typename E, int D, bool HAS_SEG, int NW, bool FUSE_DELTA>
+// W: live width, as in the dK/dV kernel.
+template <typename E, int D, bool HAS_SEG, int NW, bool FUSE_DELTA, int W>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW / 4, NW / 4)))
 void flash_bwd_dq_ring_kernel(const BwdArgs a) {
   using Tile = DqRing<D, HAS_SEG, NW>;
-  constexpr int KK = D / 16, DT = D / 32;
+  constexpr int KK = W / 16, DT = W / 32;
   constexpr int NA = 2 * KK;          // stage-A MFMAs per sub-tile
   constexpr int NB = 2 * DT;          // stage-B MFMAs per sub-tile
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -517,11 +518,11 @@ void flash_bwd_dq_ring_kernel(const BwdArgs a) {
 // Wavefronts per workgroup: at head_dim 64 the kernel fits 256 registers, and eight wavefronts (two per
 // SIMD, 256 query rows share every K / V tile) are 4 % faster than four; at head_dim 128 they spill
 // (+40 %).
-template <typename E, int D, bool HAS_SEG, bool FUSE_DELTA>
+template <typename E, int D, bool HAS_SEG, bool FUSE_DELTA, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   constexpr int NW = D == 64 ? 8 : 4;
   using Tile = DqRing<D, HAS_SEG, NW>;
-  auto kernel = flash_bwd_dq_ring_kernel<E, D, HAS_SEG, NW, FUSE_DELTA>;
+  auto kernel = flash_bwd_dq_ring_kernel<E, D, HAS_SEG, NW, FUSE_DELTA, W>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
   const int grid = ((a.T + Tile::BQ - 1) / Tile::BQ) * a.B * a.Hq;
@@ -529,17 +530,16 @@ static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+template <typename E, int D, int W = D>
+static hipError_t launch_width(const BwdArgs& a, bool fuse_delta, hipStream_t stream) {
+  if (fuse_delta) return a.seg ? launch_one<E, D, true, true, W>(a, stream) : launch_one<E, D, false, true, W>(a, stream);
+  return a.seg ? launch_one<E, D, true, false, W>(a, stream) : launch_one<E, D, false, false, W>(a, stream);
+}
+
 template <typename E>
 static hipError_t launch_for(const BwdArgs& a, int head_dim, bool fuse_delta, hipStream_t stream) {
-  const bool seg = a.seg != nullptr;
-  if (fuse_delta) {
-    if (head_dim == 128)
-      return seg ? launch_one<E, 128, true, true>(a, stream) : launch_one<E, 128, false, true>(a, stream);
-    return seg ? launch_one<E, 64, true, true>(a, stream) : launch_one<E, 64, false, true>(a, stream);
-  }
-  if (head_dim == 128)
-    return seg ? launch_one<E, 128, true, false>(a, stream) : launch_one<E, 128, false, false>(a, stream);
-  return seg ? launch_one<E, 64, true, false>(a, stream) : launch_one<E, 64, false, false>(a, stream);
+  if (head_dim == 96) return launch_width<E, 128, 96>(a, fuse_delta, stream);
+  return head_dim == 128 ? launch_width<E, 128>(a, fuse_delta, stream) : launch_width<E, 64>(a, fuse_delta, stream);
 }
 
 hipError_t launch_bwd_dq(const BwdArgs& a, int dtype, int head_dim, bool fuse_delta, hipStream_t stream) {

@@ -46,10 +46,11 @@ struct DqStream {
 // RANGED: under a sliding window or with segment ids a key block's dK/dV workgroups store the dS of
 // the query tiles [first, end) that a.kb_tbl records for it; the other blocks of the workspace hold
 // nothing and are skipped (their loads are pointed at the first block, their MFMAs left out).
-template <typename E, int D, int NW, bool RANGED>
+// W: live width, as in the dK/dV kernel.
+template <typename E, int D, int NW, bool RANGED, int W>
 __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdArgs a) {
   using Tile = DqStream<D, NW>;
-  constexpr int DT = D / 32;
+  constexpr int DT = W / 32;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
   const int tid = threadIdx.x;
@@ -247,10 +248,10 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
     }
 }
 
-template <typename E, int D, int NW, bool RANGED>
+template <typename E, int D, int NW, bool RANGED, int W>
 static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
   using Tile = DqStream<D, NW>;
-  auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED>;
+  auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED, W>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
   const int grid = (a.T / Tile::BQ) * a.B * a.Hq;
@@ -258,18 +259,23 @@ static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-template <typename E, int D>
+template <typename E, int D, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   // 8 wavefronts need two K loads per wavefront (head_dim 128) and 256-row blocks
   constexpr int NW8 = D == 128 ? 8 : 4;
   if (D == 128 && a.T % 256 == 0)
-    return a.kb_tbl ? launch_nw<E, D, NW8, true>(a, stream) : launch_nw<E, D, NW8, false>(a, stream);
-  return a.kb_tbl ? launch_nw<E, D, 4, true>(a, stream) : launch_nw<E, D, 4, false>(a, stream);
+    return a.kb_tbl ? launch_nw<E, D, NW8, true, W>(a, stream) : launch_nw<E, D, NW8, false, W>(a, stream);
+  return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
+}
+
+template <typename E>
+static hipError_t launch_for(const BwdArgs& a, int head_dim, hipStream_t stream) {
+  if (head_dim == 96) return launch_one<E, 128, 96>(a, stream);
+  return head_dim == 128 ? launch_one<E, 128>(a, stream) : launch_one<E, 64>(a, stream);
 }
 
 hipError_t launch_bwd_dq_stream(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream) {
-  if (dtype == AXL_F16) return head_dim == 128 ? launch_one<ElemF16, 128>(a, stream) : launch_one<ElemF16, 64>(a, stream);
-  return head_dim == 128 ? launch_one<ElemBf16, 128>(a, stream) : launch_one<ElemBf16, 64>(a, stream);
+  return dtype == AXL_F16 ? launch_for<ElemF16>(a, head_dim, stream) : launch_for<ElemBf16>(a, head_dim, stream);
 }
 
 }  // namespace axl
