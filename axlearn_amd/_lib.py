@@ -23,7 +23,7 @@ BWD_DS_WORKSPACE, BWD_F32_NO_PLANES, BWD_NO_SPLIT = 1, 2, 4  # AXL_BWD_* flags
 AXL_OK, AXL_ERR_INVALID_ARGUMENT, AXL_ERR_UNSUPPORTED, AXL_ERR_WORKSPACE, AXL_ERR_LAUNCH = 0, -1, -2, -3, -4
 
 
-ABI_VERSION = 8  # AXL_ATTN_ABI_VERSION of include/axl_attn.h these structures mirror
+ABI_VERSION = 9  # AXL_ATTN_ABI_VERSION of include/axl_attn.h these structures mirror
 
 
 class AxlError(RuntimeError):
@@ -65,6 +65,7 @@ class AxlFlashFwdParams(ctypes.Structure):
         ("logit_sink", ctypes.c_void_p),
         ("aux", AxlAttnAux),
         ("q_pos_offsets", ctypes.c_void_p),
+        ("bias_copy", ctypes.c_void_p),
     ]
 
 

@@ -219,6 +219,7 @@ int axl_flash_fwd(const AxlFlashFwdParams* p, void* stream) {
     return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: segment_ids must be 16-byte aligned");
   rc = check_aux("axl_flash_fwd", p->aux, p->batch, p->num_q_heads, p->q_len, p->kv_len);
   if (rc != AXL_OK) return rc;
+  if (!aligned16(p->bias_copy)) return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: bias_copy must be 16-byte aligned");
   rc = check_odd_head_dim("axl_flash_fwd", p->head_dim, p->aux.bias || p->aux.dropout_mask,
                           {&p->q_strides, &p->k_strides, &p->v_strides, &p->out_strides});
   if (rc != AXL_OK) return rc;

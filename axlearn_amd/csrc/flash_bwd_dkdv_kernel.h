@@ -372,12 +372,14 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 #define AXL_ELEM_1(R_, MASKED_)                                                                \
   {                                                                                            \
     const int r_ = (R_);                                                                       \
-    float sv_ = s_e[r_];                                                                       \
-    if (MASKED_) {                                                                             \
+    auto masked_ = [&](float x_) __attribute__((always_inline)) {                              \
       const unsigned diff_ = (unsigned)(diff0 + 16 * (r_ / 8) + (r_ % 8));                     \
-      sv_ = diff_ <= limit ? sv_ : kMasked;                                                    \
-      if (HAS_SEG) sv_ = seg_v[r_ / 4][r_ % 4] == seg_k ? sv_ : kMasked;                       \
-    }                                                                                          \
+      x_ = diff_ <= limit ? x_ : kMasked;                                                      \
+      if (HAS_SEG) x_ = seg_v[r_ / 4][r_ % 4] == seg_k ? x_ : kMasked;                         \
+      return x_;                                                                               \
+    };                                                                                         \
+    float sv_ = s_e[r_];                                                                       \
+    if (MASKED_ && !HAS_BIAS) sv_ = masked_(sv_);                                              \
     float off_ = lse_v[r_ / 4][r_ % 4]; /* -lse * log2 e */                                    \
     if constexpr (BIAS_LDS) {                                                                  \
       const unsigned bw_ = (unsigned)(uint16_t)bias_v[r_ / 4][r_ % 4] << 16;                   \
@@ -391,7 +393,11 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
       asm volatile("" : "+v"(bw_));                                                            \
       off_ = __builtin_fmaf(__builtin_bit_cast(float, bw_ << (BIAS_F32 ? 0 : 16)), kLog2e, off_); \
     }                                                                                          \
-    s_e[r_] = __builtin_fmaf(sv_, c, off_);                                                    \
+    sv_ = __builtin_fmaf(sv_, c, off_);                                                        \
+    /* behind the bias: what a masked element's bias is does not matter (a copy that the forward   \
+       kept holds nothing there) */                                                            \
+    if (MASKED_ && HAS_BIAS) sv_ = masked_(sv_);                                               \
+    s_e[r_] = sv_;                                                                             \
   }
 #define AXL_ELEM_2(R_) s_e[R_] = fast_exp2(s_e[R_]);
 #define AXL_ELEM_3(R_)                                                                         \

@@ -37,6 +37,8 @@ struct FwdArgs {
   const float* sink;  // [Hq] logit of the per-head attention sink, or nullptr
   const int32_t* q_offs;  // [B] per-sequence addition to q_off, or nullptr
   AuxArgs aux;        // dense bias / dropout mask (read only by the AUX instantiations)
+  char* bias_copy;    // bf16 bias alone: where the tiles that are read are stored again, or nullptr
+  int64_t copy_sb, copy_sh;  // its strides in BYTES (rows lie as those of the bias do)
   Strides3 qs, ks, vs, os;
   int B, T, S, Hq, Hkv;
   int mask_kind, window, q_off;
@@ -71,8 +73,9 @@ struct FwdTile {
 constexpr int kMaxSegTiles = 1024;               // key tiles whose segment ids the forward classifies
 constexpr int kSegNotUniform = -0x7fffffff - 1;  // marks a tile with more than one segment id
 
-// Optional inputs of the body: none; a bf16 bias and nothing else; whatever the arguments say.
-constexpr int kFwdPlain = 0, kFwdBias16 = 1, kFwdAux = 2;
+// Optional inputs of the body: none; a bf16 bias and nothing else; the same, and it is stored again (FwdArgs::bias_copy);
+// whatever the arguments say.
+constexpr int kFwdPlain = 0, kFwdBias16 = 1, kFwdBias16Copy = 2, kFwdAux = 3;
 
 // Partial results of the chunk form: per workgroup and wavefront the accumulators as they lie in
 // registers, [D / 8 pieces][64 lanes] float4, so that a store instruction writes 1 KB in one piece, then
@@ -177,7 +180,7 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
 template <typename E, int D, int INPUTS, int NW, bool CHUNK, int W = D>
 __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // BIAS16: a bf16 bias and nothing else, known at compile time; AUX without it: whatever there is.
-  constexpr bool AUX = INPUTS != kFwdPlain, BIAS16 = INPUTS == kFwdBias16;
+  constexpr bool AUX = INPUTS != kFwdPlain, COPY = INPUTS == kFwdBias16Copy, BIAS16 = INPUTS == kFwdBias16 || COPY;
   static_assert(!(AUX && CHUNK), "the chunk form takes no bias or dropout mask");
   using Tile = FwdTile<D, NW>;
   constexpr int KK = W / 16;  // MFMA k-steps over head_dim
@@ -301,8 +304,11 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   const uint8_t* drop_row = nullptr;
   // BIAS16: the same as a scalar base and one 32-bit offset per lane (the launcher checks that it fits).
   const char* bias_head = nullptr;
+  char* copy_head = nullptr;   // of one workgroup per row block where batch or heads share the bias
   unsigned bias_off = 0;
   if constexpr (BIAS16) {
+    if (COPY && (a.aux.bias_sb || b == 0) && (a.aux.bias_sh || h == 0))
+      copy_head = a.bias_copy + b * a.copy_sb + h * a.copy_sh;
     bias_head = a.aux.bias + b * a.aux.bias_sb + h * a.aux.bias_sh;
     bias_off = (unsigned)(q0 + l32) * (unsigned)a.aux.bias_sr + 16 * g;
   } else if constexpr (AUX) {
@@ -513,6 +519,11 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     uint2 dm[2][2] = {};  // dropout bytes of the lane's 4 runs of 8 keys
     if constexpr (BIAS16) {
       if (do_sm) {
+        if (COPY && copy_head) {
+          char* p = copy_head + (int64_t)t * (2 * Tile::BK);
+#pragma unroll
+          for (int i = 0; i < 4; i++) *(u32x4*)(p + 64 * (i / 2) + 32 * (i % 2) + bias_off) = bias_nx[i];
+        }
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -847,12 +858,18 @@ void flash_fwd_kernel(const FwdArgs a) {
 // B2 H16 T2048 D128 104 -> 68 us (plain 52), D64 73 -> 43 us (plain 31); B4 H32 T4096 D128 1.53 -> 0.80 ms
 // (plain 0.59; of it, taking the batch's workgroups of one head together, so that the bias comes from memory
 // once: 1.01 -> 0.88, no scratch reload in the FAST loop: 0.88 -> 0.80).
+//
+// COPY: the words of every tile that is read go out again right after they arrived (FwdArgs::bias_copy): the backward
+// reads the bias a second time and its caller may have refilled the buffer by then.  Only visible tiles are moved, part of
+// it under the MFMAs, in place of a pass that reads and writes every element ahead of this kernel: B2 H16 T2048 D128,
+// one bias for the batch, 85 us and 47 us of copy -> 108 us; window 256, B1: 34 and 50 us -> 34 us; B8 H32 D64 280 and
+// 92 us -> 314 us.  A form of its own: the branch alone cost the other calls 6 us of 76.
 // (Requesting the bias after the exponentials, where registers are free, made the compiler spill more
 // of the loop, 108 us.)
-template <typename E, int D>
+template <typename E, int D, bool COPY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_fwd_bias_kernel(const FwdArgs a) {
-  flash_fwd_body<E, D, kFwdBias16, 4, false>(a);
+  flash_fwd_body<E, D, COPY ? kFwdBias16Copy : kFwdBias16, 4, false>(a);
 }
 
 template <typename E, int D>
@@ -1459,6 +1476,12 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   a.q_offs = p.q_pos_offsets;
   a.scale = p.softmax_scale;
   a.d_real = p.head_dim;
+  a.bias_copy = (char*)p.bias_copy;
+  a.copy_sh = a.aux.bias_sh ? (int64_t)p.q_len * p.kv_len * 2 : 0;
+  a.copy_sb = a.aux.bias_sb ? (a.aux.bias_sh ? p.num_q_heads : 1) * (int64_t)p.q_len * p.kv_len * 2 : 0;
+  if (p.bias_copy && !(bias16 && p.dtype != AXL_F32 && !p.segment_ids && p.aux.bias_row_stride == p.kv_len))
+    return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: bias_copy needs a bf16 bias of rows without gaps, a 16-bit "
+                                          "dtype, no dropout mask and no segment_ids");
   const int width = p.head_dim <= 64 ? 64 : 128;  // the compiled width that serves this head_dim
   hipError_t err = hipSuccess;
 #define AXL_LAUNCH_FWD(KERNEL, TILE)                                                            \
@@ -1472,9 +1495,12 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   } while (0)
 #define AXL_LAUNCH_FWD16(E)                                                                     \
   do {                                                                                          \
-    if (bias16) {                                                                               \
-      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128>), FwdTile<128>);          \
-      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64>), FwdTile<64>);                         \
+    if (bias16 && p.bias_copy) {                                                                \
+      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128, true>), FwdTile<128>);    \
+      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64, true>), FwdTile<64>);                   \
+    } else if (bias16) {                                                                        \
+      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128, false>), FwdTile<128>);   \
+      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64, false>), FwdTile<64>);                  \
     } else if (width == 128) {                                                                  \
       if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, true>), FwdTile<128>);                  \
       else if (p.head_dim <= 96) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, false, 4, 96>), FwdTile<128>); \

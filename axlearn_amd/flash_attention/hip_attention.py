@@ -133,7 +133,7 @@ def mask_fn_as_bias(mask_fn: MaskFn, q_len: int, kv_len: int, device, q_pos_offs
 
 def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink=None,
             bias=None, dropout_mask=None, dropout_rate=0.0, save_residuals=True, bwd_ds_workspace=None,
-            bwd_workspace_limit_bytes=None):
+            bwd_workspace_limit_bytes=None, copy_bias=False):
     """Pads the head dim if needed and runs the differentiable kernel pair."""
     head_dim = query.shape[-1]
     width = padded_head_dim(head_dim)
@@ -145,7 +145,7 @@ def _attend(query, key, value, segment_ids, softmax_scale, mask_kind, window, lo
     if _differentiated(query, key, value, logit_sink, bias):
         out = _FlashAttentionFn.apply(
             query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink, bias, dropout_mask,
-            dropout_rate, save_residuals, bwd_ds_workspace, bwd_workspace_limit_bytes,
+            dropout_rate, save_residuals, bwd_ds_workspace, bwd_workspace_limit_bytes, copy_bias,
         )
     else:  # nothing to differentiate: no autograd node, no lse
         out, _ = ops.flash_fwd(
@@ -190,18 +190,26 @@ class _FlashAttentionFn(torch.autograd.Function):
     asks the backward to keep dS in its workspace (AXL_BWD_DS_WORKSPACE: about T*S bytes per (batch,
     head) more, 5 GEMMs instead of 7; ignored where that path does not apply), False to recompute dS
     in the dQ kernel, None to take the dS workspace whenever it fits bwd_workspace_limit_bytes (None:
-    a sixteenth of the device's memory)."""
+    a sixteenth of the device's memory).  copy_bias=True: the caller may write to the bias ahead of the backward,
+    which gets a copy of it, left by the forward kernel where that can."""
 
     @staticmethod
     def forward(ctx, query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink,
                 bias, dropout_mask, dropout_rate, save_residuals, bwd_ds_workspace=None,
-                bwd_workspace_limit_bytes=None):
+                bwd_workspace_limit_bytes=None, copy_bias=False):
         # neither is differentiated (gpu_attention.py:786)
         aux = dict(dropout_mask=dropout_mask, dropout_rate=dropout_rate)
+        kept = {}
+        if copy_bias:
+            if ops.can_copy_bias(query, bias, segment_ids, dropout_mask):
+                kept = dict(bias_copy=torch.empty_like(bias))
+            else:
+                bias = bias.clone()
         out, lse = ops.flash_fwd(
             query, key, value, softmax_scale=softmax_scale, mask_kind=mask_kind,
-            sliding_window=window, segment_ids=segment_ids, logit_sink=logit_sink, bias=bias, **aux,
+            sliding_window=window, segment_ids=segment_ids, logit_sink=logit_sink, bias=bias, **kept, **aux,
         )
+        bias = kept.get("bias_copy", bias)
         # The bias may be the caller's own tensor: saved like the others, so that writing to it ahead of the
         # backward is an error and not a wrong gradient.
         if save_residuals:
@@ -233,7 +241,7 @@ class _FlashAttentionFn(torch.autograd.Function):
             ds_workspace=ctx.bwd_ds_workspace, ds_workspace_limit=ctx.bwd_workspace_limit_bytes, **aux,
         )
         d_sink = grads[3].to(logit_sink.dtype) if logit_sink is not None else None
-        return grads[0], grads[1], grads[2], None, None, None, None, d_sink, None, None, None, None, None, None
+        return grads[0], grads[1], grads[2], None, None, None, None, d_sink, None, None, None, None, None, None, None
 
 
 # pylint: disable-next=too-many-positional-arguments
@@ -399,6 +407,7 @@ class HipFlashAttention(BaseFlashAttention):
         bias: BaseAttentionBias = input_batch["bias"]
         mask, segment_ids, explicit_bias = split(bias, MaskFnAttentionBias, SegmentIdAttentionBias)
         dense = explicit_bias.value() if explicit_bias.has_value() else None  # [B|1,H|1,T,S]
+        copy_bias = False
         kind = classify_mask_bias(mask)
         if kind is None:  # a mask fn the kernels have no closed form for: its dense value
             mask_bias = mask.value().to(torch.float32)
@@ -408,11 +417,12 @@ class HipFlashAttention(BaseFlashAttention):
             dense = dense.to(query.device)
             # Copied where the backward will read it again and the caller may have written to it by then (one buffer
             # refilled for every layer, say), and where it is a view into a larger tensor that the kernels' loads of
-            # 16 bytes cannot read.  The copy reads and writes every element: B2 H16 T2048, 134 MB of bf16, 51 us of a
-            # step of 282 us; without a backward the caller's tensor is read in place.
-            if dense.data_ptr() % 16 or (_is_the_callers(dense, explicit_bias)
-                                         and _differentiated(query, key, value, input_batch.get("logit_sink", None), dense)):
+            # 16 bytes cannot read.  Without a backward the caller's tensor is read in place.
+            if dense.data_ptr() % 16:
                 dense = dense.clone()
+            else:
+                copy_bias = (_is_the_callers(dense, explicit_bias)
+                             and _differentiated(query, key, value, input_batch.get("logit_sink", None), dense))
         seg = get_segment_ids(query=query, key=key, segment_ids=segment_ids)
         rate = float(self.cfg.dropout_rate)
         dropout_mask = None
@@ -429,4 +439,5 @@ class HipFlashAttention(BaseFlashAttention):
             bwd_ds_workspace=self.get_backend_overrides("bwd_ds_workspace", self.cfg.bwd_ds_workspace),
             bwd_workspace_limit_bytes=self.get_backend_overrides(
                 "bwd_workspace_limit_bytes", self.cfg.bwd_workspace_limit_bytes),
+            copy_bias=copy_bias,
         )

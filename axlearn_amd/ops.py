@@ -131,6 +131,15 @@ def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[_lib.AxlAttnAux
     return aux, tuple(keep)
 
 
+def can_copy_bias(q: torch.Tensor, bias: torch.Tensor, segment_ids: Optional[torch.Tensor],
+                  dropout_mask: Optional[torch.Tensor]) -> bool:
+    """Whether `flash_fwd` can leave a copy of the bias (`bias_copy`): the forms whose kernel reads a bf16 bias and
+    nothing else.  Without segment ids, for what documents hide from one batch row another may see."""
+    return (bias.dtype == torch.bfloat16 and q.dtype in (torch.bfloat16, torch.float16) and segment_ids is None
+            and dropout_mask is None and bias.is_contiguous() and bias.dim() == 4 and bias.data_ptr() % 16 == 0
+            and bias.shape[2] * bias.shape[3] < 1 << 31)
+
+
 def _seg(segment_ids: Optional[torch.Tensor]) -> Optional[torch.Tensor]:
     if segment_ids is None:
         return None
@@ -155,18 +164,27 @@ def flash_fwd(
     dropout_mask: Optional[torch.Tensor] = None,
     dropout_rate: float = 0.0,
     q_pos_offsets: Optional[torch.Tensor] = None,
+    bias_copy: Optional[torch.Tensor] = None,
 ):
     """q [B,T,Hq,D], k/v [B,S,Hkv,D] -> (out [B,T,Hq,D], lse [B,Hq,T] fp32 or None).
 
     q_pos_offsets [B] int32: per-sequence position of query row 0, added to q_pos_offset.
     logit_sink [Hq]: optional per-head sink logit (joins the softmax and lse, carries no value).
     bias [B|1,Hq|1,T,S] bf16/fp32: dense additive logit bias.  dropout_mask [B,Hq,T,S] bool/uint8
-    (True = dropped) with dropout_rate: kept probabilities are scaled by 1 / (1 - rate)."""
+    (True = dropped) with dropout_rate: kept probabilities are scaled by 1 / (1 - rate).
+    bias_copy: a tensor like the bias that receives the elements of it that the mask leaves visible, where
+    `can_copy_bias` says so."""
     b, t, hq, d, s, hkv = _check_qkv(q, k, v)
     _check_segment_ids(segment_ids, b, t, s)
+    if bias_copy is not None:
+        if bias is None or not can_copy_bias(q, bias, segment_ids, dropout_mask):
+            raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "the forward cannot copy this bias")
+        _want_shape("bias_copy", bias_copy, bias.shape)
+        if bias_copy.dtype != bias.dtype or not bias_copy.is_contiguous():
+            raise _bad("bias_copy must be contiguous and have the dtype of the bias")
     if q_pos_offsets is not None:
         _want_shape("q_pos_offsets", q_pos_offsets, (b,))
-    _require_cuda(q, k, v, segment_ids, logit_sink, bias, dropout_mask, q_pos_offsets)
+    _require_cuda(q, k, v, segment_ids, logit_sink, bias, dropout_mask, q_pos_offsets, bias_copy)
     lib = _lib.load()
     if q_pos_offsets is not None:
         q_pos_offsets = q_pos_offsets.to(torch.int32).contiguous()
@@ -183,7 +201,7 @@ def flash_fwd(
         batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
         dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind, sliding_window=int(sliding_window),
         q_pos_offset=int(q_pos_offset), softmax_scale=float(softmax_scale),
-        logit_sink=_lib.ptr(sink), aux=aux, q_pos_offsets=_lib.ptr(q_pos_offsets),
+        logit_sink=_lib.ptr(sink), aux=aux, q_pos_offsets=_lib.ptr(q_pos_offsets), bias_copy=_lib.ptr(bias_copy),
     )
     _lib.check(lib.axl_flash_fwd(ctypes.byref(p), _lib.current_stream_ptr()))
     return out, lse

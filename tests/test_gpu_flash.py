@@ -1704,3 +1704,41 @@ def test_query_tiles_of_a_key_block_shared_by_workgroups(b, t, hq, hkv, d, mask,
         assert ref.rel_l2(x.cpu(), y.cpu()) < step / 4, name
     again = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=bufs, **kw)
     assert all(torch.equal(x, y) for x, y in zip(again, got))
+
+
+@pytest.mark.parametrize("t,s,hq,hkv,d,mask,window,bias_b,bias_h,dtype", [
+    (128, 128, 4, 4, 64, "causal", None, 1, 4, torch.bfloat16),      # one row block, nothing but diagonal tiles
+    (640, 640, 4, 2, 128, "causal", None, 1, 4, torch.bfloat16),
+    (1152, 1152, 8, 8, 128, "sliding", 200, 2, 8, torch.float16),
+    (384, 640, 4, 1, 128, "none", None, 2, 1, torch.bfloat16),
+    (1024, 1024, 16, 16, 64, "sliding", 63, 1, 1, torch.bfloat16),
+])
+def test_forward_leaves_a_copy_of_the_bias(t, s, hq, hkv, d, mask, window, bias_b, bias_h, dtype):
+    """`bias_copy`: every visible element is the bias's, whatever the bias is broadcast over, and the backward's
+    results from the copy are the bits of those from the bias, though everything invisible in it is NaN."""
+    b = 2
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, dtype, s=s))
+    gen = torch.Generator("cuda").manual_seed(5)
+    bias = torch.randn(bias_b, bias_h, t, s, device="cuda", generator=gen).to(torch.bfloat16)
+    mk = {"none": ops.MASK_NONE, "causal": ops.MASK_CAUSAL, "sliding": ops.MASK_SLIDING_WINDOW}[mask]
+    kw = dict(mask_kind=mk, sliding_window=window or 0, softmax_scale=d ** -0.5)
+    out, lse = ops.flash_fwd(q, k, v, bias=bias, **kw)
+    copy = torch.full_like(bias, float("nan"))
+    assert ops.can_copy_bias(q, bias, None, None)
+    out_c, lse_c = ops.flash_fwd(q, k, v, bias=bias, bias_copy=copy, **kw)
+    assert torch.equal(out, out_c) and torch.equal(lse, lse_c)
+    diff = torch.arange(t, device="cuda")[:, None] - torch.arange(s, device="cuda")[None]
+    seen = (diff >= 0) & (diff <= (window if window is not None else 1 << 30)) if mask != "none" else torch.ones_like(diff, dtype=torch.bool)
+    assert torch.equal(copy[:, :, seen], bias[:, :, seen])
+    copy[:, :, ~seen] = float("nan")
+    out_n, lse_n = ops.flash_fwd(q, k, v, bias=copy, **kw)   # a forward that is run again on the copy
+    assert torch.equal(out, out_n) and torch.equal(lse, lse_n)
+    for ds in (False, True):
+        want = ops.flash_bwd(q, k, v, out, lse, do, bias=bias, ds_workspace=ds, **kw)
+        got = ops.flash_bwd(q, k, v, out, lse, do, bias=copy, ds_workspace=ds, **kw)
+        assert all(torch.isfinite(x.float()).all() and torch.equal(x, y) for x, y in zip(got, want)), ds
+    seg = torch.ones(b, t, dtype=torch.int32, device="cuda") if t == s else None
+    for args in (dict(bias=bias.float()), dict(bias=bias, segment_ids=seg)):
+        if "segment_ids" not in args or seg is not None:
+            with pytest.raises(ops.AxlError):
+                ops.flash_fwd(q, k, v, bias_copy=torch.empty_like(args["bias"]), **args, **kw)
