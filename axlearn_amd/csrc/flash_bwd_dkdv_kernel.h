@@ -71,9 +71,8 @@ constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than 
 // W: live width, the head_dim rounded up to a multiple of 32 (D: the width of a row in LDS).  The MFMAs and fragment
 // reads past it, whose operands or results are nothing but padding, are left out (B2 H32/8 T4096, head_dim 96 causal
 // with dS 557 -> 481 us, 80 unmasked 931 -> 775 us; the recomputing dQ kernel there 708 -> 590 us).
-template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false, int W = D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void flash_bwd_dkdv_kernel(const BwdArgs a) {
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W>
+__device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   // A bf16 bias alone comes through the tile ring like Q and dO, its elements read from LDS where they are used;
   // everything else is the plain kernel.  The other inputs (fp32 bias, dropout mask, both, a bias beside segment
   // ids, whose form of this kernel has no registers left) are fetched element by element into registers an
@@ -883,6 +882,19 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
   }  // key blocks of this workgroup
 }
 
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void flash_bwd_dkdv_kernel(const BwdArgs a) {
+  flash_bwd_dkdv_body<E, D, HAS_SEG, AUX, SPILL, D>(a);
+}
+
+// Head dims 72 to 96 of the width 128.
+template <typename E, bool HAS_SEG, bool SPILL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void flash_bwd_dkdv_w96_kernel(const BwdArgs a) {
+  flash_bwd_dkdv_body<E, 128, HAS_SEG, 0, SPILL, 96>(a);
+}
+
 // Sums the partial dK (blockIdx.y 0) and dV (1) of a split launch in the order of the splits, and scales and rounds
 // as the kernel above does at its end.  One workgroup per 32 keys, a wavefront per 32 columns of head_dim, the pieces read
 // as they were written (1 KB per instruction, four splits in flight).  Bound by the bytes.
@@ -924,7 +936,10 @@ __global__ __launch_bounds__(2 * D) void flash_bwd_dkdv_combine_kernel(const Bwd
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
-  auto kernel = flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL, W>;
+  auto kernel = [] {
+    if constexpr (W == 96) return flash_bwd_dkdv_w96_kernel<E, HAS_SEG, SPILL>;
+    else return flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
+  }();
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
   const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;

@@ -846,10 +846,17 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   }
 }
 
-template <typename E, int D, bool AUX, int NW = 4, int W = D>
+template <typename E, int D, bool AUX, int NW = 4>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(AUX ? 1 : 2, AUX ? 1 : 2)))
 void flash_fwd_kernel(const FwdArgs a) {
-  flash_fwd_body<E, D, AUX ? kFwdAux : kFwdPlain, NW, false, W>(a);
+  flash_fwd_body<E, D, AUX ? kFwdAux : kFwdPlain, NW, false>(a);
+}
+
+// Head dims 72 to 96 of the width 128.
+template <typename E>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_fwd_w96_kernel(const FwdArgs a) {
+  flash_fwd_body<E, 128, kFwdPlain, 4, false, 96>(a);
 }
 
 // A bf16 bias without a dropout mask.  Knowing that at compile time takes the run-time tests, the fp32
@@ -859,17 +866,23 @@ void flash_fwd_kernel(const FwdArgs a) {
 // (plain 0.59; of it, taking the batch's workgroups of one head together, so that the bias comes from memory
 // once: 1.01 -> 0.88, no scratch reload in the FAST loop: 0.88 -> 0.80).
 //
-// COPY: the words of every tile that is read go out again right after they arrived (FwdArgs::bias_copy): the backward
+// flash_fwd_bias_copy_kernel: the words of every tile that is read go out again right after they arrived (FwdArgs::bias_copy): the backward
 // reads the bias a second time and its caller may have refilled the buffer by then.  Only visible tiles are moved, part of
 // it under the MFMAs, in place of a pass that reads and writes every element ahead of this kernel: B2 H16 T2048 D128,
 // one bias for the batch, 85 us and 47 us of copy -> 108 us; window 256, B1: 34 and 50 us -> 34 us; B8 H32 D64 280 and
 // 92 us -> 314 us.  A form of its own: the branch alone cost the other calls 6 us of 76.
 // (Requesting the bias after the exponentials, where registers are free, made the compiler spill more
 // of the loop, 108 us.)
-template <typename E, int D, bool COPY>
+template <typename E, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_fwd_bias_kernel(const FwdArgs a) {
-  flash_fwd_body<E, D, COPY ? kFwdBias16Copy : kFwdBias16, 4, false>(a);
+  flash_fwd_body<E, D, kFwdBias16, 4, false>(a);
+}
+
+template <typename E, int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_fwd_bias_copy_kernel(const FwdArgs a) {
+  flash_fwd_body<E, D, kFwdBias16Copy, 4, false>(a);
 }
 
 template <typename E, int D>
@@ -1496,14 +1509,14 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
 #define AXL_LAUNCH_FWD16(E)                                                                     \
   do {                                                                                          \
     if (bias16 && p.bias_copy) {                                                                \
-      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128, true>), FwdTile<128>);    \
-      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64, true>), FwdTile<64>);                   \
+      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_copy_kernel<E, 128>), FwdTile<128>);    \
+      else AXL_LAUNCH_FWD((flash_fwd_bias_copy_kernel<E, 64>), FwdTile<64>);                   \
     } else if (bias16) {                                                                        \
-      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128, false>), FwdTile<128>);   \
-      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64, false>), FwdTile<64>);                  \
+      if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 128>), FwdTile<128>);   \
+      else AXL_LAUNCH_FWD((flash_fwd_bias_kernel<E, 64>), FwdTile<64>);                  \
     } else if (width == 128) {                                                                  \
       if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, true>), FwdTile<128>);                  \
-      else if (p.head_dim <= 96) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, false, 4, 96>), FwdTile<128>); \
+      else if (p.head_dim <= 96) AXL_LAUNCH_FWD((flash_fwd_w96_kernel<E>), FwdTile<128>); \
       else AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, false>), FwdTile<128>);                     \
     } else {                                                                                    \
       if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 64, true>), FwdTile<64>);                    \

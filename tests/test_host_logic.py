@@ -875,3 +875,14 @@ def test_chunk_and_bias_kernels_keep_the_distance_behind_their_assembly_mfma_cha
     """The forms of the forward for chunks over a long cache and for a bf16 bias share its body: the same check."""
     asm, _ = _device_asm("flash_fwd.hip", extra=("-mllvm", "-amdgpu-mfma-vgpr-form"))
     _assert_asm_mfma_distances(asm, r"_ZN3axl(18flash_chunk_kernel|21flash_fwd_bias_kernel)", 8)
+
+
+def test_forms_for_a_live_width_and_for_a_copied_bias_keep_their_distances():
+    """The live width 96 of the forward and of dK/dV (chains of six instead of eight MFMAs, fewer slots) and the
+    forward that stores the bias again: the same check."""
+    asm, _ = _device_asm("flash_fwd.hip", extra=("-mllvm", "-amdgpu-mfma-vgpr-form"))
+    _assert_asm_mfma_distances(asm, r"_ZN3axl(20flash_fwd_w96_kernel|26flash_fwd_bias_copy_kernel)", 6)
+    asm, remarks = _device_asm("flash_bwd_dkdv.hip")
+    _assert_asm_mfma_distances(asm, r"_ZN3axl25flash_bwd_dkdv_w96_kernel", 8)
+    blocks = [b for b in remarks.split("Function Name: ")[1:] if "flash_bwd_dkdv_w96_kernel" in b.split()[0]]
+    assert len(blocks) == 8 and all("ScratchSize [bytes/lane]: 0" in b for b in blocks)
