@@ -19,7 +19,7 @@ def config_class(cls):
 
 # Values a shallow copy may share.  (A config is copied for every kernel instance of every call, and
 # `copy.deepcopy` of its handful of plain fields took 15 us.)
-_IMMUTABLE = (type(None), bool, int, float, str)
+_IMMUTABLE = frozenset((type(None), bool, int, float, str))
 
 
 def _copy_config(cfg):
@@ -39,10 +39,10 @@ class Configurable:
         klass: Optional[type] = None
 
         def set(self, **kwargs) -> "Configurable.Config":
-            for name, value in kwargs.items():
+            for name in kwargs:
                 if name not in self.__dataclass_fields__:
                     raise AttributeError(f"{type(self).__qualname__} has no field {name!r}")
-                setattr(self, name, value)
+            self.__dict__.update(kwargs)
             return self
 
         def clone(self, **kwargs) -> "Configurable.Config":

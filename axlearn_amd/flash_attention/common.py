@@ -140,27 +140,17 @@ class BaseFlashAttention(Configurable):
     def is_supported(self, input_batch: Nested, kv_cache_type: Optional[type[BaseKVCache]]) -> bool:
         del kv_cache_type
         self._validate_input_batch(input_batch)
-        query, key = input_batch["query"], input_batch["key"]
+        query, key = input_batch["query"].shape, input_batch["key"].shape
         logit_sink = input_batch.get("logit_sink", None)
-        if query.shape[0] != key.shape[0]:
+        if query[0] != key[0]:
+            raise ValueError(f"Expects query batch size {query[0]} to be equal to key batch size {key[0]}")
+        if query[-1] != key[-1]:
+            raise ValueError(f"Expects query head dim {query[-1]} to be equal to key head dim {key[-1]}")
+        if query[2] % key[2] != 0:
+            raise ValueError(f"Expects query num heads {query[2]} to be divisible by num key heads {key[2]}")
+        if logit_sink is not None and logit_sink.shape[0] != query[2]:
             raise ValueError(
-                f"Expects query batch size {query.shape[0]} to be equal to key batch size "
-                f"{key.shape[0]}"
-            )
-        if query.shape[-1] != key.shape[-1]:
-            raise ValueError(
-                f"Expects query head dim {query.shape[-1]} to be equal to key head dim "
-                f"{key.shape[-1]}"
-            )
-        if query.shape[2] % key.shape[2] != 0:
-            raise ValueError(
-                f"Expects query num heads {query.shape[2]} to be divisible by num key heads "
-                f"{key.shape[2]}"
-            )
-        if logit_sink is not None and logit_sink.shape[0] != query.shape[2]:
-            raise ValueError(
-                f"Expects logit sink num heads {logit_sink.shape[0]} to be equal to "
-                f"num query heads {query.shape[2]}."
+                f"Expects logit sink num heads {logit_sink.shape[0]} to be equal to num query heads {query[2]}."
             )
         return True
 

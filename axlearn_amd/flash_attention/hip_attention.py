@@ -380,9 +380,10 @@ class HipFlashAttention(BaseFlashAttention):
         positions = mask.target_positions.to(query.device)
         if query.dtype != torch.float32:
             width = head_dim if runs_at_native_head_dim(query, key, value, aux=False) else padded_head_dim(head_dim)
+            query, key, value = (x.detach() if x.requires_grad else x for x in (query, key, value))
             out = ops.flash_chunk(
-                _aligned_rows(_pad_last(query.detach(), width)), _pad_last(key.detach(), width),
-                _pad_last(value.detach(), width), positions, softmax_scale=float(self.cfg.softmax_scale), mask_kind=kind[0], sliding_window=kind[1],
+                _aligned_rows(_pad_last(query, width)), _pad_last(key, width),
+                _pad_last(value, width), positions, softmax_scale=float(self.cfg.softmax_scale), mask_kind=kind[0], sliding_window=kind[1],
                 logit_sink=input_batch.get("logit_sink", None),
             )
             return out if width == head_dim else out[..., :head_dim]

@@ -61,10 +61,18 @@ def _positions(mask: MaskFnAttentionBias, batch_size: int, device) -> Tensor:
     return positions.expand(batch_size)
 
 
-def _mask_and_bias(input_batch: Nested, positions: Tensor, kv_len: int) -> Tuple[int, Optional[Tensor]]:
+def _as_they_are(mask: MaskFnAttentionBias, explicit_bias: BaseAttentionBias, query: Tensor) -> bool:
+    """Whether the call needs no tensor but the caller's own: a mask in closed form, no bias, positions the kernels
+    read in place.  (The views that the general form makes of query, positions and result took 10 us of a call.)"""
+    positions = getattr(mask, "target_positions", None)
+    return (positions is not None and positions.dim() == 2 and positions.shape[0] in (1, query.shape[0])
+            and positions.dtype in (torch.int32, torch.int64) and positions.device == query.device
+            and query.is_contiguous() and not explicit_bias.has_value() and _decode_window(mask) is not None)
+
+
+def _window_and_bias(mask: MaskFnAttentionBias, explicit_bias: BaseAttentionBias, query: Tensor, positions: Tensor,
+                     kv_len: int) -> Tuple[int, Optional[Tensor]]:
     """(sliding window for the kernel or -1, bias `[B|1, Hq|1, kv_len]` or None) of a decode call."""
-    mask, explicit_bias = split(input_batch["bias"], MaskFnAttentionBias)
-    query = input_batch["query"]
     bias = None
     if explicit_bias.has_value():
         value = explicit_bias.value().to(query.device)  # [B|1, Hq|1, 1, S]
@@ -121,10 +129,16 @@ class HipDecoding(BaseSingleStepDecoding):
 
     def __call__(self, input_batch: Nested) -> Tensor:
         query, key, value = input_batch["query"], input_batch["key"], input_batch["value"]
-        mask, _ = split(input_batch["bias"], MaskFnAttentionBias)
+        mask, explicit_bias = split(input_batch["bias"], MaskFnAttentionBias)
         batch_size, _, q_heads, head_dim = query.shape
+        if _as_they_are(mask, explicit_bias, query):
+            return ops.decode(
+                query, _as_query_dtype(key, query), _as_query_dtype(value, query), mask.target_positions,
+                softmax_scale=float(self.cfg.softmax_scale), sliding_window=_decode_window(mask),
+                lengths_are_positions=True, single_row=True,
+            )
         positions = _positions(mask, batch_size, query.device)
-        window, bias = _mask_and_bias(input_batch, positions, key.shape[1])
+        window, bias = _window_and_bias(mask, explicit_bias, query, positions, key.shape[1])
         out = ops.decode(
             query.reshape(batch_size, q_heads, head_dim), _as_query_dtype(key, query), _as_query_dtype(value, query),
             positions, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window, bias=bias,
@@ -156,10 +170,16 @@ class HipPagedAttention(BasePagedAttention):
     def __call__(self, input_batch: Nested) -> Tensor:
         query, key, value = input_batch["query"], input_batch["key"], input_batch["value"]
         page_tables = input_batch["page_tables"]
-        mask, _ = split(input_batch["bias"], MaskFnAttentionBias)
+        mask, explicit_bias = split(input_batch["bias"], MaskFnAttentionBias)
         batch_size, _, q_heads, head_dim = query.shape
+        if _as_they_are(mask, explicit_bias, query):
+            return ops.paged_decode(
+                query, _as_query_dtype(key, query), _as_query_dtype(value, query), page_tables.contiguous(),
+                mask.target_positions, softmax_scale=float(self.cfg.softmax_scale),
+                sliding_window=_decode_window(mask), lengths_are_positions=True, single_row=True,
+            )
         positions = _positions(mask, batch_size, query.device)
-        window, bias = _mask_and_bias(input_batch, positions, key.shape[2] * page_tables.shape[1])
+        window, bias = _window_and_bias(mask, explicit_bias, query, positions, key.shape[2] * page_tables.shape[1])
         out = ops.paged_decode(
             query.reshape(batch_size, q_heads, head_dim), _as_query_dtype(key, query), _as_query_dtype(value, query),
             page_tables.contiguous(), positions, softmax_scale=float(self.cfg.softmax_scale), sliding_window=window,

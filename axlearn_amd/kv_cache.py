@@ -57,6 +57,10 @@ def paged_extend_step(k_pages, v_pages, page_indices, *, k_proj, v_proj, key_pos
         raise ValueError(f"{k_proj.shape[1]=} != {key_positions.shape[1]=}")
     if k_proj.shape[1] != 1:
         raise ValueError("Currently only support single time step.")
-    ops.paged_kv_insert(k_pages, v_pages, k_proj[:, 0].to(k_pages.dtype), v_proj[:, 0].to(v_pages.dtype),
-                        page_indices, key_positions.reshape(-1).contiguous())
+    if k_proj.dim() == 4 and key_positions.dim() == 2 and key_positions.is_contiguous():
+        ops.paged_kv_insert(k_pages, v_pages, k_proj.to(k_pages.dtype), v_proj.to(v_pages.dtype), page_indices,
+                            key_positions, single_row=True)
+    else:
+        ops.paged_kv_insert(k_pages, v_pages, k_proj[:, 0].to(k_pages.dtype), v_proj[:, 0].to(v_pages.dtype),
+                            page_indices, key_positions.reshape(-1).contiguous())
     return k_pages, v_pages

@@ -7,6 +7,7 @@ call. Inputs must be CUDA(ROCm) tensors; torch is used for device memory and str
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -17,13 +18,9 @@ from axlearn_amd._lib import (
     MASK_NONE,
     MASK_SLIDING_WINDOW,
     AxlDecodeBias,
-    AxlDecodeParams,
     AxlError,
     AxlFlashBwdParams,
-    AxlFlashChunkParams,
-    AxlFlashFwdParams,
     AxlPagedDecodeParams,
-    AxlPageInsertParams,
 )
 
 __all__ = [
@@ -42,15 +39,16 @@ __all__ = [
 
 
 def _require_cuda(*tensors):
-    dev = None
+    first = None
     for t in tensors:
         if t is None:
             continue
         if not t.is_cuda:
             raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "all tensors must live on the GPU")
-        if dev is not None and t.device != dev:
-            raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, f"tensors live on different devices ({dev} and {t.device})")
-        dev = t.device
+        if first is None:
+            first, index = t, t.get_device()
+        elif t.get_device() != index:
+            raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, f"tensors live on different devices ({first.device} and {t.device})")
 
 
 def _bad(msg: str) -> AxlError:
@@ -68,16 +66,16 @@ def _check_qkv(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor):
     if q.dim() != 4 or k.dim() != 4 or v.dim() != 4:
         raise _bad(f"q, k, v must be 4-d [batch, seq, heads, head_dim], got {list(q.shape)}, {list(k.shape)}, {list(v.shape)}")
     b, t, hq, d = q.shape
-    if k.shape[0] != b or k.shape[3] != d:
+    kb, s, hkv, kd = k_shape = k.shape
+    if kb != b or kd != d:
         raise _bad(f"k {list(k.shape)} does not match q {list(q.shape)} in batch / head_dim")
-    if tuple(v.shape) != tuple(k.shape):
+    if v.shape != k_shape:
         raise _bad(f"v {list(v.shape)} must have the shape of k {list(k.shape)}")
-    hkv = k.shape[2]
     if hkv <= 0 or hq % hkv != 0:
         raise _bad(f"num_q_heads {hq} is not divisible by num_kv_heads {hkv}")
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "q, k, v must share one dtype")
-    return b, t, hq, d, k.shape[1], hkv
+    return b, t, hq, d, s, hkv
 
 
 def _check_segment_ids(segment_ids: Optional[torch.Tensor], b: int, t: int, s: int) -> None:
@@ -96,10 +94,14 @@ def _sink(logit_sink: Optional[torch.Tensor], num_heads: int) -> Optional[torch.
     return logit_sink.detach().to(torch.float32).contiguous()
 
 
-def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[_lib.AxlAttnAux, tuple]:
-    """Builds the AxlAttnAux block; returns it with the tensors it points at (keep them alive)."""
-    aux = _lib.AxlAttnAux()
-    keep = []
+_NO_AUX = (0, 0, 0, 0, 0, 0.0, 0, 0, 0, 0)
+
+
+def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[tuple, tuple]:
+    """The fields of an AxlAttnAux block, and the tensors it points at (keep them alive)."""
+    if bias is None and dropout_mask is None and not dropout_rate:
+        return _NO_AUX, ()
+    bias_part, drop_part, keep = _NO_AUX[:5], (0.0, 0, 0, 0, 0), []
     if bias is not None:
         if bias.dim() != 4 or bias.shape[0] not in (1, b) or bias.shape[1] not in (1, hq) or tuple(bias.shape[2:]) != (t, s):
             raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, f"bias must be [{b}|1, {hq}|1, {t}, {s}], got {tuple(bias.shape)}")
@@ -108,11 +110,8 @@ def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[_lib.AxlAttnAux
         if bias.stride(-1) != 1:
             bias = bias.contiguous()
         keep.append(bias)
-        aux.bias = bias.data_ptr()
-        aux.bias_batch_stride = bias.stride(0) if bias.shape[0] > 1 else 0
-        aux.bias_head_stride = bias.stride(1) if bias.shape[1] > 1 else 0
-        aux.bias_row_stride = bias.stride(2)
-        aux.bias_dtype = _lib.dtype_code(bias.dtype)
+        bias_part = (bias.data_ptr(), bias.stride(0) if bias.shape[0] > 1 else 0, bias.stride(1) if bias.shape[1] > 1 else 0,
+                     bias.stride(2), _lib.dtype_code(bias.dtype))
     if dropout_mask is not None:
         if tuple(dropout_mask.shape) != (b, hq, t, s):
             raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, f"dropout_mask must be [{b}, {hq}, {t}, {s}]")
@@ -123,12 +122,10 @@ def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[_lib.AxlAttnAux
         if dropout_mask.stride(-1) != 1:
             dropout_mask = dropout_mask.contiguous()
         keep.append(dropout_mask)
-        aux.dropout_mask = dropout_mask.data_ptr()
-        aux.drop_batch_stride, aux.drop_head_stride, aux.drop_row_stride = dropout_mask.stride()[:3]
-        aux.dropout_rate = float(dropout_rate)
+        drop_part = (float(dropout_rate), dropout_mask.data_ptr(), *dropout_mask.stride()[:3])
     elif dropout_rate:
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "dropout_rate needs a dropout_mask (the kernels draw no random numbers)")
-    return aux, tuple(keep)
+    return bias_part + drop_part, tuple(keep)
 
 
 def can_copy_bias(q: torch.Tensor, bias: torch.Tensor, segment_ids: Optional[torch.Tensor],
@@ -193,15 +190,11 @@ def flash_fwd(
     seg = _seg(segment_ids)
     sink = _sink(logit_sink, hq)
     aux, _keep = _aux(bias, dropout_mask, dropout_rate, b, hq, t, s)
-    p = AxlFlashFwdParams(
-        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), out=out.data_ptr(), lse=_lib.ptr(lse),
-        segment_ids=_lib.ptr(seg),
-        q_strides=_lib.strides4(q), k_strides=_lib.strides4(k), v_strides=_lib.strides4(v),
-        out_strides=_lib.strides4(out),
-        batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
-        dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind, sliding_window=int(sliding_window),
-        q_pos_offset=int(q_pos_offset), softmax_scale=float(softmax_scale),
-        logit_sink=_lib.ptr(sink), aux=aux, q_pos_offsets=_lib.ptr(q_pos_offsets), bias_copy=_lib.ptr(bias_copy),
+    p = _lib.fill_flash_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _lib.ptr(lse), _lib.ptr(seg),
+        *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out),
+        b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), _lib.int32(q_pos_offset),
+        float(softmax_scale), _lib.ptr(sink), *aux, _lib.ptr(q_pos_offsets), _lib.ptr(bias_copy),
     )
     _lib.check(lib.axl_flash_fwd(ctypes.byref(p), _lib.current_stream_ptr()))
     return out, lse
@@ -229,15 +222,12 @@ def flash_chunk(
         positions = positions.to(torch.int32)
     out = torch.empty((b, t, hq, d), dtype=q.dtype, device=q.device)
     sink = _sink(logit_sink, hq)
-    p = AxlFlashChunkParams(
-        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), out=out.data_ptr(),
-        q_strides=_lib.strides4(q), k_strides=_lib.strides4(k), v_strides=_lib.strides4(v),
-        out_strides=_lib.strides4(out),
-        batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
-        dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind, sliding_window=int(sliding_window),
-        softmax_scale=float(softmax_scale), logit_sink=_lib.ptr(sink), positions=positions.data_ptr(),
-        pos_batch_stride=positions.stride(0) if positions.shape[0] > 1 else 0, pos_row_stride=positions.stride(1),
-        pos_is_i64=int(positions.dtype == torch.int64),
+    p = _lib.fill_flash_chunk(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
+        *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out),
+        b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), float(softmax_scale),
+        _lib.ptr(sink), positions.data_ptr(), positions.stride(0) if positions.shape[0] > 1 else 0, positions.stride(1),
+        int(positions.dtype == torch.int64), 0, 0,
     )
     need = int(lib.axl_flash_chunk_workspace_bytes(ctypes.byref(p)))
     if need:
@@ -319,18 +309,13 @@ def flash_bwd(
     sink = _sink(logit_sink, hq)
     d_sink = torch.empty((hq,), dtype=torch.float32, device=q.device) if sink is not None else None
     aux, _keep = _aux(bias, dropout_mask, dropout_rate, b, hq, t, s)
-    p = AxlFlashBwdParams(
-        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), out=out.data_ptr(),
-        d_out=d_out.data_ptr(), lse=lse.data_ptr(), dq=dq.data_ptr(), dk=dk.data_ptr(),
-        dv=dv.data_ptr(), segment_ids=_lib.ptr(seg),
-        q_strides=_lib.strides4(q), k_strides=_lib.strides4(k), v_strides=_lib.strides4(v),
-        out_strides=_lib.strides4(out), d_out_strides=_lib.strides4(d_out),
-        dq_strides=_lib.strides4(dq), dk_strides=_lib.strides4(dk), dv_strides=_lib.strides4(dv),
-        batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
-        dtype=_lib.dtype_code(q.dtype), mask_kind=mask_kind, sliding_window=int(sliding_window),
-        q_pos_offset=int(q_pos_offset), softmax_scale=float(softmax_scale),
-        workspace=None, workspace_bytes=0, logit_sink=_lib.ptr(sink), d_logit_sink=_lib.ptr(d_sink),
-        aux=aux, flags=_bwd_flags(ds_workspace, ds_slice_kv_heads),
+    p = _lib.fill_flash_bwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), d_out.data_ptr(), lse.data_ptr(), dq.data_ptr(),
+        dk.data_ptr(), dv.data_ptr(), _lib.ptr(seg),
+        *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out), *_lib.strides4(d_out),
+        *_lib.strides4(dq), *_lib.strides4(dk), *_lib.strides4(dv),
+        b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), _lib.int32(q_pos_offset),
+        float(softmax_scale), 0, 0, _lib.ptr(sink), _lib.ptr(d_sink), *aux, _bwd_flags(ds_workspace, ds_slice_kv_heads),
     )
     ws = _bwd_workspace(lib, p, by_size or bias is not None or dropout_mask is not None, ws, q.device)
     p.workspace = ws.data_ptr()
@@ -419,7 +404,20 @@ def flash_bwd_ds_workspace_bytes(q: torch.Tensor, k: torch.Tensor, *, mask_kind:
 def default_bwd_workspace_limit(device) -> int:
     """Transient bytes the backward may take for dS when the caller states no limit: a sixteenth of the
     device's memory (18 GB of an MI355X's 288 GB)."""
-    return torch.cuda.get_device_properties(device).total_memory // 16
+    return _device_properties(device)[0] // 16
+
+
+def _device_properties(device) -> Tuple[int, int]:
+    """(bytes of memory, compute units) of a device."""
+    if isinstance(device, torch.device) and device.type == "cuda" and device.index is not None:
+        return _indexed_device_properties(device.index)
+    return _indexed_device_properties.__wrapped__(device)
+
+
+@functools.lru_cache(maxsize=None)
+def _indexed_device_properties(index) -> Tuple[int, int]:
+    p = torch.cuda.get_device_properties(index)
+    return p.total_memory, p.multi_processor_count
 
 
 def select_ds_slice(q: torch.Tensor, k: torch.Tensor, *, mask_kind: int,
@@ -442,7 +440,7 @@ def select_ds_slice(q: torch.Tensor, k: torch.Tensor, *, mask_kind: int,
                                                       ds_slice_kv_heads=heads)[0] > int(limit):
         heads -= 1
     per_head = b * (s // 128) // (2 if mask_kind == MASK_CAUSAL else 1)   # dK/dV workgroups per kv head
-    cus = torch.cuda.get_device_properties(q.device).multi_processor_count
+    cus = _device_properties(q.device)[1]
     if heads < 1 or heads * per_head < cus:
         return False, 0
     return True, int(heads)
@@ -460,13 +458,29 @@ def _decode_flags(deterministic: bool, workspace_reused: bool, lengths: torch.Te
             | (_lib.DECODE_LENGTHS_I64 if lengths.dtype == torch.int64 else 0))
 
 
-def _check_lengths(lengths: torch.Tensor, b: int, are_positions: bool) -> None:
-    _want_shape("lengths", lengths, (b,))
+def _check_lengths(lengths: torch.Tensor, b: int, are_positions: bool, single_row: bool) -> Tuple[int, int]:
+    """(pointer, stride in elements) of the lengths [B], or with `single_row` of the last column of [B|1, T] positions."""
+    if single_row:
+        if lengths.dim() != 2 or lengths.shape[0] not in (1, b) or lengths.shape[1] < 1 or not are_positions:
+            raise _bad(f"positions must be [{b}|1, T], got {list(lengths.shape)}")
+    else:
+        _want_shape("lengths", lengths, (b,))
     if are_positions:
         if lengths.dtype not in (torch.int32, torch.int64) or lengths.stride(0) < 0:
             raise _bad("positions must be int32 or int64")
     elif lengths.dtype != torch.int32:
         raise _bad("lengths must be int32")
+    if not single_row:
+        return lengths.data_ptr(), lengths.stride(0)
+    last = (lengths.shape[1] - 1) * lengths.stride(1) * (8 if lengths.dtype == torch.int64 else 4)
+    return lengths.data_ptr() + last, lengths.stride(0) if lengths.shape[0] > 1 else 0
+
+
+def _one_query(q: torch.Tensor, other: torch.Tensor, single_row: bool, names: str) -> Tuple[int, int, int]:
+    """(batch, heads, head_dim) of q [B,Hq,D], or [B,1,Hq,D] with `single_row`."""
+    if q.dim() != 3 + single_row or other.dim() != 4 or (single_row and q.shape[1] != 1):
+        raise _bad(f"q must be [B,{'1,' if single_row else ''}Hq,D] and {names}, got {list(q.shape)}, {list(other.shape)}")
+    return q.shape[0], q.shape[-2], q.shape[-1]
 
 
 def _check_decode_out_ws(q, out, workspace):
@@ -479,21 +493,17 @@ def _check_decode_out_ws(q, out, workspace):
 
 
 def _decode_bias(bias: Optional[torch.Tensor], b: int, hq: int, kv_len: int):
-    """The AxlDecodeBias block for a bias `[B|1, Hq|1, kv_len]`; returns it with the tensor it points at."""
-    blk = AxlDecodeBias()
+    """The fields of an AxlDecodeBias block for a bias `[B|1, Hq|1, kv_len]`, and the tensor it points at."""
     if bias is None:
-        return blk, None
+        return (0, 0, 0, 0), None
     if bias.dim() != 3 or bias.shape[0] not in (1, b) or bias.shape[1] not in (1, hq) or bias.shape[2] != kv_len:
         raise _bad(f"bias must be [{b}|1, {hq}|1, {kv_len}], got {list(bias.shape)}")
     if bias.dtype not in (torch.bfloat16, torch.float32):
         bias = bias.to(torch.float32)
     if bias.stride(-1) != 1:
         bias = bias.contiguous()
-    blk.bias = bias.data_ptr()
-    blk.batch_stride = bias.stride(0) if bias.shape[0] > 1 else 0
-    blk.head_stride = bias.stride(1) if bias.shape[1] > 1 else 0
-    blk.dtype = _lib.dtype_code(bias.dtype)
-    return blk, bias
+    return (bias.data_ptr(), bias.stride(0) if bias.shape[0] > 1 else 0, bias.stride(1) if bias.shape[1] > 1 else 0,
+            _lib.dtype_code(bias.dtype)), bias
 
 
 def paged_decode(
@@ -511,6 +521,7 @@ def paged_decode(
     workspace_reused: bool = False,
     bias: Optional[torch.Tensor] = None,
     lengths_are_positions: bool = False,
+    single_row: bool = False,
 ) -> torch.Tensor:
     """q [B,Hq,D]; pools [Hkv,P,page,D]; page_tables [B,pps] int32; lengths [B] int32 -> [B,Hq,D].
 
@@ -518,10 +529,10 @@ def paged_decode(
     fixes the work decomposition (bit-reproducible); `workspace_reused` promises that `workspace` was
     last touched by an earlier decode call (skips the launch that zeroes its work counter).
     bias [B|1,Hq|1,pps*page] bf16/fp32: additive logit bias per key position.  `lengths_are_positions`:
-    `lengths` holds positions of the query tokens (length - 1), int32 or int64, with any stride."""
-    if q.dim() != 3 or k_pages.dim() != 4:
-        raise _bad(f"q must be [B,Hq,D] and k_pages [Hkv,P,page,D], got {list(q.shape)}, {list(k_pages.shape)}")
-    b, hq, d = q.shape
+    `lengths` holds positions of the query tokens (length - 1), int32 or int64, with any stride.  `single_row` (with
+    it): q and the result are [B,1,Hq,D], the positions [B|1,T], of which the last column counts - a layer's own tensors
+    without a view of each."""
+    b, hq, d = _one_query(q, k_pages, single_row, "k_pages [Hkv,P,page,D]")
     hkv, num_pages, page_size, dk = k_pages.shape
     if dk != d:
         raise _bad(f"head_dim of k_pages ({dk}) differs from q's ({d})")
@@ -530,7 +541,7 @@ def paged_decode(
         raise _bad(f"num_q_heads {hq} is not divisible by num_kv_heads {hkv}")
     if page_tables.dim() != 2 or page_tables.shape[0] != b:
         raise _bad(f"page_tables must be [{b}, pages_per_seq], got {list(page_tables.shape)}")
-    _check_lengths(lengths, b, lengths_are_positions)
+    len_ptr, len_stride = _check_lengths(lengths, b, lengths_are_positions, single_row)
     if page_tables.dtype != torch.int32:
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "page_tables and lengths must be int32")
     if k_pages.dtype != q.dtype or v_pages.dtype != q.dtype:
@@ -544,17 +555,13 @@ def paged_decode(
     _require_cuda(q, k_pages, v_pages, page_tables, lengths, out, workspace, bias)
     lib = _lib.load()
     if out is None:
-        out = torch.empty((b, hq, d), dtype=q.dtype, device=q.device)
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     bias_blk, _keep = _decode_bias(bias, b, hq, page_size * page_tables.shape[1])
-    p = AxlPagedDecodeParams(
-        q=q.data_ptr(), k_pages=k_pages.data_ptr(), v_pages=v_pages.data_ptr(),
-        page_tables=page_tables.data_ptr(), lengths=lengths.data_ptr(), out=out.data_ptr(),
-        batch=b, num_q_heads=hq, num_kv_heads=hkv, head_dim=d, num_pages=num_pages,
-        page_size=page_size, pages_per_seq=page_tables.shape[1],
-        dtype=_lib.dtype_code(q.dtype), sliding_window=int(sliding_window),
-        softmax_scale=float(softmax_scale), workspace=None, workspace_bytes=0,
-        flags=_decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), bias=bias_blk,
-        lengths_stride=lengths.stride(0),
+    p = _lib.fill_paged_decode(
+        q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), page_tables.data_ptr(), len_ptr, out.data_ptr(),
+        b, hq, hkv, d, num_pages, page_size, page_tables.shape[1], _lib.dtype_code(q.dtype), _lib.int32(sliding_window),
+        float(softmax_scale), 0, 0, _decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions),
+        *bias_blk, len_stride,
     )
     need = int(lib.axl_paged_decode_workspace_bytes(ctypes.byref(p)))
     if workspace is None or workspace.numel() < need:
@@ -594,20 +601,20 @@ def decode(
     workspace_reused: bool = False,
     bias: Optional[torch.Tensor] = None,
     lengths_are_positions: bool = False,
+    single_row: bool = False,
 ) -> torch.Tensor:
     """q [B,Hq,D]; k/v [B,S,Hkv,D]; lengths [B] int32 -> [B,Hq,D].  Lengths are clamped to [0, S]; a
     sequence of length 0 yields zeros.  `deterministic` / `workspace_reused`: see `paged_decode`.
-    bias [B|1,Hq|1,S] bf16/fp32: additive logit bias per key position.  `lengths_are_positions`: as there."""
-    if q.dim() != 3 or k.dim() != 4:
-        raise _bad(f"q must be [B,Hq,D] and k [B,S,Hkv,D], got {list(q.shape)}, {list(k.shape)}")
-    b, hq, d = q.shape
-    s, hkv = k.shape[1], k.shape[2]
-    if k.shape[0] != b or k.shape[3] != d:
+    bias [B|1,Hq|1,S] bf16/fp32: additive logit bias per key position.  `lengths_are_positions`, `single_row`: as
+    there."""
+    b, hq, d = _one_query(q, k, single_row, "k [B,S,Hkv,D]")
+    kb, s, hkv, kd = k.shape
+    if kb != b or kd != d:
         raise _bad(f"k {list(k.shape)} does not match q {list(q.shape)} in batch / head_dim")
     _want_shape("v", v, k.shape)
     if hkv <= 0 or hq % hkv != 0:
         raise _bad(f"num_q_heads {hq} is not divisible by num_kv_heads {hkv}")
-    _check_lengths(lengths, b, lengths_are_positions)
+    len_ptr, len_stride = _check_lengths(lengths, b, lengths_are_positions, single_row)
     if k.dtype != q.dtype or v.dtype != q.dtype:
         raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "q, k, v must share one dtype")
     if not q.is_contiguous():
@@ -620,16 +627,12 @@ def decode(
     _require_cuda(q, k, v, lengths, out, workspace, bias)
     lib = _lib.load()
     if out is None:
-        out = torch.empty((b, hq, d), dtype=q.dtype, device=q.device)
+        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     bias_blk, _keep = _decode_bias(bias, b, hq, s)
-    p = AxlDecodeParams(
-        q=q.data_ptr(), k=k.data_ptr(), v=v.data_ptr(), lengths=lengths.data_ptr(),
-        out=out.data_ptr(), k_strides=_lib.strides4(k), v_strides=_lib.strides4(v),
-        batch=b, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
-        dtype=_lib.dtype_code(q.dtype), sliding_window=int(sliding_window),
-        softmax_scale=float(softmax_scale), workspace=None, workspace_bytes=0,
-        flags=_decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), bias=bias_blk,
-        lengths_stride=lengths.stride(0),
+    p = _lib.fill_decode(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), len_ptr, out.data_ptr(), *_lib.strides4(k), *_lib.strides4(v),
+        b, s, hq, hkv, d, _lib.dtype_code(q.dtype), _lib.int32(sliding_window), float(softmax_scale), 0, 0,
+        _decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), *bias_blk, len_stride,
     )
     need = int(lib.axl_decode_workspace_bytes(ctypes.byref(p)))
     if workspace is None or workspace.numel() < need:
@@ -649,11 +652,12 @@ def paged_kv_insert(
     v_proj: Optional[torch.Tensor],
     page_indices: torch.Tensor,
     key_positions: torch.Tensor,
+    single_row: bool = False,
 ) -> None:
     """Writes one new token per sequence into the pools, IN PLACE.
 
-    pools [Hkv,P,page,D]; k_proj/v_proj [B,Hkv,D] (any batch/head strides, dense in D);
-    page_indices [B,pps] int32; key_positions [B] int32, or [1] to use one position for all."""
+    pools [Hkv,P,page,D]; k_proj/v_proj [B,Hkv,D] (any batch/head strides, dense in D), or [B,1,Hkv,D] with
+    `single_row`; page_indices [B,pps] int32; key_positions [B] int32, or [1] to use one position for all."""
     pool = k_pages if k_pages is not None else v_pages
     proj = k_proj if k_proj is not None else v_proj
     if pool is None or proj is None:
@@ -670,25 +674,19 @@ def paged_kv_insert(
                     ("key_positions", key_positions)):
         if x is not None and not x.is_contiguous():
             raise AxlError(_lib.AXL_ERR_UNSUPPORTED, f"{name} must be contiguous")
+    row = (b, 1, hkv, d) if single_row else (b, hkv, d)
     for name, x in (("k_proj", k_proj), ("v_proj", v_proj)):
-        if x is not None and (tuple(x.shape) != (b, hkv, d) or x.stride(-1) != 1 or x.dtype != pool.dtype):
+        if x is not None and (tuple(x.shape) != row or x.stride(-1) != 1 or x.dtype != pool.dtype):
             raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, f"{name} must be [B,Hkv,D] of the pool dtype, dense in D")
     if page_indices.dtype != torch.int32 or key_positions.dtype != torch.int32:
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "page_indices and key_positions must be int32")
     if key_positions.numel() not in (1, b):
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "key_positions must hold 1 or batch values")
-    p = AxlPageInsertParams(
-        k_pages=None if k_pages is None else k_pages.data_ptr(),
-        v_pages=None if v_pages is None else v_pages.data_ptr(),
-        k_proj=None if k_proj is None else k_proj.data_ptr(),
-        v_proj=None if v_proj is None else v_proj.data_ptr(),
-        page_indices=page_indices.data_ptr(), key_positions=key_positions.data_ptr(),
-        k_proj_batch_stride=0 if k_proj is None else k_proj.stride(0),
-        k_proj_head_stride=0 if k_proj is None else k_proj.stride(1),
-        v_proj_batch_stride=0 if v_proj is None else v_proj.stride(0),
-        v_proj_head_stride=0 if v_proj is None else v_proj.stride(1),
-        batch=b, num_kv_heads=hkv, head_dim=d, num_pages=num_pages, page_size=page_size,
-        pages_per_seq=page_indices.shape[1], dtype=_lib.dtype_code(pool.dtype),
-        broadcast_positions=int(key_positions.numel() == 1 and b > 1),
+    p = _lib.fill_page_insert(
+        _lib.ptr(k_pages), _lib.ptr(v_pages), _lib.ptr(k_proj), _lib.ptr(v_proj), page_indices.data_ptr(),
+        key_positions.data_ptr(), *((0, 0) if k_proj is None else (k_proj.stride(0), k_proj.stride(-2))),
+        *((0, 0) if v_proj is None else (v_proj.stride(0), v_proj.stride(-2))),
+        b, hkv, d, num_pages, page_size, page_indices.shape[1], _lib.dtype_code(pool.dtype),
+        int(key_positions.numel() == 1 and b > 1),
     )
     _lib.check(lib.axl_paged_kv_insert(ctypes.byref(p), _lib.current_stream_ptr()))

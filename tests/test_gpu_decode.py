@@ -860,3 +860,43 @@ def test_decode_in_equal_shares(b, hq, hkv, d, pps, window):
             assert _ok(got[live], want[live]) and torch.equal(got[~live], torch.zeros_like(got[~live]))
         fixed.append(got)
     assert torch.equal(fixed[0], fixed[1]) and torch.equal(fixed[0], fixed[2])
+
+
+@pytest.mark.parametrize("dtype", [torch.int32, torch.int64])
+@pytest.mark.parametrize("shape", [(3, 1), (1, 1), (3, 4), (1, 4)])
+def test_layer_tensors_without_views_give_the_bits_of_the_views(shape, dtype):
+    """`single_row`: q [B,1,Hq,D] and positions [B|1,T] as a layer holds them, contiguous and strided."""
+    b, hq, hkv, d, page, pps = 3, 8, 2, 64, 16, 20
+    gen = torch.Generator("cuda").manual_seed(3)
+    q = torch.randn(b, 1, hq, d, device="cuda", generator=gen).to(torch.bfloat16)
+    k, v = (torch.randn(b, page * pps, hkv, d, device="cuda", generator=gen).to(torch.bfloat16) for _ in range(2))
+    kp, vp = (torch.randn(hkv, b * pps + 1, page, d, device="cuda", generator=gen).to(torch.bfloat16) for _ in range(2))
+    tables = (torch.randperm(b * pps, device="cuda") + 1).to(torch.int32).reshape(b, pps)
+    wide = torch.randint(0, page * pps, (shape[0], 2 * shape[1]), device="cuda", generator=gen, dtype=dtype)
+    for positions in (wide[:, ::2], wide[:, : shape[1]].contiguous(), wide[:, : shape[1]].t().contiguous().t()):
+        views = positions[:, -1].expand(b)
+        kw = dict(softmax_scale=0.1, lengths_are_positions=True, deterministic=True)
+        for got, want in ((ops.decode(q, k, v, positions, single_row=True, **kw), ops.decode(q[:, 0], k, v, views, **kw)),
+                          (ops.paged_decode(q, kp, vp, tables, positions, single_row=True, **kw),
+                           ops.paged_decode(q[:, 0], kp, vp, tables, views, **kw))):
+            assert got.shape == q.shape and torch.equal(got[:, 0], want)
+    for bad in (dict(q=q[:, 0]), dict(positions=wide[:, 0]), dict(positions=wide.repeat(2, 1)[: 2 if shape[0] == 1 else 4])):
+        args = dict(dict(q=q, positions=wide), **bad)
+        with pytest.raises(ops.AxlError):
+            ops.decode(args["q"], k, v, args["positions"], single_row=True, softmax_scale=0.1, lengths_are_positions=True)
+    with pytest.raises(ops.AxlError):
+        ops.decode(q, k, v, wide[:, 0].expand(b), softmax_scale=0.1, lengths_are_positions=True)   # 4-d without it
+
+
+def test_page_insert_of_a_layers_projections():
+    hkv, pages, page, d, b = 2, 9, 16, 64, 4
+    for strided in (False, True):
+        base = torch.randn(b, 3, hkv, 2 * d, device="cuda").to(torch.bfloat16)
+        proj = base[:, 1:2, :, :d] if strided else base[:, 1:2, :, :d].contiguous()
+        tables = torch.arange(1, 9, dtype=torch.int32, device="cuda").reshape(b, 2)
+        for positions in (torch.tensor([[0], [17], [31], [5]], dtype=torch.int32, device="cuda"),
+                          torch.tensor([[9]], dtype=torch.int32, device="cuda")):
+            pools = [torch.zeros(hkv, pages, page, d, dtype=torch.bfloat16, device="cuda") for _ in range(4)]
+            ops.paged_kv_insert(pools[0], pools[1], proj, proj, tables, positions, single_row=True)
+            ops.paged_kv_insert(pools[2], pools[3], proj[:, 0], proj[:, 0], tables, positions.reshape(-1))
+            assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3]) and pools[0].abs().sum() > 0

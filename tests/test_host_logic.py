@@ -886,3 +886,62 @@ def test_forms_for_a_live_width_and_for_a_copied_bias_keep_their_distances():
     _assert_asm_mfma_distances(asm, r"_ZN3axl25flash_bwd_dkdv_w96_kernel", 8)
     blocks = [b for b in remarks.split("Function Name: ")[1:] if "flash_bwd_dkdv_w96_kernel" in b.split()[0]]
     assert len(blocks) == 8 and all("ScratchSize [bytes/lane]: 0" in b for b in blocks)
+
+
+def test_split_of_a_flat_sum_is_what_the_general_form_gives():
+    class General(ab.CompositeAttentionBias):   # not the class itself: the loop over bias_and_residual
+        pass
+
+    pos = dict(target_positions=torch.arange(8)[None], source_positions=torch.arange(8)[None])
+    seg = ab.SegmentIdAttentionBias(torch.ones(2, 8, dtype=torch.int32))
+    members = [ab.CausalAttentionBias(**pos), ab.ZeroAttentionBias(), seg, ab.TensorAttentionBias(torch.randn(1, 2, 8, 8)),
+               ab.TensorAttentionBias(torch.randn(2, 1, 8, 8)), None,
+               ab.SlidingWindowAttentionBias(ab.sliding_window_causal_mask(3), sliding_window_size=3, **pos),
+               ab.BoolTensorAttentionBias(torch.ones(1, 1, 8, 8, dtype=torch.bool))]
+    classes = [(ab.MaskFnAttentionBias,), (ab.MaskFnAttentionBias, ab.SegmentIdAttentionBias), (ab.TensorAttentionBias,),
+               (ab.SegmentIdAttentionBias, ab.BoolAttentionBias), (ab.BaseAttentionBias,)]
+    outcome = lambda kind, chosen, cls: [
+        [id(m) for m in p.biases] if isinstance(p, ab.CompositeAttentionBias) else
+        (type(p), p._shape(), getattr(p, "sliding_window_size", None)) if isinstance(p, ab.MaskFnAttentionBias) or not p.has_value()
+        else id(p) for p in ab.split(kind(chosen), *cls)]
+    for bits in range(1 << len(members)):
+        chosen = [m for i, m in enumerate(members) if bits >> i & 1]
+        for cls in classes:
+            results = []
+            for kind in (ab.CompositeAttentionBias, General):
+                try:
+                    results.append(outcome(kind, chosen, cls))
+                except (NotImplementedError, ValueError, TypeError) as e:
+                    results.append(type(e))
+            if cls != (ab.BaseAttentionBias,):   # takes the composite itself
+                assert results[0] == results[1], (chosen, cls)
+
+
+def test_shapes_that_go_together_broadcast_as_torch_does():
+    for shapes in ([(1, 2, 3, 4)], [(1, 2, 3, 4), (5, 1, 3, 1)], [(0, 1), (1, 4)], [(2, 3), (1, 2, 3)], [(2,), (3,)], [(0,), (2,)]):
+        try:
+            want = tuple(torch.broadcast_shapes(*shapes))
+        except RuntimeError:
+            with pytest.raises(RuntimeError):
+                ab._broadcast_shapes(shapes)
+            continue
+        assert ab._broadcast_shapes(shapes) == want
+
+
+@pytest.mark.parametrize("cls,fill", [
+    (_lib.AxlFlashFwdParams, _lib.fill_flash_fwd), (_lib.AxlFlashChunkParams, _lib.fill_flash_chunk),
+    (_lib.AxlFlashBwdParams, _lib.fill_flash_bwd), (_lib.AxlPagedDecodeParams, _lib.fill_paged_decode),
+    (_lib.AxlDecodeParams, _lib.fill_decode), (_lib.AxlPageInsertParams, _lib.fill_page_insert)])
+def test_packed_parameter_blocks_hold_their_fields(cls, fill):
+    def leaves(c, prefix=()):
+        for name, t in c._fields_:
+            yield from leaves(t, prefix + (name,)) if issubclass(t, ctypes.Structure) else [prefix + (name,)]
+
+    paths = list(leaves(cls))
+    block = fill(*range(1, len(paths) + 1))
+    for want, path in enumerate(paths, 1):
+        value = block
+        for name in path:
+            value = getattr(value, name)
+        assert value == want, path
+    assert _lib.int32(1 << 31) == -(1 << 31) and _lib.int32((1 << 32) + 5) == 5 and _lib.int32(-7) == -7
