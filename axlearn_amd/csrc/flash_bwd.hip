@@ -409,8 +409,8 @@ static bool spill_eligible(const AxlFlashBwdParams& p) {
   return (p.dtype == AXL_BF16 || p.dtype == AXL_F16 || f32_planes(p)) &&
          (p.mask_kind == AXL_MASK_CAUSAL || p.mask_kind == AXL_MASK_SLIDING_WINDOW) && p.q_pos_offset == 0 &&
          p.q_len == p.kv_len && (p.flags & AXL_BWD_DS_WORKSPACE) &&
-         // the ranged kernel keeps the table in LDS beside its ring: 256-row blocks at head_dim 128
-         (!spill_ranged(p) || (p.kv_len / 128 <= kMaxKbRanged && (p.head_dim <= 64 || p.q_len % 256 == 0)));
+         // the ranged kernel keeps the table in LDS beside its ring
+         (!spill_ranged(p) || p.kv_len / 128 <= kMaxKbRanged);
 }
 
 // kv heads whose dS the workspace holds at a time (AXL_BWD_DS_SLICE_KV_HEADS in the flags; all of them

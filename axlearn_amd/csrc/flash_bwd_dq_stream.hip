@@ -19,9 +19,12 @@
 // tile (shared, XOR-swizzled) and each wavefront's own 4 KB of ds arrive by direct global->LDS loads
 // through a ring of buffers; dQ^T += K^T dS^T with both operands from transposing LDS reads.  The
 // kernel issues 2.5 LDS reads and half a tile load per MFMA, each of which holds up the wavefront that
-// issues it, so it runs with two wavefronts per SIMD where the shape allows (NW = 8, one workgroup of
-// 256 rows per CU, three buffers; a wavefront of the upper 128 rows has two trips more than one of
-// the lower 128) and with NW = 4 (five buffers) otherwise.
+// issues it, so at head_dim 128 it runs with two wavefronts per SIMD (NW = 8, one workgroup of 256 rows per CU,
+// three buffers; a wavefront of the upper 128 rows has two trips more than one of the lower 128).  Where the rows are
+// an odd multiple of 128, four wavefronts of the last workgroup own none and only help to load.  (Workgroups of 128 rows
+// throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
+// with segment ids they had to recompute dS: B8 H32/8 T2176 window 256 743 -> 688 us, B3 H16 T5760 window 1024 packed
+// 797 -> 752 us.)  At head_dim 64 NW = 4 (five buffers).
 #include "flash_bwd.h"
 
 namespace axl {
@@ -56,12 +59,13 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   int qb, b, h;
-  decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 32, qb, b, h);
+  decode_block(blockIdx.x, (a.T + Tile::BQ - 1) / Tile::BQ, a.B, a.Hq, a.Hkv, 32, qb, b, h);
   const int hk = h / (a.Hq / a.Hkv);
   const int q0 = qb * Tile::BQ + wave * 32;
   const int t_q = NW * qb + wave;            // this wavefront's query tile
-  int trips = 2 * ((NW * qb + NW - 1) / 4 + 1);  // 64-key tiles up to and including the last diagonal block
-  const int my_trips = __builtin_amdgcn_readfirstlane(2 * (t_q / 4 + 1));  // ... of this wavefront's own 128-row block
+  const bool live = q0 < a.T;
+  int trips = 2 * ((min(NW * qb + NW, a.T / 32) - 1) / 4 + 1);  // 64-key tiles up to and including the last diagonal block
+  const int my_trips = __builtin_amdgcn_readfirstlane(live ? 2 * (t_q / 4 + 1) : 0);  // ... of this wavefront's own 128-row block
   int trip0 = 0;                                 // first 64-key tile that any of the workgroup's query tiles has dS for
   __shared__ int2 s_rng[RANGED ? kMaxKbRanged : 1];
   __shared__ int s_first[RANGED ? NW : 1], s_last[RANGED ? NW : 1];
@@ -129,8 +133,8 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
   const int64_t k_step = (int64_t)Tile::BK * a.ks.s;
   const __bf16* k_src = (const __bf16*)a.k + b * a.ks.b + hk * a.ks.h + trip0 * k_step;
   const int G = a.Hq / a.Hkv;
-  const char* ds_src = (const char*)a.ds + ds_run_start((int64_t)b * a.Hkv + hk, a.T, G, t_q, h - hk * G) * kDsBlockBytes +
-                       (int64_t)trip0 * Tile::DS_WAVE_BYTES;
+  const char* ds_src = (const char*)a.ds + (!live ? 0 : ds_run_start((int64_t)b * a.Hkv + hk, a.T, G, t_q, h - hk * G) * kDsBlockBytes +
+                       (int64_t)trip0 * Tile::DS_WAVE_BYTES);
   const unsigned ds_lane = 16 * lane;
   const unsigned lds0 = lds_address(smem);
 #define AXL_DMA_TRIP(BUF_)                                                                         \
@@ -233,6 +237,7 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
 #undef AXL_DMA_TRIP
 #undef AXL_ADVANCE
 
+  if (!live) return;
   __bf16* dqp = (__bf16*)a.dq + b * a.dqs.b + (int64_t)(q0 + l32) * a.dqs.s + h * a.dqs.h;
 #pragma unroll
   for (int dt = 0; dt < DT; dt++)
@@ -254,18 +259,15 @@ static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
   auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED, W>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
-  const int grid = (a.T / Tile::BQ) * a.B * a.Hq;
+  const int grid = (a.T + Tile::BQ - 1) / Tile::BQ * a.B * a.Hq;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * NW), Tile::LDS_BYTES, stream, a);
   return hipGetLastError();
 }
 
 template <typename E, int D, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
-  // 8 wavefronts need two K loads per wavefront (head_dim 128) and 256-row blocks
-  constexpr int NW8 = D == 128 ? 8 : 4;
-  if (D == 128 && a.T % 256 == 0)
-    return a.kb_tbl ? launch_nw<E, D, NW8, true, W>(a, stream) : launch_nw<E, D, NW8, false, W>(a, stream);
-  return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
+  constexpr int NW = D == 128 ? 8 : 4;   // 8 wavefronts need two K loads per wavefront (head_dim 128)
+  return a.kb_tbl ? launch_nw<E, D, NW, true, W>(a, stream) : launch_nw<E, D, NW, false, W>(a, stream);
 }
 
 template <typename E>

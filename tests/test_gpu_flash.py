@@ -1082,7 +1082,7 @@ def test_ds_workspace_backward_matches_oracle(b, t, hq, hkv, d, dtype):
     (3, 640, 10, 5, 64, torch.float16, "sliding", 31, "packed"),
     # ids that come back later in the row: the key blocks that hold dS for a query tile are then not one run
     (2, 768, 6, 6, 128, torch.float16, "causal", None, "unsorted"),
-    # head_dim 128 with a length that is not a multiple of 256: the flag falls back to the recomputing path
+    # head_dim 128 with a length that is not a multiple of 256
     (1, 384, 4, 4, 128, torch.bfloat16, "sliding", 64, "packed"),
 ])
 def test_ds_workspace_backward_under_window_and_segments(b, t, hq, hkv, d, dtype, mask, window, seg):
@@ -1742,3 +1742,31 @@ def test_forward_leaves_a_copy_of_the_bias(t, s, hq, hkv, d, mask, window, bias_
         if "segment_ids" not in args or seg is not None:
             with pytest.raises(ops.AxlError):
                 ops.flash_fwd(q, k, v, bias_copy=torch.empty_like(args["bias"]), **args, **kw)
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,dtype", [
+    (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),      # one workgroup, half of its wavefronts without rows
+    (2, 384, 4, 2, 128, "causal", None, True, torch.float16),
+    (1, 640, 8, 8, 128, "sliding", 100, True, torch.bfloat16),       # pairs a multiple of 8
+    (2, 1152, 4, 4, 96, "sliding", 700, False, torch.bfloat16),
+    (1, 896, 4, 2, 128, "causal", None, False, torch.bfloat16),
+])
+def test_dq_from_stored_ds_with_rows_an_odd_multiple_of_128(b, t, hq, hkv, d, mask, window, packed, dtype):
+    """The last workgroup of 256 rows owns 128: its other wavefronts read nothing but what is there and store nothing.
+    dk and dv are the bits of the recomputing pair's (delta apart, which the two sum in different orders: dk to 1e-4), dq sums
+    the same products in another order; dq lies in a larger tensor whose rows past the end stay as they were."""
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, dtype))
+    segs = ref.packed_segment_ids(6, b, t).cuda() if packed else None
+    mk = ops.MASK_CAUSAL if mask == "causal" else ops.MASK_SLIDING_WINDOW
+    kw = dict(mask_kind=mk, sliding_window=window or 0, softmax_scale=d ** -0.5, segment_ids=segs)
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    _, dk, dv, ws = ops.flash_bwd_buffers(q, k, v, mask_kind=mk, ds_workspace=True, segment_ids=segs)
+    plain = ops.flash_bwd_buffers(q, k, v, mask_kind=mk, segment_ids=segs)
+    assert ws.numel() > plain[3].numel()
+    ws.fill_(0xff)
+    wide = torch.full((b + 1, t, hq, d), 7.0, dtype=dtype, device="cuda")
+    got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=True, buffers=(wide[:b], dk, dv, ws), **kw)
+    want = ops.flash_bwd(q, k, v, out, lse, do, buffers=plain, **kw)
+    assert torch.equal(got[2], want[2]) and (wide[b] == 7.0).all()
+    for x, y in zip(got[:2], want[:2]):
+        assert torch.isfinite(x.float()).all() and ref.rel_l2(x.cpu(), y.cpu().float()) < 1e-4
