@@ -455,14 +455,22 @@ __device__ __forceinline__ int classify_segment_groups_tbl(const int2* tbl, int 
 // `batch_fastest`: an XCD takes the pairs of one kv head after one another over the batch, for inputs that
 // the batch shares: a broadcast bias is then read by all of it while that XCD's L2 or the memory-side cache
 // holds it (kv heads a multiple of 8, so that the batch stays on one XCD).
+// `two_per_cu`: the kernel's workgroups share a CU in pairs.  A launch that all fits at once, and more than half of
+// it, then gives its second half out in ascending order: the CU that got the heaviest block of the first half gets
+// the lightest of the second, and all have about the same to do (causal, 16 query blocks: 33 tiles per CU instead of
+// 18 to 48).  In longer launches the dispatcher evens that out itself.
 __device__ __forceinline__ void decode_block(int bid, int nqb, int B, int Hq, int Hkv, int slots, int& qb,
-                                             int& b, int& h, bool batch_fastest = false) {
+                                             int& b, int& h, bool batch_fastest = false, bool two_per_cu = false) {
   const int G = Hq / Hkv;
   const int npairs = B * Hkv;
+  auto second_half_ascending = [&](int i, int n, int resident) {
+    return two_per_cu && n <= resident && i >= resident / 2 ? resident / 2 + (n - 1 - i) : i;
+  };
   if (npairs % 8 == 0) {
-    const int xcd = bid & 7, slot = bid >> 3;
+    const int xcd = bid & 7;
     const int ppx = npairs >> 3;                       // pairs per XCD
     const int per_pair = nqb * G;
+    const int slot = second_half_ascending(bid >> 3, ppx * per_pair, slots);
     const int pgn = max(1, (slots + per_pair - 1) / per_pair);  // pairs per group
     const int grp = slot / (pgn * per_pair);
     const int r = slot - grp * (pgn * per_pair);
@@ -475,6 +483,7 @@ __device__ __forceinline__ void decode_block(int bid, int nqb, int B, int Hq, in
     h = (by_head ? xcd + 8 * (i / B) : (xcd + 8 * i) % Hkv) * G + rem % G;
   } else {
     const int per_qb = B * Hq;
+    bid = second_half_ascending(bid, nqb * per_qb, 8 * slots);
     const int qb_rev = bid / per_qb, rem = bid % per_qb;
     qb = nqb - 1 - qb_rev;
     b = rem / Hq;

@@ -208,7 +208,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     qb = slot - sh.first - split * nqb;
     hk = blockIdx.x - slot * a.Hkv;
   } else {
-    decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h, BIAS16 && a.aux.bias_sb == 0);
+    decode_block(blockIdx.x, a.T / Tile::BQ, a.B, a.Hq, a.Hkv, 256 / NW, qb, b, h, BIAS16 && a.aux.bias_sb == 0, INPUTS != kFwdAux && NW == 4);
     hk = h / G;
   }
   const int q_off = CHUNK ? 0 : a.q_off + (a.q_offs ? a.q_offs[b] : 0);  // position of this sequence's query row 0
