@@ -1770,3 +1770,33 @@ def test_dq_from_stored_ds_with_rows_an_odd_multiple_of_128(b, t, hq, hkv, d, ma
     assert torch.equal(got[2], want[2]) and (wide[b] == 7.0).all()
     for x, y in zip(got[:2], want[:2]):
         assert torch.isfinite(x.float()).all() and ref.rel_l2(x.cpu(), y.cpu().float()) < 1e-4
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,ids", [
+    (1, 128, 2, 1, 64, "causal", None, "packed"),        # workgroups of four wavefronts, one row block
+    (2, 384, 4, 2, 128, "none", None, "unsorted"),       # ids that come back later in the row
+    (1, 640, 4, 4, 64, "sliding", 100, "packed"),
+    (2, 512, 64, 8, 128, "causal", None, "packed"),      # eight wavefronts (256 rows)
+    (2, 512, 64, 8, 64, "none", None, "unsorted"),
+    (2, 256, 2, 2, 128, "causal", None, "single"),       # every token a document of its own: no tile of one id
+])
+def test_float32_forward_leaves_out_keys_of_other_documents(b, t, hq, hkv, d, mask, window, ids):
+    """The key range shrinks to the documents of a workgroup's queries and tiles of one id go unmasked: the values of
+    the oracle, to the bar of every float32 test; NaN in the keys and values of a document reach no other."""
+    q, k, v, _ = _inputs(b, t, hq, hkv, d, torch.float32)
+    seg = ref.packed_segment_ids(8, b, t, max_docs=4)
+    if ids == "unsorted":
+        seg = (seg * 7) % 5 + 1
+    if ids == "single":
+        seg = torch.arange(t, dtype=torch.int32)[None].repeat(b, 1)
+    spec, kw = _mask_args(mask, window, seg)
+    out, lse = ops.flash_fwd(q.cuda(), k.cuda(), v.cuda(), softmax_scale=d ** -0.5, **kw)
+    want = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5)
+    _assert_close("out", out, want, torch.float32)
+    hidden = seg == seg[:, -1:]
+    kn, vn = (torch.where(hidden[:, :, None, None], float("nan"), x) for x in (k, v))
+    poisoned, _ = ops.flash_fwd(q.cuda(), kn.cuda(), vn.cuda(), softmax_scale=d ** -0.5, **kw)
+    if ids != "unsorted" and mask == "causal":
+        rows = 256 if t % 256 == 0 else 128
+        clean = ~torch.repeat_interleave(hidden.reshape(b, -1, rows).any(-1), rows, 1)   # row blocks without that document
+        assert torch.equal(poisoned.cpu()[clean], out.cpu()[clean])
