@@ -19,17 +19,17 @@
 // tile (shared, XOR-swizzled) and each wavefront's own 4 KB of ds arrive by direct global->LDS loads
 // through a ring of buffers; dQ^T += K^T dS^T with both operands from transposing LDS reads.  The
 // kernel issues 2.5 LDS reads and half a tile load per MFMA, each of which holds up the wavefront that
-// issues it, so at head_dim 128 it runs with two wavefronts per SIMD (NW = 8, one workgroup of 256 rows per CU,
+// issues it, so at head_dim 128 long calls run with two wavefronts per SIMD (NW = 8, one workgroup of 256 rows per CU,
 // three buffers; a wavefront of the upper 128 rows has two trips more than one of the lower 128).  Where the rows are
 // an odd multiple of 128, four wavefronts of the last workgroup own none and only help to load.  (Workgroups of 128 rows
 // throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
 // with segment ids they had to recompute dS: B8 H32/8 T2176 window 256 743 -> 688 us, B3 H16 T5760 window 1024 packed
-// 797 -> 752 us.)  At head_dim 64 NW = 4 (five buffers).
+// 797 -> 752 us.)  At head_dim 64 and in calls of at most one workgroup per CU NW = 4 (five buffers, or four).
 #include "flash_bwd.h"
 
 namespace axl {
 
-template <int D, int NW>
+template <int D, int NW, bool RANGED>
 struct DqStream {
   static constexpr int BQ = 32 * NW;         // query rows per workgroup (32 per wavefront)
   static constexpr int BK = 64;              // keys per trip
@@ -38,7 +38,7 @@ struct DqStream {
   static constexpr int DS_WAVE_BYTES = 2 * kDsBlockBytes;          // two 32-key blocks per wavefront per trip
   static constexpr int DS_BASE = K_BYTES;
   static constexpr int BUF_BYTES = K_BYTES + NW * DS_WAVE_BYTES;
-  static constexpr int NBUF = NW == 8 ? 3 : 5;
+  static constexpr int NBUF = NW == 8 ? 3 : D == 128 && RANGED ? 4 : 5;   // (the RANGED form's table lies beside the ring)
   static constexpr int WROWS = BK / NW;                            // K rows that one wavefront fetches
   static constexpr int RPI = 1024 / ROWB;                          // K rows per direct-to-LDS instruction
   static constexpr int K_DMA_PER_WAVE = WROWS / RPI;
@@ -52,7 +52,7 @@ struct DqStream {
 // W: live width, as in the dK/dV kernel.
 template <typename E, int D, int NW, bool RANGED, int W>
 __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdArgs a) {
-  using Tile = DqStream<D, NW>;
+  using Tile = DqStream<D, NW, RANGED>;
   constexpr int DT = W / 32;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
 
 template <typename E, int D, int NW, bool RANGED, int W>
 static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
-  using Tile = DqStream<D, NW>;
+  using Tile = DqStream<D, NW, RANGED>;
   auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED, W>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
@@ -266,7 +266,13 @@ static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
 
 template <typename E, int D, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
-  constexpr int NW = D == 128 ? 8 : 4;   // 8 wavefronts need two K loads per wavefront (head_dim 128)
+  // 8 wavefronts need two K loads per wavefront (head_dim 128), and more workgroups than CUs: a launch of one round
+  // lasts as long as its longest workgroup, and blocks of 128 rows are shorter and even out (causal, dQ with 256 / 128
+  // rows: B1 H32 T512 14.3 / 10.6 us, T1024 22.4 / 16.8, T2048 45.6 / 39.2, H8 T8192 159 / 132; past that B4 H32 T1024 46.4 / 52.6, B2 H32 T2048
+  // 74.5 / 83.5 us).
+  constexpr int NW = D == 128 ? 8 : 4;
+  if (NW == 8 && (int64_t)((a.T + 255) / 256) * a.B * a.Hq <= cu_count())
+    return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
   return a.kb_tbl ? launch_nw<E, D, NW, true, W>(a, stream) : launch_nw<E, D, NW, false, W>(a, stream);
 }
 

@@ -1745,11 +1745,16 @@ def test_forward_leaves_a_copy_of_the_bias(t, s, hq, hkv, d, mask, window, bias_
 
 
 @pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,dtype", [
-    (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),      # one workgroup, half of its wavefronts without rows
+    # workgroups of 128 rows: at most one of 256 per CU
+    (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),
     (2, 384, 4, 2, 128, "causal", None, True, torch.float16),
     (1, 640, 8, 8, 128, "sliding", 100, True, torch.bfloat16),       # pairs a multiple of 8
     (2, 1152, 4, 4, 96, "sliding", 700, False, torch.bfloat16),
-    (1, 896, 4, 2, 128, "causal", None, False, torch.bfloat16),
+    # workgroups of 256 rows
+    (2, 384, 80, 8, 128, "causal", None, True, torch.float16),
+    (3, 640, 32, 8, 128, "sliding", 100, False, torch.bfloat16),
+    (3, 128, 96, 3, 96, "causal", None, False, torch.bfloat16),      # half of every workgroup without rows
+    (2, 896, 36, 9, 128, "causal", None, False, torch.bfloat16),
 ])
 def test_dq_from_stored_ds_with_rows_an_odd_multiple_of_128(b, t, hq, hkv, d, mask, window, packed, dtype):
     """The last workgroup of 256 rows owns 128: its other wavefronts read nothing but what is there and store nothing.
