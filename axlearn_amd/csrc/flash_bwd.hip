@@ -425,8 +425,13 @@ static bool spill_eligible(const AxlFlashBwdParams& p) {
   return (p.dtype == AXL_BF16 || p.dtype == AXL_F16 || f32_planes(p)) &&
          (p.mask_kind == AXL_MASK_CAUSAL || p.mask_kind == AXL_MASK_SLIDING_WINDOW) && p.q_pos_offset == 0 &&
          p.q_len == p.kv_len && (p.flags & AXL_BWD_DS_WORKSPACE) &&
-         // the ranged kernel keeps the table in LDS beside its ring
-         (!spill_ranged(p) || p.kv_len / 128 <= kMaxKbRanged);
+         // The ranged kernel keeps the table in LDS beside its ring.  At head_dim 128 a length that is an odd multiple of
+         // 128 takes it from more than one workgroup of 256 rows per CU on; below that the recomputing kernel is as fast in
+         // less memory (training step, recomputing / from dS: B1 H16 T3968 window 1024 packed 197 to 204 / 193 to 210 us,
+         // B1 H8 T4224 packed 242 / 239; above it B8 H32/8 T2176 window 256 743 / 688 us).
+         (!spill_ranged(p) || (p.kv_len / 128 <= kMaxKbRanged &&
+                               (p.head_dim <= 64 || p.q_len % 256 == 0 ||
+                                (int64_t)((p.q_len + 255) / 256) * p.batch * p.num_q_heads > cu_count())));
 }
 
 // kv heads whose dS the workspace holds at a time (AXL_BWD_DS_SLICE_KV_HEADS in the flags; all of them

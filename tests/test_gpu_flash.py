@@ -1082,7 +1082,7 @@ def test_ds_workspace_backward_matches_oracle(b, t, hq, hkv, d, dtype):
     (3, 640, 10, 5, 64, torch.float16, "sliding", 31, "packed"),
     # ids that come back later in the row: the key blocks that hold dS for a query tile are then not one run
     (2, 768, 6, 6, 128, torch.float16, "causal", None, "unsorted"),
-    # head_dim 128 with a length that is not a multiple of 256
+    # head_dim 128 with a length that is not a multiple of 256: the flag falls back to the recomputing path
     (1, 384, 4, 4, 128, torch.bfloat16, "sliding", 64, "packed"),
 ])
 def test_ds_workspace_backward_under_window_and_segments(b, t, hq, hkv, d, dtype, mask, window, seg):
@@ -1747,10 +1747,9 @@ def test_forward_leaves_a_copy_of_the_bias(t, s, hq, hkv, d, mask, window, bias_
 @pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,dtype", [
     # workgroups of 128 rows: at most one of 256 per CU
     (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),
-    (2, 384, 4, 2, 128, "causal", None, True, torch.float16),
-    (1, 640, 8, 8, 128, "sliding", 100, True, torch.bfloat16),       # pairs a multiple of 8
-    (2, 1152, 4, 4, 96, "sliding", 700, False, torch.bfloat16),
     # workgroups of 256 rows
+    (1, 640, 96, 8, 128, "sliding", 100, True, torch.bfloat16),      # pairs a multiple of 8
+    (2, 1152, 32, 4, 96, "sliding", 700, False, torch.bfloat16),
     (2, 384, 80, 8, 128, "causal", None, True, torch.float16),
     (3, 640, 32, 8, 128, "sliding", 100, False, torch.bfloat16),
     (3, 128, 96, 3, 96, "causal", None, False, torch.bfloat16),      # half of every workgroup without rows
