@@ -92,6 +92,8 @@ struct DkvPart {
 hipError_t launch_bwd_dkdv(const BwdArgs& a, int dtype, int head_dim, bool aux, hipStream_t stream);
 hipError_t launch_bwd_dkdv_aux(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 hipError_t launch_bwd_dkdv_bias(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
+hipError_t launch_bwd_dkdv_split(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
+hipError_t launch_bwd_dkdv_split_bias(const BwdArgs& a, int dtype, int head_dim, hipStream_t stream);
 
 // Enqueues the streaming dQ kernel, dq = scale * dS k from the dS blocks in a.ds (with a.kb_tbl set:
 // from the blocks that table says were stored).

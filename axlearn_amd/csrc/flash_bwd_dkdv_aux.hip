@@ -5,10 +5,15 @@
 
 namespace axl {
 
+template <typename E, int D, bool HAS_SEG, int AUX>
+static hipError_t launch_form(const BwdArgs& a, hipStream_t stream) {
+  if (a.splits > 1) return a.ds ? launch_one<E, D, HAS_SEG, AUX, true, D, true>(a, stream) : launch_one<E, D, HAS_SEG, AUX, false, D, true>(a, stream);
+  return a.ds ? launch_one<E, D, HAS_SEG, AUX, true, D, false>(a, stream) : launch_one<E, D, HAS_SEG, AUX, false, D, false>(a, stream);
+}
+
 template <typename E, int D, int AUX>
 static hipError_t launch_mode(const BwdArgs& a, hipStream_t stream) {
-  if (a.ds) return a.seg ? launch_one<E, D, true, AUX, true>(a, stream) : launch_one<E, D, false, AUX, true>(a, stream);
-  return a.seg ? launch_one<E, D, true, AUX>(a, stream) : launch_one<E, D, false, AUX>(a, stream);
+  return a.seg ? launch_form<E, D, true, AUX>(a, stream) : launch_form<E, D, false, AUX>(a, stream);
 }
 
 template <typename E, int D>
@@ -16,7 +21,7 @@ static hipError_t launch_for(const BwdArgs& a, hipStream_t stream) {
   const int bias = a.aux.bias ? (a.aux.bias_f32 ? kAuxBias32 : kAuxBias16) : 0;
   switch (bias | (a.aux.drop ? kAuxDrop : 0)) {
     case kAuxBias16:  // beside segment ids
-      return a.ds ? launch_one<E, D, true, kAuxBias16, true>(a, stream) : launch_one<E, D, true, kAuxBias16>(a, stream);
+      return launch_form<E, D, true, kAuxBias16>(a, stream);
     case kAuxBias32: return launch_mode<E, D, kAuxBias32>(a, stream);
     case kAuxDrop: return launch_mode<E, D, kAuxDrop>(a, stream);
     case kAuxBias16 | kAuxDrop: return launch_mode<E, D, kAuxBias16 | kAuxDrop>(a, stream);

@@ -71,7 +71,11 @@ constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than 
 // W: live width, the head_dim rounded up to a multiple of 32 (D: the width of a row in LDS).  The MFMAs and fragment
 // reads past it, whose operands or results are nothing but padding, are left out (B2 H32/8 T4096, head_dim 96 causal
 // with dS 557 -> 481 us, 80 unmasked 931 -> 775 us; the recomputing dQ kernel there 708 -> 590 us).
-template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W>
+//
+// SPLIT: several workgroups share the query tiles of a key block (a.splits of them, plan_dkdv: launches that would leave
+// CUs idle), each leaving fp32 partial sums for flash_bwd_dkdv_combine_kernel.  A form of its own: as a run-time branch it
+// cost launches of many short workgroups 1 % (B8 H16 T8192 window 4096 packed 2.62 against 2.64 ms) in scalar registers.
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W, bool SPLIT>
 __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   // A bf16 bias alone comes through the tile ring like Q and dO, its elements read from LDS where they are used;
   // everything else is the plain kernel.  The other inputs (fp32 bias, dropout mask, both, a bias beside segment
@@ -100,10 +104,8 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   // them brings a Q / dO tile into L2, the others find it there), half as many workgroups start and
   // end, and the launch divides evenly over the CUs.
   const int npairs = a.B * a.Hkv, nkb = a.S / Tile::BKV;
-  // With a.splits > 1 (plan_dkdv: launches that would leave CUs idle) that many workgroups share the query tiles of
-  // a key block, or of both, each leaving fp32 partial sums for flash_bwd_dkdv_combine_kernel; the splits of a key
-  // block have neighbouring numbers.
-  const int nkb_wg = nkb / a.kb_per_wg * a.splits;   // (key block, split) pairs the blockIdx mapping numbers
+  const int splits = SPLIT ? a.splits : 1;         // those of a key block have neighbouring numbers
+  const int nkb_wg = nkb / a.kb_per_wg * splits;   // (key block, split) pairs the blockIdx mapping numbers
   int kb0, pair;
   if (npairs % 8 == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
@@ -118,9 +120,9 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
     pair = blockIdx.x % npairs;
   }
   int split = 0;
-  if (a.splits > 1) {
-    split = kb0 % a.splits;
-    kb0 /= a.splits;
+  if constexpr (SPLIT) {
+    split = kb0 % splits;
+    kb0 /= splits;
   }
   const int b = pair / a.Hkv, hk = pair % a.Hkv;
   for (int pass = 0; pass < a.kb_per_wg; pass++) {
@@ -171,8 +173,8 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
     // which tiles' dS this key block stores, for the streaming dQ kernel (the same for every kv head and split)
     if (a.kb_tbl && hk == 0 && split == 0 && tid == 0) a.kb_tbl[b * nkb + kb] = make_int2(t_begin, t_begin + nt);
   }
-  if (a.splits > 1) {  // this workgroup's share of the tiles
-    const int lo = nt * split / a.splits, hi = nt * (split + 1) / a.splits;
+  if constexpr (SPLIT) {  // this workgroup's share of the tiles
+    const int lo = nt * split / splits, hi = nt * (split + 1) / splits;
     t_begin += lo;
     nt = hi - lo;
   }
@@ -847,8 +849,8 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
 #undef AXL_A_FRAG
 #undef AXL_ADVANCE
 
-  if (a.splits > 1) {
-    char* part = a.part + (((int64_t)pair * nkb + kb) * a.splits + split) * (4 * DkvPart<W>::BYTES) + wave * DkvPart<W>::BYTES;
+  if constexpr (SPLIT) {
+    char* part = a.part + (((int64_t)pair * nkb + kb) * splits + split) * (4 * DkvPart<W>::BYTES) + wave * DkvPart<W>::BYTES;
 #pragma unroll
     for (int i = 0; i < 4 * DT; i++) {
       const floatx4 wk = {dk_acc[i / 4][4 * (i % 4)], dk_acc[i / 4][4 * (i % 4) + 1], dk_acc[i / 4][4 * (i % 4) + 2], dk_acc[i / 4][4 * (i % 4) + 3]};
@@ -885,14 +887,20 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void flash_bwd_dkdv_kernel(const BwdArgs a) {
-  flash_bwd_dkdv_body<E, D, HAS_SEG, AUX, SPILL, D>(a);
+  flash_bwd_dkdv_body<E, D, HAS_SEG, AUX, SPILL, D, false>(a);
 }
 
 // Head dims 72 to 96 of the width 128.
 template <typename E, bool HAS_SEG, bool SPILL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
 void flash_bwd_dkdv_w96_kernel(const BwdArgs a) {
-  flash_bwd_dkdv_body<E, 128, HAS_SEG, 0, SPILL, 96>(a);
+  flash_bwd_dkdv_body<E, 128, HAS_SEG, 0, SPILL, 96, false>(a);
+}
+
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+void flash_bwd_dkdv_split_kernel(const BwdArgs a) {
+  flash_bwd_dkdv_body<E, D, HAS_SEG, AUX, SPILL, W, true>(a);
 }
 
 // Sums the partial dK (blockIdx.y 0) and dV (1) of a split launch in the order of the splits, and scales and rounds
@@ -933,11 +941,12 @@ __global__ __launch_bounds__(2 * D) void flash_bwd_dkdv_combine_kernel(const Bwd
   }
 }
 
-template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false, int W = D>
+template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W, bool SPLIT>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
   auto kernel = [] {
-    if constexpr (W == 96) return flash_bwd_dkdv_w96_kernel<E, HAS_SEG, SPILL>;
+    if constexpr (SPLIT) return flash_bwd_dkdv_split_kernel<E, D, HAS_SEG, AUX, SPILL, W>;
+    else if constexpr (W == 96) return flash_bwd_dkdv_w96_kernel<E, HAS_SEG, SPILL>;
     else return flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
   }();
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
@@ -945,6 +954,24 @@ static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), Tile::LDS_BYTES, stream, a);
   return hipGetLastError();
+}
+
+// No bias or dropout mask; head_dim 64, 128, or 96 for the live width.
+template <typename E, bool SPLIT, int D, int W = D>
+static hipError_t launch_plain(const BwdArgs& a, hipStream_t stream) {
+  if (a.ds) return a.seg ? launch_one<E, D, true, 0, true, W, SPLIT>(a, stream) : launch_one<E, D, false, 0, true, W, SPLIT>(a, stream);
+  return a.seg ? launch_one<E, D, true, 0, false, W, SPLIT>(a, stream) : launch_one<E, D, false, 0, false, W, SPLIT>(a, stream);
+}
+template <typename E, bool SPLIT>
+static hipError_t launch_plain_width(const BwdArgs& a, int head_dim, hipStream_t stream) {
+  if (head_dim == 96) return launch_plain<E, SPLIT, 128, 96>(a, stream);
+  return head_dim == 128 ? launch_plain<E, SPLIT, 128>(a, stream) : launch_plain<E, SPLIT, 64>(a, stream);
+}
+
+// A bf16 bias and nothing else.
+template <typename E, bool SPLIT, int D>
+static hipError_t launch_bias(const BwdArgs& a, hipStream_t stream) {
+  return a.ds ? launch_one<E, D, false, kAuxBias16, true, D, SPLIT>(a, stream) : launch_one<E, D, false, kAuxBias16, false, D, SPLIT>(a, stream);
 }
 
 }  // namespace axl

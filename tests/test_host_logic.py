@@ -888,6 +888,13 @@ def test_forms_for_a_live_width_and_for_a_copied_bias_keep_their_distances():
     assert len(blocks) == 8 and all("ScratchSize [bytes/lane]: 0" in b for b in blocks)
 
 
+def test_split_dkdv_kernels_keep_their_distances():
+    """The dK/dV forms whose workgroups share a key block's query tiles: the same chains, and nothing in scratch memory."""
+    asm, remarks = _device_asm("flash_bwd_dkdv_split.hip")
+    _assert_asm_mfma_distances(asm, r"_ZN3axl27flash_bwd_dkdv_split_kernel", 32)
+    assert re.findall(r"ScratchSize \[bytes/lane\]: (\d+)", remarks) == ["0"] * 32
+
+
 def test_split_of_a_flat_sum_is_what_the_general_form_gives():
     class General(ab.CompositeAttentionBias):   # not the class itself: the loop over bias_and_residual
         pass
