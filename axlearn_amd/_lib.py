@@ -190,6 +190,12 @@ def int32(x) -> int:
     return x if -0x80000000 <= x <= 0x7fffffff else ctypes.c_int32(x).value
 
 
+def float32(x) -> float:
+    """`x` as the parameter blocks hold it: past the type's range infinite, where `struct` would raise."""
+    x = float(x)
+    return x if -3.4e38 < x < 3.4e38 else ctypes.c_float(x).value
+
+
 EXPORTED_SYMBOLS = (
     "axl_flash_fwd",
     "axl_flash_chunk",

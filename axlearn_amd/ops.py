@@ -122,7 +122,7 @@ def _aux(bias, dropout_mask, dropout_rate, b, hq, t, s) -> Tuple[tuple, tuple]:
         if dropout_mask.stride(-1) != 1:
             dropout_mask = dropout_mask.contiguous()
         keep.append(dropout_mask)
-        drop_part = (float(dropout_rate), dropout_mask.data_ptr(), *dropout_mask.stride()[:3])
+        drop_part = (_lib.float32(dropout_rate), dropout_mask.data_ptr(), *dropout_mask.stride()[:3])
     elif dropout_rate:
         raise AxlError(_lib.AXL_ERR_INVALID_ARGUMENT, "dropout_rate needs a dropout_mask (the kernels draw no random numbers)")
     return bias_part + drop_part, tuple(keep)
@@ -194,7 +194,7 @@ def flash_fwd(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), _lib.ptr(lse), _lib.ptr(seg),
         *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out),
         b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), _lib.int32(q_pos_offset),
-        float(softmax_scale), _lib.ptr(sink), *aux, _lib.ptr(q_pos_offsets), _lib.ptr(bias_copy),
+        _lib.float32(softmax_scale), _lib.ptr(sink), *aux, _lib.ptr(q_pos_offsets), _lib.ptr(bias_copy),
     )
     _lib.check(lib.axl_flash_fwd(ctypes.byref(p), _lib.current_stream_ptr()))
     return out, lse
@@ -225,7 +225,7 @@ def flash_chunk(
     p = _lib.fill_flash_chunk(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
         *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out),
-        b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), float(softmax_scale),
+        b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), _lib.float32(softmax_scale),
         _lib.ptr(sink), positions.data_ptr(), positions.stride(0) if positions.shape[0] > 1 else 0, positions.stride(1),
         int(positions.dtype == torch.int64), 0, 0,
     )
@@ -315,7 +315,7 @@ def flash_bwd(
         *_lib.strides4(q), *_lib.strides4(k), *_lib.strides4(v), *_lib.strides4(out), *_lib.strides4(d_out),
         *_lib.strides4(dq), *_lib.strides4(dk), *_lib.strides4(dv),
         b, t, s, hq, hkv, d, _lib.dtype_code(q.dtype), mask_kind, _lib.int32(sliding_window), _lib.int32(q_pos_offset),
-        float(softmax_scale), 0, 0, _lib.ptr(sink), _lib.ptr(d_sink), *aux, _bwd_flags(ds_workspace, ds_slice_kv_heads),
+        _lib.float32(softmax_scale), 0, 0, _lib.ptr(sink), _lib.ptr(d_sink), *aux, _bwd_flags(ds_workspace, ds_slice_kv_heads),
     )
     ws = _bwd_workspace(lib, p, by_size or bias is not None or dropout_mask is not None, ws, q.device)
     p.workspace = ws.data_ptr()
@@ -560,7 +560,7 @@ def paged_decode(
     p = _lib.fill_paged_decode(
         q.data_ptr(), k_pages.data_ptr(), v_pages.data_ptr(), page_tables.data_ptr(), len_ptr, out.data_ptr(),
         b, hq, hkv, d, num_pages, page_size, page_tables.shape[1], _lib.dtype_code(q.dtype), _lib.int32(sliding_window),
-        float(softmax_scale), 0, 0, _decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions),
+        _lib.float32(softmax_scale), 0, 0, _decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions),
         *bias_blk, len_stride,
     )
     need = int(lib.axl_paged_decode_workspace_bytes(ctypes.byref(p)))
@@ -631,7 +631,7 @@ def decode(
     bias_blk, _keep = _decode_bias(bias, b, hq, s)
     p = _lib.fill_decode(
         q.data_ptr(), k.data_ptr(), v.data_ptr(), len_ptr, out.data_ptr(), *_lib.strides4(k), *_lib.strides4(v),
-        b, s, hq, hkv, d, _lib.dtype_code(q.dtype), _lib.int32(sliding_window), float(softmax_scale), 0, 0,
+        b, s, hq, hkv, d, _lib.dtype_code(q.dtype), _lib.int32(sliding_window), _lib.float32(softmax_scale), 0, 0,
         _decode_flags(deterministic, workspace_reused, lengths, lengths_are_positions), *bias_blk, len_stride,
     )
     need = int(lib.axl_decode_workspace_bytes(ctypes.byref(p)))

@@ -5,6 +5,7 @@ import ctypes
 import json
 import os
 import re
+import struct
 
 import numpy as np
 import pytest
@@ -952,3 +953,6 @@ def test_packed_parameter_blocks_hold_their_fields(cls, fill):
             value = getattr(value, name)
         assert value == want, path
     assert _lib.int32(1 << 31) == -(1 << 31) and _lib.int32((1 << 32) + 5) == 5 and _lib.int32(-7) == -7
+    for x in (0.125, -1e39, 1e39, 3.4028235e38, float("inf"), float("nan")):   # as a ctypes field holds them
+        (packed,), want = struct.unpack("f", struct.pack("f", _lib.float32(x))), ctypes.c_float(x).value
+        assert packed == want or (packed != packed and want != want), x
