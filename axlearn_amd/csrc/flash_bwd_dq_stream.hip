@@ -23,8 +23,8 @@
 // three buffers; a wavefront of the upper 128 rows has two trips more than one of the lower 128).  Where the rows are
 // an odd multiple of 128, four wavefronts of the last workgroup own none and only help to load.  (Workgroups of 128 rows
 // throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
-// with segment ids they had to recompute dS: B8 H32/8 T2176 window 256 743 -> 688 us, B3 H16 T5760 window 1024 packed
-// 797 -> 752 us.)  At head_dim 64 and in calls of at most one workgroup per CU NW = 4 (five buffers, or four).
+// with segment ids they had to recompute dS, as calls of at most one workgroup per CU still do: B8 H32/8 T2176 window 256
+// 743 -> 688 us, B3 H16 T5760 window 1024 packed 797 -> 752 us.)  At head_dim 64 and in calls of at most one workgroup per CU NW = 4 (five buffers, or four).
 #include "flash_bwd.h"
 
 namespace axl {
