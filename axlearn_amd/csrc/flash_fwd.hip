@@ -1517,6 +1517,10 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   if (p.bias_copy && !(bias16 && p.dtype != AXL_F32 && !p.segment_ids && p.aux.bias_row_stride == p.kv_len))
     return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: bias_copy needs a bf16 bias of rows without gaps, a 16-bit "
                                           "dtype, no dropout mask and no segment_ids");
+  // Of a bias that the batch shares the workgroups of the first sequence store what they read: all that any sequence sees
+  // only where all are at the same offset.
+  if (p.bias_copy && p.q_pos_offsets && p.batch > 1 && !a.aux.bias_sb)
+    return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: bias_copy with q_pos_offsets needs a bias per sequence");
   const int width = p.head_dim <= 64 ? 64 : 128;  // the compiled width that serves this head_dim
   hipError_t err = hipSuccess;
 #define AXL_LAUNCH_FWD(KERNEL, TILE)                                                            \

@@ -170,12 +170,14 @@ def flash_fwd(
     bias [B|1,Hq|1,T,S] bf16/fp32: dense additive logit bias.  dropout_mask [B,Hq,T,S] bool/uint8
     (True = dropped) with dropout_rate: kept probabilities are scaled by 1 / (1 - rate).
     bias_copy: a tensor like the bias that receives the elements of it that the mask leaves visible, where
-    `can_copy_bias` says so."""
+    `can_copy_bias` says so (with q_pos_offsets a bias that the batch shares is refused: each sequence sees keys of its own)."""
     b, t, hq, d, s, hkv = _check_qkv(q, k, v)
     _check_segment_ids(segment_ids, b, t, s)
     if bias_copy is not None:
         if bias is None or not can_copy_bias(q, bias, segment_ids, dropout_mask):
             raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "the forward cannot copy this bias")
+        if q_pos_offsets is not None and b > 1 and bias.shape[0] == 1:
+            raise AxlError(_lib.AXL_ERR_UNSUPPORTED, "bias_copy with q_pos_offsets needs a bias per sequence")
         _want_shape("bias_copy", bias_copy, bias.shape)
         if bias_copy.dtype != bias.dtype or not bias_copy.is_contiguous():
             raise _bad("bias_copy must be contiguous and have the dtype of the bias")

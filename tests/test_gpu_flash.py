@@ -1744,6 +1744,30 @@ def test_forward_leaves_a_copy_of_the_bias(t, s, hq, hkv, d, mask, window, bias_
                 ops.flash_fwd(q, k, v, bias_copy=torch.empty_like(args["bias"]), **args, **kw)
 
 
+@pytest.mark.parametrize("window", [None, 200])
+def test_forward_copies_the_bias_of_sequences_at_offsets_of_their_own(window):
+    """A bias per sequence, each sequence behind a prefix of its own: what any of them sees is in the copy, and a backward
+    of one sequence at its offset gets the same bits from it.  (One bias for all is refused.)"""
+    b, t, s, hq, hkv, d = 2, 128, 512, 4, 2, 64
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, torch.bfloat16, s=s))
+    bias = torch.randn(b, hq, t, s, device="cuda", generator=torch.Generator("cuda").manual_seed(5)).to(torch.bfloat16)
+    offsets = torch.tensor([37, 384], dtype=torch.int32, device="cuda")
+    kw = dict(mask_kind=ops.MASK_CAUSAL if window is None else ops.MASK_SLIDING_WINDOW, sliding_window=window or 0, softmax_scale=d ** -0.5)
+    out, lse = ops.flash_fwd(q, k, v, bias=bias, q_pos_offsets=offsets, **kw)
+    copy = torch.full_like(bias, float("nan"))
+    out_c, lse_c = ops.flash_fwd(q, k, v, bias=bias, bias_copy=copy, q_pos_offsets=offsets, **kw)
+    assert torch.equal(out, out_c) and torch.equal(lse, lse_c)
+    for i, offset in enumerate(offsets.tolist()):
+        diff = torch.arange(t, device="cuda")[:, None] + offset - torch.arange(s, device="cuda")[None]
+        seen = (diff >= 0) & (diff <= (window if window is not None else s))
+        assert torch.equal(copy[i][:, seen], bias[i][:, seen])
+        one = lambda *xs: [x[i : i + 1] for x in xs]
+        got, want = (ops.flash_bwd(*one(q, k, v, out, lse, do), bias=x[i : i + 1], q_pos_offset=offset, **kw) for x in (copy, bias))
+        assert all(torch.equal(x, y) for x, y in zip(got, want))
+    with pytest.raises(ops.AxlError):
+        ops.flash_fwd(q, k, v, bias=bias[:1], bias_copy=copy[:1], q_pos_offsets=offsets, **kw)
+
+
 @pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,dtype", [
     # workgroups of 128 rows: at most one of 256 per CU
     (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),

@@ -956,3 +956,32 @@ def test_packed_parameter_blocks_hold_their_fields(cls, fill):
     for x in (0.125, -1e39, 1e39, 3.4028235e38, float("inf"), float("nan")):   # as a ctypes field holds them
         (packed,), want = struct.unpack("f", struct.pack("f", _lib.float32(x))), ctypes.c_float(x).value
         assert packed == want or (packed != packed and want != want), x
+
+
+def test_a_bias_that_sequences_at_offsets_of_their_own_share_is_not_copied():
+    """One workgroup per row block stores a bias that the batch shares, the one of the first sequence: at other offsets
+    others see other keys of it.  Refused ahead of any launch."""
+    from axlearn_amd import ops
+
+    lib = _lib.load()
+    s = _lib.AxlStrides(1 << 20, 1024, 128)
+    p = _lib.AxlFlashFwdParams(q=256, k=256, v=256, out=256, q_strides=s, k_strides=s, v_strides=s, out_strides=s,
+                               batch=2, q_len=128, kv_len=256, num_q_heads=4, num_kv_heads=2, head_dim=128, dtype=0,
+                               mask_kind=1, softmax_scale=1.0, q_pos_offsets=256, bias_copy=256,
+                               aux=_lib.AxlAttnAux(bias=256, bias_head_stride=128 * 256, bias_row_stride=256, bias_dtype=0))
+    assert lib.axl_flash_fwd(ctypes.byref(p), None) == _lib.AXL_ERR_UNSUPPORTED
+    assert b"q_pos_offsets" in lib.axl_last_error()
+
+    q = torch.zeros(2, 128, 4, 128, dtype=torch.bfloat16)
+    k = torch.zeros(2, 256, 2, 128, dtype=torch.bfloat16)
+    offsets = torch.tensor([0, 128], dtype=torch.int32)
+    for shape in ((1, 4, 128, 256), (1, 1, 128, 256)):
+        bias = torch.zeros(shape, dtype=torch.bfloat16)
+        with pytest.raises(_lib.AxlError, match="q_pos_offsets"):
+            ops.flash_fwd(q, k, k, mask_kind=ops.MASK_CAUSAL, bias=bias, bias_copy=torch.zeros_like(bias), q_pos_offsets=offsets)
+    # every sequence its own bias, or one sequence: copied (the next thing to fail is the device check)
+    own = torch.zeros(2, 4, 128, 256, dtype=torch.bfloat16)
+    for args, bias in (((q, k, k), own), ((q[:1], k[:1], k[:1]), own[:1])):
+        with pytest.raises(_lib.AxlError, match="GPU"):
+            ops.flash_fwd(*args, mask_kind=ops.MASK_CAUSAL, bias=bias, bias_copy=torch.zeros_like(bias),
+                          q_pos_offsets=offsets[: len(bias)])
