@@ -481,7 +481,7 @@ struct DkdvPlan {
   int kb_per_wg, splits;
 };
 constexpr int kSplitTiles = 128, kMaxSplits = 32, kMaxSplitBlocks = 512;
-static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind) {
+static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind, int64_t q_off, int max_splits) {
   // Two key blocks per workgroup under a causal mask, where a block and its mirror image see
   // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
   // environment (read once) keeps one block per workgroup.
@@ -497,9 +497,9 @@ static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind) {
   int64_t longest = 0, total = 0;
   for (int kb = 0; kb < nkb; kb++) {
     int64_t lo = 0, hi = p.q_len;
-    if (mask_kind != AXL_MASK_NONE) lo = std::max<int64_t>(0, std::min<int64_t>(p.q_len, (int64_t)kb * 128 - p.q_pos_offset));
+    if (mask_kind != AXL_MASK_NONE) lo = std::max<int64_t>(0, std::min<int64_t>(p.q_len, (int64_t)kb * 128 - q_off));
     if (mask_kind == AXL_MASK_SLIDING_WINDOW)
-      hi = std::max<int64_t>(lo, std::min<int64_t>(p.q_len, (int64_t)kb * 128 + 128 + p.sliding_window - p.q_pos_offset));
+      hi = std::max<int64_t>(lo, std::min<int64_t>(p.q_len, (int64_t)kb * 128 + 128 + p.sliding_window - q_off));
     const int64_t n = (hi - lo + 31) / 32 * G;
     longest = std::max(longest, n);
     total += n;
@@ -517,18 +517,19 @@ static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind) {
   DkdvPlan best = whole;
   double best_cost = cost(whole) / 1.2;
   for (int kpw = 1; kpw <= whole.kb_per_wg; kpw++)
-    for (int n = 2; n <= kMaxSplits && blocks * n <= kMaxSplitBlocks; n++)
+    for (int n = 2; n <= max_splits && blocks * n <= kMaxSplitBlocks; n++)
       if (cost(DkdvPlan{kpw, n}) < best_cost) {
         best = DkdvPlan{kpw, n};
         best_cost = cost(best);
       }
   return best;
 }
-// Bytes of the partial sums.  The same for every mask, so that a workspace sized without it fits: a window's calls,
-// which the size does not look at, take no more splits than there is room for.
+// Bytes of the partial sums.  The same for every mask and every offset of the queries, so that a workspace sized without
+// them fits: calls under a window or at an offset, which the size does not look at, take no more splits than there is
+// room for.
 static int max_splits(const AxlFlashBwdParams& p) {
   if (p.flags & AXL_BWD_NO_SPLIT) return 1;
-  return std::max(plan_dkdv(p, AXL_MASK_NONE).splits, plan_dkdv(p, AXL_MASK_CAUSAL).splits);
+  return std::max(plan_dkdv(p, AXL_MASK_NONE, 0, kMaxSplits).splits, plan_dkdv(p, AXL_MASK_CAUSAL, 0, kMaxSplits).splits);
 }
 static size_t split_bytes(const AxlFlashBwdParams& p) {
   const int n = max_splits(p);
@@ -570,9 +571,10 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   a.d_real = p.head_dim;
   a.stat_hq = p.num_q_heads;
   {
-    const DkdvPlan plan = plan_dkdv(p, p.mask_kind);   // of all kv heads, whatever the slices: the same sums
+    // of all kv heads, whatever the slices: the same sums
+    const DkdvPlan plan = plan_dkdv(p, p.mask_kind, p.q_pos_offset, max_splits(p));
     a.kb_per_wg = plan.kb_per_wg;
-    a.splits = std::min(plan.splits, max_splits(p));
+    a.splits = plan.splits;
   }
   const int width = p.head_dim <= 64 ? 64 : 128;   // the compiled width that serves this head_dim
   a.aux = make_aux_args(p.aux, p.softmax_scale);

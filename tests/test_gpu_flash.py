@@ -1706,6 +1706,36 @@ def test_query_tiles_of_a_key_block_shared_by_workgroups(b, t, hq, hkv, d, mask,
     assert all(torch.equal(x, y) for x, y in zip(again, got))
 
 
+@pytest.mark.parametrize("t,s,hq,hkv,d,mask,window,offset", [
+    (1024, 2048, 16, 1, 128, "causal", None, 1024),
+    (1024, 2048, 16, 2, 64, "causal", None, 0),       # key blocks that no query sees: every share is empty
+    (1024, 2048, 16, 2, 64, "sliding", 300, 1000),
+    (640, 1024, 4, 1, 128, "causal", None, 440),      # more shares would pay than the workspace has room for
+])
+def test_shared_query_tiles_behind_a_prefix(t, s, hq, hkv, d, mask, window, offset):
+    """Queries at an offset: a workspace sized without it gives the bits of the call's own, and those are the unsplit
+    call's but for the order of fp32 sums (the bounds of the test above)."""
+    q, k, v, do = (x.cuda() for x in _inputs(1, t, hq, hkv, d, torch.bfloat16, s=s))
+    kw = dict(mask_kind=ops.MASK_CAUSAL if mask == "causal" else ops.MASK_SLIDING_WINDOW, sliding_window=window or 0,
+              softmax_scale=d ** -0.5, q_pos_offset=offset)
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    bufs = ops.flash_bwd_buffers(q, k, v)
+    bufs[3].fill_(0xff)
+    got = ops.flash_bwd(q, k, v, out, lse, do, buffers=bufs, **kw)
+    own = ops.flash_bwd(q, k, v, out, lse, do, **kw)
+    assert all(torch.equal(x, y) for x, y in zip(got, own))
+    p = _lib.AxlFlashBwdParams(batch=1, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d, flags=_lib.BWD_NO_SPLIT)
+    small = _lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p))
+    assert (small < bufs[3].numel()) == (t == 1024)
+    whole = (*(torch.empty_like(x) for x in (q, k, v)), torch.empty(small, dtype=torch.uint8, device="cuda"))
+    want = ops.flash_bwd(q, k, v, out, lse, do, buffers=whole, **kw)
+    assert torch.equal(got[0], want[0])
+    for name, x, y in (("dk", got[1].float(), want[1].float()), ("dv", got[2].float(), want[2].float())):
+        rms = y.square().mean().sqrt()
+        assert ((x - y).abs() <= 2 * 2.0 ** -8 * y.abs() + 2e-5 * rms).all(), name
+        assert ref.rel_l2(x.cpu(), y.cpu()) < 2.0 ** -10, name
+
+
 @pytest.mark.parametrize("t,s,hq,hkv,d,mask,window,bias_b,bias_h,dtype", [
     (128, 128, 4, 4, 64, "causal", None, 1, 4, torch.bfloat16),      # one row block, nothing but diagonal tiles
     (640, 640, 4, 2, 128, "causal", None, 1, 4, torch.bfloat16),

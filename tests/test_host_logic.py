@@ -985,3 +985,29 @@ def test_a_bias_that_sequences_at_offsets_of_their_own_share_is_not_copied():
         with pytest.raises(_lib.AxlError, match="GPU"):
             ops.flash_fwd(*args, mask_kind=ops.MASK_CAUSAL, bias=bias, bias_copy=torch.zeros_like(bias),
                           q_pos_offsets=offsets[: len(bias)])
+
+
+@pytest.mark.parametrize("dtype", [_lib.AXL_BF16, _lib.AXL_F16, _lib.AXL_F32])
+def test_backward_workspace_is_the_same_for_every_mask_and_offset(dtype):
+    """Without dS or segment ids: a workspace sized without the mask or the offset of the queries holds every call of
+    its shapes, partial sums of dK and dV included (`flash_bwd_buffers` takes no offset)."""
+    rng = np.random.default_rng(0)
+    shapes = [(1, 640, 1024, 4, 1, 128, 440), (1, 1024, 4096, 16, 1, 64, 3072)]
+    for _ in range(300):
+        t, s = (128 * int(x) for x in rng.integers(1, 33, 2))
+        hkv = int(rng.choice([1, 2, 4, 8]))
+        shapes.append((int(rng.integers(1, 5)), t, s, hkv * int(rng.choice([1, 2, 4, 8])), hkv,
+                       int(rng.choice([64, 96, 128] if dtype != _lib.AXL_F32 else [64, 128])), int(rng.integers(-t, s + 1))))
+    lib = _lib.load()
+    split = 0
+    for b, t, s, hq, hkv, d, offset in shapes:
+        p = _lib.AxlFlashBwdParams(batch=b, q_len=t, kv_len=s, num_q_heads=hq, num_kv_heads=hkv, head_dim=d, dtype=dtype)
+        sizes = set()
+        for p.mask_kind in (0, 1, 2):
+            for p.q_pos_offset in (0, offset, s - t):
+                for p.sliding_window in (0, 100, 5000):
+                    sizes.add(lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)))
+        assert len(sizes) == 1, (b, t, s, hq, hkv, d, offset, sizes)
+        p.flags = _lib.BWD_NO_SPLIT
+        split += lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)) < sizes.pop()
+    assert (split > 30) == (dtype != _lib.AXL_F32)
