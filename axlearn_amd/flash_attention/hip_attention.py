@@ -180,6 +180,23 @@ def _is_the_callers(dense: Tensor, bias: BaseAttentionBias) -> bool:
     return True
 
 
+def _reads_per_bias_element(query: Tensor, bias: Tensor, mask_kind: int, window: int) -> float:
+    """How many times a forward reads an element of the bias, by the (batch, head) pairs that share it and the part of
+    it that the mask leaves visible.
+
+    A clone costs 0.8 us per million elements of the bias, its copy by the forward kernel 0.1 to 0.2 us per million that
+    the kernel reads, whether the workgroup stores them or not (a bigger loop).  Clone and forward / forward with the copy,
+    D128: 1 read or less B2 H16 T2048 causal, a bias per head 127 / 78 us, B4 H8 T4096 window 512, one per sequence 155 / 112;
+    4 reads B8 H32 T1024 causal, per head 177 / 157, B8 H8 T1024 causal, per sequence 45 / 45; 8 reads B8 H16 T1024 without a
+    mask, per head 114 / 127, B2 H16 T2048 causal, per sequence 67 / 73; 16 reads B1 H32 T2048 causal, one bias 66 / 72."""
+    b, _, hq, _ = query.shape
+    kv_len = bias.shape[3]
+    visible = 1.0 if mask_kind == ops.MASK_NONE else 0.5
+    if mask_kind == ops.MASK_SLIDING_WINDOW:
+        visible = min(visible, (window + 1) / kv_len)
+    return b * hq * visible / (bias.shape[0] * bias.shape[1])
+
+
 class _FlashAttentionFn(torch.autograd.Function):
     """Forward = axl_flash_fwd, backward = axl_flash_bwd.
 
@@ -191,7 +208,7 @@ class _FlashAttentionFn(torch.autograd.Function):
     head) more, 5 GEMMs instead of 7; ignored where that path does not apply), False to recompute dS
     in the dQ kernel, None to take the dS workspace whenever it fits bwd_workspace_limit_bytes (None:
     a sixteenth of the device's memory).  copy_bias=True: the caller may write to the bias ahead of the backward,
-    which gets a copy of it, left by the forward kernel where that can."""
+    which gets a copy of it, left by the forward kernel where that can and `_reads_per_bias_element` are few."""
 
     @staticmethod
     def forward(ctx, query, key, value, segment_ids, softmax_scale, mask_kind, window, logit_sink,
@@ -201,7 +218,8 @@ class _FlashAttentionFn(torch.autograd.Function):
         aux = dict(dropout_mask=dropout_mask, dropout_rate=dropout_rate)
         kept = {}
         if copy_bias:
-            if ops.can_copy_bias(query, bias, segment_ids, dropout_mask):
+            if (ops.can_copy_bias(query, bias, segment_ids, dropout_mask)
+                    and _reads_per_bias_element(query, bias, mask_kind, window) <= 4):
                 kept = dict(bias_copy=torch.empty_like(bias))
             else:
                 bias = bias.clone()

@@ -1011,3 +1011,38 @@ def test_backward_workspace_is_the_same_for_every_mask_and_offset(dtype):
         p.flags = _lib.BWD_NO_SPLIT
         split += lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p)) < sizes.pop()
     assert (split > 30) == (dtype != _lib.AXL_F32)
+
+
+@pytest.mark.parametrize("bias_shape,mask,window,by_forward", [
+    ((1, 4, 256, 256), "causal", 0, True),     # a bias per head for a batch of two
+    ((2, 4, 256, 256), "none", 0, True),
+    ((2, 1, 256, 256), "causal", 0, True),     # 4 heads, half of them visible: 2 reads of an element
+    ((1, 1, 256, 256), "none", 0, False),      # 8 reads
+    ((1, 1, 256, 256), "sliding", 31, True),   # 8 heads, an eighth visible: 1
+])
+def test_forward_copies_a_bias_where_it_is_not_read_many_times_over(monkeypatch, bias_shape, mask, window, by_forward):
+    """A bias that a backward will read again: stored by the forward where few workgroups read the same element, cloned
+    ahead of it otherwise.  Either way the backward has the values of the forward after the buffer was refilled."""
+    seen = []
+
+    def flash_fwd(q, k, v, *, bias, bias_copy=None, **kw):
+        seen.append((bias, bias_copy))
+        if bias_copy is not None:
+            bias_copy.copy_(bias)
+        return q + 0.0, torch.zeros(2, 4, 256)
+
+    monkeypatch.setattr(ops, "flash_fwd", flash_fwd)
+    monkeypatch.setattr(ops, "flash_bwd", lambda q, k, v, *a, **kw: (q * 0 + kw["bias"].float().mean(), k + 0.0, v + 0.0))
+    q, k, v = (torch.randn(2, 256, 4, 64).to(torch.bfloat16).requires_grad_(True) for _ in range(3))
+    pos = dict(target_positions=torch.arange(256)[None], source_positions=torch.arange(256)[None])
+    buffer = torch.full(bias_shape, 3.0, dtype=torch.bfloat16)
+    members = [ab.TensorAttentionBias(buffer)]
+    if mask == "causal":
+        members.append(ab.CausalAttentionBias(**pos))
+    if mask == "sliding":
+        members.append(ab.SlidingWindowAttentionBias(ab.sliding_window_causal_mask(window), sliding_window_size=window, **pos))
+    out = HipFlashAttention.default_config().instantiate()(dict(query=q, key=k, value=v, bias=ab.CompositeAttentionBias(members)))
+    buffer.fill_(-1.0)
+    assert torch.equal(torch.autograd.grad(out.sum(), q)[0], torch.full_like(q, 3.0))
+    (bias, copy), = seen
+    assert (copy is not None) == by_forward and (bias.data_ptr() == buffer.data_ptr()) == by_forward
