@@ -260,10 +260,10 @@ int axl_flash_chunk(const AxlFlashChunkParams* p, void* stream) {
 }
 
 size_t axl_flash_bwd_workspace_bytes(const AxlFlashBwdParams* p) {
-  if (!p) return 0;
+  // (not yet checked: the size divides by the heads)
+  if (!p || p->batch <= 0 || p->q_len <= 0 || p->kv_len <= 0 || p->num_q_heads <= 0 || p->num_kv_heads <= 0) return 0;
   return flash_bwd_workspace_bytes(*p);
 }
-
 
 int axl_flash_bwd(const AxlFlashBwdParams* p, void* stream) {
   return axl_flash_bwd_phases(p, AXL_BWD_DELTA | AXL_BWD_DKDV | AXL_BWD_DQ, stream);

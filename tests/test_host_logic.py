@@ -1046,3 +1046,26 @@ def test_forward_copies_a_bias_where_it_is_not_read_many_times_over(monkeypatch,
     assert torch.equal(torch.autograd.grad(out.sum(), q)[0], torch.full_like(q, 3.0))
     (bias, copy), = seen
     assert (copy is not None) == by_forward and (bias.data_ptr() == buffer.data_ptr()) == by_forward
+
+
+def test_size_queries_of_shapes_that_no_call_has_return(tmp_path):
+    """Zero or negative extents reach the backward's size query unchecked (`flash_bwd_buffers` asks for what its tensors
+    say): it returns, the call itself is what refuses them.  In a process of its own, which a fault would end."""
+    import subprocess
+    import sys
+
+    script = tmp_path / "sizes.py"
+    script.write_text(f"""
+import ctypes, itertools, sys
+sys.path.insert(0, {ROOT!r})
+from axlearn_amd import _lib
+lib = _lib.load()
+ok = dict(batch=1, q_len=1024, kv_len=1024, num_q_heads=8, num_kv_heads=1, head_dim=64)
+for bad in ({{}}, *({{name: x}} for name in ok for x in (0, -1, -1024))):
+    for dtype, mask, flags in itertools.product((0, 1, 2), (0, 1, 2), (0, 1, 1 | 1 << 8, 4)):
+        p = _lib.AxlFlashBwdParams(dtype=dtype, mask_kind=mask, flags=flags, **dict(ok, **bad))
+        lib.axl_flash_bwd_workspace_bytes(ctypes.byref(p))
+print("done")
+""")
+    done = subprocess.run([sys.executable, str(script)], capture_output=True, text=True, timeout=300)
+    assert done.returncode == 0 and done.stdout.strip() == "done", (done.returncode, done.stderr[-500:])
