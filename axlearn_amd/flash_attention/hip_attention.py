@@ -193,8 +193,8 @@ def _reads_per_bias_element(query: Tensor, bias: Tensor, mask_kind: int, window:
     kv_len = bias.shape[3]
     visible = 1.0 if mask_kind == ops.MASK_NONE else 0.5
     if mask_kind == ops.MASK_SLIDING_WINDOW:
-        visible = min(visible, (window + 1) / kv_len)
-    return b * hq * visible / (bias.shape[0] * bias.shape[1])
+        visible = min(visible, (window + 1) / max(1, kv_len))
+    return b * hq * visible / max(1, bias.shape[0] * bias.shape[1])   # (the sizes are checked by the call itself)
 
 
 class _FlashAttentionFn(torch.autograd.Function):

@@ -1069,3 +1069,22 @@ print("done")
 """)
     done = subprocess.run([sys.executable, str(script)], capture_output=True, text=True, timeout=300)
     assert done.returncode == 0 and done.stdout.strip() == "done", (done.returncode, done.stderr[-500:])
+
+
+@pytest.mark.parametrize("batch,q_heads,kv_len,bias_shape,window", [
+    (0, 4, 256, (0, 4, 256, 256), None),
+    (0, 4, 256, (1, 4, 256, 256), None),
+    (2, 4, 256, (2, 0, 256, 256), None),
+    (2, 4, 0, (1, 4, 256, 0), 31),
+])
+def test_a_bias_without_elements_is_refused_like_any_that_does_not_fit(batch, q_heads, kv_len, bias_shape, window):
+    """The choice between cloning a bias and having the forward store it divides by its sizes ahead of their check."""
+    q = torch.zeros(batch, 256, q_heads, 64, dtype=torch.bfloat16).requires_grad_(True)
+    k, v = (torch.zeros(batch, kv_len, 2, 64, dtype=torch.bfloat16) for _ in range(2))
+    pos = dict(target_positions=torch.arange(256)[None], source_positions=torch.arange(kv_len)[None])
+    members = [ab.TensorAttentionBias(torch.zeros(bias_shape, dtype=torch.bfloat16))]
+    if window is not None:
+        members.append(ab.SlidingWindowAttentionBias(ab.sliding_window_causal_mask(window), sliding_window_size=window, **pos))
+    layer = HipFlashAttention.default_config().instantiate()
+    with pytest.raises(_lib.AxlError):
+        layer(dict(query=q, key=k, value=v, bias=ab.CompositeAttentionBias(members)))
