@@ -717,6 +717,28 @@ def test_head_dims_between_the_compiled_widths(d, dtype, monkeypatch):
             _assert_close(name, got, exp, dtype)
 
 
+@pytest.mark.parametrize("d", [72, 80, 96])
+@pytest.mark.parametrize("hq,hkv", [(16, 16), (32, 2)])   # one workgroup per key block; several that share its query tiles
+@pytest.mark.parametrize("mask,window,packed", [("causal", None, False), ("sliding", 300, True), ("none", None, False)])
+def test_head_dims_that_leave_columns_out_give_the_bits_of_the_full_width(d, hq, hkv, mask, window, packed):
+    """Head dims 72 to 96 skip the last quarter of the width 128, whose products are zeros: outputs, lse and gradients
+    have the bits of the same tensors padded with zeros to 128, with dS from the workspace and recomputed."""
+    b, t = 1, 1024
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, d, torch.bfloat16))
+    segs = ref.packed_segment_ids(4, b, t, max_docs=3) if packed else None
+    _, kw = _mask_args(mask, window, segs)
+    kw["softmax_scale"] = d ** -0.5
+    wide = [torch.nn.functional.pad(x, (0, 128 - d)) for x in (q, k, v, do)]
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    out_w, lse_w = ops.flash_fwd(*wide[:3], **kw)
+    assert torch.equal(out, out_w[..., :d]) and torch.equal(lse, lse_w) and not out_w[..., d:].any()
+    for ds in (False, True):
+        got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, **kw)
+        want = ops.flash_bwd(*wide[:3], out_w, lse_w, wide[3], ds_workspace=ds, **kw)
+        for x, y in zip(got, want):
+            assert torch.equal(x, y[..., :d]) and not y[..., d:].any()
+
+
 def test_head_dim_columns_past_the_end_are_never_used():
     """head_dim 72 as a view of wider tensors whose other columns hold NaN: neither the forward nor the
     backward lets one of them into a result (the tile loads stay inside the 72 columns)."""
@@ -1706,6 +1728,59 @@ def test_query_tiles_of_a_key_block_shared_by_workgroups(b, t, hq, hkv, d, mask,
     assert all(torch.equal(x, y) for x, y in zip(again, got))
 
 
+@pytest.mark.parametrize("t,hq,hkv,d,mask,window,packed,bias,rate,dtype", [
+    (1024, 16, 1, 128, "causal", None, False, torch.float32, 0.0, torch.bfloat16),
+    (1152, 16, 1, 64, "sliding", 300, True, torch.float32, 0.0, torch.float16),
+    (1024, 16, 1, 128, "causal", None, True, None, 0.25, torch.float16),
+    (896, 32, 2, 64, "none", None, False, None, 0.1, torch.bfloat16),
+    (1280, 16, 1, 128, "sliding", 300, False, None, 0.25, torch.bfloat16),     # some shares empty
+    (1024, 16, 1, 128, "causal", None, False, torch.bfloat16, 0.25, torch.bfloat16),
+    (1152, 16, 1, 64, "causal", None, True, torch.bfloat16, 0.5, torch.bfloat16),
+    (1024, 16, 1, 64, "causal", None, False, torch.float32, 0.25, torch.bfloat16),
+    (1280, 16, 1, 128, "sliding", 300, True, torch.float32, 0.5, torch.float16),
+    (1024, 32, 2, 64, "causal", None, True, torch.bfloat16, 0.0, torch.float16),
+])
+def test_shared_query_tiles_with_a_bias_or_dropout_mask(t, hq, hkv, d, mask, window, packed, bias, rate, dtype):
+    """The forms of the split with fp32 biases, dropout masks (whose 1 / (1 - rate) the sum over the shares applies to
+    dv), both, and either beside documents: against the unsplit call, to the bounds of the test above, and against the
+    oracle's gradients, to the bar of every test."""
+    q, k, v, do = _inputs(1, t, hq, hkv, d, dtype)
+    segs = ref.packed_segment_ids(3, 1, t) if packed else None
+    spec, kw = _mask_args(mask, window, segs)
+    kw["softmax_scale"] = d ** -0.5
+    gen = torch.Generator().manual_seed(1)
+    dropped = {}
+    if bias is not None:
+        spec.dense_bias = torch.randn(1, hq, t, t, generator=gen).to(bias)
+        kw["bias"] = spec.dense_bias.cuda()
+    if rate:
+        dropped = dict(dropout_mask=torch.rand(1, hq, t, t, generator=gen) < rate, dropout_rate=rate)
+        kw.update(dropped, dropout_mask=dropped["dropout_mask"].cuda())
+    exact = ref.reference_mha_grads(q, k, v, do, spec, softmax_scale=d ** -0.5, **dropped)
+    q, k, v, do = (x.cuda() for x in (q, k, v, do))
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    step = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for ds in (False, True):
+        bufs = ops.flash_bwd_buffers(q, k, v, mask_kind=kw["mask_kind"], ds_workspace=ds, segment_ids=kw["segment_ids"])
+        p = _lib.AxlFlashBwdParams(batch=1, q_len=t, kv_len=t, num_q_heads=hq, num_kv_heads=hkv, head_dim=d,
+                                   mask_kind=kw["mask_kind"], dtype=_lib.dtype_code(dtype), segment_ids=256 if packed else None,
+                                   flags=_lib.BWD_NO_SPLIT | (_lib.BWD_DS_WORKSPACE if ds else 0))
+        small = _lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p))
+        assert small < bufs[3].numel()
+        whole = (*(torch.empty_like(x) for x in (q, k, v)), torch.empty(small, dtype=torch.uint8, device="cuda"))
+        for x in (bufs[3], whole[3]):
+            x.fill_(0xff)
+        got = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=bufs, **kw)
+        want = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=ds, buffers=whole, **kw)
+        assert torch.equal(got[0], want[0])
+        for name, x, y in (("dk", got[1].float(), want[1].float()), ("dv", got[2].float(), want[2].float())):
+            rms = y.square().mean().sqrt()
+            assert ((x - y).abs() <= 2 * step * y.abs() + 2e-5 * rms).all(), name
+            assert ref.rel_l2(x.cpu(), y.cpu()) < step / 4, name
+        for name, x, y in zip(("dq", "dk", "dv"), got, exact):
+            _assert_close(name, x, y, dtype)
+
+
 @pytest.mark.parametrize("t,s,hq,hkv,d,mask,window,offset", [
     (1024, 2048, 16, 1, 128, "causal", None, 1024),
     (1024, 2048, 16, 2, 64, "causal", None, 0),       # key blocks that no query sees: every share is empty
@@ -1840,7 +1915,7 @@ def test_dq_from_stored_ds_with_rows_an_odd_multiple_of_128(b, t, hq, hkv, d, ma
 ])
 def test_float32_forward_leaves_out_keys_of_other_documents(b, t, hq, hkv, d, mask, window, ids):
     """The key range shrinks to the documents of a workgroup's queries and tiles of one id go unmasked: the values of
-    the oracle, to the bar of every float32 test; NaN in the keys and values of a document reach no other."""
+    the oracle, to the bar of every float32 test."""
     q, k, v, _ = _inputs(b, t, hq, hkv, d, torch.float32)
     seg = ref.packed_segment_ids(8, b, t, max_docs=4)
     if ids == "unsorted":
@@ -1851,10 +1926,27 @@ def test_float32_forward_leaves_out_keys_of_other_documents(b, t, hq, hkv, d, ma
     out, lse = ops.flash_fwd(q.cuda(), k.cuda(), v.cuda(), softmax_scale=d ** -0.5, **kw)
     want = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5)
     _assert_close("out", out, want, torch.float32)
-    hidden = seg == seg[:, -1:]
-    kn, vn = (torch.where(hidden[:, :, None, None], float("nan"), x) for x in (k, v))
-    poisoned, _ = ops.flash_fwd(q.cuda(), kn.cuda(), vn.cuda(), softmax_scale=d ** -0.5, **kw)
-    if ids != "unsorted" and mask == "causal":
-        rows = 256 if t % 256 == 0 else 128
-        clean = ~torch.repeat_interleave(hidden.reshape(b, -1, rows).any(-1), rows, 1)   # row blocks without that document
+
+
+@pytest.mark.parametrize("b,hq,d", [(1, 2, 128), (1, 2, 64), (2, 40, 128), (2, 40, 64)])   # four wavefronts; eight
+@pytest.mark.parametrize("mask,window", [("causal", None), ("sliding", 700), ("none", None)])
+@pytest.mark.parametrize("cuts", [(512,), (256, 768)])
+def test_float32_documents_that_no_query_of_a_workgroup_belongs_to_are_not_read(b, hq, d, mask, window, cuts):
+    """Documents that begin where a workgroup's rows do: with NaN in the keys and values of one of them the rows of
+    the others keep every bit.  (A key that is read and masked would show: its probability is 0, and 0 NaN is NaN.)"""
+    t = 1024
+    q, k, v, _ = _inputs(b, t, hq, hq, d, torch.float32)
+    seg = torch.ones(b, t, dtype=torch.int32)
+    for cut in cuts:
+        seg[:, cut:] += 1
+    _, kw = _mask_args(mask, window, seg)
+    out, lse = ops.flash_fwd(q.cuda(), k.cuda(), v.cuda(), softmax_scale=d ** -0.5, **kw)
+    for doc in range(1, len(cuts) + 2):
+        hidden = seg == doc
+        kn, vn = (torch.where(hidden[:, :, None, None], float("nan"), x).cuda() for x in (k, v))
+        poisoned, lse_p = ops.flash_fwd(q.cuda(), kn, vn, softmax_scale=d ** -0.5, **kw)
+        clean = ~hidden
+        assert clean.any() and hidden.any()
         assert torch.equal(poisoned.cpu()[clean], out.cpu()[clean])
+        assert torch.equal(lse_p.cpu().transpose(1, 2)[clean], lse.cpu().transpose(1, 2)[clean])
+        assert poisoned.cpu()[hidden].isnan().all()
