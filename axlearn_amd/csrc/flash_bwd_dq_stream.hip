@@ -24,7 +24,8 @@
 // an odd multiple of 128, four wavefronts of the last workgroup own none and only help to load.  (Workgroups of 128 rows
 // throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
 // with segment ids they had to recompute dS, as calls of at most one workgroup per CU still do: B8 H32/8 T2176 window 256
-// 743 -> 688 us, B3 H16 T5760 window 1024 packed 797 -> 752 us.)  At head_dim 64 and in calls of at most one workgroup per CU NW = 4 (five buffers, or four).
+// 743 -> 688 us, B3 H16 T5760 window 1024 packed 797 -> 752 us.)  At head_dim 64, and in the shorter launches that launch_one
+// names, NW = 4 (five buffers, or four).
 #include "flash_bwd.h"
 
 namespace axl {
@@ -266,12 +267,22 @@ static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
 
 template <typename E, int D, int W = D>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
-  // 8 wavefronts need two K loads per wavefront (head_dim 128), and more workgroups than CUs: a launch of one round
-  // lasts as long as its longest workgroup, and blocks of 128 rows are shorter and even out (causal, dQ with 256 / 128
-  // rows: B1 H32 T512 14.3 / 10.6 us, T1024 22.4 / 16.8, T2048 45.6 / 39.2, H8 T8192 159 / 132; past that B4 H32 T1024 46.4 / 52.6, B2 H32 T2048
-  // 74.5 / 83.5 us).
+  // 8 wavefronts need two K loads per wavefront (head_dim 128).  Workgroups of 128 rows where they take one round of the
+  // CUs: it lasts as long as its longest workgroup (causal, dQ with 256 / 128 rows: B1 H32 T512 14.3 / 10.6 us, T1024 22.4 / 16.8).
+  // More rounds of them instead of one of 256 rows where lengths differ enough for the short ones to even out, causal rows from 1024 on
+  // (B1 H32 T2048 37.0 / 35.0, H8 T8192 155 / 129; B2 H32 T768 18.8 / 21.0, B8 H16 T512 18.1 / 19.2), with documents from 2048 (of three cuts B1 H32 T2048
+  // 31.0 / 29.0, of 40 20.0 / 21.7; B4 H16 T1024 23.9 / 23.1 and 18.4 / 21.5).  Past one round of 256 rows those (B4 H32 T1024
+  // 46.4 / 52.6, B2 H32 T2048 72.5 / 84.8).
+  //
+  // Under a window shorter than the sequence all workgroups do about the same and what counts are the rounds: one of 128 rows
+  // takes 0.6 to 0.7 of one of 256, so those are taken where they need no more of them (window 256: B1 H16 T2048 15.6 / 11.5,
+  // B6 H16 T640 25.7 / 21.2; the other way B1 H32 T2048 20.8 / 22.5, B2 H32 T768 16.9 / 19.7, B4 H8 T2176 25.2 / 29.1).
   constexpr int NW = D == 128 ? 8 : 4;
-  if (NW == 8 && (int64_t)((a.T + 255) / 256) * a.B * a.Hq <= cu_count())
+  const int64_t cus = cu_count(), heads = (int64_t)a.B * a.Hq, wgs8 = heads * ((a.T + 255) / 256), wgs4 = heads * (a.T / 128);
+  const bool equal = a.mask_kind == AXL_MASK_SLIDING_WINDOW && a.window < a.T;
+  const bool rows128 = equal ? (wgs4 + cus - 1) / cus <= (wgs8 + cus - 1) / cus
+                             : wgs4 <= cus || (wgs8 <= cus && a.T >= (a.kb_tbl ? 2048 : 1024));
+  if (NW == 8 && rows128)
     return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
   return a.kb_tbl ? launch_nw<E, D, NW, true, W>(a, stream) : launch_nw<E, D, NW, false, W>(a, stream);
 }

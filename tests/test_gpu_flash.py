@@ -1876,8 +1876,10 @@ def test_forward_copies_the_bias_of_sequences_at_offsets_of_their_own(window):
 @pytest.mark.parametrize("b,t,hq,hkv,d,mask,window,packed,dtype", [
     # workgroups of 128 rows: at most one of 256 per CU
     (1, 128, 2, 1, 128, "causal", None, False, torch.bfloat16),
+    # a window: workgroups of 128 rows take no more rounds of the CUs
+    (1, 640, 96, 8, 128, "sliding", 100, True, torch.bfloat16),
     # workgroups of 256 rows
-    (1, 640, 96, 8, 128, "sliding", 100, True, torch.bfloat16),      # pairs a multiple of 8
+    (1, 1152, 64, 8, 128, "sliding", 100, True, torch.bfloat16),     # pairs a multiple of 8
     (2, 1152, 32, 4, 96, "sliding", 700, False, torch.bfloat16),
     (2, 384, 80, 8, 128, "causal", None, True, torch.float16),
     (3, 640, 32, 8, 128, "sliding", 100, False, torch.bfloat16),
