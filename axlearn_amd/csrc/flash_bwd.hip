@@ -471,7 +471,10 @@ static size_t planes_bytes(const AxlFlashBwdParams& p) {
 // workgroup walks G x T / 32 tiles (batch 1, 64 / 8 heads, 1792 tokens: 56 workgroups of 480 tiles on 256 CUs).  There the
 // query tiles are split, fp32 partial sums go through the workspace and a second kernel adds them.  Costs, in tiles
 // (0.87 us at the compiled width 128, 0.5 at 64): 12 per key block that a workgroup starts and ends (11 us), 8 for
-// the second launch and 16 per 256 blocks of partial sums written and read.  The split is taken where the
+// the second launch and 16 per 256 blocks of partial sums written and read.  Workgroups that do the same take whole rounds
+// of the CUs; where their lengths differ (causal, one key block each) they even out to the mean.  (With the mean for equal ones
+// too, unmasked calls were cut in two that then took two rounds, batch 6, 8 / 1 heads, 3328 tokens: 592 us unsplit, 664 in two, 489 in
+// three, at 64: 414 / 436 / 304; batch 12, 1024 tokens: 186 unsplit, 154 in three, 114 in two.)  The split is taken where the
 // longest workgroup walks kSplitTiles or more and this estimate falls by a sixth; below that a call is bound by its
 // caller's host work (kernels of less than 110 us in a step of about 200).  Causal, bf16, dK/dV without / with the split
 // and the sum: batch 1, 8 / 1 heads, 4096 tokens 840 / 91 + 14 us; 64 / 8 heads, 1024 tokens 253 / 63 + 10 us; 32 / 8
@@ -505,12 +508,15 @@ static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind, int64_t q_o
     total += n;
   }
   const double both = mirror ? 2.0 * total / nkb : 0;   // the mirror images add up to the same for every workgroup
+  const bool equal = 10 * total >= 9 * longest * nkb;   // (all key blocks unmasked, nearly all under a window)
   if ((mirror ? both : (double)longest) < kSplitTiles) return whole;
   const double start = p.head_dim <= 64 ? 22 : 12, bytes = 16 / 256.0;   // (64: half the bytes, half the time per tile)
   auto cost = [&](const DkdvPlan& x) {
     const int64_t wgs = blocks / x.kb_per_wg * x.splits;
+    const double rounds = (double)((wgs + cus - 1) / cus);
     double c;
-    if (x.kb_per_wg == 2) c = (double)((wgs + cus - 1) / cus) * (both / x.splits + 2 * start);
+    if (x.kb_per_wg == 2) c = rounds * (both / x.splits + 2 * start);
+    else if (equal) c = rounds * ((double)longest / x.splits + start);
     else c = std::max((double)longest / x.splits + start, 1.1 * ((double)total * pairs + start * (double)wgs) / cus);
     return x.splits == 1 ? c : c + 8 + bytes * (double)(blocks * x.splits);
   };
