@@ -71,8 +71,8 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const BwdArgs a) {
 // Gradient of the per-head sink logit.  The sink's probability in row (b, h, t) is
 // exp(sink[h] - lse[b,h,t]) and it has no value row (dP = 0), so dL/dsink is
 // -sum_{b,t} exp(sink[h] - lse) * delta.  One workgroup per head; fixed summation order.  Bound by the latency
-// of its loads: 1024 threads, four rows each in flight (256 threads, a row at a time: B8 H8 T8192 124 us,
-// B6 H32 T2432 31 us).
+// of its loads: 1024 threads, four rows each in flight (256 threads, a row at a time / now: B8 H8 T8192 124 / 26 us,
+// B6 H32 T2432 31 / 9 us).
 // ---------------------------------------------------------------------------------------------
 constexpr int kDsinkThreads = 1024;
 __global__ __launch_bounds__(kDsinkThreads) void bwd_dsink_kernel(const float* __restrict__ sink,
@@ -475,8 +475,12 @@ static size_t planes_bytes(const AxlFlashBwdParams& p) {
 // of the CUs; where their lengths differ (causal, one key block each) they even out to the mean.  (With the mean for equal ones
 // too, unmasked calls were cut in two that then took two rounds, batch 6, 8 / 1 heads, 3328 tokens: 592 us unsplit, 664 in two, 489 in
 // three, at 64: 414 / 436 / 304; batch 12, 1024 tokens: 186 unsplit, 154 in three, 114 in two.)  The split is taken where the
-// longest workgroup walks kSplitTiles or more and this estimate falls by a sixth; below that a call is bound by its
-// caller's host work (kernels of less than 110 us in a step of about 200).  Causal, bf16, dK/dV without / with the split
+// longest workgroup walks kSplitTiles or more and this estimate falls by a sixth.  kSplitTiles was set where
+// about 200 us of host work, a training step of one layer alone, no longer hide the kernel.  The kernels gain below it too (dK/dV
+// unsplit / split with the sum, causal: batch 1, 8 / 2 heads, 1024 tokens 133 / 35 us; 16 / 8 heads 77 / 38; 4 / 4 heads, 4096 tokens
+// 124 / 63; batch 2, 16 / 8 heads, 1024 tokens 78 / 51), which a caller that runs ahead of the GPU would see.  The costs per tile are the plain
+// form's; fp32 biases, dropout masks and both take up to 1.5 us, and every form gains (ten forms with and without documents at 12
+// shapes, both widths, dS stored and not: 1.28 to 13.4 times).  Causal, bf16, dK/dV without / with the split
 // and the sum: batch 1, 8 / 1 heads, 4096 tokens 840 / 91 + 14 us; 64 / 8 heads, 1024 tokens 253 / 63 + 10 us; 32 / 8
 // heads, 2048 tokens 248 / 97 + 12 us; 12 / 4 heads of 64, 4096 tokens 241 / 88 + 7 us; batch 2, 8 / 1 heads with a bias,
 // 1920 tokens 427 / 58 + 12 us; batch 1, 8 / 1 heads, 16384 tokens, window 1024: 257 / 161 + 11 us.

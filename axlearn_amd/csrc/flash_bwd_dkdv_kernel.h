@@ -74,7 +74,8 @@ constexpr int kNotUniformDkv = -0x7fffffff - 1;  // marks a tile with more than 
 //
 // SPLIT: several workgroups share the query tiles of a key block (a.splits of them, plan_dkdv: launches that would leave
 // CUs idle), each leaving fp32 partial sums for flash_bwd_dkdv_combine_kernel.  A form of its own: as a run-time branch it
-// cost launches of many short workgroups 1 % (B8 H16 T8192 window 4096 packed 2.62 against 2.64 ms) in scalar registers.
+// kept 26 more scalar registers of the unsplit kernel spilled (B8 H16 T8192 window 4096 packed 2.64 against 2.62 ms,
+// no more than runs differ by).
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W, bool SPLIT>
 __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   // A bf16 bias alone comes through the tile ring like Q and dO, its elements read from LDS where they are used;
