@@ -35,6 +35,7 @@ struct BwdArgs {
                 // place of the slices past it (finite values that only ever meet those zeros or end up in
                 // output columns that are not stored), stores leave the columns past it out.
   int kb_per_wg;  // key blocks (of 128 keys) a dK/dV workgroup works through: 1, or 2 (a block and its mirror image)
+  int pair_group; // 16-bit dK/dV: (batch, kv head) pairs that an XCD works through together (dkdv_pair_group)
   int splits;     // 16-bit dK/dV: workgroups that share the query tiles of a key block (plan_dkdv); with more than
   char* part;     // one, the workspace's partial sums, DkvPart<width>::BYTES per (pair, key block, split, wavefront)
   AuxArgs aux;  // dense bias / dropout mask (read only by the AUX instantiations)

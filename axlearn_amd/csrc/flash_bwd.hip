@@ -491,10 +491,13 @@ constexpr int kSplitTiles = 128, kMaxSplits = 32, kMaxSplitBlocks = 512;
 static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind, int64_t q_off, int max_splits) {
   // Two key blocks per workgroup under a causal mask, where a block and its mirror image see
   // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
-  // environment (read once) keeps one block per workgroup.
+  // environment (read once) keeps one block per workgroup.  Not with segment ids: documents end where they like, the
+  // two shares add up to anything, and the longer workgroups leave the longer tail (training step, two / one: B6 H32/8
+  // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; of 25 packed causal shapes none
+  // lost more than runs differ by).
   static const bool single = [] { const char* e = getenv("AXL_DKDV_KB_PER_WG"); return e && e[0] == '1'; }();
   const int nkb = p.kv_len / 128;
-  const bool mirror = !single && mask_kind == AXL_MASK_CAUSAL && nkb % 2 == 0;
+  const bool mirror = !single && mask_kind == AXL_MASK_CAUSAL && nkb % 2 == 0 && !p.segment_ids;
   const DkdvPlan whole{mirror ? 2 : 1, 1};
   if (p.dtype == AXL_F32 || nkb < 1) return whole;
   const int64_t pairs = (int64_t)p.batch * p.num_kv_heads, blocks = pairs * nkb;
@@ -556,6 +559,17 @@ size_t flash_bwd_workspace_bytes(const AxlFlashBwdParams& p) {
          (spill_eligible(p) ? spill_bytes(p) : 0) + (kWsAlign - 16);
 }
 
+// Pairs that an XCD works through together in the dK/dV kernel: two (one costs balance, more lose the sharing of Q / dO rows
+// through L2: B8 H16 T8192 causal packed 5.43 ms, all together 5.67), but all of them under a causal mask with one key
+// block per workgroup where the whole launch is at most six rounds of the XCD's CUs.  There the tail weighs more: the late
+// key blocks of every pair, the short ones, then come last (training step, two / all: B5 H32/8 T2560 packed 1061 / 965 us, B5
+// H64/8 T2432 D96 1999 / 1903, B6 H32/8 T1408 packed 479 / 438; unmasked, where early blocks are no longer, it went either way).
+static int dkdv_pair_group(const BwdArgs& a) {
+  const int64_t per_xcd = (int64_t)a.B * a.Hkv / 8 * (a.S / 128) * a.splits;
+  const bool all = a.mask_kind == AXL_MASK_CAUSAL && a.kb_per_wg == 1 && per_xcd <= 6 * cu_count() / 8;
+  return all ? std::max(1, a.B * a.Hkv / 8) : 2;
+}
+
 int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream) {
   const int dt = p.dtype;
   BwdArgs a;
@@ -586,6 +600,7 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
     a.kb_per_wg = plan.kb_per_wg;
     a.splits = plan.splits;
   }
+  a.pair_group = dkdv_pair_group(a);
   const int width = p.head_dim <= 64 ? 64 : 128;   // the compiled width that serves this head_dim
   a.aux = make_aux_args(p.aux, p.softmax_scale);
   const bool aux = p.aux.bias || p.aux.dropout_mask;
@@ -646,6 +661,7 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
       BwdArgs s = a;
       s.Hkv = min(slice, p.num_kv_heads - h0);
       s.Hq = s.Hkv * G;
+      s.pair_group = dkdv_pair_group(s);
       const int64_t hq0 = (int64_t)h0 * G;
       s.q = (const char*)a.q + hq0 * a.qs.h * es;
       s.dout = (const char*)a.dout + hq0 * a.dos.h * es;

@@ -31,10 +31,6 @@
 
 #include "flash_bwd.h"
 
-#ifndef AXL_DKDV_PG
-#define AXL_DKDV_PG 2
-#endif
-
 namespace axl {
 
 // BIAS: with the bf16 bias of the tile's queries and the workgroup's keys beside it.
@@ -95,9 +91,9 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
 
   const int G = a.Hq / a.Hkv;
   // blockIdx -> (key block, batch, kv head).  When the (batch, kv head) pairs divide evenly over the
-  // 8 XCDs (workgroup i is dispatched to XCD i % 8), an XCD works through one pair after the other,
-  // so the workgroups that run together stream the same Q / dO rows through that XCD's L2; within a
-  // pair the earliest key blocks (most queries under a causal mask) come first.
+  // 8 XCDs (workgroup i is dispatched to XCD i % 8), an XCD works through a.pair_group pairs together, one such group
+  // after the other, so the workgroups that run together stream the same Q / dO rows through that XCD's L2; within a
+  // group the earliest key blocks (most queries under a causal mask) come first.
   // With a.kb_per_wg == 2 a workgroup works through TWO key blocks of its pair, one after the other:
   // block kb0 of the first half and its mirror image nkb - 1 - kb0.  Under a causal mask the two see
   // complementary shares of the queries, so every workgroup of the launch walks the same number of
@@ -111,10 +107,10 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   if (npairs % 8 == 0) {
     const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
     const int ppx = npairs >> 3;                     // pairs per XCD
-    const int grp = slot / (AXL_DKDV_PG * nkb_wg);   // group of AXL_DKDV_PG pairs worked through together
-    const int r = slot - grp * (AXL_DKDV_PG * nkb_wg);
-    const int pg = min(AXL_DKDV_PG, ppx - grp * AXL_DKDV_PG);
-    pair = xcd + 8 * (grp * AXL_DKDV_PG + r % pg);
+    const int grp = slot / (a.pair_group * nkb_wg);
+    const int r = slot - grp * (a.pair_group * nkb_wg);
+    const int pg = min(a.pair_group, ppx - grp * a.pair_group);  // the last group may be smaller
+    pair = xcd + 8 * (grp * a.pair_group + r % pg);
     kb0 = r / pg;
   } else {
     kb0 = blockIdx.x / npairs;

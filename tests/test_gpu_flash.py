@@ -1952,3 +1952,33 @@ def test_float32_documents_that_no_query_of_a_workgroup_belongs_to_are_not_read(
         assert torch.equal(poisoned.cpu()[clean], out.cpu()[clean])
         assert torch.equal(lse_p.cpu().transpose(1, 2)[clean], lse.cpu().transpose(1, 2)[clean])
         assert poisoned.cpu()[hidden].isnan().all()
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,packed", [
+    (3, 384, 16, 8, False),    # three pairs per XCD, all together
+    (2, 512, 8, 8, True),      # an even number of key blocks, one per workgroup because of the documents
+    (5, 640, 8, 8, True),      # five pairs, all together
+    (8, 3200, 8, 8, False),    # past six rounds of an XCD's CUs: two pairs at a time
+    (7, 3584, 8, 8, True),     # the last group is a single pair
+])
+def test_pairs_worked_through_together_give_the_bits_of_each_sequence(b, t, hq, hkv, packed):
+    """The order in which the dK/dV kernel's workgroups take (sequence, kv head, key block) does not show in the results:
+    a batch gives the bits of its sequences one by one (no room for partial sums, whose split depends on the batch)."""
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, 64, torch.bfloat16))
+    segs = ref.packed_segment_ids(5, b, t).cuda() if packed else None
+
+    def grads(rows):
+        x = [y[rows] for y in (q, k, v, do)]
+        ids = None if segs is None else segs[rows]
+        kw = dict(mask_kind=ops.MASK_CAUSAL, softmax_scale=0.125, segment_ids=ids)
+        p = _lib.AxlFlashBwdParams(batch=x[0].shape[0], q_len=t, kv_len=t, num_q_heads=hq, num_kv_heads=hkv, head_dim=64,
+                                   mask_kind=ops.MASK_CAUSAL, dtype=_lib.dtype_code(torch.bfloat16),
+                                   segment_ids=256 if packed else None, flags=_lib.BWD_NO_SPLIT)
+        ws = torch.empty(_lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device="cuda")
+        out, lse = ops.flash_fwd(*x[:3], **kw)
+        return ops.flash_bwd(*x[:3], out, lse, x[3], buffers=(*(torch.empty_like(y) for y in x[:3]), ws), **kw)
+
+    whole = grads(slice(0, b))
+    for i in range(b):
+        for name, got, want in zip(("dq", "dk", "dv"), whole, grads(slice(i, i + 1))):
+            assert torch.equal(got[i], want[0]), (name, i)
