@@ -475,10 +475,12 @@ static size_t planes_bytes(const AxlFlashBwdParams& p) {
 // of the CUs; where their lengths differ (causal, one key block each) they even out to the mean.  (With the mean for equal ones
 // too, unmasked calls were cut in two that then took two rounds, batch 6, 8 / 1 heads, 3328 tokens: 592 us unsplit, 664 in two, 489 in
 // three, at 64: 414 / 436 / 304; batch 12, 1024 tokens: 186 unsplit, 154 in three, 114 in two.)  The split is taken where the
-// longest workgroup walks kSplitTiles or more and this estimate falls by a sixth.  kSplitTiles was set where
-// about 200 us of host work, a training step of one layer alone, no longer hide the kernel.  The kernels gain below it too (dK/dV
-// unsplit / split with the sum, causal: batch 1, 8 / 2 heads, 1024 tokens 133 / 35 us; 16 / 8 heads 77 / 38; 4 / 4 heads, 4096 tokens
-// 124 / 63; batch 2, 16 / 8 heads, 1024 tokens 78 / 51), which a caller that runs ahead of the GPU would see.  The costs per tile are the plain
+// longest workgroup walks kSplitTiles or more and this estimate falls by a sixth.  Below kSplitTiles the
+// kernels gain too (dK/dV unsplit / split with the sum, causal: batch 1, 8 / 8 heads, 1280 tokens 56 / 36 us, 40 tiles; batch 2,
+// 32 / 8 heads, 384 tokens 50 / 33, 64 tiles), but there the forward and the whole backward take no more than the 100 us in which
+// a training step of one layer is called, and a caller would only pay for the launch; above it they take longer (batch 1, 64 / 8 heads,
+// 256 tokens, 96 tiles: backward 111 / 42 us; batch 5, 8 / 1 heads, 512 tokens, window 256 with an fp32 bias: 138 / 55 us; batch 3,
+// 12 / 4 heads, 1024 tokens: 136 / 77 us).  The costs per tile are the plain
 // form's; fp32 biases, dropout masks and both take up to 1.5 us, and every form gains (ten forms with and without documents at 12
 // shapes, both widths, dS stored and not: 1.28 to 13.4 times).  Causal, bf16, dK/dV without / with the split
 // and the sum: batch 1, 8 / 1 heads, 4096 tokens 840 / 91 + 14 us; 64 / 8 heads, 1024 tokens 253 / 63 + 10 us; 32 / 8
@@ -487,7 +489,7 @@ static size_t planes_bytes(const AxlFlashBwdParams& p) {
 struct DkdvPlan {
   int kb_per_wg, splits;
 };
-constexpr int kSplitTiles = 128, kMaxSplits = 32, kMaxSplitBlocks = 512;
+constexpr int kSplitTiles = 84, kMaxSplits = 32, kMaxSplitBlocks = 512;
 static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind, int64_t q_off, int max_splits) {
   // Two key blocks per workgroup under a causal mask, where a block and its mirror image see
   // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
