@@ -25,16 +25,27 @@ heads to make them divisible by a mesh axis, so it is the identity here.
 from __future__ import annotations
 
 import dataclasses
+import logging
 from typing import Any, Callable, Optional
 
 import torch
 
+from axlearn_amd import _host
 from axlearn_amd.attention_bias import BaseAttentionBias
 from axlearn_amd.config import Configurable, config_class
+from axlearn_amd.flash_attention import utils
+from axlearn_amd.flash_attention.hip_attention import HipFlashAttention, _attend
+from axlearn_amd.flash_attention.hip_decoding import HipDecoding, HipPagedAttention
 from axlearn_amd.flash_attention.utils import flash_attention_implementation
 from axlearn_amd.kv_cache import BaseKVCache
 
 Tensor = torch.Tensor
+
+
+def _usual_dispatch(backend: str) -> bool:
+    """Whether the dispatch of `backend` is the one that `_host.attend` stands for, and says nothing about its choice."""
+    return (backend == "gpu" and utils.BACKENDS.get("gpu") == [HipDecoding, HipFlashAttention]
+            and utils.PAGED_ATTN_BACKENDS.get("gpu") == [HipPagedAttention] and not logging.root.isEnabledFor(logging.INFO))
 
 
 class FlashAttention(Configurable):
@@ -74,8 +85,20 @@ class FlashAttention(Configurable):
         request (layer.py:278-285).  This package computes nothing outside its HIP kernels: without a
         fallback such a request raises."""
         cfg = self._config  # read only: no copy per call
-        attention_logit_biases = attention_logit_biases.astype(q_proj.dtype)
         softmax_scale = cfg.softmax_scale if cfg.softmax_scale is not None else 1.0
+        if not (is_training and cfg.dropout_rate) and _usual_dispatch(cfg.backend):
+            # the calls that need nothing but their own tensors, in native code; the others as written out below
+            native = _host.attend(q_proj, k_proj, v_proj, attention_logit_biases, page_indices, kv_cache_type, logit_sink,
+                                  softmax_scale, cfg.gpu_block_size or 128)
+            if native is not None:
+                if native[0] is not None:
+                    return native
+                if not cfg.backend_overrides:
+                    _, output_probs, mask_kind, window, segment_ids, dense = native
+                    outputs = _attend(q_proj, k_proj, v_proj, segment_ids, softmax_scale, mask_kind, window, logit_sink,
+                                      bias=dense, copy_bias=dense is not None)
+                    return outputs, output_probs
+        attention_logit_biases = attention_logit_biases.astype(q_proj.dtype)
         flash_specs = flash_attention_implementation(
             backend=cfg.backend,
             query=q_proj,

@@ -49,7 +49,10 @@ def paged_extend_step(k_pages, v_pages, page_indices, *, k_proj, v_proj, key_pos
     """The pool update of `PagedKVCache.extend_step` (paged_kv_cache.py:183-240) for one decode step:
     k_proj, v_proj [batch, 1, num_heads, head_dim] are cast to the pool dtype and written at
     key_positions [batch or 1, 1]; both pools are updated by one kernel launch, in place."""
-    from axlearn_amd import ops
+    from axlearn_amd import _host, ops
+
+    if _host.page_insert(k_pages, v_pages, k_proj, v_proj, page_indices, key_positions):
+        return k_pages, v_pages
 
     if k_proj.shape != v_proj.shape:
         raise ValueError(f"{k_proj.shape=} != {v_proj.shape=}")

@@ -12,7 +12,7 @@ from typing import Optional, Tuple
 
 import torch
 
-from axlearn_amd import _lib
+from axlearn_amd import _host, _lib
 from axlearn_amd._lib import (
     MASK_CAUSAL,
     MASK_NONE,
@@ -171,6 +171,10 @@ def flash_fwd(
     (True = dropped) with dropout_rate: kept probabilities are scaled by 1 / (1 - rate).
     bias_copy: a tensor like the bias that receives the elements of it that the mask leaves visible, where
     `can_copy_bias` says so (with q_pos_offsets a bias that the batch shares is refused: each sequence sees keys of its own)."""
+    if return_lse and dropout_mask is None and not dropout_rate and q_pos_offsets is None and q_pos_offset == 0:
+        result = _host.flash_fwd(q, k, v, segment_ids, logit_sink, softmax_scale, mask_kind, sliding_window, bias, bias_copy)
+        if result is not None:
+            return result
     b, t, hq, d, s, hkv = _check_qkv(q, k, v)
     _check_segment_ids(segment_ids, b, t, s)
     if bias_copy is not None:
@@ -277,6 +281,13 @@ def flash_bwd(
     `default_bwd_workspace_limit`, a sixteenth of the device's memory), whole or in slices of kv
     heads that still fill the GPU.  A workspace that there is no room for (on the device, or in `buffers`) gives
     way to a smaller one as `_bwd_workspace` says."""
+    if (phases == 7 and buffers is None and ds_workspace is None and dropout_mask is None and not dropout_rate
+            and q_pos_offset == 0):
+        limit = ds_workspace_limit if ds_workspace_limit is not None else default_bwd_workspace_limit(q.device)
+        result = _host.flash_bwd(q, k, v, out, lse, d_out, segment_ids, logit_sink, softmax_scale, mask_kind, sliding_window,
+                                 limit, bias)
+        if result is not None:
+            return result
     b, t, hq, d, s, hkv = _check_qkv(q, k, v)
     _check_segment_ids(segment_ids, b, t, s)
     by_size = ds_workspace is None
