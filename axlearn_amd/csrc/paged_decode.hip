@@ -24,7 +24,8 @@
 //     of the second, so probabilities never leave registers;
 //   * each run inside one (sequence, kv head) yields one partial record (o, m, l) in an fp32
 //     workspace (the reference stores partial o in the query dtype, gpu_paged_attention.py:272)
-//     and a second small kernel merges the records of a (sequence, kv head) in context order.
+//     and a second small kernel merges the records of a (sequence, kv head) in context order; short
+//     calls do without it, the last workgroup of a pair merges them (finish_pairs).
 // Work is handed out by timing, so the grouping of the fp32 partial sums - not the set of keys -
 // can differ between two calls; the AXL_DECODE_DETERMINISTIC flag of the call (or
 // AXL_DECODE_DETERMINISTIC=1 in the environment, read once, as the default for every call) selects
@@ -34,7 +35,10 @@
 // position is length-1, so a sliding window w also masks keys with (length-1) - j > w.  A page
 // index outside the pool reads as zeros and a negative one counts from the end of the pool, as the
 // reference's gather does (kv_cache/paged_kv_cache.py:32).
+#include <algorithm>
+#include <atomic>
 #include <mutex>
+#include <random>
 
 #include "common.h"
 
@@ -75,6 +79,8 @@ struct DecArgs {
   int even;                    // equal shares of the live tiles instead of blocks (see the head of this file)
   int n_wg;                    // ... over this many workgroups
   int min_share;               // ... of at least this many tiles
+  uint64_t call_id;            // ... of the split kernel that merges its records itself (finish_pairs; else 0)
+  uint64_t* ws_flag;           // ... [records]: call_id once the record is complete
 };
 
 // Tokens per tile: the unit the kernels stream and compute on.  A pool page of 16 << page_shift
@@ -157,7 +163,157 @@ struct DecTile {
   static constexpr int LDS_BYTES = NEXT_BASE + 16;
   static constexpr int RED_O_PITCH = D + 4;              // floats per (wave, head) row of the epilogue
   static_assert(4 * GP * RED_O_PITCH * 4 <= RING_BYTES, "epilogue staging must fit in the ring");
+  static_assert(256 * 24 <= RING_BYTES, "a merge's exchange must fit in the ring");
 };
+
+// Partial results between workgroups: written and read past the XCD's own L2 where another workgroup of the same
+// launch reads them (DEVICE; the L2s are not coherent inside a launch), else as everything is.
+template <bool DEVICE>
+__device__ __forceinline__ float read_record(const float* p) {
+  if constexpr (DEVICE) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return *p;
+}
+template <bool DEVICE>
+__device__ __forceinline__ float4 read_record4(const float* p) {
+  if constexpr (DEVICE) {
+    union { unsigned long long u[2]; float4 f; } x;
+    x.u[0] = __hip_atomic_load((const unsigned long long*)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    x.u[1] = __hip_atomic_load((const unsigned long long*)p + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return x.f;
+  } else {
+    return *(const float4*)p;
+  }
+}
+__device__ __forceinline__ void write_record(float* p, float x, bool device) {
+  if (device) __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = x;
+}
+
+// The threads' partial sums in a merge, with their maxima and row sums.
+template <int NT>
+struct MergeLds {
+  float4 part[NT];
+  float m[NT], l[NT];
+};
+
+constexpr int kMergeBatch = 8;   // records in flight per thread
+
+// Merges `nl` records of pair (b, hv), the i-th of them record_of(i), in that order, by NT threads: the result.
+template <typename E, int D, int GP, int NT, bool DEVICE, typename F>
+__device__ __forceinline__ void merge_records(const DecArgs& a, int b, int hv, int nl, F record_of, MergeLds<NT>& lds, int tid) {
+  // Output: G*D floats = n4 groups of four.  With fewer groups than threads the records are dealt
+  // to `ways` slices of threads (record ci to slice ci % ways), kBatch of them in flight per thread,
+  // and the slices' partial results are merged in slice order.
+  constexpr int kBatch = kMergeBatch;
+  const float c = a.scale * kLog2e;
+  const int hk = hv / a.ngrp, grp = hv - hk * a.ngrp;
+  const int gcount = min(16, a.G - 16 * grp);   // query heads of this group
+  const int hbase = hk * a.G + 16 * grp;
+  const int n4 = gcount * D / 4;
+  const int per = min(n4, NT);
+  const int ways = NT / per;
+  for (int base = 0; base < n4; base += per) {
+    const int way = tid / per, col = base + tid % per;
+    const bool live = way < ways && col < n4;
+    const int gq = live ? (4 * col) / D : 0;
+    float4 acc = {0.f, 0.f, 0.f, 0.f};
+    float m = kNegInf, l = 0.f;
+    if (live) {
+      for (int c0 = way; c0 < nl; c0 += kBatch * ways) {
+        float4 o[kBatch];
+        float mb[kBatch], lb[kBatch];
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) {
+          // past the end: the batch's first record again, with a weight of zero
+          const int ci = c0 + i * ways;
+          const int64_t r = record_of(ci < nl ? ci : c0);
+          o[i] = read_record4<DEVICE>(a.ws_o + r * (GP * D) + 4 * col);
+          mb[i] = read_record<DEVICE>(a.ws_m + r * GP + gq);
+          lb[i] = read_record<DEVICE>(a.ws_l + r * GP + gq);
+        }
+        float mn = m;
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) mn = fmaxf(mn, mb[i]);
+        const float f0 = fast_exp2((m - mn) * c);
+        acc.x *= f0; acc.y *= f0; acc.z *= f0; acc.w *= f0;
+        l *= f0;
+        m = mn;
+#pragma unroll
+        for (int i = 0; i < kBatch; i++) {
+          if (c0 + i * ways < nl) {
+            const float f = fast_exp2((mb[i] - mn) * c);
+            acc.x += o[i].x * f; acc.y += o[i].y * f; acc.z += o[i].z * f; acc.w += o[i].w * f;
+            l += lb[i] * f;
+          }
+        }
+      }
+    }
+    if (base > 0) __syncthreads();  // the exchange of the previous pass has been read
+    lds.part[tid] = acc;
+    lds.m[tid] = m;
+    lds.l[tid] = l;
+    __syncthreads();
+    if (live && way == 0) {
+      float mw = m;
+      for (int w = 1; w < ways; w++) mw = fmaxf(mw, lds.m[w * per + tid]);
+      const float f0 = fast_exp2((m - mw) * c);
+      acc.x *= f0; acc.y *= f0; acc.z *= f0; acc.w *= f0;
+      l *= f0;
+      for (int w = 1; w < ways; w++) {
+        const float4 p = lds.part[w * per + tid];
+        const float f = fast_exp2((lds.m[w * per + tid] - mw) * c);
+        acc.x += p.x * f; acc.y += p.y * f; acc.z += p.z * f; acc.w += p.w * f;
+        l += lds.l[w * per + tid] * f;
+      }
+      // An empty context (length 0, or no key inside the window) has no record: the output is zeros,
+      // as with the reference's o / (l + eps) (gpu_decoding.py:282, gpu_paged_attention.py:291-293).
+      const float inv = l > 0.f ? 1.f / l : 0.f;
+      const int dcol = 4 * col - gq * D;   // column inside the head: the ones past head_dim are padding
+      const int64_t at = ((int64_t)b * a.Hq + hbase + gq) * a.d_real + dcol;
+      if (dcol < a.d_real) {
+        if constexpr (std::is_same_v<E, ElemF32>) {
+          *(float4*)((float*)a.out + at) = float4{acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
+        } else {
+          union { bf16x2 p[2]; uint2 u; } pk;
+          pk.p[0] = E::pack(acc.x * inv, acc.y * inv);
+          pk.p[1] = E::pack(acc.z * inv, acc.w * inv);
+          *(uint2*)(a.out + at) = pk.u;
+        }
+      }
+    }
+  }
+}
+
+// Equal shares, merged by the split kernel itself (MERGE): the workgroup calls this with the (at most two) pairs of which
+// it left a record, after its threads' record stores.  It marks its records as complete and merges a pair whose records all
+// are: of the workgroups of a pair the last one to mark finds all the others' marks, for a mark is at the memory that
+// all XCDs share before the marks are read.  (Two that mark at the same time may both find all: they store the same bits.)
+// A mark is the number of the call, which no workspace can hold from before, so nothing has to be zeroed; a captured launch, which
+// is replayed with its number, takes the merge kernel (launch_common).  Saves that kernel and its launch: decode of one sequence of 1024
+// tokens, 8 heads, 12.6 -> 11.0 us, 4 sequences in 128-token pages under a window of 1024, 8 heads of 64, with their page insert
+// 19.6 -> 18.0.
+template <typename E, int D, int GP>
+__device__ __forceinline__ void finish_pairs(const DecArgs& a, const int* pfx, const int* lens, int unit, int share,
+                                             const int (&pairs)[2], int n_pairs, MergeLds<256>& lds, int tid) {
+  wait_vmem_le<0>();   // this thread's records are complete
+  __syncthreads();
+  if (tid < n_pairs)
+    __hip_atomic_store(&a.ws_flag[blockIdx.x + pairs[tid]], a.call_id, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  wait_vmem_le<0>();
+  __syncthreads();
+  for (int i = 0; i < n_pairs; i++) {
+    const int pair = i == 0 ? pairs[0] : pairs[1], b = pair / a.Hv, hv = pair - b * a.Hv;
+    int u0, u1;
+    live_units(a, lens[b], unit, u0, u1);
+    const int first = pfx[b] * a.Hv + hv * (u1 - u0);
+    const int w0 = first / share, n = (first + u1 - u0 - 1) / share - w0 + 1;   // its workgroups, at most kMaxChunks
+    bool done = true;
+    if (tid < n) done = __hip_atomic_load(&a.ws_flag[w0 + tid + pair], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == a.call_id;
+    if (!__syncthreads_and(done)) continue;
+    merge_records<E, D, GP, 256, true>(a, b, hv, n, [&](int j) { return w0 + j + pair; }, lds, tid);
+    __syncthreads();
+  }
+}
 
 // Split-K kernel.  Per page a wavefront computes
 //   S^T = K Q^T     (v_mfma_f32_16x16x32_bf16, A = K rows from LDS, B = Q^T held in registers),
@@ -165,7 +321,10 @@ struct DecTile {
 // in the "transposed" form where lane l owns query head l%16 and the tokens 4*(l/16)..+3 of the
 // page: the accumulator layout of S^T is exactly the B-operand layout of the second product, so
 // probabilities never leave registers, and every softmax statistic is per lane.
-template <typename E, int D, int GP, bool PAGED, int NST, bool BIAS>
+//
+// MERGE: equal shares, whose records the kernel merges itself.  A form of its own: as a run-time branch it cost the long calls, which
+// draw their blocks, 1.3 us (5 sequences of up to 13568 tokens, 32 heads, 128.9 -> 130.5 us).
+template <typename E, int D, int GP, bool PAGED, int NST, bool BIAS, bool MERGE>
 __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   using Tile = DecTile<D, GP, NST>;
   constexpr int KSTEPS = D / 32;        // MFMA k-steps over head_dim for S^T
@@ -261,6 +420,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   int* s_page = s_next + 3;  // next page of the segment to hand to a wavefront
   if (tid == 0) *s_page = 4 * NST;
   __syncthreads();
+  int merge_pairs[2] = {0, 0}, n_merge = 0;   // pairs of which this workgroup leaves a record
   int run_e = blockIdx.x * run0;
   int run_end = min(run_e + run0, n_blocks);
   int handed = n_wg * run0;  // estimate of how many blocks have been handed out
@@ -557,7 +717,7 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   } else {
     for (int idx = tid; idx < GP * D; idx += 256) {
       const int gq = idx / D, d = idx % D;
-      out_ws[idx] = red_o[gq][d] + red_o[GP + gq][d] + red_o[2 * GP + gq][d] + red_o[3 * GP + gq][d];
+      write_record(out_ws + idx, red_o[gq][d] + red_o[GP + gq][d] + red_o[2 * GP + gq][d] + red_o[3 * GP + gq][d], MERGE);
     }
   }
   if (!whole && tid < GP) {
@@ -565,8 +725,12 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
     float lw = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; w++) lw += red_l[w][tid] * fast_exp2((red_m[w][tid] - mw) * c);
-    a.ws_m[slot * GP + tid] = mw;
-    a.ws_l[slot * GP + tid] = lw;
+    write_record(a.ws_m + slot * GP + tid, mw, MERGE);
+    write_record(a.ws_l + slot * GP + tid, lw, MERGE);
+  }
+  if (MERGE && !whole) {
+    merge_pairs[n_merge > 0] = b * a.Hv + hv;
+    n_merge++;
   }
   // Table entries of the segment's chunks: the record at its first chunk, "none" at the others.
   for (int i = tid; i < seg && !a.even; i += 256) a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + cl + i] = i == 0 ? (int)slot : -1;
@@ -581,6 +745,17 @@ __global__ __launch_bounds__(256) void decode_split_kernel(const DecArgs a) {
   handed = run_e + s_next[1];
   __syncthreads();  // s_next is rewritten at the end of the next run
   }  // runs
+  if constexpr (MERGE) {
+    if (blockIdx.x == 0 && tid == 0) a.ticket[0] = 0;   // as the merge kernel leaves it
+    // Pairs without a live key belong to no workgroup.
+    for (int pair = blockIdx.x; pair < a.B * a.Hv; pair += n_wg) {
+      const int b = pair / a.Hv;
+      int t0, t1;
+      live_tiles(a, lens[b], t0, t1);
+      if (t0 == t1) merge_records<E, D, GP, 256, true>(a, b, pair - b * a.Hv, 0, [](int) { return 0; }, *(MergeLds<256>*)smem, tid);
+    }
+    if (n_merge > 0) finish_pairs<E, D, GP>(a, pfx, lens, unit, share, merge_pairs, n_merge, *(MergeLds<256>*)smem, tid);
+  }
 }
 
 // Zeroes the work counter ahead of the split kernel when the workspace comes with unknown contents
@@ -598,17 +773,13 @@ __global__ __launch_bounds__(64) void decode_plan_kernel(int* ticket) {
 // that after the list of records there is one round trip and one exchange through LDS (statistics first, then
 // weights, then slices: three round trips and eight barriers).  8 x 8 pairs of 8 records 7.4 -> 5.3 us, 64 x 8 pairs of
 // up to 64 records 17.2 -> 12.0 us.
-template <typename E, int D, int GP>
-__global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
+template <typename E, int D, int GP, int NT>
+__global__ __launch_bounds__(NT) void decode_combine_kernel(const DecArgs a) {
   __shared__ int s_raw[kMaxChunks];       // the record table row
   __shared__ int s_list[kMaxChunks];      // records of this (sequence, kv head), in chunk order
   __shared__ int s_count;
-  __shared__ float4 s_part[256];          // the threads' partial sums, with their maxima and row sums
-  __shared__ float s_pm[256], s_pl[256];
+  __shared__ MergeLds<NT> lds;
   const int hv = blockIdx.x, b = blockIdx.y;
-  const int hk = hv / a.ngrp, grp = hv - hk * a.ngrp;
-  const int gcount = min(16, a.G - 16 * grp);   // query heads of this group
-  const int hbase = hk * a.G + 16 * grp;
   const int tid = threadIdx.x;
   const int len = length_of(a, b);
   int ch0, ch1;
@@ -616,11 +787,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
   int nc = ch1 - ch0;                     // live chunks = upper bound on records of this (b, hk)
   // The split kernel has finished: leave the work counter at zero for the next call on this workspace.
   if (hv == 0 && b == 0 && tid == 0) a.ticket[0] = 0;
-  const float c = a.scale * kLog2e;
   if (a.even) {
     // Where the pair's units lie in the list says which workgroups took them.
     int before[2] = {0, 0}, all[2] = {0, 0};   // of blocks, of tiles
-    for (int i = tid; i < a.B; i += 256) {
+    for (int i = tid; i < a.B; i += NT) {
       const int l = length_of(a, i);
 #pragma unroll
       for (int k = 0; k < 2; k++) {
@@ -630,7 +800,8 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
         before[k] += i < b ? u1 - u0 : 0;
       }
     }
-    __shared__ int s_sum[4][4];
+    constexpr int W = NT / 64;
+    __shared__ int s_sum[4][W];
 #pragma unroll
     for (int k = 0; k < 2; k++) {
 #pragma unroll
@@ -644,11 +815,16 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
       }
     }
     __syncthreads();
-    auto sum4 = [&](int k) { return s_sum[k][0] + s_sum[k][1] + s_sum[k][2] + s_sum[k][3]; };
-    const EvenPlan p = even_plan(a, sum4(2) * a.Hv, sum4(3) * a.Hv);
+    auto sum = [&](int k) {
+      int x = 0;
+#pragma unroll
+      for (int w = 0; w < W; w++) x += s_sum[k][w];
+      return x;
+    };
+    const EvenPlan p = even_plan(a, sum(2) * a.Hv, sum(3) * a.Hv);
     live_units(a, len, p.unit, ch0, ch1);
     nc = ch1 - ch0;
-    const int first = sum4(p.unit == 1 ? 1 : 0) * a.Hv + hv * nc;
+    const int first = sum(p.unit == 1 ? 1 : 0) * a.Hv + hv * nc;
     const int w0 = first / p.share, w1 = nc > 0 ? (first + nc - 1) / p.share : w0 - 1;
     if (w0 == w1) return;                 // one workgroup had all of it and stored the result
     const int n = min(w1 - w0 + 1, kMaxChunks);
@@ -656,7 +832,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
     if (tid == 0) s_count = n;
   } else {
   // The whole table row in one round trip, then compacted in chunk order by one wavefront.
-  s_raw[tid] = tid < nc ? a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + tid] : -1;
+  if (tid < kMaxChunks) s_raw[tid] = tid < nc ? a.ws_tab[((int64_t)b * a.Hv + hv) * a.nch + tid] : -1;
   __syncthreads();
   if (tid < 64) {
     int count = 0;
@@ -670,84 +846,7 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(const DecArgs a) {
   }
   }
   __syncthreads();
-  const int nl = s_count;
-  // Output: G*D floats = n4 groups of four.  With fewer groups than threads the records are dealt
-  // to `ways` slices of threads (record ci to slice ci % ways), kBatch of them in flight per thread,
-  // and the slices' partial results are merged in slice order.
-  constexpr int kBatch = 8;
-  const int n4 = gcount * D / 4;
-  const int per = min(n4, 256);
-  const int ways = 256 / per;
-  for (int base = 0; base < n4; base += per) {
-    const int way = tid / per, col = base + tid % per;
-    const bool live = way < ways && col < n4;
-    const int gq = live ? (4 * col) / D : 0;
-    float4 acc = {0.f, 0.f, 0.f, 0.f};
-    float m = kNegInf, l = 0.f;
-    if (live) {
-      for (int c0 = way; c0 < nl; c0 += kBatch * ways) {
-        float4 o[kBatch];
-        float mb[kBatch], lb[kBatch];
-#pragma unroll
-        for (int i = 0; i < kBatch; i++) {
-          // past the end: the batch's first record again, with a weight of zero
-          const int ci = c0 + i * ways;
-          const int64_t r = s_list[ci < nl ? ci : c0];
-          o[i] = *(const float4*)(a.ws_o + r * (GP * D) + 4 * col);
-          mb[i] = a.ws_m[r * GP + gq];
-          lb[i] = a.ws_l[r * GP + gq];
-        }
-        float mn = m;
-#pragma unroll
-        for (int i = 0; i < kBatch; i++) mn = fmaxf(mn, mb[i]);
-        const float f0 = fast_exp2((m - mn) * c);
-        acc.x *= f0; acc.y *= f0; acc.z *= f0; acc.w *= f0;
-        l *= f0;
-        m = mn;
-#pragma unroll
-        for (int i = 0; i < kBatch; i++) {
-          if (c0 + i * ways < nl) {
-            const float f = fast_exp2((mb[i] - mn) * c);
-            acc.x += o[i].x * f; acc.y += o[i].y * f; acc.z += o[i].z * f; acc.w += o[i].w * f;
-            l += lb[i] * f;
-          }
-        }
-      }
-    }
-    if (base > 0) __syncthreads();  // the exchange of the previous pass has been read
-    s_part[tid] = acc;
-    s_pm[tid] = m;
-    s_pl[tid] = l;
-    __syncthreads();
-    if (live && way == 0) {
-      float mw = m;
-      for (int w = 1; w < ways; w++) mw = fmaxf(mw, s_pm[w * per + tid]);
-      const float f0 = fast_exp2((m - mw) * c);
-      acc.x *= f0; acc.y *= f0; acc.z *= f0; acc.w *= f0;
-      l *= f0;
-      for (int w = 1; w < ways; w++) {
-        const float4 p = s_part[w * per + tid];
-        const float f = fast_exp2((s_pm[w * per + tid] - mw) * c);
-        acc.x += p.x * f; acc.y += p.y * f; acc.z += p.z * f; acc.w += p.w * f;
-        l += s_pl[w * per + tid] * f;
-      }
-      // An empty context (length 0, or no key inside the window) has no record: the output is zeros,
-      // as with the reference's o / (l + eps) (gpu_decoding.py:282, gpu_paged_attention.py:291-293).
-      const float inv = l > 0.f ? 1.f / l : 0.f;
-      const int dcol = 4 * col - gq * D;   // column inside the head: the ones past head_dim are padding
-      const int64_t at = ((int64_t)b * a.Hq + hbase + gq) * a.d_real + dcol;
-      if (dcol < a.d_real) {
-        if constexpr (std::is_same_v<E, ElemF32>) {
-          *(float4*)((float*)a.out + at) = float4{acc.x * inv, acc.y * inv, acc.z * inv, acc.w * inv};
-        } else {
-          union { bf16x2 p[2]; uint2 u; } pk;
-          pk.p[0] = E::pack(acc.x * inv, acc.y * inv);
-          pk.p[1] = E::pack(acc.z * inv, acc.w * inv);
-          *(uint2*)(a.out + at) = pk.u;
-        }
-      }
-    }
-  }
+  merge_records<E, D, GP, NT, false>(a, b, hv, s_count, [&](int i) { return s_list[i]; }, lds, tid);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -936,11 +1035,22 @@ static int64_t capacity_tiles(int tiles, int window) {
 // (a query may leave it out): with one there are no more tiles, in shares of 8 or more.
 static size_t even_ws_bytes(int64_t pairs, int tiles, int gp, int width) {
   const int64_t wgs = (pairs * tiles + 7) / 8, slots = 2 * (int64_t)cu_count();
-  return ws_bytes(1, 1, (int)((wgs < slots ? wgs : slots) + pairs), gp, width);
+  const int records = (int)((wgs < slots ? wgs : slots) + pairs);
+  return ws_bytes(1, 1, records, gp, width) + (size_t)records * sizeof(uint64_t);   // behind the table, which is not used: flags
 }
 // The workgroups' records must not push a call whose blocks fit it past the buffer of axl_paged_decode_static
 // (thousands of pairs of a block each; blocks are drawn there).
 static bool even_fits(size_t even, size_t drawn) { return even <= drawn || even <= AXL_PAGED_DECODE_STATIC_MAX_BYTES; }
+
+// The split kernel merges the records itself (finish_pairs) where its workgroups are short and a pair's records are a
+// round or two of loads: the marks and the records' way past the L2 take 1.5 us more there than in a kernel of its own, which costs 3 us
+// and its launch; 4 us and more where the memory system is loaded, and one workgroup of 256 threads is slow with many
+// records.  (Call, own kernel / by the split kernel: 420 tiles in shares of 8, 9 records 12.9 / 11.0 us; 10 280 tiles in shares of 20
+// 25.1 / 24.1; 9552 in 20, 31 records 21.9 / 21.1; 16 384 in 36 30.4 / 32.5; 8 sequences of 2000 to 8190 tokens, shares of 64,
+// 40.6 / 42.1; shares of 8, 39 records of 8 heads 25.1 / 29.8.)  The kernel of its own takes 1024 threads from four rounds on
+// (108 records of 8 heads 24.0 -> 18.8 us, 240 40.2 -> 26.6, 8 pairs of 65 65.8 -> 60.5; with few records, or hundreds of
+// pairs of them, it would lose 1 to 3 us).
+constexpr int kMergeShare = 24, kMergeRounds = 2, kManyRounds = 4, kManyThreads = 1024;
 
 // Equal shares (see the head of this file) where the capacity makes them at most 256 tiles, the page ids a
 // segment keeps in registers.  Measured at 8 sequences of 2000 to 8190 tokens, 8 kv heads (40 tiles a
@@ -948,7 +1058,7 @@ static bool even_fits(size_t even, size_t drawn) { return even <= drawn || even 
 // equal shares, and the call is two launches instead of three; at 64 sequences of up to 32768 tokens (1024
 // tiles a workgroup) drawing is 4 % faster.  Fills in the launch's part of `a`; a.B, a.Hv, a.pps, a.window
 // and a.nch are set.
-static void plan_even(DecArgs& a, bool deterministic) {
+static void plan_even(DecArgs& a, bool deterministic, int& merge_rounds, bool& merge_here) {
   const int64_t pair = capacity_tiles(a.pps, a.window), total = pair * a.B * a.Hv;
   const int slots = 2 * cu_count();
   // at least 8 tiles (one round of the wavefronts' rings: a shorter share ends no sooner), and few enough
@@ -958,11 +1068,19 @@ static void plan_even(DecArgs& a, bool deterministic) {
   a.n_wg = (int)(total < (int64_t)slots * a.min_share ? (total + a.min_share - 1) / a.min_share : slots);
   const int64_t share = ((total + a.n_wg - 1) / a.n_wg + 3) & ~(int64_t)3;
   a.even = a.B <= kMaxBatch && share <= 256 && a.min_share <= 256;
+  // records a pair can have, by equal shares or a block each, and the rounds of loads in which 256 threads merge them
+  const int64_t records = std::max((pair + share - 1) / share + 1, std::min<int64_t>(pair / a.chunk_pages + 2, a.n_wg));
+  merge_rounds = (int)((records * std::min(a.G, 16) * width_of(a.d_real) / 4 + kMergeBatch * 256 - 1) / (kMergeBatch * 256));
+  merge_here = !a.bias && share <= kMergeShare && merge_rounds <= kMergeRounds;
   // A deterministic call keeps to the blocks, whose bits depend on a pair's own keys alone: equal shares only
   // where the shapes leave no more blocks than workgroups.
   if (deterministic && (int64_t)a.B * a.Hv * a.nch > a.n_wg) a.even = 0;
   const int gp = gp_of(a.G, a.bias != nullptr), width = width_of(a.d_real);
   if (!even_fits(even_ws_bytes((int64_t)a.B * a.Hv, a.pps, gp, width), ws_bytes(a.B, a.Hv, a.nch, gp, width))) a.even = 0;
+  if (!a.even) {
+    merge_rounds = 1;   // runs, mostly of several blocks: few records
+    merge_here = false;
+  }
 }
 
 static size_t ws_bytes_for(int batch, int hq, int hkv, int d, int tiles, bool bias, int dtype) {
@@ -1014,6 +1132,27 @@ static bool deterministic_by_default() {
   return v;
 }
 
+// A number of its own for every call of every process: marks of an earlier call, or whatever else a workspace holds, are
+// not taken for this call's.
+static uint64_t next_call_id() {
+  static std::atomic<uint64_t> next{[] {
+    std::random_device r;
+    return ((uint64_t)r() << 32) ^ r();
+  }()};
+  const uint64_t id = next.fetch_add(1, std::memory_order_relaxed);
+  return id ? id : next.fetch_add(1, std::memory_order_relaxed);
+}
+
+// Whether what is enqueued becomes part of a graph (also where that cannot be asked).
+static bool is_captured(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+    (void)hipGetLastError();
+    return true;
+  }
+  return status != hipStreamCaptureStatusNone;
+}
+
 template <typename E, bool PAGED>
 static int launch_common(DecArgs a, int flags, hipStream_t stream, const char* who) {
   const int D = width_of(a.d_real);
@@ -1031,12 +1170,16 @@ static int launch_common(DecArgs a, int flags, hipStream_t stream, const char* w
   a.ws_o += kWsHeaderFloats;
   float* ws = a.ws_o;
   a.deterministic = (flags & AXL_DECODE_DETERMINISTIC) != 0 || deterministic_by_default();
-  plan_even(a, a.deterministic);
+  int merge_rounds;
+  bool merge_here;
+  plan_even(a, a.deterministic, merge_rounds, merge_here);
   const size_t records = a.even ? (size_t)a.n_wg + (size_t)a.B * a.Hv : (size_t)a.B * a.Hv * a.nch;
   const size_t n_o = records * gp * D, n_s = records * gp;
   a.ws_m = ws + n_o;
   a.ws_l = ws + n_o + n_s;
   a.ws_tab = (int32_t*)(ws + n_o + 2 * n_s);
+  a.ws_flag = (uint64_t*)(ws + n_o + 2 * n_s);
+  a.call_id = merge_here && !is_captured(stream) ? next_call_id() : 0;
   // Two workgroups fit a CU (LDS); the split kernel is persistent and strides over its work items.
   const dim3 grid(a.even ? a.n_wg : 2 * cu_count());
   hipError_t err = hipSuccess;
@@ -1045,11 +1188,16 @@ static int launch_common(DecArgs a, int flags, hipStream_t stream, const char* w
 #define AXL_DEC(E, DD, GG, NS, BB)                                                              \
   do {                                                                                          \
     using Tile = DecTile<DD, GG, NS>;                                                           \
-    auto kern = decode_split_kernel<E, DD, GG, PAGED, NS, BB>;                                  \
+    auto kern = BB || !s.call_id ? decode_split_kernel<E, DD, GG, PAGED, NS, BB, false>         \
+                                 : decode_split_kernel<E, DD, GG, PAGED, NS, BB, !BB>;          \
     err = allow_dynamic_lds((const void*)kern, Tile::LDS_BYTES);                                \
     if (err == hipSuccess) {                                                                    \
       hipLaunchKernelGGL(kern, grid, dim3(256), Tile::LDS_BYTES, stream, s);                    \
-      hipLaunchKernelGGL((decode_combine_kernel<E, DD, GG>), cgrid, dim3(256), 0, stream, s);   \
+      if (s.call_id) break;                                                                     \
+      if (merge_rounds >= kManyRounds)                                                          \
+        hipLaunchKernelGGL((decode_combine_kernel<E, DD, GG, kManyThreads>), cgrid, dim3(kManyThreads), 0, stream, s); \
+      else                                                                                      \
+        hipLaunchKernelGGL((decode_combine_kernel<E, DD, GG, 256>), cgrid, dim3(256), 0, stream, s); \
     }                                                                                           \
   } while (0)
   // The kernels keep per-sequence tables in LDS: larger batches go in slices of kMaxBatch (each
@@ -1110,7 +1258,7 @@ static int launch_f32(DecArgs a, hipStream_t stream, const char* who) {
 #define AXL_DEC32(DD, GG)                                                                          \
   do {                                                                                              \
     hipLaunchKernelGGL((decode_split_f32_kernel<DD, GG, PAGED>), grid, dim3(256), 0, stream, a);    \
-    hipLaunchKernelGGL((decode_combine_kernel<ElemF32, DD, GG>), cgrid, dim3(256), 0, stream, a);   \
+    hipLaunchKernelGGL((decode_combine_kernel<ElemF32, DD, GG, 256>), cgrid, dim3(256), 0, stream, a); \
   } while (0)
   if (D == 128 && gp == 4) AXL_DEC32(128, 4);
   else if (D == 128 && gp == 8) AXL_DEC32(128, 8);

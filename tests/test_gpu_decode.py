@@ -900,3 +900,64 @@ def test_page_insert_of_a_layers_projections():
             ops.paged_kv_insert(pools[0], pools[1], proj, proj, tables, positions, single_row=True)
             ops.paged_kv_insert(pools[2], pools[3], proj[:, 0], proj[:, 0], tables, positions.reshape(-1))
             assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3]) and pools[0].abs().sum() > 0
+
+
+@pytest.mark.parametrize("b,hq,hkv,s,d,window,dtype", [
+    (1, 8, 8, 1024, 128, -1, torch.float16),     # a block of 8 tiles each, 8 records to a pair
+    (3, 12, 4, 8704, 64, 1024, torch.bfloat16),  # under a window, shares of 8 that end inside pairs
+    (33, 12, 4, 2003, 96, -1, torch.bfloat16),   # shares over several pairs, some held whole
+    (1, 16, 1, 700, 80, -1, torch.bfloat16),     # 16 heads: two rounds of records
+    (2, 24, 1, 500, 128, -1, torch.float16),     # two groups of heads to a kv head
+    (2, 32, 8, 9538, 128, -1, torch.bfloat16),   # 30 records of 4 heads
+    (1, 8, 1, 13728, 128, -1, torch.bfloat16),   # 108 records: a merge kernel of 1024 threads
+])
+def test_records_merged_by_the_split_kernel(b, hq, hkv, s, d, window, dtype):
+    """Short calls merge their records without a kernel of its own, except in a captured graph, whose launches are replayed
+    with their arguments: against the oracle, on a workspace of NaN patterns and on what the call before left there, some
+    sequences empty, two calls at a time on streams of their own, and replays with the inputs changed in between."""
+    gen = torch.Generator().manual_seed(7)
+    q, k, v = (torch.randn(shape, generator=gen).to(dtype) for shape in ((b, hq, d), (b, s, hkv, d), (b, s, hkv, d)))
+    lengths = torch.randint(1, s + 1, (b,), generator=gen, dtype=torch.int32)
+    lengths[0] = s
+    if b > 1:
+        lengths[-1] = 0
+    scale = d ** -0.5
+    # what the blocks of another decomposition can differ by: each rounds its probabilities and its result
+    bar = 1e-2 if dtype == torch.bfloat16 else 1.25e-3
+
+    def want(q):
+        live = lengths > 0
+        full = torch.zeros(b, hq, d, dtype=torch.float64)
+        full[live] = ref.reference_decode(q[live][:, None], k[live], v[live], lengths[live], softmax_scale=scale,
+                                          sliding_window=None if window < 0 else window)[:, 0].double()
+        return full
+
+    args = [x.cuda() for x in (q, k, v, lengths)]
+    need = 1 << 26
+    workspaces = [torch.full((need,), 0xFF, dtype=torch.uint8, device="cuda") for _ in range(3)]
+    first, other = want(q), want(-q)
+    call = lambda x, ws, **kw: ops.decode(x, *args[1:], softmax_scale=scale, sliding_window=window, workspace=ws, **kw)
+    for _ in range(3):
+        for x, exact in ((args[0], first), (-args[0], other)):
+            assert ref.rel_l2(call(x, workspaces[0]).cpu().double(), exact) <= bar
+    det = [call(args[0], ws, deterministic=True) for ws in workspaces[:2]]
+    assert torch.equal(*det) and ref.rel_l2(det[0].cpu().double(), first) <= bar
+    torch.cuda.synchronize()
+    streams, outs = [torch.cuda.Stream() for _ in range(2)], [[], []]
+    for _ in range(20):
+        for i in range(2):
+            with torch.cuda.stream(streams[i]):
+                outs[i].append(call(args[0], workspaces[i]))
+    torch.cuda.synchronize()
+    for got in outs[0] + outs[1]:
+        assert ref.rel_l2(got.cpu().double(), first) <= bar
+    x, out = args[0].clone(), torch.empty_like(args[0])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(x, workspaces[2], out=out)
+    for sign, exact in ((1, first), (-1, other), (1, first)):
+        x.copy_(sign * args[0])
+        call(x, workspaces[0])   # eager work between the replays
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ref.rel_l2(out.cpu().double(), exact) <= bar
