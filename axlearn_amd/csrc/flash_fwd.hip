@@ -177,22 +177,28 @@ __device__ __forceinline__ ChunkShare chunk_share(const FwdArgs& a, int lane, in
 // W: live width, the head_dim rounded up to a multiple of 32 (D: the width of a row in LDS).  The MFMAs and fragment
 // reads past it, whose operands or results are nothing but padding, are left out: bound by the matrix cores' power as the
 // width 128, with a quarter of their work less (B2 H32 T4096, head_dim 96 causal 272 -> 231 us, 80 unmasked 510 -> 442 us).
-template <typename E, int D, int INPUTS, int NW, bool CHUNK, int W = D>
+//
+// KS: groups of NW wavefronts that share the keys of the same NW * 32 query rows, each walking its part of them with tiles of its
+// own, and are merged at the end through LDS (flash_fwd_keys_kernel).
+template <typename E, int D, int INPUTS, int NW, bool CHUNK, int W = D, int KS = 1>
 __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // BIAS16: a bf16 bias and nothing else, known at compile time; AUX without it: whatever there is.
   constexpr bool AUX = INPUTS != kFwdPlain, COPY = INPUTS == kFwdBias16Copy, BIAS16 = INPUTS == kFwdBias16 || COPY;
   static_assert(!(AUX && CHUNK), "the chunk form takes no bias or dropout mask");
+  static_assert(KS == 1 || (KS == 2 && !AUX && !CHUNK), "two groups of wavefronts: the plain form");
   using Tile = FwdTile<D, NW>;
   constexpr int KK = W / 16;  // MFMA k-steps over head_dim
   constexpr int DT = W / 32;  // 32-row output tiles over head_dim
   constexpr int CPR = D / 8;  // 16-byte chunks per row
-  extern __shared__ __attribute__((aligned(16))) char smem[];
+  extern __shared__ __attribute__((aligned(16))) char smem_all[];
+  const int tid = threadIdx.x;
+  const int wave_all = __builtin_amdgcn_readfirstlane(tid >> 6), key_group = KS > 1 ? wave_all / NW : 0;
+  const int wave = wave_all - key_group * NW, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+  char* const smem = smem_all + key_group * Tile::LDS_BYTES;
   char* const k_lds = smem;
   char* const v_lds = smem + 2 * Tile::TILE_BYTES;
   char* const seg_lds = smem + Tile::SEG_BASE;
 
-  const int tid = threadIdx.x;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
   int qb, b, h, hk, split = 0, nsplit = 1;
   const int G = a.Hq / a.Hkv;
   if constexpr (CHUNK) {
@@ -282,7 +288,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   // all 32 queries of a wavefront carry needs no segment mask.
   __shared__ int s_tile_id[kMaxSegTiles];
   int seg_t0 = 0;          // tile that s_tile_id[0] describes
-  if (seg_k) seg_t0 = classify_segment_groups<Tile::BK, 64 * NW>(seg_q, seg_k, tid, k_begin, k_end, s_tile_id, kMaxSegTiles,
+  if (seg_k) seg_t0 = classify_segment_groups<Tile::BK, 64 * NW * KS>(seg_q, seg_k, tid, k_begin, k_end, s_tile_id, kMaxSegTiles,
                                                             kSegNotUniform);
   int t_begin = k_begin / Tile::BK;
   int t_end = (k_end + Tile::BK - 1) / Tile::BK;
@@ -290,6 +296,13 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     const int per = (t_end - t_begin + nsplit - 1) / nsplit;
     t_begin = min(t_end, t_begin + split * per);
     t_end = min(t_end, t_begin + per);
+  }
+  int idle_barriers = 0;       // of the group with fewer tiles, a barrier to a tile
+  if constexpr (KS == 2) {
+    const int first = (t_end - t_begin + 1) / 2;
+    idle_barriers = key_group == 0 ? 0 : 2 * first - (t_end - t_begin);
+    if (key_group == 0) t_end = t_begin + first;
+    else t_begin += first;
   }
   bool seg_fast = false;   // this wavefront's queries share one id and the table covers the tiles
   int wq_id = 0;
@@ -334,7 +347,7 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
   float m_run = kNegInf;  // running row max of the raw (unscaled) logits
   float l_run = 0.f;      // this lane's share of the running row sum (lanes l and l^32 split it)
   const float c = a.scale * kLog2e;
-  if (a.sink && split == 0) {
+  if (a.sink && split == 0 && key_group == 0) {
     // The sink is one more logit per row, with no value row (attention.py:608-626): it enters the
     // running softmax state as an already-processed key of weight exp(sink - m) = 1.
     m_run = a.sink[h] / a.scale;
@@ -673,12 +686,15 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
       for (int n = 0; n < NSL; n++) {
         if (n + kAhead < NSL) kfr[n + kAhead] = AXL_K_FRAG(kt, (n + kAhead) / 2, (n + kAhead) % 2);
         if constexpr (FAST) {
-          constexpr int kPairs = Tile::DMA_PER_WAVE / 2;
-          if (n % 2 == 0 && n / 2 < kPairs) issue_k_pair(t_k2, buf, n);
-          if (n % 2 == 0 && n / 2 >= kPairs && n / 2 < 2 * kPairs) issue_v_pair(t + 1, buf ^ 1, n - 2 * kPairs);
+          // a pair every second slot, or every slot where there are more than fit that way
+          constexpr int kPairs = Tile::DMA_PER_WAVE / 2, kStep = 4 * kPairs < NSL ? 2 : 1;
+          static_assert(2 * kPairs * kStep < NSL, "the loads of a tile fit its slots");
+          if (n % kStep == 0 && n / kStep < kPairs) issue_k_pair(t_k2, buf, 2 * (n / kStep));
+          if (n % kStep == 0 && n / kStep >= kPairs && n / kStep < 2 * kPairs)
+            issue_v_pair(t + 1, buf ^ 1, 2 * (n / kStep - kPairs));
           // the ids of tile t+2 for a general tile that may follow (every wavefront fetches the same
           // 256 bytes: no branch on the wavefront number inside the slot sequence)
-          if (n == 4 * kPairs && seg_k)
+          if (n == 2 * kPairs * kStep && seg_k)
             dma16s_first16(seg_off(), seg_k + t_k2 * Tile::BK, lds0 + Tile::SEG_BASE + (t_k2 % Tile::NSEG) * (Tile::BK * 4));
           // The chain in vector registers where the next tile's softmax reads it, started from a
           // literal zero: no register is cleared and none is copied.  (The 16 P V MFMAs of this tile lie
@@ -808,7 +824,36 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
 #undef AXL_S_PLAIN
 
   // Epilogue: out = acc / l ; lse = m*scale + ln(l).
-  const float l_tot = xor32_sum(l_run);
+  float l_tot = xor32_sum(l_run);
+  if constexpr (KS == 2) {
+    // The second group leaves its accumulators, maxima and sums where its tiles were, the first one takes them over.
+    constexpr int kWaveBytes = 32 * W * 4;
+    for (int i = 0; i < idle_barriers; i++) __syncthreads();
+    __syncthreads();
+    char* const part = smem_all + Tile::LDS_BYTES + wave * kWaveBytes;
+    floatx2* const stats = (floatx2*)(smem_all + Tile::LDS_BYTES + Tile::SEG_BASE) + 32 * wave + l32;
+    static_assert(NW * kWaveBytes <= Tile::SEG_BASE && NW * 256 <= Tile::LDS_BYTES - Tile::SEG_BASE, "the second group's results");
+    if (key_group == 1) {
+      if (g == 0) *stats = floatx2{m_run, l_tot};
+#pragma unroll
+      for (int i = 0; i < 4 * DT; i++)
+        *(floatx4*)(part + i * 1024 + 16 * lane) =
+            floatx4{o[i / 4][4 * (i % 4)], o[i / 4][4 * (i % 4) + 1], o[i / 4][4 * (i % 4) + 2], o[i / 4][4 * (i % 4) + 3]};
+    }
+    __syncthreads();
+    if (key_group == 1) return;
+    const floatx2 other = *stats;
+    const float mx = fmaxf(m_run, other[0]);
+    const float f0 = fast_exp2((m_run - mx) * c), f1 = fast_exp2((other[0] - mx) * c);
+    m_run = mx;
+    l_tot = l_tot * f0 + other[1] * f1;
+#pragma unroll
+    for (int i = 0; i < 4 * DT; i++) {
+      const floatx4 x = *(const floatx4*)(part + i * 1024 + 16 * lane);
+#pragma unroll
+      for (int j = 0; j < 4; j++) o[i / 4][4 * (i % 4) + j] = o[i / 4][4 * (i % 4) + j] * f0 + x[j] * f1;
+    }
+  }
   if constexpr (CHUNK) {
     if (nsplit > 1) {
       if (q0 >= chunk_rows) return;
@@ -850,6 +895,21 @@ template <typename E, int D, bool AUX, int NW = 4>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(AUX ? 1 : 2, AUX ? 1 : 2)))
 void flash_fwd_kernel(const FwdArgs a) {
   flash_fwd_body<E, D, AUX ? kFwdAux : kFwdPlain, NW, false>(a);
+}
+
+// Launches of few row blocks: workgroups of 64 rows, whose four wavefronts are two groups that share the keys.  A launch of at most
+// a workgroup of 128 rows per CU lasts as long as its longest one walks; this doubles the workgroups and halves the walk, at one
+// wavefront per SIMD as before (the same with 128 rows and eight wavefronts, two per SIMD, gained nothing below 2048
+// keys: 16.3 -> 17.6 us at 512, 66 -> 59 at 4096).  Kernel, us, causal D128 unless said, 128 rows / 64 rows and two groups: up to half as
+// many blocks of 128 rows as CUs: B1 H32 T512 16.3 / 12.4, B1 H8 T1024 22.1 / 15.9, T2048 36.0 / 25.5, D64 T512 10.4 / 8.7, window
+// 256 B2 H8 T1024 16.1 / 11.2, unmasked B1 H16 T768 19.5 / 13.9, documents B1 H8 T1536 17.3 / 13.6, three short ones D80 T384 9.1 / 8.6.
+// Up to as many as CUs two workgroups follow one another on a CU; causal, long and short walks even out: B1 H32 T1024
+// 25.0 / 24.3, B1 H16 T2048 39.5 / 33.7, B1 H8 T4096 68.7 / 53.8, D64 45.7 / 32.8 - but unmasked, under a window, with documents or
+// below 1024 keys it loses (B2 H16 T768 unmasked 20.3 / 26.0, B1 H64 T512 18.1 / 19.8).
+template <typename E, int D, int W>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void flash_fwd_keys_kernel(const FwdArgs a) {
+  flash_fwd_body<E, D, kFwdPlain, 2, false, W, 2>(a);
 }
 
 // Head dims 72 to 96 of the width 128.
@@ -1523,6 +1583,12 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
     return set_error(AXL_ERR_UNSUPPORTED, "axl_flash_fwd: bias_copy with q_pos_offsets needs a bias per sequence");
   const int width = p.head_dim <= 64 ? 64 : 128;  // the compiled width that serves this head_dim
   hipError_t err = hipSuccess;
+  const int64_t blocks = (int64_t)(p.q_len / 128) * p.batch * p.num_q_heads;
+// Launches that leave CUs idle, or a CU with one workgroup of the longest walk: flash_fwd_keys_kernel (its comment has both
+  // sides' times).  Not for rows at offsets of their own: a chunk of rows padded into blocks gives the chunk kernel's bits.
+  const bool share_keys = !aux && !p.q_pos_offsets && p.kv_len > 256 &&
+                          (2 * blocks <= cu_count() ||
+                           (blocks <= cu_count() && p.mask_kind == AXL_MASK_CAUSAL && !p.segment_ids && p.kv_len >= 1024));
 #define AXL_LAUNCH_FWD(KERNEL, TILE)                                                            \
   do {                                                                                          \
     err = allow_dynamic_lds((const void*)KERNEL, TILE::LDS_BYTES);                              \
@@ -1532,9 +1598,23 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
       err = hipGetLastError();                                                                  \
     }                                                                                           \
   } while (0)
+#define AXL_LAUNCH_FWD_KEYS(E, DD, WW)                                                          \
+  do {                                                                                          \
+    auto kernel = flash_fwd_keys_kernel<E, DD, WW>;                                             \
+    constexpr int lds = 2 * FwdTile<DD, 2>::LDS_BYTES;                                          \
+    err = allow_dynamic_lds((const void*)kernel, lds);                                          \
+    if (err == hipSuccess) {                                                                    \
+      hipLaunchKernelGGL(kernel, dim3(2 * (int)blocks), dim3(256), lds, stream, a);             \
+      err = hipGetLastError();                                                                  \
+    }                                                                                           \
+  } while (0)
 #define AXL_LAUNCH_FWD16(E)                                                                     \
   do {                                                                                          \
-    if (bias16 && p.bias_copy) {                                                                \
+    if (share_keys) {                                                                           \
+      if (width == 64) AXL_LAUNCH_FWD_KEYS(E, 64, 64);                                          \
+      else if (p.head_dim <= 96) AXL_LAUNCH_FWD_KEYS(E, 128, 96);                               \
+      else AXL_LAUNCH_FWD_KEYS(E, 128, 128);                                                    \
+    } else if (bias16 && p.bias_copy) {                                                                \
       if (width == 128) AXL_LAUNCH_FWD((flash_fwd_bias_copy_kernel<E, 128>), FwdTile<128>);    \
       else AXL_LAUNCH_FWD((flash_fwd_bias_copy_kernel<E, 64>), FwdTile<64>);                   \
     } else if (bias16) {                                                                        \

@@ -1967,6 +1967,8 @@ def test_pairs_worked_through_together_give_the_bits_of_each_sequence(b, t, hq, 
     q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, 64, torch.bfloat16))
     segs = ref.packed_segment_ids(5, b, t).cuda() if packed else None
 
+    forward = ops.flash_fwd(q, k, v, mask_kind=ops.MASK_CAUSAL, softmax_scale=0.125, segment_ids=segs)
+
     def grads(rows):
         x = [y[rows] for y in (q, k, v, do)]
         ids = None if segs is None else segs[rows]
@@ -1975,10 +1977,43 @@ def test_pairs_worked_through_together_give_the_bits_of_each_sequence(b, t, hq, 
                                    mask_kind=ops.MASK_CAUSAL, dtype=_lib.dtype_code(torch.bfloat16),
                                    segment_ids=256 if packed else None, flags=_lib.BWD_NO_SPLIT)
         ws = torch.empty(_lib.load().axl_flash_bwd_workspace_bytes(ctypes.byref(p)), dtype=torch.uint8, device="cuda")
-        out, lse = ops.flash_fwd(*x[:3], **kw)
+        out, lse = (y[rows] for y in forward)
         return ops.flash_bwd(*x[:3], out, lse, x[3], buffers=(*(torch.empty_like(y) for y in x[:3]), ws), **kw)
 
     whole = grads(slice(0, b))
     for i in range(b):
         for name, got, want in zip(("dq", "dk", "dv"), whole, grads(slice(i, i + 1))):
             assert torch.equal(got[i], want[0]), (name, i)
+
+
+@pytest.mark.parametrize("b,t,s,hq,hkv,d,dtype,mask,window,packed,offset", [
+    (1, 384, 384, 4, 2, 128, torch.bfloat16, "causal", None, False, 0),     # one to six tiles, odd numbers of them
+    (2, 512, 512, 4, 1, 64, torch.float16, "causal", None, True, 0),        # documents: ranges of one tile and of many
+    (1, 640, 640, 3, 3, 128, torch.float16, "sliding", 0, False, 0),        # two tiles at most, the second group's none or one
+    (1, 1152, 1152, 4, 4, 96, torch.bfloat16, "sliding", 300, True, 0),     # a width below the compiled one
+    (2, 768, 768, 8, 2, 72, torch.bfloat16, "none", None, False, 0),
+    (1, 128, 1024, 4, 2, 128, torch.bfloat16, "causal", None, False, 700),  # few rows behind a prefix
+    (1, 384, 1920, 2, 1, 64, torch.bfloat16, "none", None, False, 0),
+    (1, 2048, 2048, 16, 4, 128, torch.bfloat16, "causal", None, False, 0),  # as many row blocks of 128 as CUs
+    (1, 1024, 1024, 24, 8, 80, torch.float16, "causal", None, False, 0),
+])
+@pytest.mark.parametrize("sink", [False, True])
+def test_forward_of_few_row_blocks(b, t, s, hq, hkv, d, dtype, mask, window, packed, offset, sink):
+    """Launches that leave CUs idle: two groups of wavefronts share the keys of 64 rows.  out and lse against the oracle, twice
+    the same bits."""
+    q, k, v, _ = _inputs(b, t, hq, hkv, d, dtype, s=s)
+    segs = ref.packed_segment_ids(6, b, t, max_docs=5) if packed else None
+    spec, kw = _mask_args(mask, window, segs)
+    spec.target_positions, spec.source_positions = torch.arange(t)[None] + offset, torch.arange(s)[None]
+    kw.update(softmax_scale=d ** -0.5, q_pos_offset=offset)
+    more = {}
+    if sink:
+        more = dict(logit_sink=ref.normal_tensor(8, (hq,), torch.float32))
+    want, want_lse = ref.reference_mha(q, k, v, spec, softmax_scale=d ** -0.5, return_lse=True, **more)
+    kw.update({n: x.cuda() for n, x in more.items()})
+    q, k, v = (x.cuda() for x in (q, k, v))
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    _assert_close("out", out, want, dtype)
+    assert ref.max_abs(lse.cpu(), want_lse) < 1e-3 * max(1.0, float(want_lse.abs().max()))
+    again, lse2 = ops.flash_fwd(q, k, v, **kw)
+    assert torch.equal(out, again) and torch.equal(lse, lse2)
