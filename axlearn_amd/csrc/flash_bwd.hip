@@ -493,13 +493,10 @@ constexpr int kSplitTiles = 84, kMaxSplits = 32, kMaxSplitBlocks = 512;
 static DkdvPlan plan_dkdv(const AxlFlashBwdParams& p, int mask_kind, int64_t q_off, int max_splits) {
   // Two key blocks per workgroup under a causal mask, where a block and its mirror image see
   // complementary shares of the queries (an even number of blocks); AXL_DKDV_KB_PER_WG=1 in the
-  // environment (read once) keeps one block per workgroup.  Not with segment ids: documents end where they like, the
-  // two shares add up to anything, and the longer workgroups leave the longer tail (training step, two / one: B6 H32/8
-  // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; of 25 packed causal shapes none
-  // lost more than runs differ by).
+  // environment (read once) keeps one block per workgroup.
   static const bool single = [] { const char* e = getenv("AXL_DKDV_KB_PER_WG"); return e && e[0] == '1'; }();
   const int nkb = p.kv_len / 128;
-  const bool mirror = !single && mask_kind == AXL_MASK_CAUSAL && nkb % 2 == 0 && !p.segment_ids;
+  const bool mirror = !single && mask_kind == AXL_MASK_CAUSAL && nkb % 2 == 0;
   const DkdvPlan whole{mirror ? 2 : 1, 1};
   if (p.dtype == AXL_F32 || nkb < 1) return whole;
   const int64_t pairs = (int64_t)p.batch * p.num_kv_heads, blocks = pairs * nkb;
@@ -599,7 +596,13 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
   {
     // of all kv heads, whatever the slices: the same sums
     const DkdvPlan plan = plan_dkdv(p, p.mask_kind, p.q_pos_offset, max_splits(p));
-    a.kb_per_wg = plan.kb_per_wg;
+    // Unsplit, one key block per workgroup with segment ids: documents end where they like, the shares of a block and its
+    // mirror image add up to anything, and the longer workgroups leave the longer tail (training step, two / one: B6 H32/8
+    // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; of 25 packed causal shapes none
+    // lost more than runs differ by).  The choice to split looks at the mirrored form all the same: the sizes of the key blocks it
+    // weighs are those without documents (B2 H32/8 T2048 D64 packed, split / whole by the longest key block 215 / 237 us).
+    const bool one = plan.splits == 1 && p.segment_ids;
+    a.kb_per_wg = one ? 1 : plan.kb_per_wg;
     a.splits = plan.splits;
   }
   a.pair_group = dkdv_pair_group(a);
