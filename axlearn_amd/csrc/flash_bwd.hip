@@ -601,7 +601,10 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
     // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; of 25 packed causal shapes none
     // lost more than runs differ by).  The choice to split looks at the mirrored form all the same: the sizes of the key blocks it
     // weighs are those without documents (B2 H32/8 T2048 D64 packed, split / whole by the longest key block 215 / 237 us).
-    const bool one = plan.splits == 1 && p.segment_ids;
+    // One also where two workgroups share a CU, each busy in the other's gaps (head_dim 64 without a bias or dropout mask: step,
+    // two / one, B3 H8 T1024 68.1 / 60.4 us, B7 H32 T256 56.5 / 52.7, B6 H64/8 T3328 3489 / 3301, B4 H32/8 T4096 1500 / 1512).
+    const bool two_per_cu = dt != AXL_F32 && p.head_dim <= 64 && !p.aux.bias && !p.aux.dropout_mask;
+    const bool one = plan.splits == 1 && (p.segment_ids || two_per_cu);
     a.kb_per_wg = one ? 1 : plan.kb_per_wg;
     a.splits = plan.splits;
   }

@@ -881,10 +881,22 @@ __device__ __forceinline__ void flash_bwd_dkdv_body(const BwdArgs& a) {
   }  // key blocks of this workgroup
 }
 
+// At head_dim 64 two workgroups fit a CU (251 registers, 51 KB of LDS): starts and ends of key blocks, 10 us of the 60 of a short
+// one, and the waits of a tile lie under the other workgroup's loop.  dK/dV at B7 H32 T512 60.0 -> 47.7 us; training steps B4 H32/8 T4096
+// 1617 -> 1500 us, B2 H32 T2176 300 -> 271, T2048 unmasked 370 -> 343, H16 window 1024 B4 T4096 490 -> 455, B1 T16384 3015 -> 2745.
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL = false>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, D == 64 && AUX == 0 && !HAS_SEG ? 2 : 1)))
 void flash_bwd_dkdv_kernel(const BwdArgs a) {
   flash_bwd_dkdv_body<E, D, HAS_SEG, AUX, SPILL, D, false>(a);
+}
+
+// The same with segment ids, whose 275 registers do not fit twice: 1 to 14 of them spilled.  Pays for itself where a kv head has
+// one query head and there are two and a half rounds of key blocks or more, us: B4 H16 T4096 595 -> 565, T2048 unmasked 313 -> 284, T1408
+// 148 -> 138, B8 T640 112 -> 104; not with longer walks (B8 H32/8 T4096 2160 / 2218, H64/8 T2048 1382 / 1426) or fewer (B8 H8/1 T5376 1490 / 1650).
+template <typename E, bool SPILL>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_bwd_dkdv_seg64_kernel(const BwdArgs a) {
+  flash_bwd_dkdv_body<E, 64, true, 0, SPILL, 64, false>(a);
 }
 
 // Head dims 72 to 96 of the width 128.
@@ -941,14 +953,16 @@ __global__ __launch_bounds__(2 * D) void flash_bwd_dkdv_combine_kernel(const Bwd
 template <typename E, int D, bool HAS_SEG, int AUX, bool SPILL, int W, bool SPLIT>
 static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   using Tile = DkvTile<D, bias_through_lds(HAS_SEG, AUX)>;
-  auto kernel = [] {
+  const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;
+  auto kernel = [&] {
     if constexpr (SPLIT) return flash_bwd_dkdv_split_kernel<E, D, HAS_SEG, AUX, SPILL, W>;
     else if constexpr (W == 96) return flash_bwd_dkdv_w96_kernel<E, HAS_SEG, SPILL>;
+    else if constexpr (D == 64 && HAS_SEG && AUX == 0)
+      return a.Hq == a.Hkv && 2 * (int64_t)grid >= 5 * (int64_t)cu_count() ? flash_bwd_dkdv_seg64_kernel<E, SPILL> : flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
     else return flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
   }();
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
-  const int blocks = (a.S / Tile::BKV) * a.B * a.Hkv, grid = blocks / a.kb_per_wg * a.splits;
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), Tile::LDS_BYTES, stream, a);
   return hipGetLastError();
 }

@@ -2017,3 +2017,28 @@ def test_forward_of_few_row_blocks(b, t, s, hq, hkv, d, dtype, mask, window, pac
     assert ref.max_abs(lse.cpu(), want_lse) < 1e-3 * max(1.0, float(want_lse.abs().max()))
     again, lse2 = ops.flash_fwd(q, k, v, **kw)
     assert torch.equal(out, again) and torch.equal(lse, lse2)
+
+
+@pytest.mark.parametrize("b,t,h,mask,window,dtype", [
+    (5, 1024, 16, "causal", None, torch.bfloat16),    # the smallest number of key blocks
+    (9, 640, 16, "sliding", 200, torch.float16),
+    (4, 1408, 16, "none", None, torch.bfloat16),
+])
+@pytest.mark.parametrize("ds", [False, True])
+def test_dkdv_of_documents_with_two_workgroups_per_cu(b, t, h, mask, window, dtype, ds):
+    """head_dim 64, one query head per kv head, two and a half rounds of key blocks: the form with two workgroups per CU gives the
+    bits of the sequences one by one, which take the other one."""
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, h, h, 64, dtype))
+    segs = ref.packed_segment_ids(6, b, t).cuda()
+    _, kw = _mask_args(mask, window, None)
+    kw.pop("segment_ids", None)
+    forward = ops.flash_fwd(q, k, v, softmax_scale=0.125, segment_ids=segs, **kw)   # (of few sequences it has other bits)
+
+    def grads(rows):
+        x = [y[rows] for y in (q, k, v, *forward, do)]
+        return ops.flash_bwd(*x, softmax_scale=0.125, segment_ids=segs[rows], ds_workspace=ds and mask != "none", **kw)
+
+    whole = grads(slice(0, b))
+    for i in range(b):
+        for name, got, want in zip(("dq", "dk", "dv"), whole, grads(slice(i, i + 1))):
+            assert torch.equal(got[i], want[0]), (name, i)

@@ -817,6 +817,15 @@ def test_forward_kernel_keeps_the_distance_behind_its_assembly_mfma_chains():
     _assert_asm_mfma_distances(asm, r"_ZN3axl16flash_fwd_kernel", 4)
 
 
+def test_forms_for_few_row_blocks_and_for_two_workgroups_per_cu_keep_the_distance():
+    """The same check for the forward whose groups of wavefronts share the keys and for the dK/dV form of documents at
+    head_dim 64, which spills: nothing comes between a chain and its distance there either."""
+    asm, _ = _device_asm("flash_fwd.hip", extra=("-mllvm", "-amdgpu-mfma-vgpr-form"))
+    _assert_asm_mfma_distances(asm, r"_ZN3axl21flash_fwd_keys_kernel", 6)
+    asm, _ = _device_asm("flash_bwd_dkdv.hip")
+    _assert_asm_mfma_distances(asm, r"_ZN3axl27flash_bwd_dkdv_seg64_kernel", 4)
+
+
 def test_ffi_shim_and_jax_side_stay_in_step_with_the_abi():
     """csrc/ffi_shim.cc and flash_attention/jax_ffi.py only build and run under stand-ins here
     (test_jax_side.py: no jaxlib headers, no jax), so the pair is also checked from its text:
