@@ -25,7 +25,8 @@
 // throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
 // with segment ids they had to recompute dS, as calls of at most one workgroup per CU still do: B8 H32/8 T2176 window 256
 // 743 -> 688 us, B3 H16 T5760 window 1024 packed 797 -> 752 us.)  At head_dim 64, and in the shorter launches that launch_one
-// names, NW = 4 (five buffers, or four).
+// names, NW = 4 (five buffers, or four; at head_dim 64 three, with which two workgroups fit a CU: B7 H32 T512 27.0 -> 22.5 us,
+// training steps, beside what dK/dV gained, B8 H32/8 T4096 window 256 833 -> 787 us, B8 H12/4 T2176 packed 360 -> 342).
 #include "flash_bwd.h"
 
 namespace axl {
@@ -39,7 +40,7 @@ struct DqStream {
   static constexpr int DS_WAVE_BYTES = 2 * kDsBlockBytes;          // two 32-key blocks per wavefront per trip
   static constexpr int DS_BASE = K_BYTES;
   static constexpr int BUF_BYTES = K_BYTES + NW * DS_WAVE_BYTES;
-  static constexpr int NBUF = NW == 8 ? 3 : D == 128 && RANGED ? 4 : 5;   // (the RANGED form's table lies beside the ring)
+  static constexpr int NBUF = NW == 8 || D == 64 ? 3 : RANGED ? 4 : 5;   // (the RANGED form's table lies beside the ring)
   static constexpr int WROWS = BK / NW;                            // K rows that one wavefront fetches
   static constexpr int RPI = 1024 / ROWB;                          // K rows per direct-to-LDS instruction
   static constexpr int K_DMA_PER_WAVE = WROWS / RPI;
