@@ -897,6 +897,14 @@ void flash_fwd_kernel(const FwdArgs a) {
   flash_fwd_body<E, D, AUX ? kFwdAux : kFwdPlain, NW, false>(a);
 }
 
+// The general form at head_dim 64 with two workgroups per CU, 13 of its 268 registers spilled: for launches of more than one round of
+// those (fp32 bias, B8 H32/8 T1920 716 -> 561 us a call; in one round it takes longer, training step B2 H16 T2048 463 / 476).
+template <typename E>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void flash_fwd_aux64_kernel(const FwdArgs a) {
+  flash_fwd_body<E, 64, kFwdAux, 4, false>(a);
+}
+
 // Launches of few row blocks: workgroups of 64 rows, whose four wavefronts are two groups that share the keys.  A launch of at most
 // a workgroup of 128 rows per CU lasts as long as its longest one walks; this doubles the workgroups and halves the walk, at one
 // wavefront per SIMD as before (the same with 128 rows and eight wavefronts, two per SIMD, gained nothing below 2048
@@ -1625,7 +1633,8 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
       else if (p.head_dim <= 96) AXL_LAUNCH_FWD((flash_fwd_w96_kernel<E>), FwdTile<128>); \
       else AXL_LAUNCH_FWD((flash_fwd_kernel<E, 128, false>), FwdTile<128>);                     \
     } else {                                                                                    \
-      if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 64, true>), FwdTile<64>);                    \
+      if (aux && blocks > 2 * cu_count()) AXL_LAUNCH_FWD(flash_fwd_aux64_kernel<E>, FwdTile<64>); \
+      else if (aux) AXL_LAUNCH_FWD((flash_fwd_kernel<E, 64, true>), FwdTile<64>);               \
       else AXL_LAUNCH_FWD((flash_fwd_kernel<E, 64, false>), FwdTile<64>);                       \
     }                                                                                           \
   } while (0)

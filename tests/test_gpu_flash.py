@@ -2042,3 +2042,23 @@ def test_dkdv_of_documents_with_two_workgroups_per_cu(b, t, h, mask, window, dty
     for i in range(b):
         for name, got, want in zip(("dq", "dk", "dv"), whole, grads(slice(i, i + 1))):
             assert torch.equal(got[i], want[0]), (name, i)
+
+
+@pytest.mark.parametrize("drop", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_general_forward_with_two_workgroups_per_cu(dtype, drop):
+    """head_dim 64 with an fp32 bias or a dropout mask, more than one round of row blocks: the bits of the sequences one by one,
+    which take one workgroup per CU."""
+    b, t, h = 3, 1408, 16
+    q, k, v, _ = (x.cuda() for x in _inputs(b, t, h, h, 64, dtype))
+    bias = ref.normal_tensor(5, (1, h, t, t), torch.float32).cuda()
+    mask = (torch.rand(b, h, t, t, generator=torch.Generator().manual_seed(3)) < 0.1).to(torch.uint8).cuda() if drop else None
+
+    def forward(rows):
+        more = dict(dropout_mask=mask[rows], dropout_rate=0.1) if drop else {}
+        return ops.flash_fwd(q[rows], k[rows], v[rows], mask_kind=ops.MASK_CAUSAL, softmax_scale=0.125, bias=bias, **more)
+
+    out, lse = forward(slice(0, b))
+    for i in range(b):
+        one, one_lse = forward(slice(i, i + 1))
+        assert torch.equal(out[i], one[0]) and torch.equal(lse[i], one_lse[0]), i
