@@ -25,13 +25,13 @@
 // throughout, as such calls had, cost a training step 1 to 2 % at B2 H64/8 T3200 and B4 H32/8 T1152; under a window or
 // with segment ids they had to recompute dS, as calls of at most one workgroup per CU still do: B8 H32/8 T2176 window 256
 // 743 -> 688 us, B3 H16 T5760 window 1024 packed 797 -> 752 us.)  At head_dim 64, and in the shorter launches that launch_one
-// names, NW = 4 (five buffers, or four; at head_dim 64 three, with which two workgroups fit a CU: B7 H32 T512 27.0 -> 22.5 us,
+// names, NW = 4 (five buffers, or four; at head_dim 64 three in long launches, with which two workgroups fit a CU: B7 H32 T512 27.0 -> 22.5 us,
 // training steps, beside what dK/dV gained, B8 H32/8 T4096 window 256 833 -> 787 us, B8 H12/4 T2176 packed 360 -> 342).
 #include "flash_bwd.h"
 
 namespace axl {
 
-template <int D, int NW, bool RANGED>
+template <int D, int NW, bool RANGED, bool TWO>
 struct DqStream {
   static constexpr int BQ = 32 * NW;         // query rows per workgroup (32 per wavefront)
   static constexpr int BK = 64;              // keys per trip
@@ -40,7 +40,7 @@ struct DqStream {
   static constexpr int DS_WAVE_BYTES = 2 * kDsBlockBytes;          // two 32-key blocks per wavefront per trip
   static constexpr int DS_BASE = K_BYTES;
   static constexpr int BUF_BYTES = K_BYTES + NW * DS_WAVE_BYTES;
-  static constexpr int NBUF = NW == 8 || D == 64 ? 3 : RANGED ? 4 : 5;   // (the RANGED form's table lies beside the ring)
+  static constexpr int NBUF = NW == 8 || TWO ? 3 : RANGED ? 4 : 5;   // (the RANGED form's table lies beside the ring)
   static constexpr int WROWS = BK / NW;                            // K rows that one wavefront fetches
   static constexpr int RPI = 1024 / ROWB;                          // K rows per direct-to-LDS instruction
   static constexpr int K_DMA_PER_WAVE = WROWS / RPI;
@@ -52,9 +52,10 @@ struct DqStream {
 // the query tiles [first, end) that a.kb_tbl records for it; the other blocks of the workspace hold
 // nothing and are skipped (their loads are pointed at the first block, their MFMAs left out).
 // W: live width, as in the dK/dV kernel.
-template <typename E, int D, int NW, bool RANGED, int W>
+// TWO: three buffers, two workgroups per CU (head_dim 64).
+template <typename E, int D, int NW, bool RANGED, int W, bool TWO>
 __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdArgs a) {
-  using Tile = DqStream<D, NW, RANGED>;
+  using Tile = DqStream<D, NW, RANGED, TWO>;
   constexpr int DT = W / 32;
   extern __shared__ __attribute__((aligned(16))) char smem[];
 
@@ -255,10 +256,10 @@ __global__ __launch_bounds__(64 * NW) void flash_bwd_dq_stream_kernel(const BwdA
     }
 }
 
-template <typename E, int D, int NW, bool RANGED, int W>
+template <typename E, int D, int NW, bool RANGED, int W, bool TWO = false>
 static hipError_t launch_nw(const BwdArgs& a, hipStream_t stream) {
-  using Tile = DqStream<D, NW, RANGED>;
-  auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED, W>;
+  using Tile = DqStream<D, NW, RANGED, TWO>;
+  auto kernel = flash_bwd_dq_stream_kernel<E, D, NW, RANGED, W, TWO>;
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
   if (err != hipSuccess) return err;
   const int grid = (a.T + Tile::BQ - 1) / Tile::BQ * a.B * a.Hq;
@@ -283,6 +284,11 @@ static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   const bool equal = a.mask_kind == AXL_MASK_SLIDING_WINDOW && a.window < a.T;
   const bool rows128 = equal ? (wgs4 + cus - 1) / cus <= (wgs8 + cus - 1) / cus
                              : wgs4 <= cus || (wgs8 <= cus && a.T >= (a.kb_tbl ? 2048 : 1024));
+  // Two workgroups per CU where there is more than one round of them: in one it counts what the longest takes, which the other slows
+  // down (B2 H16 T2048 D64, 512 workgroups: 49.5 us with one per CU, 57.3 with two; B7 H32 T512, 896: 27.0 / 22.5).
+  if constexpr (D == 64)
+    if (wgs4 > 2 * cus)
+      return a.kb_tbl ? launch_nw<E, D, 4, true, W, true>(a, stream) : launch_nw<E, D, 4, false, W, true>(a, stream);
   if (NW == 8 && rows128)
     return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
   return a.kb_tbl ? launch_nw<E, D, NW, true, W>(a, stream) : launch_nw<E, D, NW, false, W>(a, stream);
