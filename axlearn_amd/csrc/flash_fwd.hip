@@ -843,8 +843,10 @@ __device__ __forceinline__ void flash_fwd_body(const FwdArgs& a) {
     __syncthreads();
     if (key_group == 1) return;
     const floatx2 other = *stats;
-    const float mx = fmaxf(m_run, other[0]);
-    const float f0 = fast_exp2((m_run - mx) * c), f1 = fast_exp2((other[0] - mx) * c);
+    // A group that saw no key has no say in the maximum, and the larger of two counts in full whatever it is: a sink may
+    // be infinite, and infinity less itself is no weight.
+    const float m_other = other[1] == 0.f ? m_run : other[0], mx = fmaxf(m_run, m_other);
+    const float f0 = m_run == mx ? 1.f : fast_exp2((m_run - mx) * c), f1 = m_other == mx ? 1.f : fast_exp2((m_other - mx) * c);
     m_run = mx;
     l_tot = l_tot * f0 + other[1] * f1;
 #pragma unroll

@@ -2062,3 +2062,25 @@ def test_general_forward_with_two_workgroups_per_cu(dtype, drop):
     for i in range(b):
         one, one_lse = forward(slice(i, i + 1))
         assert torch.equal(out[i], one[0]) and torch.equal(lse[i], one_lse[0]), i
+
+
+@pytest.mark.parametrize("t,s,mask,window,offset", [
+    (768, 768, "causal", None, 0),
+    (640, 640, "sliding", 100, 0),       # of some rows one group sees no key
+    (128, 512, "sliding", 100, 1000),    # no row sees a key
+])
+def test_sinks_without_bounds_in_launches_of_few_row_blocks(t, s, mask, window, offset):
+    """Sinks that are infinite, or become so in units of the logits: what the form without key sharing gives, which a call with
+    positions per sequence takes.  A sink of plus infinity takes all the weight (zeros), one of minus infinity none."""
+    # (with minus infinity a row whose first tile is masked for it has no running maximum, in either form)
+    none = float("-inf") if mask == "causal" else -1e35
+    sinks = torch.tensor([float("inf"), 3e38, none, -1e30, 0.5], device="cuda")
+    q, k, v, _ = (x.cuda() for x in _inputs(1, t, len(sinks), len(sinks), 64, torch.bfloat16, s=s))
+    _, kw = _mask_args(mask, window, None)
+    kw.update(softmax_scale=0.125, logit_sink=sinks)
+    out, lse = ops.flash_fwd(q, k, v, q_pos_offset=offset, **kw)
+    want, want_lse = ops.flash_fwd(q, k, v, q_pos_offsets=torch.tensor([offset], device="cuda"), **kw)
+    assert not want[:, :, :2].any() and (want_lse[:, :2] == float("inf")).all() and not want.isnan().any()
+    # each form rounds its probabilities and its result to bf16: twice the oracle's bar for one of them
+    torch.testing.assert_close(out, want, rtol=0, atol=2 * BF16_MAX_ABS)
+    torch.testing.assert_close(lse, want_lse, rtol=1e-5, atol=1e-5)
