@@ -914,8 +914,9 @@ void flash_fwd_aux64_kernel(const FwdArgs a) {
 // many blocks of 128 rows as CUs: B1 H32 T512 16.3 / 12.4, B1 H8 T1024 22.1 / 15.9, T2048 36.0 / 25.5, D64 T512 10.4 / 8.7, window
 // 256 B2 H8 T1024 16.1 / 11.2, unmasked B1 H16 T768 19.5 / 13.9, documents B1 H8 T1536 17.3 / 13.6, three short ones D80 T384 9.1 / 8.6.
 // Up to as many as CUs two workgroups follow one another on a CU; causal, long and short walks even out: B1 H32 T1024
-// 25.0 / 24.3, B1 H16 T2048 39.5 / 33.7, B1 H8 T4096 68.7 / 53.8, D64 45.7 / 32.8 - but unmasked, under a window, with documents or
-// below 1024 keys it loses (B2 H16 T768 unmasked 20.3 / 26.0, B1 H64 T512 18.1 / 19.8).
+// 25.0 / 24.3, B1 H16 T2048 39.5 / 33.7, B1 H8 T4096 68.7 / 53.8, D64 45.7 / 32.8 - but unmasked, under a window, with documents,
+// below 1024 rows or behind a prefix, where every row walks much the same, it loses (B2 H16 T768 unmasked 20.3 / 26.0, B1 H64 T512
+// 18.1 / 19.8, B1 H64/8 512 rows behind 2304 keys 52 / 58, B1 H32/8 D96 896 rows behind 3456 64 / 76).
 template <typename E, int D, int W>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2)))
 void flash_fwd_keys_kernel(const FwdArgs a) {
@@ -1594,11 +1595,13 @@ int launch_flash_fwd(const AxlFlashFwdParams& p, hipStream_t stream) {
   const int width = p.head_dim <= 64 ? 64 : 128;  // the compiled width that serves this head_dim
   hipError_t err = hipSuccess;
   const int64_t blocks = (int64_t)(p.q_len / 128) * p.batch * p.num_q_heads;
-// Launches that leave CUs idle, or a CU with one workgroup of the longest walk: flash_fwd_keys_kernel (its comment has both
+  // Launches that leave CUs idle, or a CU with one workgroup of the longest walk: flash_fwd_keys_kernel (its comment has both
   // sides' times).  Not for rows at offsets of their own: a chunk of rows padded into blocks gives the chunk kernel's bits.
+  // From half as many row blocks as CUs on, long and short walks have to even out: rows from the first position on.
   const bool share_keys = !aux && !p.q_pos_offsets && p.kv_len > 256 &&
                           (2 * blocks <= cu_count() ||
-                           (blocks <= cu_count() && p.mask_kind == AXL_MASK_CAUSAL && !p.segment_ids && p.kv_len >= 1024));
+                           (blocks <= cu_count() && p.mask_kind == AXL_MASK_CAUSAL && !p.segment_ids && p.q_pos_offset == 0 &&
+                            p.q_len >= 1024 && p.kv_len >= p.q_len));
 #define AXL_LAUNCH_FWD(KERNEL, TILE)                                                            \
   do {                                                                                          \
     err = allow_dynamic_lds((const void*)KERNEL, TILE::LDS_BYTES);                              \

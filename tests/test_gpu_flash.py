@@ -2084,3 +2084,23 @@ def test_sinks_without_bounds_in_launches_of_few_row_blocks(t, s, mask, window, 
     # each form rounds its probabilities and its result to bf16: twice the oracle's bar for one of them
     torch.testing.assert_close(out, want, rtol=0, atol=2 * BF16_MAX_ABS)
     torch.testing.assert_close(lse, want_lse, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("b,t,s,h,mask,offset,shared", [
+    (1, 512, 2816, 64, "causal", 2304, False),   # behind a prefix every row block walks much the same
+    (1, 1024, 1152, 32, "causal", 128, False),
+    (1, 1024, 1024, 32, "causal", 0, True),
+    (1, 896, 1024, 32, "causal", 0, False),      # the keys past the rows are not walked
+    (1, 512, 2816, 32, "causal", 2304, True),    # half as many blocks as CUs: whatever the walks
+    (2, 1024, 1024, 16, "none", 0, False),
+])
+def test_which_launches_of_few_row_blocks_share_the_keys(b, t, s, h, mask, offset, shared):
+    """By the bits, on a GPU of 256 CUs: those of the form without key sharing, which a call with positions per sequence takes,
+    or others."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
+    q, k, v, _ = (x.cuda() for x in _inputs(b, t, h, 8, 64, torch.bfloat16, s=s))
+    _, kw = _mask_args(mask, None, None)
+    out, lse = ops.flash_fwd(q, k, v, softmax_scale=0.125, q_pos_offset=offset, **kw)
+    want, want_lse = ops.flash_fwd(q, k, v, softmax_scale=0.125, q_pos_offsets=torch.full((b,), offset, device="cuda"), **kw)
+    assert (torch.equal(out, want) and torch.equal(lse, want_lse)) is not shared
+    _assert_close("out", out, want.cpu(), torch.bfloat16)
