@@ -1047,10 +1047,16 @@ static bool even_fits(size_t even, size_t drawn) { return even <= drawn || even 
 // and its launch; 4 us and more where the memory system is loaded, and one workgroup of 256 threads is slow with many
 // records.  (Call, own kernel / by the split kernel: 420 tiles in shares of 8, 9 records 12.9 / 11.0 us; 10 280 tiles in shares of 20
 // 25.1 / 24.1; 9552 in 20, 31 records 21.9 / 21.1; 16 384 in 36 30.4 / 32.5; 8 sequences of 2000 to 8190 tokens, shares of 64,
-// 40.6 / 42.1; shares of 8, 39 records of 8 heads 25.1 / 29.8.)  The kernel of its own takes 1024 threads from four rounds on
+// 40.6 / 42.1; shares of 8, 39 records of 8 heads 25.1 / 29.8.)  A workgroup whose share ends inside a pair is the last one of
+// two pairs as often as not and merges one after the other.  In shares of 8 that takes longer than the kernel (16 heads, one
+// sequence of 1000 tokens in a cache of 1006, 126 shares for 128 blocks, 14.7 / 16.6 us; window 1024 of 6000, 8 heads 14.7 / 16.4; 4
+// sequences of 991, 16 heads 17.8 / 20.8), so there every block the call can have must find a workgroup, and not all that the
+// GPU holds at once (512 blocks of 32 heads 14.1 / 14.9).  In shares of 12 to 20 the two are even, and the call gains where it
+// turns out to have fewer blocks than workgroups (4224 to 8448 tiles: 0.92 to 1.03; in 24 up to 1.08).  The kernel of its own
+// takes 1024 threads from four rounds on
 // (108 records of 8 heads 24.0 -> 18.8 us, 240 40.2 -> 26.6, 8 pairs of 65 65.8 -> 60.5; with few records, or hundreds of
 // pairs of them, it would lose 1 to 3 us).
-constexpr int kMergeShare = 24, kMergeRounds = 2, kManyRounds = 4, kManyThreads = 1024;
+constexpr int kMergeShare = 20, kMergeRounds = 2, kManyRounds = 4, kManyThreads = 1024;
 
 // Equal shares (see the head of this file) where the capacity makes them at most 256 tiles, the page ids a
 // segment keeps in registers.  Measured at 8 sequences of 2000 to 8190 tokens, 8 kv heads (40 tiles a
@@ -1071,7 +1077,10 @@ static void plan_even(DecArgs& a, bool deterministic, int& merge_rounds, bool& m
   // records a pair can have, by equal shares or a block each, and the rounds of loads in which 256 threads merge them
   const int64_t records = std::max((pair + share - 1) / share + 1, std::min<int64_t>(pair / a.chunk_pages + 2, a.n_wg));
   merge_rounds = (int)((records * std::min(a.G, 16) * width_of(a.d_real) / 4 + kMergeBatch * 256 - 1) / (kMergeBatch * 256));
-  merge_here = !a.bias && share <= kMergeShare && merge_rounds <= kMergeRounds;
+  // blocks a pair can have: under a window they may begin and end inside one
+  const int64_t blocks = a.window >= 0 ? std::min<int64_t>(a.nch, (pair + a.chunk_pages - 2) / a.chunk_pages + 1) : a.nch;
+  const bool block_each = blocks * a.B * a.Hv <= a.n_wg && a.n_wg < slots;
+  merge_here = !a.bias && merge_rounds <= kMergeRounds && share <= kMergeShare && (block_each || share > a.min_share);
   // A deterministic call keeps to the blocks, whose bits depend on a pair's own keys alone: equal shares only
   // where the shapes leave no more blocks than workgroups.
   if (deterministic && (int64_t)a.B * a.Hv * a.nch > a.n_wg) a.even = 0;

@@ -902,19 +902,24 @@ def test_page_insert_of_a_layers_projections():
             assert torch.equal(pools[0], pools[2]) and torch.equal(pools[1], pools[3]) and pools[0].abs().sum() > 0
 
 
-@pytest.mark.parametrize("b,hq,hkv,s,d,window,dtype", [
-    (1, 8, 8, 1024, 128, -1, torch.float16),     # a block of 8 tiles each, 8 records to a pair
-    (3, 12, 4, 8704, 64, 1024, torch.bfloat16),  # under a window, shares of 8 that end inside pairs
-    (33, 12, 4, 2003, 96, -1, torch.bfloat16),   # shares over several pairs, some held whole
-    (1, 16, 1, 700, 80, -1, torch.bfloat16),     # 16 heads: two rounds of records
-    (2, 24, 1, 500, 128, -1, torch.float16),     # two groups of heads to a kv head
-    (2, 32, 8, 9538, 128, -1, torch.bfloat16),   # 30 records of 4 heads
-    (1, 8, 1, 13728, 128, -1, torch.bfloat16),   # 108 records: a merge kernel of 1024 threads
+@pytest.mark.parametrize("b,hq,hkv,s,d,window,dtype,marks", [
+    (1, 8, 8, 1024, 128, -1, torch.float16, True),     # a block of 8 tiles each, 8 records to a pair
+    (3, 12, 4, 8704, 64, 1024, torch.bfloat16, True),  # under a window, blocks of 16 tiles
+    (33, 12, 4, 2003, 96, -1, torch.bfloat16, False),  # shares over several pairs, some held whole
+    (1, 16, 1, 700, 80, -1, torch.bfloat16, True),     # 16 heads: two rounds of records
+    (2, 24, 1, 500, 128, -1, torch.float16, True),     # two groups of heads to a kv head
+    (2, 32, 8, 9538, 128, -1, torch.bfloat16, True),   # 30 records of 4 heads
+    (4, 16, 16, 1536, 64, -1, torch.float16, True),    # shares of 12 that end inside pairs: two to merge
+    (1, 16, 16, 1006, 128, -1, torch.bfloat16, False),     # shares of 8 that would, two blocks more than workgroups
+    (1, 8, 8, 6000, 64, 1024, torch.bfloat16, False),      # the same under a window
+    (1, 8, 1, 13728, 128, -1, torch.bfloat16, False),  # 108 records: a merge kernel of 1024 threads
 ])
-def test_records_merged_by_the_split_kernel(b, hq, hkv, s, d, window, dtype):
+def test_records_merged_by_the_split_kernel(b, hq, hkv, s, d, window, dtype, marks):
     """Short calls merge their records without a kernel of its own, except in a captured graph, whose launches are replayed
     with their arguments: against the oracle, on a workspace of NaN patterns and on what the call before left there, some
-    sequences empty, two calls at a time on streams of their own, and replays with the inputs changed in between."""
+    sequences empty, two calls at a time on streams of their own, and replays with the inputs changed in between.  Which form
+    ran (on a GPU of 256 CUs) shows in the workspace: marks are one number in the places of all pairs, which counts the calls."""
+    assert torch.cuda.get_device_properties(0).multi_processor_count == 256
     gen = torch.Generator().manual_seed(7)
     q, k, v = (torch.randn(shape, generator=gen).to(dtype) for shape in ((b, hq, d), (b, s, hkv, d), (b, s, hkv, d)))
     lengths = torch.randint(1, s + 1, (b,), generator=gen, dtype=torch.int32)
@@ -940,6 +945,20 @@ def test_records_merged_by_the_split_kernel(b, hq, hkv, s, d, window, dtype):
     for _ in range(3):
         for x, exact in ((args[0], first), (-args[0], other)):
             assert ref.rel_l2(call(x, workspaces[0]).cpu().double(), exact) <= bar
+
+    def marks_left(calls):
+        """How many words of 64 bits hold the same number after the second of `calls`, and one less after the first."""
+        left = []
+        for one in calls:
+            one()
+            torch.cuda.synchronize()
+            left.append(workspaces[0].view(torch.int64).clone())
+        numbers = left[1][left[1] - left[0] == 1]
+        return int(numbers.unique(return_counts=True)[1].max()) if len(numbers) else 0
+
+    again = lambda: call(args[0], workspaces[0])
+    some = max(2, b * hkv)   # (sums of two calls may differ by one unit in a few places too)
+    assert (marks_left([again, again]) >= some) is marks
     det = [call(args[0], ws, deterministic=True) for ws in workspaces[:2]]
     assert torch.equal(*det) and ref.rel_l2(det[0].cpu().double(), first) <= bar
     torch.cuda.synchronize()
@@ -955,6 +974,10 @@ def test_records_merged_by_the_split_kernel(b, hq, hkv, s, d, window, dtype):
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         call(x, workspaces[2], out=out)
+    replayed = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(replayed):
+        call(args[0], workspaces[0])
+    assert marks_left([replayed.replay, replayed.replay]) < some
     for sign, exact in ((1, first), (-1, other), (1, first)):
         x.copy_(sign * args[0])
         call(x, workspaces[0])   # eager work between the replays
