@@ -598,13 +598,18 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
     const DkdvPlan plan = plan_dkdv(p, p.mask_kind, p.q_pos_offset, max_splits(p));
     // Unsplit, one key block per workgroup with segment ids: documents end where they like, the shares of a block and its
     // mirror image add up to anything, and the longer workgroups leave the longer tail (training step, two / one: B6 H32/8
-    // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; of 25 packed causal shapes none
-    // lost more than runs differ by).  The choice to split looks at the mirrored form all the same: the sizes of the key blocks it
+    // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; backward, B2 H64/8 T6400 D96 of six documents
+    // 2472 / 1673, B1 H16 T9472 861 / 721).  Rows of one document, which the launch cannot tell from others, lose 1 to 2 %
+    // (backward, B4 H32/8 T4096 1714 / 1743, B8 H16 T2048 581 / 589; of long documents with one query head a kv head and a bias
+    // up to 8, B4 H16 T2048 D64 310 / 336).  Not in float32, where it went either way, and further down than up (backward, B4 H16
+    // T1024 D64 of four documents 164 / 213, B2 H32 T2048 of one 986 / 1094, B1 H32 T2048 D64 of four 314 / 361; B2 H32/8 T2048
+    // of three 1222 / 1160).
+    // The choice to split looks at the mirrored form all the same: the sizes of the key blocks it
     // weighs are those without documents (B2 H32/8 T2048 D64 packed, split / whole by the longest key block 215 / 237 us).
     // One also where two workgroups share a CU, each busy in the other's gaps (head_dim 64 without a bias or dropout mask: step,
     // two / one, B3 H8 T1024 68.1 / 60.4 us, B7 H32 T256 56.5 / 52.7, B6 H64/8 T3328 3489 / 3301, B4 H32/8 T4096 1500 / 1512).
-    const bool two_per_cu = dt != AXL_F32 && p.head_dim <= 64 && !p.aux.bias && !p.aux.dropout_mask;
-    const bool one = plan.splits == 1 && (p.segment_ids || two_per_cu);
+    const bool two_per_cu = p.head_dim <= 64 && !p.aux.bias && !p.aux.dropout_mask;
+    const bool one = dt != AXL_F32 && plan.splits == 1 && (p.segment_ids || two_per_cu);
     a.kb_per_wg = one ? 1 : plan.kb_per_wg;
     a.splits = plan.splits;
   }
