@@ -607,8 +607,15 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
     // The choice to split looks at the mirrored form all the same: the sizes of the key blocks it
     // weighs are those without documents (B2 H32/8 T2048 D64 packed, split / whole by the longest key block 215 / 237 us).
     // One also where two workgroups share a CU, each busy in the other's gaps (head_dim 64 without a bias or dropout mask: step,
-    // two / one, B3 H8 T1024 68.1 / 60.4 us, B7 H32 T256 56.5 / 52.7, B6 H64/8 T3328 3489 / 3301, B4 H32/8 T4096 1500 / 1512).
-    const bool two_per_cu = p.head_dim <= 64 && !p.aux.bias && !p.aux.dropout_mask;
+    // two / one, B3 H8 T1024 68.1 / 60.4 us, B7 H32 T256 56.5 / 52.7, B6 H64/8 T3328 3489 / 3301, B4 H32/8 T4096 1500 / 1512).  In one
+    // round of those, up to 512 key blocks, only where the starts and ends of key blocks weigh: it lasts as long as the
+    // longest walk, which the mirrored form halves (dK/dV, two / one, by the tiles of the longest walk: 16 B8 H8 T512 26.1 / 18.7,
+    // 64 B16 H32/8 T512 75 / 68, 128 B7 H32/8 T1024 110 / 107, 192 B8 H12/4 T2048 162 / 159; 256 from 0.97 to 1.02; 384 B3 H12/4 T4096
+    // 256 / 269, 512 B2 H32/8 T4096 395 / 402, 1152 B1 H12/4 T12288 724 / 766, 2048 B1 H64/8 T8192 1527 / 1583).
+    const int64_t key_blocks = (int64_t)p.batch * p.num_kv_heads * (p.kv_len / 128);
+    const int64_t longest = (int64_t)p.num_q_heads / p.num_kv_heads * ((p.q_len + 31) / 32);
+    const bool two_per_cu = p.head_dim <= 64 && !p.aux.bias && !p.aux.dropout_mask &&
+                            (key_blocks > 2 * (int64_t)cu_count() || longest < 256);
     const bool one = dt != AXL_F32 && plan.splits == 1 && (p.segment_ids || two_per_cu);
     a.kb_per_wg = one ? 1 : plan.kb_per_wg;
     a.splits = plan.splits;
