@@ -285,10 +285,15 @@ static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   const bool rows128 = equal ? (wgs4 + cus - 1) / cus <= (wgs8 + cus - 1) / cus
                              : wgs4 <= cus || (wgs8 <= cus && a.T >= (a.kb_tbl ? 2048 : 1024));
   // Two workgroups per CU where there is more than one round of them: in one it counts what the longest takes, which the other slows
-  // down (B2 H16 T2048 D64, 512 workgroups: 49.5 us with one per CU, 57.3 with two; B7 H32 T512, 896: 27.0 / 22.5).
-  if constexpr (D == 64)
-    if (wgs4 > 2 * cus)
+  // down (B2 H16 T2048 D64, 512 workgroups: 49.5 us with one per CU, 57.3 with two; B7 H32 T512, 896: 27.0 / 22.5).  And where a
+  // workgroup walks few keys, so that its start and end weigh more than the depth of the ring (one / two, causal: T256 to T1152
+  // 16.0 / 11.8 to 22.4 / 21.4, T1664 28.1 / 27.7, T2048 132 / 136, T2560 38.4 / 40.2, T4096 126 / 137, T10240 179 / 190; of three
+  // documents T512 28.0 / 22.4, T2560 31.5 / 29.1, T3456 43.6 / 41.0, T4096 75.8 / 80.8; window 1024 of T4608 77.8 / 74.1).
+  if constexpr (D == 64) {
+    const int64_t keys = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? min((int64_t)a.T, (int64_t)a.window + 128) : a.T;
+    if (wgs4 > 2 * cus && keys <= (a.seg ? 3584 : 1920))
       return a.kb_tbl ? launch_nw<E, D, 4, true, W, true>(a, stream) : launch_nw<E, D, 4, false, W, true>(a, stream);
+  }
   if (NW == 8 && rows128)
     return a.kb_tbl ? launch_nw<E, D, 4, true, W>(a, stream) : launch_nw<E, D, 4, false, W>(a, stream);
   return a.kb_tbl ? launch_nw<E, D, NW, true, W>(a, stream) : launch_nw<E, D, NW, false, W>(a, stream);

@@ -2104,3 +2104,26 @@ def test_which_launches_of_few_row_blocks_share_the_keys(b, t, s, h, mask, offse
     want, want_lse = ops.flash_fwd(q, k, v, softmax_scale=0.125, q_pos_offsets=torch.full((b,), offset, device="cuda"), **kw)
     assert (torch.equal(out, want) and torch.equal(lse, want_lse)) is not shared
     _assert_close("out", out, want.cpu(), torch.bfloat16)
+
+
+@pytest.mark.parametrize("b,t,hq,hkv,mask,window,packed,dtype", [
+    (9, 512, 16, 16, "causal", None, False, torch.bfloat16),    # 576 workgroups, the smallest number of whole sequences
+    (3, 1920, 16, 4, "causal", None, False, torch.float16),     # the longest walk
+    (4, 1152, 16, 4, "sliding", 200, False, torch.bfloat16),    # with the table of query tiles
+    (5, 896, 16, 16, "causal", None, True, torch.float16),
+])
+def test_dq_from_ds_with_two_workgroups_per_cu(b, t, hq, hkv, mask, window, packed, dtype):
+    """head_dim 64, more than one round of two workgroups of 128 rows per CU: dQ of three buffers has the bits of the sequences
+    one by one, which take one workgroup per CU with four or five."""
+    q, k, v, do = (x.cuda() for x in _inputs(b, t, hq, hkv, 64, dtype))
+    assert b * hq * t // 128 > 2 * torch.cuda.get_device_properties(0).multi_processor_count
+    segs = ref.packed_segment_ids(6, b, t).cuda() if packed else None
+    _, kw = _mask_args(mask, window, None)
+    kw.update(softmax_scale=0.125, segment_ids=segs)
+    out, lse = ops.flash_fwd(q, k, v, **kw)
+    dq = ops.flash_bwd(q, k, v, out, lse, do, ds_workspace=True, **kw)[0]
+    for i in range(b):
+        rows = slice(i, i + 1)
+        kw["segment_ids"] = segs[rows] if packed else None
+        one = ops.flash_bwd(*(x[rows] for x in (q, k, v, out, lse, do)), ds_workspace=True, **kw)[0]
+        assert torch.equal(dq[rows], one), i
