@@ -891,8 +891,11 @@ void flash_bwd_dkdv_kernel(const BwdArgs a) {
 }
 
 // The same with segment ids, whose 275 registers do not fit twice: 1 to 14 of them spilled.  Pays for itself where a kv head has
-// one query head and there are two and a half rounds of key blocks or more, us: B4 H16 T4096 595 -> 565, T2048 unmasked 313 -> 284, T1408
-// 148 -> 138, B8 T640 112 -> 104; not with longer walks (B8 H32/8 T4096 2160 / 2218, H64/8 T2048 1382 / 1426) or fewer (B8 H8/1 T5376 1490 / 1650).
+// one query head and there are two and a half rounds of key blocks or more, us: B4 H16 T2048 unmasked 313 -> 284, causal B8 T640
+// 112 -> 104; not with longer walks (B8 H32/8 T4096 2160 / 2218, H64/8 T2048 1382 / 1426) or fewer (B8 H8/1 T5376 1490 / 1650).
+// Nor under a mask that leaves a key block more than 1280 rows, unless most are another document's: dK/dV, one per CU / two, causal B8
+// H32 T512 to T1152 of one to six documents 0.82 to 0.98, T1408 of one 298 / 318, of six 205 / 192, B8 H16 T2816 of one, whole
+// backward, 800 / 868, B4 H8 T2688 of one 185 / 212.  Unmasked 0.85 to 0.92 at all lengths to 5504, window 256 and 1024 0.92 to 1.02.
 template <typename E, bool SPILL>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void flash_bwd_dkdv_seg64_kernel(const BwdArgs a) {
@@ -957,8 +960,11 @@ static hipError_t launch_one(const BwdArgs& a, hipStream_t stream) {
   auto kernel = [&] {
     if constexpr (SPLIT) return flash_bwd_dkdv_split_kernel<E, D, HAS_SEG, AUX, SPILL, W>;
     else if constexpr (W == 96) return flash_bwd_dkdv_w96_kernel<E, HAS_SEG, SPILL>;
-    else if constexpr (D == 64 && HAS_SEG && AUX == 0)
-      return a.Hq == a.Hkv && 2 * (int64_t)grid >= 5 * (int64_t)cu_count() ? flash_bwd_dkdv_seg64_kernel<E, SPILL> : flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
+    else if constexpr (D == 64 && HAS_SEG && AUX == 0) {
+      const int64_t rows = a.mask_kind == AXL_MASK_SLIDING_WINDOW ? min((int64_t)a.T, (int64_t)a.window + 128) : a.T;
+      return a.Hq == a.Hkv && 2 * (int64_t)grid >= 5 * (int64_t)cu_count() && (a.mask_kind == AXL_MASK_NONE || rows <= 1280)
+                 ? flash_bwd_dkdv_seg64_kernel<E, SPILL> : flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
+    }
     else return flash_bwd_dkdv_kernel<E, D, HAS_SEG, AUX, SPILL>;
   }();
   hipError_t err = allow_dynamic_lds((const void*)kernel, Tile::LDS_BYTES);
