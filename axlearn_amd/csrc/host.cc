@@ -24,6 +24,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/forward_grad.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/headeronly/version.h>
 
 #include "../../include/axl_attn.h"
 
@@ -584,5 +585,10 @@ PyMODINIT_FUNC PyInit__axl_host() {
   s_segments = PyUnicode_InternFromString("segment_ids");
   s_dtype = PyUnicode_InternFromString("dtype");
   s_internal_value = PyUnicode_InternFromString("_internal_value");
-  return PyModule_Create(&module);
+  PyObject* const m = PyModule_Create(&module);
+  if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
 }

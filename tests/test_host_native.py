@@ -29,8 +29,8 @@ def _fields(block):
 
 
 @pytest.fixture
-def through_python(monkeypatch):
-    """Calls go through Python on CPU tensors that pass for the GPU's; the list of blocks that reach the C ABI."""
+def recorded(monkeypatch):
+    """CPU tensors pass for the GPU's; the list of blocks that reach the C ABI."""
     real, seen = _lib.load(), []
 
     class Recorder:
@@ -43,11 +43,21 @@ def through_python(monkeypatch):
     monkeypatch.setattr(_lib, "current_stream_ptr", lambda: 0)
     monkeypatch.setattr(torch.Tensor, "is_cuda", True)
     monkeypatch.setattr(ops, "_device_properties", lambda device: (288 << 30, 256))
+    return seen
+
+
+def _without_native_calls(monkeypatch):
     for name in ("attend", "flash_fwd", "flash_bwd"):
         monkeypatch.setattr(_host, name, lambda *a: None)
     monkeypatch.setattr(_host, "page_insert", lambda *a: False)
+
+
+@pytest.fixture
+def through_python(monkeypatch, recorded):
+    """Calls go through Python on CPU tensors that pass for the GPU's; the list of blocks that reach the C ABI."""
+    _without_native_calls(monkeypatch)
     logging.disable(logging.WARNING)
-    yield seen
+    yield recorded
     logging.disable(logging.NOTSET)
 
 
@@ -245,6 +255,55 @@ def test_calls_that_something_looks_at_by_its_operations_go_through_python():
     assert seen and not any(seen)
     assert taken()
     assert _host.load().attend(x, x, x, bias, None, None, None, 0.125, 128, False) is None   # not on the GPU
+
+
+def _no_extension(monkeypatch, tmp_path, how):
+    monkeypatch.setattr(_host, "_module", None)
+    monkeypatch.setattr(_host, "_absent", False)
+    if how == "missing":
+        monkeypatch.setattr(_host, "PATH", str(tmp_path / "_axl_host.so"))
+    elif how == "not a library":
+        (tmp_path / "_axl_host.so").write_bytes(b"\x7fELF")
+        monkeypatch.setattr(_host, "PATH", str(tmp_path / "_axl_host.so"))
+    elif how == "another torch":
+        monkeypatch.setattr(torch, "__version__", "1.13.0+rocm5.2")
+    else:
+        def load():
+            raise RuntimeError("libaxl_attn_hip.so is missing.")
+        monkeypatch.setattr(_lib, "load", load)
+
+
+@pytest.mark.parametrize("how", ["missing", "not a library", "another torch"])
+def test_without_the_extension_calls_reach_the_kernels_through_python(monkeypatch, tmp_path, caplog, recorded, how):
+    """The extension is not there, or does not load here: every call takes the way through Python, which says so once."""
+    _no_extension(monkeypatch, tmp_path, how)
+    with pytest.raises((RuntimeError, ImportError)):
+        _host.load()
+    x, pool = torch.zeros(1, 128, 2, 64, dtype=torch.bfloat16), torch.zeros(2, 4, 16, 64, dtype=torch.bfloat16)
+    layer = FlashAttention.default_config().set(softmax_scale=0.125).instantiate()
+    q = x.clone().requires_grad_(True)
+    with caplog.at_level(logging.WARNING):
+        out, _ = layer.compute_attention(q_proj=q, k_proj=x, v_proj=x, attention_logit_biases=ab.CompositeAttentionBias([]))
+        out.backward(x)
+        paged_extend_step(pool, pool.clone(), torch.zeros(1, 2, dtype=torch.int32), k_proj=x[:, :1], v_proj=x[:, :1],
+                          key_positions=torch.zeros(1, 1, dtype=torch.int32))
+    assert len(recorded) == 3 and q.grad.shape == q.shape   # forward, backward, insert
+    assert len([r for r in caplog.records if "host path" in r.getMessage()]) == 1
+
+
+@pytest.mark.parametrize("how", ["missing", "another torch", "no kernel library"])
+def test_without_libraries_what_needs_none_is_answered(monkeypatch, tmp_path, how):
+    """A request that no kernel supports goes to the fallback, and sizes that do not fit together are refused in Python."""
+    _no_extension(monkeypatch, tmp_path, how)
+    layer = FlashAttention.default_config().set(softmax_scale=0.125).instantiate()
+    x = torch.zeros(1, 100, 2, 64)
+    call = lambda k, **kw: layer.compute_attention(q_proj=x, k_proj=k, v_proj=k, attention_logit_biases=ab.CompositeAttentionBias([]), **kw)
+    answer = (torch.ones(1), None)
+    assert call(x, fallback=lambda **kw: answer) is answer
+    with pytest.raises(ValueError):
+        call(torch.zeros(2, 100, 2, 64))
+    with pytest.raises(ValueError):
+        paged_extend_step(x, x, torch.zeros(1, 2, dtype=torch.int32), k_proj=x, v_proj=x[:, :1], key_positions=torch.zeros(1, 1))
 
 
 @pytest.mark.gpu
