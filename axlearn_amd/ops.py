@@ -282,7 +282,7 @@ def flash_bwd(
     heads that still fill the GPU.  A workspace that there is no room for (on the device, or in `buffers`) gives
     way to a smaller one as `_bwd_workspace` says."""
     if (phases == 7 and buffers is None and ds_workspace is None and dropout_mask is None and not dropout_rate
-            and q_pos_offset == 0):
+            and q_pos_offset == 0 and q.is_cuda):   # (other devices have no memory to ask for: refused below)
         limit = ds_workspace_limit if ds_workspace_limit is not None else default_bwd_workspace_limit(q.device)
         result = _host.flash_bwd(q, k, v, out, lse, d_out, segment_ids, logit_sink, softmax_scale, mask_kind, sliding_window,
                                  limit, bias)

@@ -306,6 +306,14 @@ def test_without_libraries_what_needs_none_is_answered(monkeypatch, tmp_path, ho
         paged_extend_step(x, x, torch.zeros(1, 2, dtype=torch.int32), k_proj=x, v_proj=x[:, :1], key_positions=torch.zeros(1, 1))
 
 
+def test_backward_by_the_size_rule_refuses_cpu_tensors_as_the_other_calls_do():
+    x, lse = torch.zeros(1, 128, 2, 64, dtype=torch.bfloat16), torch.zeros(1, 2, 128)
+    with pytest.raises(_lib.AxlError, match="must live on the GPU"):
+        ops.flash_bwd(x, x, x, x, lse, x, ds_workspace=None)
+    with pytest.raises(_lib.AxlError, match="does not match"):   # sizes first, whatever the device
+        ops.flash_bwd(x, x[..., :32], x, x, lse, x, mask_kind=ops.MASK_CAUSAL, ds_workspace=None)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["decode", "paged", "chunk", "self", "train", "train_bias", "train_bias_f16"])
 def test_native_calls_give_the_bits_of_those_through_python(kind):
