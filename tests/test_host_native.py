@@ -316,8 +316,9 @@ def test_backward_by_the_size_rule_refuses_cpu_tensors_as_the_other_calls_do():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("kind", ["decode", "paged", "chunk", "self", "train", "train_bias", "train_bias_f16"])
-def test_native_calls_give_the_bits_of_those_through_python(kind):
-    """On a stream of their own, each behind work that its inputs wait for."""
+def test_native_calls_give_the_bits_of_those_through_python(kind, monkeypatch):
+    """On a stream of their own, each behind work that its inputs wait for; every step of them native, and none of those through
+    Python."""
     gen = torch.Generator("cuda").manual_seed(0)
     b, hq, hkv, d, s = 2, 8, 2, 128, 512
     t = dict(decode=1, paged=1, chunk=40).get(kind, s)
@@ -352,17 +353,27 @@ def test_native_calls_give_the_bits_of_those_through_python(kind):
         return [out, *torch.autograd.grad(out, leaves, d_out)]
 
     torch.cuda.synchronize()
-    side = torch.cuda.Stream()
-    with torch.cuda.stream(side):
-        got = [call() for _ in range(3)]
-    side.synchronize()
-    root = logging.getLogger()
-    level = root.level
-    root.setLevel(logging.INFO)   # the dispatch speaks: everything through Python
-    try:
+    side, taken = torch.cuda.Stream(), []
+
+    def noted(name, native):
+        def f(*a):
+            result = native(*a)
+            if result is not None and result is not False:
+                taken.append(name)
+            return result
+        return f
+
+    with monkeypatch.context() as m:
+        for name in ("attend", "flash_fwd", "flash_bwd", "page_insert"):
+            m.setattr(_host, name, noted(name, getattr(_host, name)))
+        with torch.cuda.stream(side):
+            got = [call() for _ in range(3)]
+        side.synchronize()
+    steps = dict(paged=["page_insert", "attend"]).get(kind, ["attend", "flash_fwd", "flash_bwd"] if kind.startswith("train") else ["attend"])
+    assert taken == 3 * steps
+    with monkeypatch.context() as m:
+        _without_native_calls(m)
         want = call()
-    finally:
-        root.setLevel(level)
     torch.cuda.synchronize()
     for outs in got:
         assert all(torch.equal(x, y) for x, y in zip(outs, want))
