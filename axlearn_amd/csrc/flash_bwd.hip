@@ -601,7 +601,7 @@ int launch_flash_bwd(const AxlFlashBwdParams& p, int phases, hipStream_t stream)
     // T4096 2830 / 2642 us, B5 H12/4 T1792 D96 275 / 233, B8 H8/1 T5376 D64 1578 / 1376; backward, B2 H64/8 T6400 D96 of six documents
     // 2472 / 1673, B1 H16 T9472 861 / 721).  Rows of one document, which the launch cannot tell from others, lose 1 to 2 %
     // (backward, B4 H32/8 T4096 1714 / 1743, B8 H16 T2048 581 / 589; of long documents with one query head a kv head and a bias
-    // up to 8, B4 H16 T2048 D64 310 / 336).  Not in float32, where it went either way, and further down than up (backward, B4 H16
+    // up to 9, B4 H16 T2048 D64 310 / 336).  Not in float32, where it went either way, and further down than up (backward, B4 H16
     // T1024 D64 of four documents 164 / 213, B2 H32 T2048 of one 986 / 1094, B1 H32 T2048 D64 of four 314 / 361; B2 H32/8 T2048
     // of three 1222 / 1160).
     // The choice to split looks at the mirrored form all the same: the sizes of the key blocks it

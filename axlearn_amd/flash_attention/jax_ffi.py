@@ -164,7 +164,7 @@ def _flash_bwd(softmax_scale, mask_kind, sliding_window, dropout_rate, res, d_ou
         # Too large for the automatic choice in one piece: the dS of as many kv heads at a time as fit
         # (AXL_BWD_DS_SLICE_KV_HEADS(n) = n << 8 in the flags; the kernels then run slice after slice),
         # if a slice still gives each of the 256 CUs a dK/dV workgroup; else the recomputing pair.
-        per_head = b * (s // 128) // (2 if mask_kind == 1 else 1)   # AXL_MASK_CAUSAL: two key blocks per workgroup
+        per_head = b * (s // 128) // (2 if mask_kind == 1 else 1)   # AXL_MASK_CAUSAL: up to two key blocks per workgroup
         heads = hkv - 1
         while heads >= 1 and _bwd_workspace_bytes(*size_args, flags | (heads << 8)) > BWD_WORKSPACE_LIMIT_BYTES:
             heads -= 1

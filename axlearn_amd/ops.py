@@ -439,7 +439,8 @@ def select_ds_slice(q: torch.Tensor, k: torch.Tensor, *, mask_kind: int,
     executed GEMMs instead of 7) when that path applies to these shapes and its workspace fits `limit`
     bytes - whole (slice 0), or of as many kv heads at a time as fit, provided a slice still gives every
     CU a dK/dV workgroup (batch * heads * kv_len / 256 of them under a causal mask, twice that under a
-    window); else the recomputing pair."""
+    window; counted as two key blocks to a workgroup where the launcher gives it one as well, with segment ids or
+    at head_dim 64); else the recomputing pair."""
     with_ds, without = flash_bwd_ds_workspace_bytes(q, k, mask_kind=mask_kind, segment_ids=segment_ids)
     if with_ds == without:
         return False, 0
@@ -452,7 +453,7 @@ def select_ds_slice(q: torch.Tensor, k: torch.Tensor, *, mask_kind: int,
     while heads >= 1 and flash_bwd_ds_workspace_bytes(q, k, mask_kind=mask_kind, segment_ids=segment_ids,
                                                       ds_slice_kv_heads=heads)[0] > int(limit):
         heads -= 1
-    per_head = b * (s // 128) // (2 if mask_kind == MASK_CAUSAL else 1)   # dK/dV workgroups per kv head
+    per_head = b * (s // 128) // (2 if mask_kind == MASK_CAUSAL else 1)   # dK/dV workgroups per kv head, at least
     cus = _device_properties(q.device)[1]
     if heads < 1 or heads * per_head < cus:
         return False, 0
