@@ -2000,7 +2000,7 @@ def test_pairs_worked_through_together_give_the_bits_of_each_sequence(b, t, hq, 
 @pytest.mark.parametrize("sink", [False, True])
 def test_forward_of_few_row_blocks(b, t, s, hq, hkv, d, dtype, mask, window, packed, offset, sink):
     """Launches that leave CUs idle: two groups of wavefronts share the keys of 64 rows.  out and lse against the oracle, twice
-    the same bits."""
+    the same bits, and not those of the form without key sharing, which a call with positions per sequence takes."""
     q, k, v, _ = _inputs(b, t, hq, hkv, d, dtype, s=s)
     segs = ref.packed_segment_ids(6, b, t, max_docs=5) if packed else None
     spec, kw = _mask_args(mask, window, segs)
@@ -2017,6 +2017,9 @@ def test_forward_of_few_row_blocks(b, t, s, hq, hkv, d, dtype, mask, window, pac
     assert ref.max_abs(lse.cpu(), want_lse) < 1e-3 * max(1.0, float(want_lse.abs().max()))
     again, lse2 = ops.flash_fwd(q, k, v, **kw)
     assert torch.equal(out, again) and torch.equal(lse, lse2)
+    if window != 0:   # (one key a row: nothing is rounded)
+        kw.update(q_pos_offset=0, q_pos_offsets=torch.full((b,), offset, device="cuda"))
+        assert not torch.equal(out, ops.flash_fwd(q, k, v, **kw)[0])
 
 
 @pytest.mark.parametrize("b,t,h,mask,window,dtype", [
